@@ -66,6 +66,7 @@ template <typename T>
 __device__ __forceinline__ FZ_GLB T* glb(T* p) { return (FZ_GLB T*)p; }
 
 // ---------------------------------------------------------------- small device helpers
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct BitW {  // LSB-first FSE bitstream writer (zfse/bitstream.h)
@@ -1493,25 +1494,7 @@ __global__ void __launch_bounds__(256) k_o1_dtables(const uint8_t* stream, const
 }
 
 
-// ---- order-1 tANS decoding split by bit position ----------------------------------------------
-// A chain's bitstream is cut into subsequences of sub_bits bits. Subsequence r owns the symbols
-// whose decoding starts at a read position B in (b_{r+1}, b_r], b_r = pos0 - r * sub_bits; the
-// last one owns everything below b_{R-1}.
-//
-// A decoder started at a wrong state on a wrong boundary falls into step with the true one after
-// some hundreds of symbols (both land on the same read position, state and context). What breaks
-// plain speculation is the escape symbol: the context after it depends on the sign of the escaped
-// code, which sits in the side stream at an index (the number of escapes before) that a
-// subsequence does not know. So each subsequence decodes from a *set* of possible start states and
-// follows both contexts after every escape; branches that reach the same read position, state and
-// context are merged. The result is a small graph: every escape met is a node with two out-edges
-// (escaped code >= 0 / < 0), every start state an origin edge, and every edge ends at the next node
-// on its branch or at an exit state, carrying the number of symbols decoded along it. The exit
-// states of a subsequence are the start set of the next; rounds repeat for subsequences whose
-// start set changed, and do not depend on escape indices. A walk per chain then follows the true
-// path through the graphs with the real escape signs (cost proportional to the escapes), giving
-// every subsequence its exact start, escape index and output offset; k_o1d_out decodes from those.
-// Subsequences whose graph outgrows its capacity are decoded exactly by the walk instead.
+// A chain that is decoded from its start (k_o1d_dense).
 struct O1DecChain {
     uint64_t off, len;      // stream bytes
     uint64_t lo, hi;        // output codes
@@ -1519,45 +1502,8 @@ struct O1DecChain {
     uint64_t dset;          // table set (segment)
     int64_t pos0;           // read position after the initial state
     uint32_t x0;            // initial state
-    uint32_t nsub;          // subsequences
-    uint64_t tfirst;        // first subsequence (global index)
-    int64_t sub_bits;
-    uint32_t hot0;          // the walk keeps the tables of contexts hot0 .. hot0 + 3 in LDS
     uint32_t pad;
 };
-
-struct O1DecState {  // where a subsequence starts, or where it left off
-    int64_t B;
-    uint32_t X;
-    uint32_t ctx;
-};
-
-__device__ inline int o1d_chain_of(const O1DecChain* ch, int nch, uint64_t t) {
-    int lo = 0, hi = nch;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (ch[mid].tfirst <= t) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
-// One decoder step; returns the code. r.pos is the read position; ovf_lim guards the side-stream index.
-__device__ inline int o1d_step(const DEntry* dt, BitWin& r, uint32_t& X, uint32_t& ctx, uint64_t& e,
-                               const int16_t* ovf, uint64_t ovf_lim, bool& bad) {
-    const DEntry d = dt[(size_t)ctx * (1u << kO1Log) + (X & ((1u << kO1Log) - 1))];
-    X = d.newState + bwin_read(r, d.nbBits & 15u);
-    int code;
-    if (d.symbol == 255) {
-        if (e < ovf_lim) code = ovf[e];
-        else { code = 32767; bad = true; }
-        e++;
-    } else {
-        const unsigned s = d.symbol;
-        code = (int)((s >> 1) ^ (~(s & 1) + 1));
-    }
-    ctx = (uint32_t)o1_ctx(code);
-    return code;
-}
 
 // Sequential decoding of a stretch of one chain from a bitstream window staged in LDS, for the
 // walk and for dense chains. win[k + kWinPad] holds chain byte wlo + k; the kWinPad bytes below are
@@ -1570,6 +1516,8 @@ constexpr int kDenseOut = 4096;     // dense chains: codes per round
 constexpr int kDenseOvf = 2048;     // dense chains: escaped values per round
 constexpr int kDnOvfLast = kDenseOvf - 1;
 
+
+constexpr int kSeqLanes = 64;       // the sequential decoders run as one wave
 
 struct SeqState {
     int64_t B;      // read position (bits below are unread)
@@ -1637,10 +1585,22 @@ __device__ __forceinline__ uint64_t seq_decode(SeqState& S, const FZ_LDS uint8_t
     return k;
 }
 
+__device__ __forceinline__ uint32_t uniform32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return (uint64_t)uniform32((uint32_t)v) | (uint64_t)uniform32((uint32_t)(v >> 32)) << 32;
+}
+
+// LDS accesses of one wave on either side stay in order (the hardware keeps a wave's LDS operations in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Copies chain bytes [w0, hi) into win, where w0 <= lo - kWinPad is the nearest chain byte below
 // whose device address is 16-byte aligned, so that whole aligned 16-byte blocks move (one load per
 // block; blocks that cross the chain's first or last byte go byte by byte, and bytes outside
-// [0, len) read as zero). Returns w0: win[i] holds chain byte w0 + i. win must hold
+// [0, len) read as zero), by one wave. Returns w0: win[i] holds chain byte w0 + i. win must hold
 // hi - lo + kWinPad + 32 bytes.
 __device__ __forceinline__ int64_t stage_window(FZ_LDS uint8_t* win, const uint8_t* cb, int64_t len, int64_t lo,
                                                 int64_t hi) {
@@ -1650,11 +1610,12 @@ __device__ __forceinline__ int64_t stage_window(FZ_LDS uint8_t* win, const uint8
     // kStageBatch blocks per lane are loaded before any is stored, so their loads are in flight
     // together (a window is a dozen or so blocks per lane)
     constexpr int kStageBatch = 8;
-    for (int64_t q0 = 0; q0 < nblk; q0 += (int64_t)blockDim.x * kStageBatch) {
+    const int lane = (int)(threadIdx.x & (kSeqLanes - 1));
+    for (int64_t q0 = 0; q0 < nblk; q0 += (int64_t)kSeqLanes * kStageBatch) {
         u32x4 v[kStageBatch];
 #pragma unroll
         for (int b = 0; b < kStageBatch; b++) {
-            const int64_t q = q0 + (int64_t)b * blockDim.x + threadIdx.x;
+            const int64_t q = q0 + (int64_t)b * kSeqLanes + lane;
             const int64_t c0 = w0 + 16 * q;
             if (q < nblk && c0 >= 0 && c0 + 16 <= len) {
                 v[b] = *reinterpret_cast<const u32x4*>(cb + c0);
@@ -1677,354 +1638,775 @@ __device__ __forceinline__ int64_t stage_window(FZ_LDS uint8_t* win, const uint8
         }
 #pragma unroll
         for (int b = 0; b < kStageBatch; b++) {
-            const int64_t q = q0 + (int64_t)b * blockDim.x + threadIdx.x;
+            const int64_t q = q0 + (int64_t)b * kSeqLanes + lane;
             if (q < nblk) *reinterpret_cast<FZ_LDS u32x4*>(win + 16 * q) = v[b];
         }
     }
     return w0;
 }
 
-constexpr int kSeqLanes = 64;  // the sequential decoders run as one wave
 
-// Graph capacity. Where escapes are dense the branches that follow wrong signs keep meeting
-// spurious escapes and the graph grows without bound; such subsequences give up early and are
-// decoded exactly by the walk.
-constexpr int kGBr = 16;     // live branches
-constexpr int kGNode = 24;   // escapes per subsequence graph
-constexpr int kGPend = 48;   // open edges
-constexpr uint64_t kGWork = 2;  // decode steps per graph, in average subsequences
-
-struct O1GEdge {
-    int32_t tgt;   // >= 0: node, < 0: exit -1-tgt
-    uint32_t sym;  // symbols decoded along the edge (the escape ending it included)
+// ---- order-1 tANS decoding split by bit position ----------------------------------------------
+// A chain's bitstream is cut into parts of sub_bits bits. Part r owns the symbols whose decoding
+// starts at a read position B in (b_{r+1}, b_r], b_r = pos0 - r * sub_bits; the last one owns
+// everything below b_{R-1}. The state in which the true decoder enters a part (its read position is
+// 0..12 bits below b_r, tANS state, context) is unknown; what is computed for every part at once is a
+// small set of states that holds it:
+//  * warm-up (k_o1s_warm): a few decoders per part start at guessed states some thousand symbols ahead
+//    of it. Two decoders that meet in position, state and context stay together, so their distinct
+//    states at the boundary are few, and the true one is mostly among them.
+//  * graphs (k_o1s_graph): every start state of a part is followed to the part's end. The context
+//    after an escape depends on the sign of the escaped code, which sits in the side stream at an
+//    index that a decoder started mid-chain does not know, so an escape is a node with two out-edges,
+//    and decoders that meet at one share it. The states in which the paths leave the part are
+//    possible entries of the next one: the following rounds add those that its set lacks. A part
+//    whose set holds the true entry so passes it on, and within two or three rounds nearly every set
+//    does. Where escapes are frequent the sets saturate after one round: the states that can be
+//    reached by any sequence of signs are few tens and contain the true one (512^3 field, REL 1e-3,
+//    segment 0, an escape in 48 symbols: 36 states a part at most, 132 nodes on average).
+//  * walk (k_o1s_walk, one workgroup per chain): the true path through the graphs with the real escape
+//    signs, giving every part its exact entry, escape index and output offset; a part whose set or
+//    graph lacks it is decoded exactly on the way.
+//  * output (k_o1s_out): every part decodes from its entry into its place.
+// States at a part's boundary are packed in 32 bits: bits below the boundary << 17 | context << 13 |
+// state; the low 17 bits index the segment's tables.
+struct O1Split {
+    const uint8_t* cb;    // the chain's bytes
+    const uint32_t* dt;   // its segment's tables (DEntry, kO1Ctx x 2^kO1Log)
+    const int16_t* ov;    // its escaped codes
+    int16_t* out;         // its codes
+    int* err;
+    uint64_t m, novf;     // codes, escaped codes
+    int64_t len, pos0;    // bytes, read position after the initial state
+    uint64_t tfirst;      // first part (index over all chains)
+    uint64_t cfirst;      // first slot of its candidate arrays (cap a part)
+    uint64_t wfirst;      // first warm-up lane (a multiple of 64)
+    uint64_t gfirst;      // first graph wave, over all chains
+    uint64_t lo;          // first code in the call's code array (alignment of the output)
+    uint32_t x0, nsub, sub_bits, warm_bits;
+    uint32_t lgk;         // 1 << lgk warm-up decoders a part
+    uint32_t cap;         // candidates a part holds at most
+    uint32_t parts;       // parts a graph wave takes
+    uint32_t max_sym;     // symbols an edge may hold
+    uint32_t warm_steps;  // pairs of steps a warm-up decoder takes at most
+    uint32_t hot0;        // the walk keeps the tables of contexts hot0 .. hot0 + 3 in LDS
+    uint32_t cls;         // graph size class
 };
 
-struct O1StartSet {
-    O1DecState s[kGBr];
-    int n;
-    int pad;
+constexpr int kSplitRounds = 3;
+// Edges: target (16 bits: node, numbered through all rounds of its graph wave, or kSplitExit | exit),
+// symbols decoded << 16.
+constexpr uint32_t kSplitExit = 0xF000u, kSplitFail = 0xFFFFFFFFu;
+constexpr uint32_t kSplitMaxSym = 0xFFFEu;
+constexpr uint32_t kSplitMaxCap = 128;  // candidates a part holds at most
+constexpr int kSplitMaxParts = 16;   // parts a graph wave takes at most
+constexpr int kSplitMaxOrig = 256;   // origins it takes at most (parts * cap)
+
+// Arrays shared by the kernels of one decode.
+struct O1SplitWs {
+    uint32_t* cand;              // start states of every part
+    uint32_t* edge;              // their edges
+    uint32_t* exits;             // states in which paths leave the part
+    uint16_t* hdr;               // [kSplitRounds][parts]: start states | exits << 8 after the round
+    uint8_t* n0;                 // [parts]: start states from the warm-up
+    uint2* wave;                 // [graph waves][kSplitRounds]: first node in pool (~0: no room there), nodes
+    uint2* pool;                 // nodes: edges for an escaped code >= 0 / < 0
+    unsigned int* pool_used;
+    uint64_t pool_cap;
+    uint64_t nparts;
+    uint32_t* res_state;         // [parts]: entry, escape index and output offset on the true path
+    uint64_t* res_e;
+    uint64_t* res_off;
 };
 
-struct O1Graph {
-    O1DecState exit[kGBr];
-    int nexit, nnode, status, norigin;  // status 0: complete, else capacity or step budget exceeded
-    O1DecState ostate[kGBr];            // the start states the graph was built from
-    O1GEdge origin[kGBr];
-    O1GEdge node[kGNode][2];
-};
-
-__device__ inline bool o1d_same(const O1DecState& a, const O1DecState& b) {
-    return a.B == b.B && a.X == b.X && a.ctx == b.ctx;
-}
-
-// Starts of round 1: the true start for subsequence 0; elsewhere the state a decoder reaches at the
-// subsequence boundary after warming up over the preceding `warm` bits from a guessed state (it has
-// almost always fallen into step by then; after an escape it follows the positive sign).
-// A decoder started in state X0 (context 0) at bit w and run down to the first symbol start at or
-// below b (after an escape it follows the positive sign). Symbols that read no bits do not move
-// the position (a context with one symbol), so the run is bounded; one that never gets there
-// returns position b.
-__device__ O1DecState o1d_warm(const uint8_t* cb, const DEntry* dt, int64_t w, int64_t b, uint32_t X0) {
-    BitWin rd = bwin_at(cb, w);
-    uint32_t X = X0 & ((1u << kO1Log) - 1), cx = 0;
-    uint64_t guard = (uint64_t)(w - b) * 4 + 4096;
-    while (rd.pos > b && guard--) {
-        const DEntry d = dt[(size_t)cx * (1u << kO1Log) + (X & ((1u << kO1Log) - 1))];
-        X = d.newState + bwin_read(rd, d.nbBits & 15u);
-        const unsigned nc = d.nbBits >> 4;
-        cx = nc == 15 ? 13u : nc;
+__device__ inline int o1s_chain(const O1Split* ch, int nch, uint64_t x, uint64_t O1Split::*first) {
+    int lo = 0, hi = nch;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (ch[mid].*first <= x) lo = mid; else hi = mid;
     }
-    return O1DecState{rd.pos > b ? b : rd.pos, X & ((1u << kO1Log) - 1), cx};
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
-__global__ void __launch_bounds__(256) k_o1d_init(const uint8_t* in, const O1DecChain* ch, int nch, uint64_t nsub,
-                                                  const DEntry* dt_all, int64_t warm_subs, O1StartSet* start,
-                                                  uint8_t* run) {
-    const uint64_t t = (uint64_t)xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= nsub) return;
-    const O1DecChain c = ch[o1d_chain_of(ch, nch, t)];
-    const uint64_t r = t - c.tfirst;
-    O1StartSet ss;
-    ss.n = 1;
-    ss.pad = 0;
-    if (r == 0) {
-        ss.s[0] = O1DecState{c.pos0, c.x0, 0};
-    } else {
+// Backward bit reader over aligned 32-bit words of a chain: bits [32 j, 32 j + have) are in w (its
+// low end first), the word below is in flight. Bits below the chain's first read as zero, as do the
+// words below it, which are not touched.
+struct ChainWords {
+    const uint32_t* d4;   // the aligned word that holds the chain's first byte
+    uint32_t m0;          // its bits that belong to the chain
+    int32_t shift;        // bit 0 of the chain in it
+    __device__ explicit ChainWords(const uint8_t* cb) {
+        const uint32_t o = (uint32_t)(uintptr_t)cb & 3u;
+        d4 = reinterpret_cast<const uint32_t*>(cb - o);
+        m0 = ~0u << (8 * o);
+        shift = (int32_t)(8 * o);
+    }
+    __device__ __forceinline__ uint32_t word(int64_t j) const {
+        const uint32_t v = glb(d4)[j < 0 ? 0 : j];
+        return j > 0 ? v : (j == 0 ? v & m0 : 0u);
+    }
+};
+struct WordBits {
+    uint64_t w;
+    int32_t have;
+    int64_t j;
+    uint32_t nxt;
+    // reads from chain bit position B downward (B > 0)
+    __device__ __forceinline__ void init(const ChainWords& c, int64_t B) {
+        const int64_t a = B + c.shift;
+        j = ((a + 31) >> 5) - 2;
+        w = ((uint64_t)c.word(j + 1) << 32) | c.word(j);
+        have = (int32_t)(a - 32 * j);
+        nxt = c.word(j - 1);
+    }
+    // at least 32 bits; enough for two steps of at most 13
+    __device__ __forceinline__ void refill(const ChainWords& c) {
+        if (have < 32) {
+            w = (w << 32) | nxt;
+            have += 32;
+            j--;
+            nxt = c.word(j - 1);
+        }
+    }
+    __device__ __forceinline__ uint32_t take(uint32_t nb) {
+        have -= (int32_t)nb;
+        return (uint32_t)(w >> ((uint32_t)have & 63u)) & ((1u << nb) - 1u);
+    }
+};
+
+// Guessed start states: any spread will do, the same ones in every run.
+__device__ __forceinline__ uint32_t o1s_mix(uint32_t x) {
+    x ^= x >> 16;
+    x *= 0x7feb352du;
+    x ^= x >> 15;
+    x *= 0x846ca68bu;
+    return x ^ (x >> 16);
+}
+
+// One lane per guessed decoder; the 2^lgk lanes of a part sit in one wave and drop duplicates at the
+// boundary. After an escape each lane picks a sign at random, so that lanes which have met can part
+// again and cover the states reachable by other signs.
+__global__ void __launch_bounds__(256) k_o1s_warm(const O1Split* ch, int nch, uint64_t nlanes, O1SplitWs ws) {
+    const uint64_t g = (uint64_t)xcd_block() * blockDim.x + threadIdx.x;
+    if (g >= nlanes) return;  // whole waves: nlanes is a multiple of 64
+    const O1Split& c = ch[o1s_chain(ch, nch, g & ~63ull, &O1Split::wfirst)];
+    const uint32_t K = 1u << c.lgk;
+    const uint64_t local = g - c.wfirst;
+    const uint64_t r = local >> c.lgk;
+    const uint32_t k = (uint32_t)local & (K - 1);
+    const bool valid = r > 0 && r < c.nsub;
+    uint32_t state = ~0u;
+    if (valid) {
+        const ChainWords cw(c.cb);
+        const uint32_t* dt = c.dt;
         const int64_t b = c.pos0 - (int64_t)r * c.sub_bits;
-        const int64_t w = min<int64_t>(c.pos0, b + warm_subs * c.sub_bits);
-        const DEntry* dt = dt_all + c.dset * kO1Ctx * (1u << kO1Log);
-        // a warm-up that never got there starts at the boundary (the walk then decodes it exactly)
-        ss.s[0] = o1d_warm(in + c.off, dt, w, b, (uint32_t)(r * 2654435761u));
+        uint32_t seed = o1s_mix((uint32_t)local * 2654435761u + 12345u);
+        int64_t B = b + c.warm_bits;
+        uint32_t idx;
+        if (B >= c.pos0) {  // near the chain's start: from its true state
+            B = c.pos0;
+            idx = c.x0 & ((1u << kO1Log) - 1);
+        } else {
+            B -= seed % 13u;
+            idx = (((seed >> 8) % (uint32_t)kO1Ctx) << kO1Log) | ((seed >> 16) & ((1u << kO1Log) - 1));
+        }
+        int32_t rem = (int32_t)(B - b);
+        WordBits rd;
+        rd.init(cw, B);
+        // a context whose one symbol reads no bits would never get there
+        uint32_t guard = c.warm_steps;
+        auto step = [&]() {
+            if (rem <= 0) return;
+            const uint32_t raw = glb(dt)[idx];
+            const uint32_t nb = (raw >> 24) & 15u;
+            rem -= (int32_t)nb;
+            const uint32_t x = (raw & ((1u << kO1Log) - 1)) + rd.take(nb);
+            uint32_t cx = raw >> 28;
+            if (cx == 15u) {
+                seed = seed * 1664525u + 1013904223u;
+                cx = 13u + (seed >> 31);
+            }
+            idx = (cx << kO1Log) | (x & ((1u << kO1Log) - 1));
+        };
+        while (rem > 0 && guard--) {
+            rd.refill(cw);
+            step();
+            step();
+        }
+        if (rem <= 0) state = ((uint32_t)-rem << 17) | idx;
     }
-    start[t] = ss;
-    run[t] = 1;
+    bool keep = state != ~0u;
+    const int lane = threadIdx.x & 63, base = lane & ~(int)(K - 1);
+    for (uint32_t i = 0; i < K; i++) {
+        const uint32_t o = __shfl(state, base + (int)i);
+        keep = keep && !(i < k && o == state);
+    }
+    const uint64_t grp = (K == 64 ? ~0ull : ((1ull << K) - 1) << base) & __ballot(keep);
+    const uint32_t n = min((uint32_t)__popcll(grp), c.cap);
+    const uint32_t at = (uint32_t)__popcll(grp & ((1ull << lane) - 1));
+    const uint64_t slot = c.cfirst + r * c.cap;
+    if (r == 0 && k == 0) {
+        ws.cand[slot] = c.x0 & ((1u << kO1Log) - 1);  // the chain starts in context 0
+        ws.n0[c.tfirst] = 1;
+    }
+    if (valid) {
+        if (keep && at < c.cap) ws.cand[slot + at] = state;
+        if (k == 0) ws.n0[c.tfirst + r] = (uint8_t)n;
+    }
 }
 
-// Graph of one subsequence from its start set (all but the last subsequence of each chain). One lane
-// per subsequence; while a single branch is live (most of the time) its state stays in registers,
-// otherwise branches and open edges live in LDS, one column per lane.
-constexpr int kGLanes = 64;
-
-__global__ void __launch_bounds__(kGLanes) k_o1d_graph(const uint8_t* in, const O1DecChain* ch, int nch, uint64_t nsub,
-                                                       const DEntry* dt_all, const uint8_t* run,
-                                                       const O1StartSet* start, O1Graph* graph) {
-    __shared__ int64_t bB[kGBr][kGLanes];
-    __shared__ uint32_t bX[kGBr][kGLanes];
-    __shared__ uint32_t bN[kGBr][kGLanes];  // symbols decoded on the branch
-    __shared__ uint8_t bC[kGBr][kGLanes];   // context
-    __shared__ int32_t pS[kGPend][kGLanes]; // open edge: >= 0 origin slot, < 0 node edge -1-(2 node + sign)
-    __shared__ uint8_t pB[kGPend][kGLanes]; // its branch
-    __shared__ uint32_t pC[kGPend][kGLanes];// branch count where it started
-    const int l = threadIdx.x;
-    const uint64_t t = (uint64_t)xcd_block() * blockDim.x + l;
-    if (t >= nsub || !run[t]) return;
-    const O1DecChain c = ch[o1d_chain_of(ch, nch, t)];
-    const uint64_t r = t - c.tfirst;
-    if (r + 1 >= c.nsub) return;
-    const DEntry* dt = dt_all + c.dset * kO1Ctx * (1u << kO1Log);
-    const uint8_t* buf = in + c.off;
-    const int64_t stop = c.pos0 - (int64_t)(r + 1) * c.sub_bits;
-    const uint32_t cap = (uint32_t)min<uint64_t>(c.hi - c.lo, 0xFFFFFFFFull);
-    // A step budget: kGWork times the symbols a subsequence holds on average, plus a margin. Graphs
-    // that keep several branches live across the whole subsequence cost up to kGBr times one exact
-    // decode; past the budget the walk decodes the subsequence exactly instead (status 5).
-    const uint64_t expect = c.pos0 > 0 ? (uint64_t)c.sub_bits * (c.hi - c.lo) / (uint64_t)c.pos0 : 0;
-    const uint64_t budget = kGWork * expect + 512;
-    uint64_t work = 0;
-    O1Graph& G = graph[t];
-    int nb = 0, np = 0, nexit = 0, nnode = 0, status = 0;
-    {
-        const O1StartSet& ss = start[t];
-        const int n0 = min(ss.n, kGBr);
-        for (int o = 0; o < n0; o++) {
-            const O1DecState s0 = ss.s[o];
-            G.ostate[o] = s0;
-            bB[nb][l] = s0.B; bX[nb][l] = s0.X; bC[nb][l] = (uint8_t)s0.ctx; bN[nb][l] = 0;
-            pS[np][l] = o; pB[np][l] = (uint8_t)nb; pC[np][l] = 0;
-            np++;
-            nb++;
+// The graphs of the parts of one wave, from this round's new start states. A lane takes one edge at a
+// time (a start state, or a node and a sign), decodes to the next escape or the part's end, and looks
+// the state it met up in a hash table in LDS: a new escape state is a new node and two more edges. The
+// edges still to take are the tail of the node list, so there is no queue. Parts share a wave where
+// their edges are few (chains without escapes have a handful of start states). Steps run eight at a
+// time between looks at the table; a lane that has met its end waits for the rest.
+// NC: nodes a wave holds at most; past it, and where a table or the pool is full, the edges left stay
+// marked and the walk decodes such parts exactly.
+template <int NC>
+__global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, uint32_t nwaves, int round, O1SplitWs ws) {
+    constexpr uint32_t kSlots = NC <= 128 ? 512 : 2 * NC;
+    __shared__ unsigned long long key[kSlots];  // 1 << 63 | part << 43 | (bits above the end + 64) << 17 | ctx << 13 | state
+    __shared__ uint16_t val[kSlots];            // node, or kSplitExit | exit
+    __shared__ uint16_t list[NC];               // node -> slot
+    __shared__ uint2 nodes[NC];
+    __shared__ uint32_t ost[kSplitMaxOrig];
+    __shared__ uint16_t oat[kSplitMaxOrig];     // part << 8 | slot
+    __shared__ uint32_t nex[kSplitMaxParts], ncand[kSplitMaxParts];
+    const uint32_t l = threadIdx.x;
+    const uint64_t below = (1ull << l) - 1;
+    if (xcd_block() >= nwaves) return;
+    const uint64_t gw = ch[0].gfirst + xcd_block();
+    const O1Split& c = ch[o1s_chain(ch, nch, gw, &O1Split::gfirst)];
+    const uint32_t wl = (uint32_t)(gw - c.gfirst);
+    const uint32_t p0 = wl * c.parts;
+    const uint32_t np = min(c.parts, c.nsub - 1 - p0);  // the last part has no graph
+    const uint32_t cap = c.cap;
+    const uint64_t t0 = c.tfirst + p0, c0 = c.cfirst + (uint64_t)p0 * cap;
+    uint16_t* hdr = ws.hdr + (uint64_t)round * ws.nparts;
+    for (uint32_t i = l; i < kSlots; i += 64) key[i] = 0;
+    // this round's start states
+    uint32_t no = 0;
+    for (uint32_t p = 0; p < np; p++) {
+        const uint64_t t = t0 + p, cs = c0 + (uint64_t)p * cap;
+        uint32_t n = 0, ne = 0;
+        if (round == 0) {
+            n = ws.n0[t];
+            for (uint32_t i = l; i < n; i += 64) {
+                ost[no + i] = ws.cand[cs + i];
+                oat[no + i] = (uint16_t)(p << 8 | i);
+            }
+            no += n;
+        } else {
+            const uint32_t h = (hdr - ws.nparts)[t];
+            n = h & 255u;
+            ne = h >> 8;
+            if (p0 + p > 0) {
+                // exits of the part before that its latest round added, less those already in the set
+                const uint32_t e1 = (hdr - ws.nparts)[t - 1] >> 8;
+                const uint32_t e0 = round > 1 ? (hdr - 2 * ws.nparts)[t - 1] >> 8 : 0u;
+                const uint32_t nold = n;
+                for (uint32_t i0 = e0; i0 < e1; i0 += 64) {
+                    const uint32_t i = i0 + l;
+                    bool keep = i < e1;
+                    const uint32_t x = keep ? ws.exits[cs - cap + i] : 0u;
+                    for (uint32_t q = 0; q < nold; q++) keep = keep && ws.cand[cs + q] != x;
+                    const uint64_t mk = __ballot(keep);
+                    const uint32_t at = n + (uint32_t)__popcll(mk & below);
+                    if (keep && at < cap) {
+                        ws.cand[cs + at] = x;
+                        ost[no + (at - n)] = x;
+                        oat[no + (at - n)] = (uint16_t)(p << 8 | at);
+                    }
+                    const uint32_t add = min((uint32_t)__popcll(mk), cap - n);
+                    n += add;
+                    no += add;
+                }
+            }
+        }
+        if (l == 0) {
+            ncand[p] = n;
+            nex[p] = ne;
         }
     }
-    auto close_edges = [&](int b, int32_t tgt) {
-        for (int k = 0; k < np;) {
-            if (pB[k][l] == b) {
-                const O1GEdge e{tgt, bN[b][l] - pC[k][l]};
-                const int32_t sl = pS[k][l];
-                if (sl >= 0) G.origin[sl] = e;
-                else { const int q = -1 - sl; G.node[q >> 1][q & 1] = e; }
-                np--;
-                pS[k][l] = pS[np][l]; pB[k][l] = pB[np][l]; pC[k][l] = pC[np][l];
+    __syncthreads();
+    uint32_t id0 = 0;  // nodes of earlier rounds
+    for (int z = 0; z < round; z++) id0 += ws.wave[gw * kSplitRounds + z].y;
+    if (no == 0) {
+        for (uint32_t p = l; p < np; p += 64) hdr[t0 + p] = (uint16_t)(ncand[p] | nex[p] << 8);
+        if (l == 0) ws.wave[gw * kSplitRounds + round] = make_uint2(0, 0);
+        return;
+    }
+    for (uint32_t i = l; i < no; i += 64) ws.edge[c0 + (uint64_t)(oat[i] >> 8) * cap + (oat[i] & 255u)] = kSplitFail;
+    // returns the slot of k, and whether it was put there now; kSlots: the table is full
+    auto insert = [&](unsigned long long k, bool& fresh) -> uint32_t {
+        uint32_t s = ((uint32_t)(k >> 32) * 0x9E3779B1u ^ (uint32_t)k * 0x85EBCA6Bu) >> 8;
+        fresh = false;
+        for (int q = 0; q < 128; q++, s++) {
+            s &= kSlots - 1;
+            const unsigned long long old = atomicCAS(&key[s], 0ull, k);
+            if (old == 0) { fresh = true; return s; }
+            if (old == k) return s;
+        }
+        return kSlots;
+    };
+    // exits of earlier rounds
+    if (round > 0)
+        for (uint32_t p = 0; p < np; p++)
+            for (uint32_t i = l; i < nex[p]; i += 64) {
+                const uint32_t x = ws.exits[c0 + (uint64_t)p * cap + i];
+                bool fresh;
+                const uint32_t s = insert(1ull << 63 | (unsigned long long)p << 43 |
+                                              (unsigned long long)(64u - (x >> 17)) << 17 | (x & 0x1FFFFu), fresh);
+                if (s < kSlots) val[s] = (uint16_t)(kSplitExit | i);
+            }
+    __syncthreads();
+    const ChainWords cw(c.cb);
+    const uint32_t* dt = c.dt;
+    const int64_t stop0 = c.pos0 - (int64_t)(p0 + 1) * c.sub_bits;  // end of the wave's first part
+    uint32_t head = 0, tail = no, nn = 0;  // edges taken, edges known, nodes
+    bool active = false;
+    uint32_t task = 0, p = 0, idx = 0, nsym = 0;
+    int32_t rem = 0;
+    WordBits rd{0, 0, 0, 0};
+    for (;;) {
+        const uint64_t idle = __ballot(!active);
+        const uint32_t mine = head + (uint32_t)__popcll(idle & below);
+        bool run = active;
+        if (!active && mine < tail) {
+            task = mine;
+            if (task < no) {
+                const uint32_t x = ost[task];
+                p = oat[task] >> 8;
+                rem = (int32_t)c.sub_bits - (int32_t)(x >> 17);
+                idx = x & 0x1FFFFu;
             } else {
-                k++;
+                const uint32_t q = task - no;
+                const unsigned long long k = key[list[q >> 1]];
+                p = (uint32_t)(k >> 43) & 15u;
+                rem = (int32_t)((uint32_t)(k >> 17) & 0x3FFFFFFu) - 64;
+                idx = ((13u + (q & 1u)) << kO1Log) | ((uint32_t)k & ((1u << kO1Log) - 1));
+            }
+            nsym = 0;
+            active = true;
+            run = rem > 0;
+            if (run) rd.init(cw, stop0 - (int64_t)p * c.sub_bits + rem);
+        }
+        head = min(tail, head + (uint32_t)__popcll(idle));
+        if (__ballot(active) == 0) break;
+        bool esc = false, dead = false;
+        auto step = [&]() {
+            if (!run) return;
+            const uint32_t raw = glb(dt)[idx];
+            const uint32_t nb = (raw >> 24) & 15u;
+            rem -= (int32_t)nb;
+            const uint32_t x = (raw + rd.take(nb)) & ((1u << kO1Log) - 1);
+            idx = (raw >> 28 << kO1Log) | x;
+            nsym++;
+            esc = raw >> 28 == 15u;
+            run = rem > 0 && !esc;
+        };
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (run) rd.refill(cw);
+            step();
+            step();
+        }
+        if (run && nsym > c.max_sym) {
+            run = false;
+            dead = true;  // a stretch of many symbols in few bits: the walk takes it
+        }
+        // lanes that met an escape or the end
+        const bool ev = active && !run;
+        if (__ballot(ev) == 0) continue;
+        bool fresh = false;
+        uint32_t slot = kSlots;
+        if (ev && !dead)
+            slot = insert(1ull << 63 | (unsigned long long)p << 43 | (unsigned long long)(uint32_t)(rem + 64) << 17 |
+                              (idx | (esc ? 0xFu << kO1Log : 0u)), fresh);
+        const uint64_t nmask = __ballot(fresh && esc);
+        const uint32_t id = nn + (uint32_t)__popcll(nmask & below);
+        const bool full = nn + (uint32_t)__popcll(nmask) > (uint32_t)NC;
+        if (fresh) {
+            if (esc) {
+                if (id < (uint32_t)NC) {
+                    val[slot] = (uint16_t)(id0 + id);
+                    list[id] = (uint16_t)slot;
+                    nodes[id] = make_uint2(kSplitFail, kSplitFail);
+                }
+            } else {
+                const uint32_t e = atomicAdd(&nex[p], 1u);
+                if (e < cap) {
+                    ws.exits[c0 + (uint64_t)p * cap + e] = ((uint32_t)-rem << 17) | idx;
+                    val[slot] = (uint16_t)(kSplitExit | e);
+                } else {
+                    val[slot] = 0xFFFFu;
+                }
             }
         }
-    };
-    auto drop_branch = [&](int b) {
-        nb--;
-        if (b != nb) {
-            bB[b][l] = bB[nb][l]; bX[b][l] = bX[nb][l]; bC[b][l] = bC[nb][l]; bN[b][l] = bN[nb][l];
-            for (int k = 0; k < np; k++)
-                if (pB[k][l] == nb) pB[k][l] = (uint8_t)b;
+        __syncthreads();
+        if (full) break;
+        if (ev) {
+            const uint32_t v = slot < kSlots ? val[slot] : 0xFFFFu;
+            const uint32_t e = v == 0xFFFFu || nsym > kSplitMaxSym ? kSplitFail : v | nsym << 16;
+            if (task < no) ws.edge[c0 + (uint64_t)(oat[task] >> 8) * cap + (oat[task] & 255u)] = e;
+            else if ((task - no) & 1u) nodes[(task - no) >> 1].y = e;
+            else nodes[(task - no) >> 1].x = e;
+            active = false;
         }
-    };
-    auto exit_branch = [&](int b) {
-        const O1DecState sb{bB[b][l], bX[b][l], bC[b][l]};
-        int x = 0;
-        while (x < nexit && !o1d_same(G.exit[x], sb)) x++;
-        if (x == nexit) {
-            if (nexit == kGBr) { status = 1; return; }
-            G.exit[nexit++] = sb;
-        }
-        close_edges(b, -1 - x);
-        drop_branch(b);
-    };
-    // an escape decoded on branch b: new node, both contexts continue
-    auto fork_branch = [&](int b) {
-        if (nnode == kGNode) { status = 2; return; }
-        if (nb == kGBr) { status = 3; return; }
-        if (np + 2 > kGPend) { status = 4; return; }
-        const int n = nnode++;
-        close_edges(b, n);
-        bB[nb][l] = bB[b][l]; bX[nb][l] = bX[b][l]; bN[nb][l] = bN[b][l];
-        bC[b][l] = 13;   // escaped code >= 128
-        bC[nb][l] = 14;  // escaped code <= -128
-        pS[np][l] = -1 - 2 * n; pB[np][l] = (uint8_t)b; pC[np][l] = bN[b][l]; np++;
-        pS[np][l] = -1 - (2 * n + 1); pB[np][l] = (uint8_t)nb; pC[np][l] = bN[b][l]; np++;
-        nb++;
-    };
-    while (nb > 0 && status == 0) {
-        if (work > budget) {
-            status = 5;
-            break;
-        }
-        if (nb == 1) {  // single branch: registers only
-            BitWin rd = bwin_at(buf, bB[0][l]);
-            uint32_t X = bX[0][l], cx = bC[0][l], cnt = bN[0][l];
-            const uint32_t cnt0 = cnt;
-            bool esc = false;
-            while (rd.pos > stop && cnt < cap) {
-                const DEntry d = dt[(size_t)cx * (1u << kO1Log) + (X & ((1u << kO1Log) - 1))];
-                X = d.newState + bwin_read(rd, d.nbBits & 15u);
-                cnt++;
-                if (d.symbol == 255) { esc = true; break; }
-                const unsigned sy = d.symbol;
-                cx = (uint32_t)o1_ctx((int)((sy >> 1) ^ (~(sy & 1) + 1)));
-            }
-            bB[0][l] = rd.pos; bX[0][l] = X; bC[0][l] = (uint8_t)cx; bN[0][l] = cnt;
-            work += cnt - cnt0;
-            if (esc) fork_branch(0);
-            else exit_branch(0);
-            continue;
-        }
-        int i = 0;
-        for (int j = 1; j < nb; j++)
-            if (bB[j][l] > bB[i][l]) i = j;
-        if (bB[i][l] <= stop || bN[i][l] >= cap) {
-            exit_branch(i);
-            continue;
-        }
-        const uint32_t cx0 = bC[i][l], X0 = bX[i][l];
-        const DEntry d = dt[(size_t)cx0 * (1u << kO1Log) + (X0 & ((1u << kO1Log) - 1))];
-        work++;
-        BitWin rd = bwin_at(buf, bB[i][l]);
-        const uint32_t X = d.newState + bwin_read(rd, d.nbBits & 15u);
-        const int64_t B = rd.pos;
-        bB[i][l] = B; bX[i][l] = X; bN[i][l] = bN[i][l] + 1;
-        if (d.symbol == 255) {
-            fork_branch(i);
-            continue;
-        }
-        const unsigned sy = d.symbol;
-        const uint32_t cx = (uint32_t)o1_ctx((int)((sy >> 1) ^ (~(sy & 1) + 1)));
-        bC[i][l] = (uint8_t)cx;
-        for (int j = 0; j < nb; j++) {
-            if (j == i || bB[j][l] != B || bX[j][l] != X || bC[j][l] != cx) continue;
-            const uint32_t di = bN[i][l], dj = bN[j][l];
-            for (int k = 0; k < np; k++)
-                if (pB[k][l] == i) { pC[k][l] += dj - di; pB[k][l] = (uint8_t)j; }
-            drop_branch(i);
-            break;
+        nn += (uint32_t)__popcll(nmask);
+        tail = no + 2 * nn;
+        __syncthreads();
+    }
+    __syncthreads();
+    nn = min(nn, (uint32_t)NC);
+    uint32_t at = 0;
+    if (nn) {
+        if (l == 0) at = atomicAdd(ws.pool_used, nn);
+        at = __builtin_amdgcn_readfirstlane(at);
+        if ((uint64_t)at + nn <= ws.pool_cap) {
+            for (uint32_t i = l; i < nn; i += 64) ws.pool[at + i] = nodes[i];
+        } else {
+            at = ~0u;  // the walk finds no node and decodes such parts exactly
         }
     }
-    G.nexit = nexit;
-    G.nnode = nnode;
-    G.status = status;
-    G.norigin = min(start[t].n, kGBr);
+    if (l == 0) ws.wave[gw * kSplitRounds + round] = make_uint2(at, nn);
+    for (uint32_t i = l; i < np; i += 64) hdr[t0 + i] = (uint16_t)(ncand[i] | min(nex[i], cap) << 8);
 }
 
-// Next round's start sets from this round's exits; counts the subsequences to run again.
-__global__ void __launch_bounds__(256) k_o1d_glink(const O1DecChain* ch, int nch, uint64_t nsub, const O1Graph* graph,
-                                                   O1StartSet* start, uint8_t* run, unsigned int* nrun) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nsub) return;
-    const O1DecChain c = ch[o1d_chain_of(ch, nch, t)];
-    const uint64_t r = t - c.tfirst;
-    uint8_t go = 0;
-    if (r > 0) {
-        const O1Graph& g = graph[t - 1];
-        O1StartSet& ss = start[t];
-        if (g.status == 0) {
-            bool same = ss.n == g.nexit;
-            for (int k = 0; same && k < g.nexit; k++) same = o1d_same(ss.s[k], g.exit[k]);
-            if (!same) {
-                ss.n = g.nexit;
-                for (int k = 0; k < g.nexit; k++) ss.s[k] = g.exit[k];
-                go = 1;
-            }
-        }
-        if (go && r + 1 < c.nsub) atomicAdd(nrun, 1u);
-    }
-    run[t] = go;
-}
+// One workgroup per chain; wave 0 walks, the others stage what it needs next in LDS: the sets and nodes
+// of whole graph waves ("units" of c.parts parts), a buffer of units while the walk is in the other.
+// The walk is one LDS round trip per escape and three per part. A part that the graph does not hold is
+// decoded exactly; the tables of four contexts then take the place of both buffers. (Staging one part at
+// a time, behind two dependent device loads, cost 1.5 us a part and 0.35 us an escape: 512^3 field at
+// REL 1e-3 23.2 ms a call, counts of 101 x 128 x 150 11.3 ms.)
+constexpr int kWalkThreads = 512;
+constexpr uint32_t kWalkBuf = 65536;   // bytes of one buffer
+constexpr int64_t kWalkStage = 4096;   // bitstream bytes staged per window of an exact decode
+// Nodes of a unit that are staged, by size class; the rest are read from memory.
+__device__ __forceinline__ uint32_t walk_nodes(uint32_t cls) { return cls == 0 ? 64u : cls == 1 ? 512u : 1024u; }
 
-// One workgroup per chain: the true path through the graphs. Gives every subsequence its start
-// state, escape index and output offset (relative to the chain). A subsequence without a usable
-// graph (capacity exceeded, or a start state missing from its set) is decoded exactly here, by one
-// lane, with the tables of four consecutive contexts staged in LDS: the window the chain's segment
-// uses most (by the stationary distribution of its context chain; 11..14, the contexts after large
-// codes, where escapes are dense).
-constexpr int64_t kWalkStage = 16384;          // bitstream bytes staged per window
-
-__global__ void __launch_bounds__(kSeqLanes) k_o1d_walk(const uint8_t* in, const O1DecChain* ch, int nch,
-                                                        const DEntry* dt_all, const int16_t* ovf,
-                                                        const O1Graph* graph, O1DecState* res_start, uint64_t* res_e,
-                                                        uint64_t* res_off, unsigned int* stats, int* err) {
-    __shared__ uint32_t hot[kWalkCtxN << kO1Log];
+__global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, int nch, O1SplitWs ws, unsigned int* stats) {
+    __shared__ __align__(16) uint32_t mem[2 * kWalkBuf / 4];  // two buffers, or the hot tables
     __shared__ __align__(16) uint32_t stage32[(kWalkStage + kWinPad + 32) / 4 + 4];
-    uint8_t* stage = reinterpret_cast<uint8_t*>(stage32);
+    __shared__ uint32_t sh_miss, sh_stop;
+    static_assert(2 * kWalkBuf / 4 >= (uint32_t)kWalkCtxN << kO1Log, "the tables fit in the buffers");
     const int q = blockIdx.x;
     if (q >= nch) return;
-    const O1DecChain c = ch[q];
-    const uint32_t* dt = reinterpret_cast<const uint32_t*>(dt_all + c.dset * kO1Ctx * (1u << kO1Log));
-    for (uint32_t i = threadIdx.x; i < (kWalkCtxN << kO1Log); i += blockDim.x)
-        hot[i] = dt[((size_t)c.hot0 << kO1Log) + i];
-    __syncthreads();
-    const uint8_t* cb = in + c.off;
-    const int16_t* ov = ovf + c.ovf_base;
-    const bool lead = threadIdx.x == 0;
-    // every lane walks the same path (the values stay wave-uniform); lane 0 does the stores
-    SeqState z{c.pos0, c.x0, 0, 0, false};
-    uint64_t off = 0;
-    const uint64_t m = c.hi - c.lo;
-    for (uint64_t r = 0; r < c.nsub; r++) {
-        const uint64_t t = c.tfirst + r;
-        if (lead) {
-            res_start[t] = O1DecState{z.B, z.X, z.cx};
-            res_e[t] = z.e;
-            res_off[t] = off;
+    const O1Split c = ch[q];
+    const uint32_t tid = threadIdx.x, l = tid & 63u, wv = tid >> 6;
+    const bool lead = tid == 0;
+    const uint32_t P = c.parts, pc = P * c.cap;  // candidates of a unit
+    const uint32_t NS = walk_nodes(c.cls);
+    // a unit's words: nodes (first, for their alignment), cand, edge, exits, start states of each part,
+    // nodes staged
+    const uint32_t o_cand = 2 * NS, o_edge = o_cand + pc, o_exit = o_edge + pc, o_n = o_exit + pc,
+                   o_ns = o_n + kSplitMaxParts, unit_words = o_ns + 4;
+    const uint32_t U = (kWalkBuf / 4) / unit_words;  // units a buffer
+    const uint32_t ngraph = c.nsub - 1, nunit = (ngraph + P - 1) / P;
+    const uint16_t* hdr = ws.hdr + (uint64_t)(kSplitRounds - 1) * ws.nparts + c.tfirst;
+    FZ_LDS uint32_t* const lmem = lds(mem);
+    const FZ_GLB u32x2* pool = glb(reinterpret_cast<const u32x2*>(ws.pool));
+    auto stage_units = [&](uint32_t u0, FZ_LDS uint32_t* buf, uint32_t w0, uint32_t nw) {  // by waves w0 .. w0 + nw - 1
+        const uint32_t u1 = min(nunit, u0 + U);
+        for (uint32_t u = u0 + (wv - w0); u < u1; u += nw) {
+            FZ_LDS uint32_t* b = buf + (u - u0) * unit_words;
+            const uint2* rw = ws.wave + (c.gfirst + u) * kSplitRounds;
+            uint2 rd[kSplitRounds];
+#pragma unroll
+            for (int z = 0; z < kSplitRounds; z++) rd[z] = rw[z];
+            // the last unit's sets end with the chain's
+            const uint64_t cs = c.cfirst + (uint64_t)u * pc;
+            const uint32_t nc = min(pc, (c.nsub - u * P) * c.cap);
+            for (uint32_t i = l; i < nc; i += 128) {
+                const uint32_t k = min(i + 64, nc - 1);
+                const uint32_t v0 = glb(ws.cand)[cs + i], v1 = glb(ws.edge)[cs + i], v2 = glb(ws.exits)[cs + i];
+                const uint32_t v3 = glb(ws.cand)[cs + k], v4 = glb(ws.edge)[cs + k], v5 = glb(ws.exits)[cs + k];
+                b[o_cand + i] = v0;
+                b[o_edge + i] = v1;
+                b[o_exit + i] = v2;
+                b[o_cand + k] = v3;
+                b[o_edge + k] = v4;
+                b[o_exit + k] = v5;
+            }
+            if (l < P && u * P + l < ngraph) b[o_n + l] = glb(hdr)[u * P + l] & 255u;
+            // the nodes of all rounds, one after another, eight loads a lane in flight
+            uint32_t ns = 0;
+            bool room = true;
+#pragma unroll
+            for (int z = 0; z < kSplitRounds; z++) {
+                const uint32_t n = room && rd[z].x != ~0u ? min(rd[z].y, NS - ns) : 0u;
+                for (uint32_t i0 = 0; i0 < n; i0 += 512) {
+                    u32x2 v[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) v[j] = pool[rd[z].x + min(i0 + 64u * j + l, n - 1)];
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if (i0 + 64u * j + l < n) {
+                            b[2 * (ns + i0 + 64u * j + l)] = v[j].x;
+                            b[2 * (ns + i0 + 64u * j + l) + 1] = v[j].y;
+                        }
+                }
+                room = room && n == rd[z].y;
+                ns += n;
+            }
+            if (l == 0) b[o_ns] = ns;
         }
-        if (r + 1 == c.nsub) break;
-        // the graph is usable when it is complete and was built from a start set holding the true
-        // start, also when later rounds moved that subsequence's start set on
-        const O1Graph& g = graph[t];
-        const O1DecState zs{z.B, z.X, z.cx};
-        int o = -1;
-        if (g.status == 0)
-            for (int k = 0; k < g.norigin; k++)
-                if (o1d_same(g.ostate[k], zs)) { o = k; break; }
-        if (o >= 0) {
-            O1GEdge ed = g.origin[o];
-            off += ed.sym;
-            int guard = 0;
-            while (ed.tgt >= 0 && guard++ <= kGNode) {
-                const int sign = (z.e < c.novf) ? (ov[z.e] < 0) : 0;
-                z.e++;
-                ed = g.node[ed.tgt][sign];
-                off += ed.sym;
+    };
+    // an edge of a node that is not staged
+    auto far_edge = [&](uint32_t u, uint32_t tgt, uint32_t neg) -> uint32_t {
+        const uint2* rw = ws.wave + (c.gfirst + u) * kSplitRounds;
+        for (int z = 0; z < kSplitRounds; z++) {
+            const uint2 v = rw[z];
+            if (tgt < v.y) return v.x == ~0u ? kSplitFail : glb(reinterpret_cast<const uint32_t*>(ws.pool))[2 * ((uint64_t)v.x + tgt) + neg];
+            tgt -= v.y;
+        }
+        return kSplitFail;
+    };
+    uint32_t cur = c.x0 & ((1u << kO1Log) - 1);
+    uint64_t e = 0, off = 0;
+    // signs of 64 escaped codes from index eb on (bit k: code eb + k is negative), the next 64 in flight
+    uint64_t eb = 0, signs = 0;
+    int vnext = 0;
+    auto sign_load = [&](uint64_t at) { return at + l < c.novf ? (int)glb(c.ov)[at + l] : 0; };
+    if (wv == 0) {
+        signs = __ballot(sign_load(0) < 0);
+        vnext = sign_load(64);
+    }
+    uint32_t r = 0;        // part the walk is at
+    uint32_t u0 = 0, cb = 0;  // first unit of the current buffer, which one it is
+    const uint32_t nwaves = kWalkThreads / 64;
+    if (ngraph) stage_units(0, lmem, 0, nwaves);
+    if (lead) sh_stop = 0;
+    while (r < ngraph) {
+        if (lead) sh_miss = 0;
+        __syncthreads();
+        const uint32_t r_end = min(ngraph, (u0 + U) * P);
+        if (wv > 0) {
+            stage_units(u0 + U, lmem + (cb ^ 1u) * (kWalkBuf / 4), 1, nwaves - 1);
+        } else {
+            const FZ_LDS uint32_t* buf = lmem + cb * (kWalkBuf / 4);
+            uint32_t u = u0, pu = r - u0 * P;
+            while (pu >= P) { pu -= P; u++; }
+            bool miss = false;
+            for (; r < r_end; r++) {
+                const FZ_LDS uint32_t* b = buf + (u - u0) * unit_words;
+                if (lead) {
+                    ws.res_state[c.tfirst + r] = cur;
+                    ws.res_e[c.tfirst + r] = e;
+                    ws.res_off[c.tfirst + r] = off;
+                }
+                const uint32_t n = __builtin_amdgcn_readfirstlane(b[o_n + pu]);
+                const uint32_t ns = __builtin_amdgcn_readfirstlane(b[o_ns]);
+                uint32_t ed = kSplitFail;
+                bool found = false;
+                for (uint32_t i = 0; i < n && !found; i += 64) {
+                    const uint64_t mk = __ballot(i + l < n && b[o_cand + pu * c.cap + i + l] == cur);
+                    if (mk) {
+                        found = true;
+                        ed = b[o_edge + pu * c.cap + i + (uint32_t)__builtin_ctzll(mk)];
+                    }
+                }
+                ed = __builtin_amdgcn_readfirstlane(ed);
+                // every escape is one hop: node, sign, next edge. All of it is wave-uniform and kept in
+                // scalar registers; signs holds those of 64 escapes, k the next one's place in it
+                uint64_t pe = uniform64(e), sg = uniform64(signs);
+                uint64_t po = off + (ed >> 16);
+                uint32_t tgt = ed & 0xFFFFu, k = uniform32((uint32_t)min<uint64_t>(pe - eb, 128)), guard = 0;
+                while (tgt < kSplitExit) {
+                    if (k >= 64) {
+                        if (k < 128) {
+                            eb += 64;
+                            k -= 64;
+                            signs = __ballot(vnext < 0);
+                        } else {
+                            eb = pe;
+                            k = 0;
+                            signs = __ballot(sign_load(eb) < 0);
+                        }
+                        vnext = sign_load(eb + 64);
+                        sg = uniform64(signs);
+                    }
+                    const uint32_t k0 = k;
+                    uint32_t sum = 0;
+                    if (tgt < ns) {
+                        do {
+                            ed = uniform32(b[2 * tgt + ((uint32_t)(sg >> k) & 1u)]);
+                            sum += ed >> 16;
+                            tgt = ed & 0xFFFFu;
+                            k++;
+                        } while (tgt < ns && k < 64);
+                    } else {
+                        ed = uniform32(far_edge(u, tgt, (uint32_t)(sg >> k) & 1u));
+                        sum = ed >> 16;
+                        tgt = ed & 0xFFFFu;
+                        k++;
+                    }
+                    po += sum;
+                    pe += k - k0;
+                    guard += k - k0;
+                    if (guard > 65536u) {  // a loop of escapes that read no bits
+                        ed = kSplitFail;
+                        break;
+                    }
+                }
+                if (ed == kSplitFail) {
+                    if (lead) {
+                        atomicAdd(&stats[found ? 0 : 1], 1u);  // no whole path in the graph / entry not in the set
+                        atomicAdd(&stats[6 + q], 1u);          // per chain
+                    }
+                    miss = true;
+                    break;
+                }
+                cur = __builtin_amdgcn_readfirstlane(b[o_exit + pu * c.cap + (ed & 0xFFFu)]);
+                e = pe;
+                off = po;
+                if (off > c.m) {  // a corrupt stream
+                    if (lead) {
+                        *c.err = 1;
+                        sh_stop = 1;
+                    }
+                    break;
+                }
+                if (++pu == P) { pu = 0; u++; }
             }
-            if (ed.tgt >= 0 || -1 - ed.tgt >= g.nexit) {
-                if (lead) *err = 1;
-                return;
-            }
-            const O1DecState x = g.exit[-1 - ed.tgt];
-            z.B = x.B; z.X = x.X; z.cx = x.ctx;
+            if (lead) sh_miss = miss ? r + 1 : 0;
+        }
+        __syncthreads();
+        if (sh_stop) return;
+        const uint32_t miss = sh_miss;
+        if (!miss) {
+            u0 += U;
+            cb ^= 1u;
+            r = r_end;
             continue;
         }
-        if (lead) {
-            atomicAdd(&stats[g.status ? 0 : 1], 1u);  // capacity exceeded / start state not in the set
-            if (g.status) atomicAdd(&stats[1 + g.status], 1u);
-            atomicAdd(&stats[6 + q], 1u);  // per chain
+        // exact decode of part r = miss - 1, the bitstream staged in LDS window by window
+        r = miss - 1;
+        for (uint32_t i = tid; i < (uint32_t)kWalkCtxN << kO1Log; i += kWalkThreads)
+            mem[i] = glb(c.dt)[((size_t)c.hot0 << kO1Log) + i];
+        __syncthreads();
+        if (wv == 0) {
+            const int64_t b = c.pos0 - (int64_t)r * c.sub_bits, stop = b - c.sub_bits;
+            SeqState z{b - (int64_t)(cur >> 17), cur & ((1u << kO1Log) - 1), (cur >> kO1Log) & 15u, e, false};
+            uint8_t* st8 = reinterpret_cast<uint8_t*>(stage32);
+            while (z.B > stop && off < c.m && !z.bad) {
+                const int64_t hi = min<int64_t>(c.len, (z.B + 7) / 8 + 1);
+                const int64_t lo = max<int64_t>(0, hi - kWalkStage);
+                wave_lds_order();
+                const int64_t w0 = stage_window(lds(st8), c.cb, c.len, lo, hi);
+                wave_lds_order();
+                // window reads reach 64 bits below the read position: stay above the staged bytes
+                // unless they start at the chain's first byte
+                const int64_t floor_bits = lo == 0 ? INT64_MIN : lo * 8 + 64;
+                off += seq_decode(z, lds(st8), w0 + kWinPad, max<int64_t>(stop, floor_bits), c.m - off, lds(mem), c.hot0,
+                                  c.dt, nullptr, 0, 0, c.ov, c.novf, nullptr);
+            }
+            e = z.e;
+            const int64_t d = stop - z.B;
+            if (z.bad || d < 0 || d > 12 || off > c.m) {  // a corrupt stream: its codes ran out inside the part
+                if (lead) {
+                    *c.err = 1;
+                    sh_stop = 1;
+                }
+            }
+            cur = ((uint32_t)d & 15u) << 17 | z.cx << kO1Log | (z.X & ((1u << kO1Log) - 1));
         }
-        // exact decode of this subsequence down to `stop`, the bitstream staged in LDS window by
-        // window
-        const int64_t stop = c.pos0 - (int64_t)(r + 1) * c.sub_bits;
-        while (z.B > stop && off < m && !z.bad) {
-            const int64_t hi = min<int64_t>((int64_t)c.len, (z.B + 7) / 8 + 1);
-            const int64_t lo = max<int64_t>(0, hi - (int64_t)kWalkStage);
-            __syncthreads();
-            const int64_t w0 = stage_window(lds(stage), cb, (int64_t)c.len, lo, hi);
-            __syncthreads();
-            // window reads reach 64 bits below the read position: stay above the staged bytes unless
-            // they start at the chain's first byte (bits below it read as zero)
-            const int64_t floor_bits = lo == 0 ? INT64_MIN : lo * 8 + 64;
-            off += seq_decode(z, lds(stage), w0 + kWinPad, max<int64_t>(stop, floor_bits), m - off, lds(hot), c.hot0, dt, nullptr, 0, 0,
-                              ov, c.novf, nullptr);
-        }
-        if (z.bad) {
-            if (lead) *err = 1;
-            return;
+        __syncthreads();
+        if (sh_stop) return;
+        r++;
+        u0 = r / P;
+        cb = 0;
+        if (r < ngraph) stage_units(u0, lmem, 0, nwaves);
+    }
+    if (lead) {  // the last part
+        ws.res_state[c.tfirst + r] = cur;
+        ws.res_e[c.tfirst + r] = e;
+        ws.res_off[c.tfirst + r] = off;
+    }
+}
+
+// Final pass: every part decodes from its entry into its place in the code array. Its code count is
+// the distance to the next part's output offset, so codes leave in aligned 64-byte runs (32 codes
+// packed in registers, four 16-byte stores) between a head and a tail written one by one.
+__global__ void __launch_bounds__(256) k_o1s_out(const O1Split* ch, int nch, O1SplitWs ws) {
+    const uint64_t t = (uint64_t)xcd_block() * blockDim.x + threadIdx.x;
+    if (t >= ws.nparts) return;
+    int q = 0;
+    {
+        int hi = nch;
+        while (hi - q > 1) {
+            const int mid = (q + hi) >> 1;
+            if (ch[mid].tfirst <= t) q = mid; else hi = mid;
         }
     }
+    const O1Split& c = ch[q];
+    if (*c.err) return;  // the walk stopped short: entries are missing
+    const uint64_t r = t - c.tfirst;
+    const bool last = r + 1 >= c.nsub;
+    const uint64_t m = c.m;
+    const uint64_t o0 = ws.res_off[t], o1 = last ? m : ws.res_off[t + 1];
+    if (o0 > o1 || o1 > m) {  // offsets from a corrupt stream
+        *c.err = 1;
+        return;
+    }
+    const uint32_t s = ws.res_state[t];
+    uint64_t e = ws.res_e[t];
+    const uint64_t novf = c.novf;
+    const uint32_t* dt = c.dt;
+    const int16_t* ov = c.ov;
+    const ChainWords cw(c.cb);
+    const int64_t b = c.pos0 - (int64_t)r * c.sub_bits, B0 = b - (int64_t)(s >> 17);
+    uint32_t idx = s & 0x1FFFFu;
+    WordBits rd;
+    rd.init(cw, B0);
+    bool bad = false;
+    uint32_t nb = 0;  // bits of the latest symbol
+    auto step = [&]() -> uint32_t {
+        const uint32_t raw = glb(dt)[idx];
+        nb = (raw >> 24) & 15u;
+        const uint32_t x = (raw + rd.take(nb)) & ((1u << kO1Log) - 1);
+        uint32_t cx = raw >> 28;
+        const uint32_t sy = (raw >> 16) & 0xFFu;
+        int code = (int)((sy >> 1) ^ (~(sy & 1) + 1));
+        if (cx == 15u) {
+            if (e < novf) code = glb(ov)[e];
+            else { code = 32767; bad = true; }
+            e++;
+            cx = (uint32_t)o1_ctx(code);
+        }
+        idx = (cx << kO1Log) | x;
+        return (uint32_t)code & 0xFFFFu;
+    };
+    int16_t* out = c.out;
+    uint64_t i = o0;
+    const uint64_t iend = o1;
+    const uint64_t a0 = ((uintptr_t)out >> 1) & 31;  // 64-byte alignment of the code array
+    while (i < iend && ((i + a0) & 31)) {
+        rd.refill(cw);
+        out[i++] = (int16_t)step();
+    }
+    while (i + 32 <= iend) {
+        uint32_t w[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            rd.refill(cw);
+            const uint32_t a = step();
+            w[j] = a | (step() << 16);
+        }
+        uint32_t* o = reinterpret_cast<uint32_t*>(out + i);
+#pragma unroll
+        for (int j = 0; j < 16; j += 4)
+            *reinterpret_cast<u32x4*>(o + j) = u32x4{w[j], w[j + 1], w[j + 2], w[j + 3]};
+        i += 32;
+    }
+    while (i < iend) {
+        rd.refill(cw);
+        out[i++] = (int16_t)step();
+    }
+    // the part's symbols are those that start above the next boundary
+    const int64_t pos = 32 * rd.j + rd.have - cw.shift, stop = b - (int64_t)c.sub_bits;
+    if (bad || (last && e != novf) || (!last && o1 > o0 && (pos > stop || pos + (int64_t)nb <= stop))) *c.err = 1;
 }
 
 // Decoding-table entries of the dense-chain decoder. Contexts are renumbered so that the four
@@ -2420,58 +2802,6 @@ __global__ void __launch_bounds__(kSeqLanes) k_o1d_dense(const uint8_t* in, cons
 // The chains of many calls (the batched decompress), one workgroup a chain.
 __global__ void __launch_bounds__(kSeqLanes) k_o1d_dense_jobs(const DenseJob* jobs) {
     dense_chain(DenseJobSrc{jobs + blockIdx.x});
-}
-
-
-// Final pass: every subsequence decodes from its settled start into its place in the code array.
-// Its code count is the distance to the next subsequence's output offset, so codes leave in
-// aligned 64-byte runs (32 codes packed in registers, four 16-byte stores) between a head and a
-// tail written one by one: whole lines reach L2 instead of two bytes at a time.
-__global__ void __launch_bounds__(256) k_o1d_out(const uint8_t* in, const O1DecChain* ch, int nch, uint64_t nsub,
-                                                 const DEntry* dt_all, const int16_t* ovf, const O1DecState* start,
-                                                 const uint64_t* e_start, const uint64_t* res_off, int16_t* out,
-                                                 int* err) {
-    const uint64_t t = (uint64_t)xcd_block() * blockDim.x + threadIdx.x;
-    if (t >= nsub) return;
-    const O1DecChain c = ch[o1d_chain_of(ch, nch, t)];
-    const uint64_t r = t - c.tfirst;
-    const DEntry* dt = dt_all + c.dset * kO1Ctx * (1u << kO1Log);
-    const bool last = r + 1 >= c.nsub;
-    const int64_t stop = last ? INT64_MIN : c.pos0 - (int64_t)(r + 1) * c.sub_bits;
-    const uint64_t m = c.hi - c.lo;
-    const uint64_t o0 = res_off[t], o1 = last ? m : res_off[t + 1];
-    if (o0 > o1 || o1 > m) {  // offsets from a corrupt stream
-        *err = 1;
-        return;
-    }
-    O1DecState s = start[t];
-    uint64_t e = e_start[t];
-    uint64_t i = c.lo + o0;
-    const uint64_t iend = c.lo + o1;
-    bool bad = false;
-    BitWin rd = bwin_at(in + c.off, s.B);
-    int64_t before = rd.pos;  // read position before the latest symbol
-    auto step = [&]() -> uint32_t {
-        before = rd.pos;
-        return (uint32_t)o1d_step(dt, rd, s.X, s.ctx, e, ovf + c.ovf_base, c.novf, bad) & 0xFFFFu;
-    };
-    while (i < iend && (i & 31)) out[i++] = (int16_t)step();
-    while (i + 32 <= iend) {
-        uint32_t w[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const uint32_t a = step();
-            w[j] = a | (step() << 16);
-        }
-        uint32_t* o = reinterpret_cast<uint32_t*>(out + i);
-#pragma unroll
-        for (int j = 0; j < 16; j += 4)
-            *reinterpret_cast<u32x4*>(o + j) = u32x4{w[j], w[j + 1], w[j + 2], w[j + 3]};
-        i += 32;
-    }
-    while (i < iend) out[i++] = (int16_t)step();
-    // the subsequence's symbols are those that start above the next boundary
-    if (bad || (last && e != c.novf) || (!last && o1 > o0 && (rd.pos > stop || before <= stop))) *err = 1;
 }
 
 
@@ -3223,29 +3553,15 @@ static void fse_dec_multi(const std::vector<FseDecItem>& items, int* err, DevAre
     sync(st);  // blks is read by the copy above
 }
 
-// Order-1 tANS chains (7 values each: stream offset, bytes, out lo, out hi, escape offset, table
-// set, escape count) decoded in parallel subsequences; see k_o1d_round.
-// More than this many escapes per 4096 symbols on average: the chain is decoded from its start.
-constexpr uint64_t kDenseEscapes = 8;
-// Symbols per subsequence (about): each graph round decodes this many per lane, so it sets the
-// latency of a round; a decoder started at a guessed state falls into step within about a
-// thousand symbols, so start sets settle within a few rounds.
-constexpr double kSubSymbols = 1024;
-// Graph rounds before the walk; subsequences whose start sets are still moving are decoded exactly
-// by the walk.
-constexpr uint64_t kMaxRounds = 6;
-// Subsequences of warm-up before the first round's start states.
-constexpr int64_t kWarmSubs = 4;
-// Chains below this many bits a symbol are decoded from their start.
-constexpr double kSeqBitsPerSymbol = 2.5;
-// So are chains of at most this many symbols (fields up to about 128^3, one segment of four chains):
-// the sequential decoder takes about 85 ns a symbol on one CU, while the warm-up, graph rounds and
-// walk cost several milliseconds on many CUs whatever the length. Measured per call on k^-3 fields
-// (REL 1e-2 / 1e-3 / 1e-4): 64^3 15.0 / 7.0 / 10.0 ms against 9.8 / 7.0 / 10.1 decoded from the
-// start, 128^3 84.7 / 45.1 / 51.5 against 65.6 / 47.9 / 51.5, 200^3 243 / 169 / 182 against
-// 235 / 185 / 182; many such fields decoded side by side gain most, the sequential chains
-// occupying four CUs a field.
-constexpr uint64_t kSeqShortSymbols = 1ull << 19;
+// Order-1 tANS chains are given as 7 values each: stream offset, bytes, out lo, out hi, escape offset,
+// table set, escape count.
+// Chains of fewer symbols, or of fewer bits a symbol (where decoders started at guessed states hardly
+// ever meet), are decoded from their start.
+constexpr uint64_t kSplitMinSymbols = 8192;
+constexpr double kSplitMinBits = 2.5;
+// In the batched decompress, so are chains of at most this many: many fields' sequential chains run
+// side by side in one launch.
+constexpr uint64_t kDeferSymbols = 1ull << 19;
 
 // Stationary distribution of segment g's context chain (a code's context follows from the previous
 // code; an escape leads to 13 or 14, counted half each), from the normalized counts of its 15
@@ -3290,9 +3606,7 @@ static void context_shares(const uint8_t* host, uint64_t nf_off, double pi[kO1Ct
 
 // The four consecutive contexts the walk keeps in LDS for a chain of the segment at nf_off: the
 // window with the largest share (ties: the higher window, so 11..14 where escapes dominate).
-static uint32_t hot_window(const uint8_t* host, uint64_t nf_off) {
-    double pi[kO1Ctx];
-    context_shares(host, nf_off, pi);
+static uint32_t hot_window(const double pi[kO1Ctx]) {
     uint32_t best = kWalkCtx0;
     double bw = -1;
     for (int h = kO1Ctx - kWalkCtxN; h >= 0; h--) {
@@ -3361,28 +3675,87 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st) {
     FZ_HIP(hipGetLastError());
 }
 
+// How a chain is decoded: from its start by one workgroup (k_o1d_dense), or split into parts. The
+// split decoder follows, for every part, all states that its entry may be; what that costs is the
+// number of such states that live side by side, estimated from the chain's tables:
+//   mu   rate per symbol at which two decoders meet. It falls with the bits a symbol takes (a step
+//        replaces that many bits of the 13-bit state): 5e-4 at 7.4 bits, 3e-4 at 6.2, 5e-5 at 3.2
+//        (measured on k^-3 fields), so 8e-6 * 2^(0.85 bits).
+//   pe   escapes per symbol by the tables, which is what a decoder off the true path meets. Every escape doubles the paths and meeting halves them: about 1 + 2 pe / mu live ones
+//        (counted on the CPU: 24 at 7.8 bits and an escape in 175 symbols, 130 at 7.4 and one in 36,
+//        over 900 at 3.0 and one in 250).
+// Split chains, by size class of the graph kernel; kSplitNone: from the start.
+enum { kSplitFew = 0, kSplitSome = 1, kSplitMany = 2, kSplitNone = 3 };
+constexpr int kSplitNodes[3] = {128, 512, 1024};
+struct SplitPlan {
+    int cls = kSplitNone;
+    double nodes = 0;  // nodes a symbol
+    uint32_t lgk = 0, warm = 0, cap = 0, parts = 0, sub = 0;  // warm, sub in symbols
+};
+static SplitPlan split_plan(uint64_t m, uint64_t novf, double bits, const double pi[kO1Ctx], const uint8_t* norm,
+                            bool keep_short) {
+    SplitPlan s;
+    // a chain of few symbols is done sooner from its start than the split decoder's launches take
+    if (m < (keep_short ? 4096u : kSplitMinSymbols) || bits < kSplitMinBits) return s;
+    double pe = 0;
+    for (int a = 0; a < kO1Ctx; a++) {
+        int16_t v;
+        memcpy(&v, norm + 2 * ((size_t)a * kO1Sym + 255), 2);
+        pe += pi[a] * (v < 0 ? 1.0 : (double)v) / (double)(1u << kO1Log);
+    }
+    // the first chain of a segment holds most of its escapes (the coarse levels)
+    pe = std::max(pe, 0.25 * (double)novf / (double)m);
+    const double mu = 8e-6 * std::exp2(0.85 * bits);
+    const double live = 1.0 + 2.0 * pe / mu;
+    if (novf * 8 > m || live > (bits >= 6.0 ? 200.0 : bits >= 4.5 ? 60.0 : 10.0)) return s;
+    s.nodes = 1.5 * pe * live;
+    if (pe < 1.0 / 1024 && live <= 10.0) {
+        // Few states: long parts, and guessed decoders enough, early enough, for the true entry to be
+        // among their states in most parts before the first round (CPU counts on k^-3 fields, parts
+        // that the walk decodes exactly after three rounds: 6.2 bits, 8 decoders 512 symbols ahead 1 of
+        // 2000; 3.2 bits, 64 decoders 2048 ahead 2 of 750, 32 decoders 7).
+        s.cls = kSplitFew;
+        s.sub = m >= (1u << 20) ? (bits >= 5.5 ? 1024 : 2048) : m >= (1u << 18) ? 1024 : m >= (1u << 16) ? 512 : 256;
+        s.warm = bits >= 5.5 ? 512 : 2048;
+        s.lgk = bits >= 6.0 ? 3 : bits >= 5.5 ? 4 : 6;
+        s.cap = s.lgk <= 4 ? 16 : 32;
+        s.parts = s.lgk <= 4 ? 16 : 8;
+        while (s.parts > 1 && s.parts * s.nodes * s.sub > kSplitNodes[kSplitFew] / 3) s.parts /= 2;
+    } else {
+        // Escapes saturate the sets in a round or two whatever they start from: short parts and a short
+        // warm-up (same counts: none of 500 parts left at 16 decoders 256 symbols ahead).
+        s.sub = 256;
+        s.warm = 256;
+        s.lgk = 4;
+        const double nodes = s.nodes * s.sub;
+        // the estimate is about twice what is counted; past its table a graph is lost to the walk
+        if (nodes > 1.5 * kSplitNodes[kSplitMany]) return s;
+        s.cls = nodes <= kSplitNodes[kSplitSome] / 4 ? kSplitSome : kSplitMany;
+        s.cap = s.cls == kSplitSome ? 64 : kSplitMaxCap;
+        s.parts = s.cls == kSplitMany ? 1 : nodes <= kSplitNodes[kSplitSome] / 16 ? 4 : nodes <= kSplitNodes[kSplitSome] / 8 ? 2 : 1;
+    }
+    return s;
+}
+
 // defer: the sequential chains are handed to it instead of launched (their decode then runs in
 // dense_batch_run, after the work this call has queued on st).
 static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const std::vector<uint64_t>& chains,
                                const std::vector<uint64_t>& nf_off, const DEntry* dt, const int16_t* ovf, int16_t* out,
                                int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer) {
     const int nch = (int)(chains.size() / 7);
-    std::vector<O1DecChain> hc, hd;
-    uint64_t nsub = 0, stream_bytes = 0, ncodes = 0, dense_bytes = 0, dense_codes = 0;
-    // segments holding a dense chain: their context-13/14 tables give escapes a high probability, so
-    // a decoder off the true path (a wrong sign, a wrong start) meets spurious escapes at every turn
-    // and graphs overflow even where real escapes are few; chains there that have escapes at all are
-    // decoded from their start as well
-    std::vector<uint64_t> dense_seg;
-    for (int q = 0; q < nch; q++) {
-        const uint64_t* c = &chains[7 * q];
-        const uint64_t m = c[3] - c[2];
-        if (m && c[6] * 4096 > kDenseEscapes * m) dense_seg.push_back(c[5]);
-    }
-    auto in_dense_seg = [&](uint64_t g) { return std::find(dense_seg.begin(), dense_seg.end(), g) != dense_seg.end(); };
-    // FALCONS_O1_SEQUENTIAL=1 decodes every chain from its start (the dense-chain decoder)
+    std::vector<O1Split> hc;
+    std::vector<O1DecChain> hd;
+    std::vector<SplitPlan> plans;
+    std::vector<uint64_t> seg_of, novf_of;
+    uint64_t dense_bytes = 0, dense_codes = 0, stream_bytes = 0, ncodes = 0;
+    // FALCONS_O1_SEQUENTIAL=1 decodes every chain from its start; FALCONS_O1_PARALLEL_SHORT=1 splits
+    // short chains too (the tests of either decoder on small fields)
     const char* seq_env = getenv("FALCONS_O1_SEQUENTIAL");
     const bool all_seq = seq_env && atoi(seq_env) != 0;
+    const char* par_env = getenv("FALCONS_O1_PARALLEL_SHORT");
+    const bool keep_short = par_env && atoi(par_env) != 0;
+    double pi[kO1Ctx];
+    uint64_t pi_seg = ~0ull;
     for (int q = 0; q < nch; q++) {
         const uint64_t* c = &chains[7 * q];
         const uint64_t m = c[3] - c[2];
@@ -3396,47 +3769,47 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             x0 = (x0 << 1) | (bit >= 0 ? ((b[bit >> 3] >> (bit & 7)) & 1u) : 0u);
         }
         const int64_t pos0 = top - (int64_t)kO1Log;
-        if (all_seq || c[6] * 4096 > kDenseEscapes * m || (in_dense_seg(c[5]) && c[6] * 16384 > m)) {
-            hd.push_back(O1DecChain{c[0], c[1], c[2], c[3], c[4], c[6], c[5], pos0, x0, 1, 0, 0, kWalkCtx0, 0});
+        const double bits = (double)std::max<int64_t>(pos0, 0) / (double)m;
+        if (pi_seg != c[5]) {
+            context_shares(host, nf_off[c[5]], pi);
+            pi_seg = c[5];
+        }
+        SplitPlan sp;
+        if (!all_seq && !(defer && m <= kDeferSymbols)) sp = split_plan(m, c[6], bits, pi, host + nf_off[c[5]], keep_short);
+        if (sp.cls == kSplitNone) {
+            hd.push_back(O1DecChain{c[0], c[1], c[2], c[3], c[4], c[6], c[5], pos0, x0, 0});
             dense_bytes += c[1];
             dense_codes += m;
             continue;
         }
-        // about 1024 symbols per subsequence
-        const double bits_per_sym = std::max(1.0, (double)std::max<int64_t>(pos0, 1) / (double)m);
-        const int64_t sub = std::max<int64_t>(2048, (int64_t)(bits_per_sym * kSubSymbols));
-        const uint64_t ns = std::max<int64_t>(1, (pos0 + sub - 1) / sub);
-        hc.push_back(O1DecChain{c[0], c[1], c[2], c[3], c[4], c[6], c[5], pos0, x0, (uint32_t)ns, 0, sub,
-                                hot_window(host, nf_off[c[5]]), 0});
+        O1Split k{};
+        k.cb = dev + c[0];
+        k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
+        k.ov = ovf + c[4];
+        k.out = out + c[2];
+        k.err = err;
+        k.m = m;
+        k.novf = c[6];
+        k.len = (int64_t)c[1];
+        k.pos0 = pos0;
+        k.x0 = x0;
+        k.sub_bits = (uint32_t)std::max(2048.0, bits * sp.sub);
+        k.nsub = (uint32_t)std::max<int64_t>(1, (pos0 + k.sub_bits - 1) / k.sub_bits);
+        k.warm_bits = (uint32_t)(bits * sp.warm) + 64;
+        k.warm_steps = 2 * sp.warm;
+        k.lgk = sp.lgk;
+        k.cap = sp.cap;
+        k.parts = sp.parts;
+        k.max_sym = 8 * sp.sub;
+        k.hot0 = hot_window(pi);
+        k.cls = (uint32_t)sp.cls;
+        hc.push_back(k);
+        plans.push_back(sp);
+        seg_of.push_back(c[5]);
+        stream_bytes += c[1];
+        ncodes += m;
     }
-    // Chains of fewer than 2.5 bits a symbol go to the sequential decoder as well: there a decoder
-    // started from a guessed state seldom falls into step with the true one (few bits are read per
-    // symbol), so subsequence start sets do not settle and the walk would decode most subsequences
-    // one after another anyway, more slowly. So do short chains (kSeqShortSymbols).
-    {
-        // FALCONS_O1_PARALLEL_SHORT=1 keeps short chains on the parallel decoder (its tests on small fields)
-        const char* par_env = getenv("FALCONS_O1_PARALLEL_SHORT");
-        const bool short_seq = !(par_env && atoi(par_env) != 0);
-        std::vector<O1DecChain> keep;
-        for (O1DecChain c : hc) {
-            const double bps = (double)c.pos0 / (double)(c.hi - c.lo);
-            if ((c.nsub > 2 && bps < kSeqBitsPerSymbol) || (short_seq && c.hi - c.lo <= kSeqShortSymbols)) {
-                c.nsub = 1;
-                c.sub_bits = 0;
-                hd.push_back(c);
-                dense_bytes += c.len;
-                dense_codes += c.hi - c.lo;
-                continue;
-            }
-            c.tfirst = nsub;
-            keep.push_back(c);
-            stream_bytes += c.len;
-            ncodes += c.hi - c.lo;
-            nsub += c.nsub;
-        }
-        hc.swap(keep);
-    }
-    // dense chains run beside the rest, on the auxiliary stream when there is one
+    // sequential chains run beside the rest, on the auxiliary stream when there is one
     hipStream_t dst = aux.stream ? aux.stream : st;
     const bool stats_on = getenv("FALCONS_DECODE_STATS") != nullptr;
     uint64_t* dense_times = nullptr;  // per sequential chain: clock at start and end (statistics only)
@@ -3486,53 +3859,78 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     } join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
     if (hc.empty()) return;
     const int nc = (int)hc.size();
-    O1DecChain* dch = ws.take<O1DecChain>(nc);
-    O1StartSet* start = ws.take<O1StartSet>(nsub);
-    O1Graph* graph = ws.take<O1Graph>(nsub);
-    O1DecState* res_start = ws.take<O1DecState>(nsub);
-    uint64_t* res_e = ws.take<uint64_t>(nsub);
-    uint64_t* res_off = ws.take<uint64_t>(nsub);
-    uint8_t* run = ws.take<uint8_t>(nsub);
-    unsigned int* nrun = ws.take<unsigned int>(1);
-    unsigned int* stats = ws.take<unsigned int>(6 + nc);
-    FZ_HIP(hipMemsetAsync(stats, 0, (6 + nc) * sizeof(unsigned int), st));
-    h2d(dch, hc.data(), hc.size(), st);
-    uint64_t rounds = 0;
-    FZ_LAUNCH("o1_decode_init", 0, k_o1d_init, dim3(nblk(nsub)), dim3(256), 0, st, dev, dch, nc, nsub, dt,
-              (int64_t)kWarmSubs, start, run);
-    FZ_HIP(hipGetLastError());
-    // start sets settle like the states of a single decoder: every round settles at least the next
-    // subsequence of every chain
-    for (uint64_t round = 0; round < kMaxRounds; round++) {
-        FZ_LAUNCH("o1_decode_graph", 0, k_o1d_graph, dim3(nblk(nsub, kGLanes)), dim3(kGLanes), 0, st, dev, dch, nc, nsub,
-                  dt, run, start, graph);
-        FZ_HIP(hipGetLastError());
-        FZ_HIP(hipMemsetAsync(nrun, 0, sizeof(unsigned int), st));
-        FZ_LAUNCH("o1_decode_link", 0, k_o1d_glink, dim3(nblk(nsub)), dim3(256), 0, st, dch, nc, nsub, graph, start,
-                  run, nrun);
-        FZ_HIP(hipGetLastError());
-        unsigned int h = 0;
-        d2h(&h, nrun, 1, st);
-        rounds = round + 1;
-        if (!h) break;
+    // chains of one size class side by side, for one launch each
+    std::vector<int> order(nc);
+    for (int q = 0; q < nc; q++) order[q] = q;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hc[x].cls < hc[y].cls; });
+    std::vector<O1Split> sc(nc);
+    uint64_t nparts = 0, ncand = 0, nlanes = 0, nwaves = 0;
+    double pool = 0;
+    int cls_first[4] = {0, 0, 0, 0};
+    uint64_t cls_waves[3] = {0, 0, 0};
+    for (int i = 0; i < nc; i++) {
+        O1Split& k = sc[i] = hc[order[i]];
+        const SplitPlan& sp = plans[order[i]];
+        const uint64_t nw = (k.nsub - 1 + k.parts - 1) / k.parts;
+        k.tfirst = nparts;
+        k.cfirst = ncand;
+        k.wfirst = nlanes;
+        k.gfirst = nwaves;
+        nparts += k.nsub;
+        ncand += (uint64_t)k.nsub * k.cap;
+        nlanes += (((uint64_t)k.nsub << k.lgk) + 63) & ~63ull;
+        nwaves += nw;
+        cls_waves[k.cls] += nw;
+        for (uint32_t z = k.cls + 1; z < 4; z++) cls_first[z] = i + 1;
+        // twice what the estimate gives for two rounds, and some for each wave
+        pool += 4.0 * sp.nodes * (double)k.m + 16.0 * (double)nw;
     }
-    FZ_LAUNCH("o1_decode_walk", 0, k_o1d_walk, dim3(nc), dim3(kSeqLanes), 0, st, dev, dch, nc, dt, ovf, graph, res_start,
-              res_e, res_off, stats, err);
+    O1Split* dch = ws.take<O1Split>(nc);
+    O1SplitWs W{};
+    W.cand = ws.take<uint32_t>(ncand);
+    W.edge = ws.take<uint32_t>(ncand);
+    W.exits = ws.take<uint32_t>(ncand);
+    W.hdr = ws.take<uint16_t>(nparts * kSplitRounds);
+    W.n0 = ws.take<uint8_t>(nparts);
+    W.wave = ws.take<uint2>((nwaves + 1) * kSplitRounds);
+    W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, 0xF0000000ull);
+    W.pool = ws.take<uint2>(W.pool_cap);
+    W.nparts = nparts;
+    W.res_state = ws.take<uint32_t>(nparts);
+    W.res_e = ws.take<uint64_t>(nparts);
+    W.res_off = ws.take<uint64_t>(nparts);
+    unsigned int* stats = ws.take<unsigned int>(8 + nc);
+    W.pool_used = stats + 6 + nc;
+    h2d(dch, sc.data(), sc.size(), st);
+    FZ_HIP(hipMemsetAsync(stats, 0, (8 + nc) * sizeof(unsigned int), st));
+    FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(nlanes)), dim3(256), 0, st, dch, nc, nlanes, W);
+    for (int round = 0; round < kSplitRounds; round++)
+        for (int z = 2; z >= 0; z--) {
+            const int c0 = cls_first[z], cn = cls_first[z + 1] - c0;
+            const uint32_t nw = (uint32_t)cls_waves[z];
+            if (!cn || !nw) continue;
+            if (z == kSplitFew)
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[0]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+            else if (z == kSplitSome)
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[1]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+            else
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[2]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+        }
+    FZ_LAUNCH("o1_split_walk", 0, k_o1s_walk, dim3(nc), dim3(kWalkThreads), 0, st, dch, nc, W, stats);
+    FZ_LAUNCH("o1_split_out", stream_bytes + ncodes * 2, k_o1s_out, dim3(nblk(nparts)), dim3(256), 0, st, dch, nc, W);
     FZ_HIP(hipGetLastError());
-    FZ_LAUNCH("o1_decode_out", stream_bytes + ncodes * 2, k_o1d_out, dim3(nblk(nsub)), dim3(256), 0, st, dev, dch, nc,
-              nsub, dt, ovf, res_start, res_e, res_off, out, err);
-    if (getenv("FALCONS_DECODE_STATS")) {
-        std::vector<unsigned int> hsv(6 + nc);
-        d2h(hsv.data(), stats, 6 + nc, st);
+    if (stats_on) {
+        std::vector<unsigned int> hsv(8 + nc);
+        d2h(hsv.data(), stats, 8 + nc, st);
         const unsigned int* hs = hsv.data();
         fprintf(stderr, "[o1 decode] chains (chain:exact subsequences/subsequences/escapes/bits a symbol/segment/"
                         "first LDS context of the walk):");
         for (int q = 0; q < nc; q++)
-            fprintf(stderr, " %d:%u/%u/esc%llu/b%.2f/s%llu/h%u", q, hs[6 + q], hc[q].nsub, (unsigned long long)hc[q].novf,
-                    (double)hc[q].pos0 / (double)std::max<uint64_t>(1, hc[q].hi - hc[q].lo),
-                    (unsigned long long)hc[q].dset, hc[q].hot0);
+            fprintf(stderr, " %d:%u/%u/esc%llu/b%.2f/s%llu/h%u", q, hs[6 + q], sc[q].nsub, (unsigned long long)sc[q].novf,
+                    (double)sc[q].pos0 / (double)std::max<uint64_t>(1, sc[q].m), (unsigned long long)seg_of[order[q]],
+                    sc[q].hot0);
         fprintf(stderr, "\n");
-        fprintf(stderr, "[o1 decode] %zu dense chains decoded from their start:", hd.size());
+        fprintf(stderr, "[o1 decode] %zu chains decoded from their start:", hd.size());
         for (const O1DecChain& c : hd)
             fprintf(stderr, " b%.2f/s%llu/esc%llu", (double)c.pos0 / (double)std::max<uint64_t>(1, c.hi - c.lo),
                     (unsigned long long)c.dset, (unsigned long long)c.novf);
@@ -3544,21 +3942,18 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             fprintf(stderr, "[o1 decode] sequential chains (ms / ns a symbol / share of symbols in LDS contexts):");
             for (size_t q = 0; q < hd.size(); q++) {
                 const double ms = (double)(tt[2 * q + 1] - tt[2 * q]) / 1e5;  // 100 MHz clock
-                double pi[kO1Ctx];
-                context_shares(host, nf_off[hd[q].dset], pi);
-                double hs = 0;
-                for (int r = 0; r < kWalkCtxN; r++) hs += pi[maps[q].perm[r]];
-                fprintf(stderr, " %.1f/%.0f/%.3f", ms, ms * 1e6 / (double)std::max<uint64_t>(1, hd[q].hi - hd[q].lo), hs);
+                double ps[kO1Ctx];
+                context_shares(host, nf_off[hd[q].dset], ps);
+                double share = 0;
+                for (int r = 0; r < kWalkCtxN; r++) share += ps[maps[q].perm[r]];
+                fprintf(stderr, " %.1f/%.0f/%.3f", ms, ms * 1e6 / (double)std::max<uint64_t>(1, hd[q].hi - hd[q].lo), share);
             }
             fprintf(stderr, "\n");
         }
-        fprintf(stderr, "[o1 decode] %d chains, %llu subsequences, %llu rounds, walk decoded %u subsequences "
-                        "exactly (%u graphs over capacity [exits %u, nodes %u, branches %u, open edges %u], %u start "
-                        "states outside the set)\n",
-                nc, (unsigned long long)nsub, (unsigned long long)rounds, hs[0] + hs[1], hs[0], hs[2], hs[3], hs[4],
-                hs[5], hs[1]);
+        fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
+                        "entries outside the set), %u nodes of %llu\n",
+                nc, (unsigned long long)nparts, hs[0] + hs[1], hs[0], hs[1], hs[6 + nc], (unsigned long long)W.pool_cap);
     }
-    FZ_HIP(hipGetLastError());
 }
 
 // Where the parts of an entropy stream sit (RleFseEncoder::save / encode, RleFse:897-982, 1072), read
