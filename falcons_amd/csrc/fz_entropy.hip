@@ -69,6 +69,18 @@ __device__ __forceinline__ FZ_GLB T* glb(T* p) { return (FZ_GLB T*)p; }
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+__device__ __forceinline__ uint32_t uniform32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return (uint64_t)uniform32((uint32_t)v) | (uint64_t)uniform32((uint32_t)(v >> 32)) << 32;
+}
+
+// LDS accesses of one wave on either side stay in order (the hardware keeps a wave's LDS operations in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 struct BitW {  // LSB-first FSE bitstream writer (zfse/bitstream.h)
     uint8_t* buf;
     uint64_t pos;
@@ -1494,29 +1506,11 @@ __global__ void __launch_bounds__(256) k_o1_dtables(const uint8_t* stream, const
 }
 
 
-// A chain that is decoded from its start (k_o1d_dense).
-struct O1DecChain {
-    uint64_t off, len;      // stream bytes
-    uint64_t lo, hi;        // output codes
-    uint64_t ovf_base, novf;
-    uint64_t dset;          // table set (segment)
-    int64_t pos0;           // read position after the initial state
-    uint32_t x0;            // initial state
-    uint32_t pad;
-};
-
-// Sequential decoding of a stretch of one chain from a bitstream window staged in LDS, for the
-// walk and for dense chains. win[k + kWinPad] holds chain byte wlo + k; the kWinPad bytes below are
+// Exact decoding of a stretch of one chain from a bitstream window staged in LDS, for the walk. win[k + kWinPad] holds chain byte wlo + k; the kWinPad bytes below are
 // zero when the window starts at the chain's first byte. The decoding tables of contexts
 // hot0 .. hot0 + kWalkCtxN - 1 sit in LDS (hot), the others are read from device memory.
 constexpr int kWalkCtx0 = 11, kWalkCtxN = 4;  // contexts 11..14: after large codes, where escapes are dense
 constexpr int kWinPad = 16;
-constexpr int kDenseStage = 12288;  // dense chains: bitstream bytes per window
-constexpr int kDenseOut = 4096;     // dense chains: codes per round
-constexpr int kDenseOvf = 2048;     // dense chains: escaped values per round
-constexpr int kDnOvfLast = kDenseOvf - 1;
-
-
 constexpr int kSeqLanes = 64;       // the sequential decoders run as one wave
 
 struct SeqState {
@@ -1526,10 +1520,8 @@ struct SeqState {
     bool bad;
 };
 
-// Decodes while the read position stays above `until` (bits), at most `max_n` symbols. Escaped
-// codes come from vbuf[e - ve0] (LDS) when vbuf is given, decoding stopping after the escape that
-// reaches ve1 unless ve1 is the end of the chain's escapes; without vbuf they are read from ov.
-// Writes each code to obuf[k] when obuf is given. Returns the symbols decoded.
+// Decodes while the read position stays above `until` (bits), at most `max_n` symbols, for the symbols
+// and escapes it counts: escaped codes are read from ov. Returns the symbols decoded.
 //
 // Per symbol: the table entry (state, context) and the two window words that hold the 32 bits below
 // the read position are independent LDS reads; the entry gives the bit count, the next state base,
@@ -1537,8 +1529,7 @@ struct SeqState {
 // offsets into the window. One LDS round trip and a few dozen scalar operations per symbol.
 __device__ __forceinline__ uint64_t seq_decode(SeqState& S, const FZ_LDS uint8_t* win, int64_t wlo, int64_t until,
                                                uint64_t max_n, const FZ_LDS uint32_t* hot, uint32_t hot0,
-                                               const uint32_t* dtg, const FZ_LDS int16_t* vbuf, uint64_t ve0,
-                                               uint64_t ve1, const int16_t* ov, uint64_t novf, FZ_LDS int16_t* obuf) {
+                                               const uint32_t* dtg, const int16_t* ov, uint64_t novf) {
     const FZ_LDS uint32_t* w32 = reinterpret_cast<const FZ_LDS uint32_t*>(win);
     const int64_t base = (wlo - kWinPad) * 8;  // bit 0 of the window
     int32_t p = (int32_t)(S.B - base);
@@ -1547,7 +1538,6 @@ __device__ __forceinline__ uint64_t seq_decode(SeqState& S, const FZ_LDS uint8_t
     const int32_t lim = (int32_t)((raised ? base + 32 : until) - base);
     uint32_t X = S.X, cx = S.cx;
     uint64_t e = S.e;
-    const uint64_t elim = (vbuf && ve1 < novf) ? ve1 : ~0ull;
     const uint32_t kmax = (uint32_t)min<uint64_t>(max_n, 0x7FFFFFFFull);
     uint32_t k = 0;
     while (p > lim && k < kmax) {
@@ -1557,44 +1547,26 @@ __device__ __forceinline__ uint64_t seq_decode(SeqState& S, const FZ_LDS uint8_t
         uint32_t raw = hot[(min(hc, (uint32_t)kWalkCtxN - 1) << kO1Log) + xi];
         const uint64_t w = (uint64_t)w32[j] | ((uint64_t)w32[j + 1] << 32);
         if (hc >= (uint32_t)kWalkCtxN) raw = dtg[((size_t)cx << kO1Log) + xi];
-        const uint32_t nb = (raw >> 24) & 15u, sym = (raw >> 16) & 0xFFu;
+        const uint32_t nb = (raw >> 24) & 15u;
         p -= (int32_t)nb;
         X = (raw & 0xFFFFu) + ((uint32_t)(w >> (uint32_t)(p - 32 * j)) & ((1u << nb) - 1u));
-        int code = (int)((sym >> 1) ^ (~(sym & 1) + 1));
         cx = raw >> 28;
         if (cx == 15u) {
-            if (e >= novf) { S.bad = true; code = 32767; }
-            else code = vbuf ? (int)vbuf[e - ve0 < (uint64_t)kDenseOvf ? e - ve0 : 0] : (int)ov[e];
+            int code = 32767;
+            if (e >= novf) S.bad = true;
+            else code = (int)ov[e];
             cx = (uint32_t)o1_ctx(code);
             e++;
-            if (e >= elim) {
-                if (obuf) obuf[k] = (int16_t)code;
-                k++;
-                break;
-            }
         }
-        if (obuf) obuf[k] = (int16_t)code;
         k++;
     }
     // stopped below the staged bytes while symbols remain: the stream runs past its first bit
-    if (raised && p <= lim && k < kmax && (vbuf == nullptr || e < elim)) S.bad = true;
+    if (raised && p <= lim && k < kmax) S.bad = true;
     S.B = base + p;
     S.X = X;
     S.cx = cx;
     S.e = e;
     return k;
-}
-
-__device__ __forceinline__ uint32_t uniform32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    return (uint64_t)uniform32((uint32_t)v) | (uint64_t)uniform32((uint32_t)(v >> 32)) << 32;
-}
-
-// LDS accesses of one wave on either side stay in order (the hardware keeps a wave's LDS operations in
-// order; this keeps the compiler from moving them).
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // Copies chain bytes [w0, hi) into win, where w0 <= lo - kWinPad is the nearest chain byte below
@@ -2300,7 +2272,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
                 // unless they start at the chain's first byte
                 const int64_t floor_bits = lo == 0 ? INT64_MIN : lo * 8 + 64;
                 off += seq_decode(z, lds(st8), w0 + kWinPad, max<int64_t>(stop, floor_bits), c.m - off, lds(mem), c.hot0,
-                                  c.dt, nullptr, 0, 0, c.ov, c.novf, nullptr);
+                                  c.dt, c.ov, c.novf);
             }
             e = z.e;
             const int64_t d = stop - z.B;
@@ -2409,401 +2381,442 @@ __global__ void __launch_bounds__(256) k_o1s_out(const O1Split* ch, int nch, O1S
     if (bad || (last && e != novf) || (!last && o1 > o0 && (pos > stop || pos + (int64_t)nb <= stop))) *c.err = 1;
 }
 
-// Decoding-table entries of the dense-chain decoder. Contexts are renumbered so that the four
-// kept in LDS (kWalkCtx0 ..) come first: 0..3 are those, 4..14 are contexts 0..10, 15 follows an
-// escape. The LDS tables of the four interleave by state: the entry of (state X, context r < 4)
-// sits at byte X * 16 + r * 4. Entry: [31] set when the next context is not in LDS, [30:22] the
-// decoded code (signed), [21:18] the bit count, [17] set for an escape, [16:0]: the byte offset of
-// the next entry less the read bits times 16 (next state base * 16 + next context * 4), where an
-// escape leaves the context term 0 (the escaped value's sign picks context 13 or 14, renumbered 2
-// or 3); with [31] set: next state base * 16 + (renumbered next context - 4).
-constexpr uint32_t kDnSlow = 1u << 31, kDnEsc = 1u << 17;
-// The renumbering of one dense chain: the four contexts most often in use on it (by the
-// stationary distribution of its segment's tables) come first and have their tables in LDS.
-// inv[context] is the renumbered context (inv[15] = 15 for an escape), perm[r] the context of r;
-// esc marks chains decoded with the escape-dense step (contexts 13 and 14 then among the first four).
-struct DenseMap {
-    uint8_t inv[16];
-    uint8_t perm[16];
+// ---- chains decoded from their start ------------------------------------------------------------
+// Chains that cannot be split (dense escapes, or few bits a symbol) are decoded by one workgroup each,
+// from the first symbol to the last. What bounds them is one dependent table lookup after another, so
+// the wave that makes the lookups (wave 0) does nothing else: it logs the states it goes through, and
+// of the other waves one turns a log into codes (symbols, escaped values, places in the output) while
+// the next is being written, and one stages bits and escape signs ahead.
+//
+// Lookups go to re-encoded tables, four contexts of them in LDS, the others in device memory. Entry:
+//   [4:0]   31 - bits read: the shift that brings them down from the top of the 31 next bits
+//   [8:5]   bits read
+//   [12:9]  context after the symbol where it is not in LDS (15: an escape)
+//   [13]    an escape, with both contexts that can follow in slots 0 and 1: the sign of the escaped
+//           value, held at the same bit, picks one
+//   [14]    the next lookup is not in LDS (or an escape whose contexts are not in slots 0 and 1)
+//   [31:16] slot << 13 | next state less the bits read
+// so the next address is three operations from the entry, and everything else (bit buffer, sign
+// register, test for the rare path) fits under the latency of the LDS read. Measured on the 512^3 field
+// at REL 1e-4, 60 chains of 2.24 M symbols with an escape in two, 3% of the lookups not in LDS: 134 ms
+// (60 ns a symbol; 204 ms with one wave for all of it).
+// Symbols of more than half probability read no bits most of the time. In chains of few bits a symbol
+// an entry stands for up to kSerialRun such steps and the one after them (they need no bits, so the
+// state alone decides them): the log then holds one state for all of them, and its expansion walks
+// them again, 64 states at a time. Measured on the 256x384x384 float64 front field (0.3-0.4 bits a
+// symbol, 4 to 5 symbols a lookup): 39 ms (202 ms).
+constexpr uint32_t kSerialSlow = 1u << 14, kSerialEsc = 1u << 13;
+constexpr int kSerialHot = 4;            // contexts in LDS
+constexpr int kSerialRun = 7;            // steps without bits an entry stands for at most
+constexpr uint32_t kSerialGroup = 6;     // steps between refills of the bit buffer
+constexpr uint32_t kSerialLog = 1020;    // states a round logs at most
+constexpr uint32_t kSerialRing = 2048;   // words of bitstream in LDS: two rounds of 13 bits a step and more
+constexpr uint32_t kSerialSigns = 128;   // words of escape signs in LDS, likewise
+constexpr int kSerialThreads = 192;
+// Log values: the byte address of a state's entry in LDS, or one of these and (context << 13 | state) << 2
+// for an entry in device memory or a single step.
+constexpr uint32_t kLogCold = 1u << 22, kLogSingle = 1u << 23;
+
+// Which contexts of a segment are in LDS: perm(slot) for slots 0 .. 3, inv(context) its slot (4 and more:
+// not there). esc: contexts 13 and 14 are in slots 0 and 1.
+struct SerialMap {
+    uint64_t inv_nibbles;
+    uint32_t perm_bytes;
     uint32_t esc;
+    uint32_t run;  // steps without bits an entry takes in
+    uint32_t pad;
+    __host__ __device__ uint32_t inv(uint32_t c) const { return (uint32_t)(inv_nibbles >> (4 * c)) & 15u; }
+    __host__ __device__ uint32_t perm(uint32_t slot) const { return (perm_bytes >> (8 * slot)) & 255u; }
 };
-__device__ __forceinline__ uint32_t dense_entry(uint32_t raw, const DenseMap& dm) {
-    const uint32_t sy = (raw >> 16) & 0xFFu;
-    const uint32_t code = (sy >> 1) ^ (~(sy & 1u) + 1u);
-    const uint32_t ns = raw & ((1u << kO1Log) - 1);
-    const uint32_t r = dm.inv[raw >> 28];
-    const uint32_t low = r == 15u ? kDnEsc | (ns << 4)
-                                  : r < (uint32_t)kWalkCtxN ? (ns << 4) | (r << 2) : kDnSlow | (ns << 4) | (r - kWalkCtxN);
-    return low | ((code & 0x1FFu) << 22) | (((raw >> 24) & 15u) << 18);
-}
-
-// Dense-format copies of the tables of renumbered contexts 4..14 for each dense chain: grid
-// (chains, 11).
-// Cold table blockIdx.y of one chain: the entries of renumbered context kWalkCtxN + y, re-encoded.
-__device__ __forceinline__ void dense_cold_table(const DEntry* dt_seg, const DenseMap& dm, uint32_t* dtd_chain) {
-    const uint32_t* dt = reinterpret_cast<const uint32_t*>(dt_seg) + ((size_t)dm.perm[kWalkCtxN + blockIdx.y] << kO1Log);
-    uint32_t* o = dtd_chain + (size_t)blockIdx.y * (1u << kO1Log);
-    for (uint32_t i = threadIdx.x; i < (1u << kO1Log); i += blockDim.x) o[i] = dense_entry(dt[i], dm);
-}
-__global__ void __launch_bounds__(256) k_o1d_dense_tables(const O1DecChain* ch, const DEntry* dt_all,
-                                                          const DenseMap* maps, uint32_t* dtd) {
-    const O1DecChain c = ch[blockIdx.x];
-    const DenseMap dm = maps[blockIdx.x];
-    dense_cold_table(dt_all + c.dset * kO1Ctx * (1u << kO1Log), dm,
-                     dtd + (size_t)blockIdx.x * kWalkCtx0 * (1u << kO1Log));
-}
-
-// A sequential chain of any call, with the call's buffers: the batched decompress collects the
-// chains of many fields and decodes them in one launch (k_o1d_dense_jobs).
-struct DenseJob {
-    const uint8_t* in;   // the call's entropy stream (chain offsets count from here)
-    const DEntry* dt;    // the call's decoding tables, every segment
-    const int16_t* ovf;  // the call's escaped codes
-    int16_t* out;        // the call's codes
+struct SerialTables {   // one segment's tables to re-encode
+    const uint32_t* dt;
+    uint32_t* et;
+    SerialMap map;
+};
+struct SerialJob {
+    const uint8_t* cb;   // the chain's bytes
+    const uint32_t* dt;  // its segment's decoding tables
+    const uint32_t* et;  // the re-encoded ones, by context
+    const int16_t* ov;   // its escaped codes
+    int16_t* out;        // its codes
     int* err;
-    uint32_t* dtd;       // this chain's cold tables (kWalkCtx0 tables)
-    O1DecChain c;
-    DenseMap dm;
-};
-__global__ void __launch_bounds__(256) k_o1d_dense_tables_jobs(const DenseJob* jobs) {
-    const DenseJob& j = jobs[blockIdx.x];
-    const DenseMap dm = j.dm;
-    dense_cold_table(j.dt + j.c.dset * kO1Ctx * (1u << kO1Log), dm, j.dtd);
-}
-
-__device__ __forceinline__ uint32_t lds_u32(const FZ_LDS uint8_t* base, uint32_t off) {
-    return *reinterpret_cast<const FZ_LDS uint32_t*>(base + off);
-}
-
-// The state machine of seq_decode for dense chains (escaped values from vbuf, codes to obuf).
-// The bits below the read position sit in a 64-bit buffer refilled from the LDS window once per
-// four steps (four steps read at most 60 bits); each step is one LDS read and a dozen scalar
-// operations unless the next context's table is in device memory or the symbol is an escape.
-// The last steps before a window, output or escape limit run one by one with every check.
-// E is the entry of the current state on entry and on return.
-template <bool kEscInline>
-__device__ __forceinline__ uint64_t dense_decode(SeqState& S, uint32_t& E, const FZ_LDS uint8_t* win, int64_t wlo,
-                                                 int64_t until,
-                                                 uint64_t max_n, const FZ_LDS uint8_t* hotb, const uint32_t* dtd,
-                                                 const FZ_LDS int16_t* vbuf, uint64_t ve0, uint64_t ve1,
-                                                 uint64_t novf, FZ_LDS int16_t* obuf, uint32_t r13, uint32_t r14) {
-    const FZ_LDS uint32_t* w32 = reinterpret_cast<const FZ_LDS uint32_t*>(win);
-    const int64_t base = (wlo - kWinPad) * 8;
-    int32_t p = (int32_t)(S.B - base);
-    const bool raised = until < base + 32;
-    const int32_t lim = (int32_t)((raised ? base + 32 : until) - base);
-    uint64_t e = S.e;
-    const uint64_t elim = ve1 < novf ? ve1 : ~0ull;
-    const uint32_t kmax = (uint32_t)min<uint64_t>(max_n, 0x7FFFFFFFull);
-    uint32_t k = 0;
-    bool bad = S.bad, stop = false;
-    // the entry of the current state
-    auto fetch = [&](uint32_t X, uint32_t r) -> uint32_t {
-        return r < (uint32_t)kWalkCtxN ? lds_u32(hotb, (X << 4) | (r << 2))
-                                       : dtd[((size_t)(r - kWalkCtxN) << kO1Log) + X];
-    };
-    asm volatile("" : "+v"(E));
-    // The next escaped value and the renumbered context it leads to (r13 or r14 by its sign; an
-    // escaped code has magnitude 128 or more), read before an escape needs them. Past the side
-    // stream's end the value is 32767 (the escape is then an error).
-    auto esc_value = [&](uint64_t ei) -> int {
-        const uint64_t q = ei - ve0;
-        return ei < novf ? (int)vbuf[q < (uint64_t)kDenseOvf ? q : 0] : 32767;
-    };
-    auto ctx_term = [&](int v) -> uint32_t { return v < 0 ? r14 : r13; };
-    int nval = esc_value(e);
-    uint32_t nterm = ctx_term(nval);
-    uint64_t buf = 0;
-    int32_t prel = 0;
-    // bits [p - prel, p) of the window into buf (p >= 33 wherever this runs)
-    auto refill = [&]() {
-        const int32_t lo = max(p - 64, 0);
-        const int32_t j0 = lo >> 5;
-        const uint32_t w0 = w32[j0], w1 = w32[j0 + 1], w2 = w32[j0 + 2];
-        const uint32_t sh = (uint32_t)lo & 31u;
-        buf = (uint64_t)__builtin_amdgcn_alignbit(w1, w0, sh) | ((uint64_t)__builtin_amdgcn_alignbit(w2, w1, sh) << 32);
-        prel = p - lo;
-    };
-    // One step. The table entry, the bit buffer and the read position stay in vector registers (the
-    // values are the same in every lane): scalar arithmetic on them would put a lane-to-scalar move
-    // and its latency on the critical path of every step. Only the rare-path test reads E into a
-    // scalar register; escapes and entries whose next table is in device memory take that path.
-    // stop is set after the escape that reaches elim (in a group of four, which starts with
-    // e + 4 <= elim, only by its last step).
-    auto step = [&]() -> uint32_t {
-        const uint32_t nb = (E >> 18) & 15u;
-        prel -= (int32_t)nb;
-        const uint32_t bits = (uint32_t)(buf >> ((uint32_t)prel & 63u)) & ((1u << nb) - 1u);
-        int code = __builtin_amdgcn_sbfe((int)E, 22, 9);
-        // the next hot entry, read before the rare-path test (its address stays inside the tables
-        // for every entry)
-        uint32_t nx = lds_u32(hotb, (E & 0x1FFFFu) + (bits << 4));
-        const uint32_t Es = __builtin_amdgcn_readfirstlane(E);
-        if (__builtin_expect((Es & (kDnSlow | kDnEsc)) != 0, 0)) {
-            const uint32_t X = (((E >> 4) & ((1u << kO1Log) - 1)) + bits) & ((1u << kO1Log) - 1);
-            if (Es & kDnEsc) {
-                // the next entry is read before the following escaped value
-                if (e >= novf) bad = true;
-                code = nval;
-                nx = fetch(X, nterm);
-                e++;
-                if (e >= elim) stop = true;
-                nval = esc_value(e);
-                nterm = ctx_term(nval);
-            } else {
-                nx = dtd[((size_t)(Es & 15u) << kO1Log) + X];
-            }
-        }
-        E = nx;
-        asm volatile("" : "+v"(E));
-        return (uint32_t)code & 0xFFFFu;
-    };
-    // The step for escape-dense chains (r13 and r14 then in LDS): an escape is handled without a
-    // branch. The escaped values come from vbuf by a running index kept in a vector register, read
-    // one step ahead; the index is folded back into e after every group.
-    uint32_t vi = (uint32_t)(e - ve0);  // index into vbuf of the next escaped value
-    asm volatile("" : "+v"(vi));
-    auto step_esc = [&]() -> uint32_t {
-        const uint32_t nb = (E >> 18) & 15u;
-        prel -= (int32_t)nb;
-        const uint32_t bits = (uint32_t)(buf >> ((uint32_t)prel & 63u)) & ((1u << nb) - 1u);
-        const bool esc = (E & kDnEsc) != 0;
-        const int code = esc ? nval : __builtin_amdgcn_sbfe((int)E, 22, 9);
-        uint32_t nx = lds_u32(hotb, (E & 0x1FFFFu) + (bits << 4) + (esc ? nterm << 2 : 0u));
-        vi += esc ? 1u : 0u;
-        nval = (int)vbuf[min(vi, (uint32_t)kDnOvfLast)];
-        nterm = ctx_term(nval);
-        const uint32_t Es = __builtin_amdgcn_readfirstlane(E);
-        if (__builtin_expect((Es & kDnSlow) != 0, 0)) {
-            const uint32_t X = (((E >> 4) & ((1u << kO1Log) - 1)) + bits) & ((1u << kO1Log) - 1);
-            nx = dtd[((size_t)(Es & 15u) << kO1Log) + X];
-        }
-        E = nx;
-        asm volatile("" : "+v"(E));
-        return (uint32_t)code & 0xFFFFu;
-    };
-    // groups of four steps after one refill; g groups at a time stay clear of the window floor (a
-    // group reads at most 60 bits), the output limit and the escape limit
-    for (;;) {
-        uint32_t g = p > lim + 60 ? (uint32_t)((p - lim - 61) / 60 + 1) : 0u;
-        g = min(g, (kmax - k) / 4);
-        if (elim != ~0ull) g = (uint32_t)min<uint64_t>(g, (elim - e) / 4);
-        if (g == 0) break;
-        // k is a multiple of four here (groups start at 0 and take four codes each)
-        for (; g; g--) {
-            refill();
-            const int32_t lo = p - prel;
-            uint32_t c0, c1, c2, c3;
-            if constexpr (kEscInline) {
-                c0 = step_esc();
-                c1 = step_esc();
-                c2 = step_esc();
-                c3 = step_esc();
-                e = ve0 + __builtin_amdgcn_readfirstlane(vi);
-                stop = e >= elim;
-            } else {
-                c0 = step();
-                c1 = step();
-                c2 = step();
-                c3 = step();
-            }
-            *reinterpret_cast<FZ_LDS uint64_t*>(obuf + k) = (uint64_t)(c0 | (c1 << 16)) | ((uint64_t)(c2 | (c3 << 16)) << 32);
-            k += 4;
-            p = lo + prel;
-            if (stop) break;
-        }
-        if (stop) break;
-    }
-    if (kEscInline) {
-        // the values consumed in groups past the side stream's end: an error, as in the step
-        if (e > novf) bad = true;
-        nval = esc_value(e);
-        nterm = ctx_term(nval);
-    }
-    while (!stop && p > lim && k < kmax) {
-        refill();
-        const int32_t lo = p - prel;
-        obuf[k] = (int16_t)step();
-        k++;
-        p = lo + prel;
-    }
-    if (raised && p <= lim && k < kmax && !stop) bad = true;
-    S.B = base + p;
-    S.e = e;
-    S.bad = bad;
-    return k;
-}
-
-// A chain whose escapes are dense (the coarse levels of a tight bound) cannot be split: every few
-// dozen symbols the next context depends on an escape whose index in the side stream is unknown
-// to a decoder that starts mid-chain. One workgroup decodes such a chain from its start, every lane
-// running the same (wave-uniform) state machine: the tables of contexts 11-14, which hold most of
-// the symbols after large codes, a window of the bitstream, a window of the escaped values and a
-// buffer of decoded codes sit in LDS; the workgroup refills the windows and writes the codes out
-// between rounds.
-
-// Where the workgroup of a sequential chain of the batched decompress finds its chain, its segment's
-// tables, its renumbering, its cold tables and its call's buffers.
-struct DenseJobSrc {
-    const DenseJob* j;
-    __device__ O1DecChain chain() const { return j->c; }
-    __device__ const uint32_t* tables(const O1DecChain& c) const {
-        return reinterpret_cast<const uint32_t*>(j->dt + c.dset * kO1Ctx * (1u << kO1Log));
-    }
-    __device__ const uint32_t* cold() const { return j->dtd; }
-    __device__ DenseMap map() const { return j->dm; }
-    __device__ const uint8_t* in() const { return j->in; }
-    __device__ const int16_t* ovf() const { return j->ovf; }
-    __device__ int16_t* out() const { return j->out; }
-    __device__ int* err() const { return j->err; }
+    uint64_t* times;     // statistics: 100 MHz clock at its start and end (or null)
+    uint64_t m, novf;    // codes, escaped codes
+    int64_t pos0;        // read position after the initial state
+    uint32_t x0;         // initial state
+    uint32_t pad;
+    SerialMap map;
 };
 
-// One sequential chain, by the workgroup (the body of k_o1d_dense, its values from src).
-template <class Src>
-__device__ __forceinline__ void dense_chain(const Src& src) {
-    __shared__ uint32_t hot[kWalkCtxN << kO1Log];
-    __shared__ __align__(16) uint32_t stage32[(kDenseStage + kWinPad + 32) / 4 + 4];
-    uint8_t* stage = reinterpret_cast<uint8_t*>(stage32);
-    __shared__ __align__(16) int16_t obuf[kDenseOut];
-    __shared__ int16_t vbuf[kDenseOvf];
-    const O1DecChain c = src.chain();
-    const uint32_t* dt = src.tables(c);
-    const uint32_t* dtd = src.cold();
-    const DenseMap dm = src.map();
-    const uint8_t* in = src.in();
-    const int16_t* ovf = src.ovf();
-    int16_t* out = src.out();
-    int* err = src.err();
-    // interleaved by state: hot[X * 4 + r] holds (state X, renumbered context r)
-    for (uint32_t i = threadIdx.x; i < (kWalkCtxN << kO1Log); i += blockDim.x)
-        hot[i] = dense_entry(dt[((size_t)dm.perm[i & 3u] << kO1Log) + (i >> 2)], dm);
-    __syncthreads();
-    const uint8_t* cb = in + c.off;
-    const int16_t* ov = ovf + c.ovf_base;
-    const uint64_t m = c.hi - c.lo;
-    SeqState z{c.pos0, c.x0, 0, 0, false};
-    const bool esc_dense = dm.esc != 0;
-    const uint32_t r13 = dm.inv[13], r14 = dm.inv[14];
-    // the chain starts in context 0
-    const uint32_t r0 = dm.inv[0], x0 = c.x0 & ((1u << kO1Log) - 1);
-    uint32_t E = r0 < (uint32_t)kWalkCtxN ? hot[(x0 << 2) | r0] : dtd[((size_t)(r0 - kWalkCtxN) << kO1Log) + x0];
-    uint64_t i = 0;
-    while (i < m && !z.bad) {
-        const int64_t hi = min<int64_t>((int64_t)c.len, (z.B + 7) / 8 + 1);
-        const int64_t lo = max<int64_t>(0, hi - (int64_t)kDenseStage);
-        const uint64_t e0 = z.e, ve = min<uint64_t>(c.novf, e0 + kDenseOvf);
-        __syncthreads();
-        const int64_t w0 = stage_window(lds(stage), cb, (int64_t)c.len, lo, hi);
-        {
-            // the round's escaped values, eight loads per lane in flight at a time
-            const uint32_t nv = (uint32_t)(ve - e0);  // at most kDenseOvf
-            for (uint32_t k0 = 0; k0 < nv; k0 += blockDim.x * 8u) {
-                int16_t t[8];
+// grid (contexts, segments)
+__global__ void __launch_bounds__(256) k_o1d_tables(const SerialTables* tabs) {
+    const SerialTables& t = tabs[blockIdx.y];
+    const SerialMap dm = t.map;
+    const FZ_GLB uint32_t* dt = glb(t.dt);
+    for (uint32_t i = threadIdx.x; i < (1u << kO1Log); i += blockDim.x) {
+        uint32_t raw = dt[blockIdx.x << kO1Log | i];
+        for (uint32_t k = 0; k < dm.run && (raw >> 24) < 0xF0u && ((raw >> 24) & 15u) == 0; k++)
+            raw = dt[raw >> 28 << kO1Log | (raw & ((1u << kO1Log) - 1))];
+        const uint32_t nb = (raw >> 24) & 15u, ns = raw & ((1u << kO1Log) - 1), cx = raw >> 28;
+        uint32_t e = (31u - nb) | nb << 5 | ns << 16;
+        if (cx == 15u) e |= dm.esc ? kSerialEsc : kSerialSlow | 15u << 9;
+        else if (dm.inv(cx) < kSerialHot) e |= dm.inv(cx) << (16 + kO1Log);
+        else e |= kSerialSlow | cx << 9;
+        t.et[blockIdx.x << kO1Log | i] = e;
+    }
+}
+
+// `groups` times kSerialGroup lookups of wave 0 from the state cur (its entry is E): logs the states whose
+// entries it takes, moves the read position p down and counts the escapes in el. kEsc: escapes are taken
+// in the entries (SerialMap::esc). All values are the same in every lane; they stay in vector registers
+// except for the rare-path test, whose reads of E go to a scalar register under the lookup's latency.
+// Cycles a step on a synthetic table without rare entries (2.4 GHz): 76 for the lookup chain alone, 27
+// more with escapes, 25 with the rare-path test; a refill of the bit buffer every 4 steps costs 26 a step
+// and every 6 steps 17, the escape count kept as an end bit in the sign register (no add a step) saves 9.
+template <bool kEsc>
+__device__ __forceinline__ void serial_groups(uint32_t& E_, uint32_t& cur_, uint32_t& p_, uint32_t& el_, uint32_t groups,
+                                              const FZ_LDS uint32_t* hot, const FZ_LDS uint32_t* ring,
+                                              const FZ_LDS uint32_t* signs, FZ_LDS uint32_t* lg,
+                                              const FZ_GLB uint32_t* et, const SerialMap& dm) {
+    const FZ_LDS uint8_t* lh = reinterpret_cast<const FZ_LDS uint8_t*>(hot);
+    uint32_t E = E_, cur = cur_, p = p_, el = el_, sgn = 0, ess = 0;
+    asm volatile("" : "+v"(E), "+v"(cur), "+v"(p), "+v"(el));
+    uint32_t phase = 0;
+    for (uint32_t g = 0; g < groups; g++) {
+        // eighteen signs from bit 13 up and an end bit, enough for three groups; the end bit's place
+        // tells how many were taken
+        if (kEsc && phase == 0) {
+            el += g ? (uint32_t)__builtin_clz(sgn) : 0u;
+            const FZ_LDS uint32_t* sw = signs + ((el >> 5) & (kSerialSigns - 1));
+            sgn = __builtin_amdgcn_alignbit(sw[1], sw[0], el & 31u) << 13 | 1u << 31;
+            phase = 3;
+        }
+        phase--;
+        // the 96 bits below the read position: six steps read at most 78
+        const FZ_LDS uint32_t* w = ring + (((p - 96u) >> 5) & (kSerialRing - 1));
+        const uint32_t w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3], sh = p & 31u;
+        uint64_t buf = (uint64_t)__builtin_amdgcn_alignbit(w3, w2, sh) << 32 | __builtin_amdgcn_alignbit(w2, w1, sh);
+        const uint32_t rest = __builtin_amdgcn_alignbit(w1, w0, sh);
+        uint32_t w31 = (uint32_t)(buf >> 32) >> 1, sgn13 = kEsc ? sgn & kSerialEsc : 0u;
+        asm volatile("" : "+v"(w31), "+v"(sgn13));
+        uint32_t states[kSerialGroup];
+        uint32_t nbs = 0;
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint32_t k = k0 + (uint32_t)b * blockDim.x + threadIdx.x;
-                    t[b] = k < nv ? ov[e0 + k] : (int16_t)0;
+        for (int k = 0; k < (int)kSerialGroup; k++) {
+            // in issue order: the next lookup, what its latency hides, the rare path
+            states[k] = cur;
+            const uint32_t Es = __builtin_amdgcn_readfirstlane(E);
+            const uint32_t t = w31 >> (E & 31u);
+            const uint32_t base = E >> 16;
+            uint32_t at = (t + (kEsc ? (sgn13 & E) | base : base)) << 2;
+            uint32_t nx = *reinterpret_cast<const FZ_LDS uint32_t*>(lh + at);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t nb = (E >> 5) & 15u;
+            buf <<= nb;
+            nbs += nb;
+            if (k == 2) buf |= ((uint64_t)rest << 31) >> (63u - nbs);  // at most 39 bits have gone
+            w31 = (uint32_t)(buf >> 32) >> 1;
+            if (kEsc) {
+                sgn >>= (E >> 13) & 1u;
+                sgn13 = sgn & kSerialEsc;
+            }
+            // both ready before the lookup returns (they would be computed where they are used, after it)
+            asm volatile("" : "+v"(w31), "+v"(sgn13));
+            __builtin_amdgcn_sched_barrier(0);
+            if (__builtin_expect((Es & kSerialSlow) != 0, 0)) {
+                const uint32_t x = base + t;
+                uint32_t c2 = (Es >> 9) & 15u;
+                if (!kEsc && c2 == 15u) {  // an escape: its sign from the ring
+                    const uint32_t ei = uniform32(el + ess);
+                    c2 = 13u + (uniform32(signs[(ei >> 5) & (kSerialSigns - 1)] >> (ei & 31u)) & 1u);
+                    ess++;
+                    const uint32_t r = dm.inv(c2);
+                    if (r < (uint32_t)kSerialHot) {
+                        at = (r << kO1Log | x) << 2;
+                        nx = *reinterpret_cast<const FZ_LDS uint32_t*>(lh + at);
+                        c2 = 15u;
+                    }
                 }
+                if (kEsc || c2 != 15u) {
+                    at = kLogCold | (c2 << kO1Log | x) << 2;
+                    nx = (et + (c2 << kO1Log))[x];
+                }
+            }
+            cur = at;
+            E = nx;
+        }
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint32_t k = k0 + (uint32_t)b * blockDim.x + threadIdx.x;
-                    if (k < nv) vbuf[k] = t[b];
+        for (int k = 0; k < (int)kSerialGroup; k += 2)
+            *reinterpret_cast<FZ_LDS u32x2*>(lg + kSerialGroup * g + k) = u32x2{states[k], states[k + 1]};
+        p -= nbs;
+    }
+    E_ = E;
+    cur_ = cur;
+    p_ = p;
+    el_ = kEsc ? el + (uint32_t)__builtin_clz(sgn) : el + ess;
+}
+
+__global__ void __launch_bounds__(kSerialThreads) k_o1d_serial(const SerialJob* jobs) {
+    __shared__ uint32_t hot[kSerialHot << kO1Log];
+    __shared__ uint32_t ring[kSerialRing + 3];     // word j of the chain at j mod kSerialRing; the first three again at the end
+    __shared__ uint32_t signs[kSerialSigns + 1];   // signs of escapes 32 w .. 32 w + 31 at w mod kSerialSigns; likewise
+    __shared__ __align__(16) uint32_t log[2][kSerialLog + 4];
+    // written by one wave for the others' next round, by the round's parity
+    __shared__ uint32_t sh_n[2], sh_fin[2];
+    __shared__ uint64_t sh_e[2], sh_done[2];
+    __shared__ int64_t sh_a[2];
+    const SerialJob& J = jobs[blockIdx.x];
+    const uint32_t tid = threadIdx.x, l = tid & 63u, wv = tid >> 6;
+    if (J.times && tid == 0) J.times[0] = __builtin_amdgcn_s_memrealtime();
+    const SerialMap dm = J.map;
+    const uint64_t m = J.m, novf = J.novf;
+    const FZ_GLB uint32_t* dt = glb(J.dt);
+    const FZ_GLB uint32_t* et = glb(J.et);
+    const FZ_GLB int16_t* ov = glb(J.ov);
+    const ChainWords cw(J.cb);
+    const uint32_t maxc = dm.run + 1;
+    {
+        u32x4* h = reinterpret_cast<u32x4*>(hot);
+        for (uint32_t i = tid; i < (uint32_t)kSerialHot << (kO1Log - 2); i += kSerialThreads)
+            h[i] = *reinterpret_cast<const FZ_GLB u32x4*>(et + (dm.perm(i >> (kO1Log - 2)) << kO1Log) +
+                                                          4 * (i & ((1u << (kO1Log - 2)) - 1)));
+    }
+    // stages words [lo, hi) by n lanes of which this is the i-th
+    auto stage_words = [&](int64_t lo, int64_t hi, uint32_t i, uint32_t n) {
+        for (int64_t j0 = lo; j0 < hi; j0 += 4 * (int64_t)n) {
+            uint32_t v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int64_t j = j0 + q * (int64_t)n + i;
+                v[q] = j < hi ? cw.word(j) : 0u;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int64_t j = j0 + q * (int64_t)n + i;
+                const uint32_t r = (uint32_t)j & (kSerialRing - 1);
+                if (j < hi) {
+                    ring[r] = v[q];
+                    if (r < 3) ring[kSerialRing + r] = v[q];
                 }
             }
         }
-        __syncthreads();
-        const int64_t floor_bits = lo == 0 ? INT64_MIN : lo * 8 + 64;
-        const uint64_t nk =
-            esc_dense ? dense_decode<true>(z, E, lds(stage), w0 + kWinPad, floor_bits, min<uint64_t>(m - i, kDenseOut),
-                                           lds(reinterpret_cast<const uint8_t*>(hot)), dtd, lds(vbuf), e0, ve, c.novf,
-                                           lds(obuf), r13, r14)
-                      : dense_decode<false>(z, E, lds(stage), w0 + kWinPad, floor_bits, min<uint64_t>(m - i, kDenseOut),
-                                            lds(reinterpret_cast<const uint8_t*>(hot)), dtd, lds(vbuf), e0, ve, c.novf,
-                                            lds(obuf), r13, r14);
-        __syncthreads();
-        for (uint64_t k = threadIdx.x; k < nk; k += blockDim.x) out[c.lo + i + k] = obuf[k];
-        i += nk;
-    }
-    if (threadIdx.x == 0 && (z.bad || i != m || z.e != c.novf)) *err = 1;
-}
-
-// The chains of one call. Its body is dense_chain's, written out: as a call of the template the
-// compiler allocates this kernel's registers differently, and it measured 1% slower (192.3-192.6 ms
-// against 193.8-194.8 ms a launch on the 512^3 field, the same box).
-__global__ void __launch_bounds__(kSeqLanes) k_o1d_dense(const uint8_t* in, const O1DecChain* ch, const DEntry* dt_all,
-                                                         const DenseMap* maps, const uint32_t* dtd_all,
-                                                         const int16_t* ovf, int16_t* out, int* err,
-                                                         uint64_t* times) {
-    // times (statistics only, else null): the 100 MHz clock at the chain's start and end
-    if (times && threadIdx.x == 0) times[2 * blockIdx.x] = __builtin_amdgcn_s_memrealtime();
-    __shared__ uint32_t hot[kWalkCtxN << kO1Log];
-    __shared__ __align__(16) uint32_t stage32[(kDenseStage + kWinPad + 32) / 4 + 4];
-    uint8_t* stage = reinterpret_cast<uint8_t*>(stage32);
-    __shared__ __align__(16) int16_t obuf[kDenseOut];
-    __shared__ int16_t vbuf[kDenseOvf];
-    const O1DecChain c = ch[blockIdx.x];
-    const uint32_t* dt = reinterpret_cast<const uint32_t*>(dt_all + c.dset * kO1Ctx * (1u << kO1Log));
-    const uint32_t* dtd = dtd_all + (size_t)blockIdx.x * kWalkCtx0 * (1u << kO1Log);
-    const DenseMap dm = maps[blockIdx.x];
-    // interleaved by state: hot[X * 4 + r] holds (state X, renumbered context r)
-    for (uint32_t i = threadIdx.x; i < (kWalkCtxN << kO1Log); i += blockDim.x)
-        hot[i] = dense_entry(dt[((size_t)dm.perm[i & 3u] << kO1Log) + (i >> 2)], dm);
-    __syncthreads();
-    const uint8_t* cb = in + c.off;
-    const int16_t* ov = ovf + c.ovf_base;
-    const uint64_t m = c.hi - c.lo;
-    SeqState z{c.pos0, c.x0, 0, 0, false};
-    const bool esc_dense = dm.esc != 0;
-    const uint32_t r13 = dm.inv[13], r14 = dm.inv[14];
-    // the chain starts in context 0
-    const uint32_t r0 = dm.inv[0], x0 = c.x0 & ((1u << kO1Log) - 1);
-    uint32_t E = r0 < (uint32_t)kWalkCtxN ? hot[(x0 << 2) | r0] : dtd[((size_t)(r0 - kWalkCtxN) << kO1Log) + x0];
-    uint64_t i = 0;
-    while (i < m && !z.bad) {
-        const int64_t hi = min<int64_t>((int64_t)c.len, (z.B + 7) / 8 + 1);
-        const int64_t lo = max<int64_t>(0, hi - (int64_t)kDenseStage);
-        const uint64_t e0 = z.e, ve = min<uint64_t>(c.novf, e0 + kDenseOvf);
-        __syncthreads();
-        const int64_t w0 = stage_window(lds(stage), cb, (int64_t)c.len, lo, hi);
-        {
-            // the round's escaped values, eight loads per lane in flight at a time
-            const uint32_t nv = (uint32_t)(ve - e0);  // at most kDenseOvf
-            for (uint32_t k0 = 0; k0 < nv; k0 += blockDim.x * 8u) {
-                int16_t t[8];
+    };
+    // stages the signs of escapes [from, to), multiples of 64, by one wave
+    auto stage_signs = [&](uint64_t from, uint64_t to) {
+        for (uint64_t e = from; e < to; e += 256) {
+            int v[4];
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint32_t k = k0 + (uint32_t)b * blockDim.x + threadIdx.x;
-                    t[b] = k < nv ? ov[e0 + k] : (int16_t)0;
-                }
+            for (int q = 0; q < 4; q++) {
+                const uint64_t k = e + 64 * q + l;
+                v[q] = k < novf ? (int)ov[k] : 0;
+            }
 #pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint32_t k = k0 + (uint32_t)b * blockDim.x + threadIdx.x;
-                    if (k < nv) vbuf[k] = t[b];
+            for (int q = 0; q < 4; q++) {
+                const uint64_t mk = __ballot(v[q] < 0);
+                const uint32_t w = (uint32_t)((e + 64 * q) >> 5) & (kSerialSigns - 1);
+                if (l < 2 && e + 64 * q < to) {
+                    signs[w + l] = (uint32_t)(mk >> (32 * l));
+                    if (w + l == 0) signs[kSerialSigns] = (uint32_t)mk;
                 }
             }
         }
-        __syncthreads();
-        const int64_t floor_bits = lo == 0 ? INT64_MIN : lo * 8 + 64;
-        const uint64_t nk =
-            esc_dense ? dense_decode<true>(z, E, lds(stage), w0 + kWinPad, floor_bits, min<uint64_t>(m - i, kDenseOut),
-                                           lds(reinterpret_cast<const uint8_t*>(hot)), dtd, lds(vbuf), e0, ve, c.novf,
-                                           lds(obuf), r13, r14)
-                      : dense_decode<false>(z, E, lds(stage), w0 + kWinPad, floor_bits, min<uint64_t>(m - i, kDenseOut),
-                                            lds(reinterpret_cast<const uint8_t*>(hot)), dtd, lds(vbuf), e0, ve, c.novf,
-                                            lds(obuf), r13, r14);
-        __syncthreads();
-        for (uint64_t k = threadIdx.x; k < nk; k += blockDim.x) out[c.lo + i + k] = obuf[k];
-        i += nk;
+    };
+    // read positions count from the aligned word that holds the chain's first byte
+    constexpr int64_t kRoundBits = 13 * (int64_t)(kSerialLog + 4);
+    const int64_t a0 = J.pos0 + cw.shift;
+    auto words_for = [&](int64_t a) { return (a - 2 * kRoundBits - 128) >> 5; };
+    int64_t staged = words_for(a0);  // words from here up are in the ring
+    uint64_t esigns = 4 * 1024 - 64 * 4;
+    stage_words(staged, (a0 + 31) >> 5, tid, kSerialThreads);
+    if (wv == 2) stage_signs(0, esigns);
+    if (tid == 0) {
+        sh_n[0] = sh_n[1] = 0;
+        sh_fin[0] = sh_fin[1] = 0;
+        sh_a[0] = a0;
+        sh_e[0] = 0;
+        sh_done[0] = 0;
     }
-    if (threadIdx.x == 0 && (z.bad || i != m || z.e != c.novf)) *err = 1;
-    if (times && threadIdx.x == 0) times[2 * blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime();
+    // wave 0
+    int64_t a = a0;
+    uint64_t e = 0, steps = 0;        // escapes, entries taken
+    uint32_t before = 0;              // entries of the round that is being expanded
+    uint32_t cx = 0, X = J.x0 & ((1u << kO1Log) - 1);  // state, where it is not in cur
+    uint32_t cur = 0, E = 0;          // log value of the current state, its entry
+    bool have = false;                // cur and E hold the state
+    // wave 1
+    uint64_t done = 0, eo = 0;
+    bool bad = false;
+    __syncthreads();
+    for (uint32_t round = 0;; round++) {
+        const uint32_t par = round & 1u;
+        if (wv == 0) {
+            if (!uniform32(sh_fin[par])) {
+                // symbols left for certain: those not expanded yet count as many as they can be
+                const uint64_t known = uniform64(sh_done[par]);
+                const uint64_t used = known + (uint64_t)maxc * before;
+                const uint64_t left = maxc == 1 ? m - steps : used < m ? m - used : 0;
+                const uint32_t groups = (uint32_t)min<uint64_t>(kSerialLog / kSerialGroup, left / (kSerialGroup * maxc));
+                FZ_LDS uint32_t* lg = lds(log[par]);
+                uint32_t n = 0;
+                bool fin = false;
+                if (groups) {
+                    if (!have) {
+                        const uint32_t r = dm.inv(cx);
+                        cur = r < (uint32_t)kSerialHot ? (r << kO1Log | X) << 2 : kLogCold | (cx << kO1Log | X) << 2;
+                        E = et[cx << kO1Log | X];
+                        have = true;
+                    }
+                    uint32_t p = (uint32_t)a;  // wraps: only its place in the ring matters
+                    uint32_t el = (uint32_t)e;
+                    if (dm.esc) serial_groups<true>(E, cur, p, el, groups, lds(hot), lds(ring), lds(signs), lg, et, dm);
+                    else serial_groups<false>(E, cur, p, el, groups, lds(hot), lds(ring), lds(signs), lg, et, dm);
+                    n = kSerialGroup * groups;
+                    a -= (int64_t)uniform32((uint32_t)a - p);
+                    e += uniform32(el - (uint32_t)e);
+                } else if (before == 0 || maxc == 1) {
+                    // the last few symbols, one step at a time
+                    const uint32_t rest = (uint32_t)(maxc == 1 ? m - steps : known < m ? m - known : 0);
+                    if (have) {
+                        const uint32_t c = uniform32(cur);
+                        cx = c & kLogCold ? (c >> (kO1Log + 2)) & 15u : dm.perm(c >> (kO1Log + 2));
+                        X = (c >> 2) & ((1u << kO1Log) - 1);
+                    }
+                    for (; n < rest; n++) {
+                        const uint32_t raw = uniform32(dt[cx << kO1Log | X]);
+                        lg[n] = kLogSingle | (cx << kO1Log | X) << 2;
+                        const uint32_t nb = (raw >> 24) & 15u;
+                        a -= nb;
+                        const FZ_LDS uint32_t* w = lds(ring) + ((uint32_t)(a >> 5) & (kSerialRing - 1));
+                        const uint32_t bits = __builtin_amdgcn_alignbit(w[1], w[0], (uint32_t)a & 31u) & ((1u << nb) - 1u);
+                        X = uniform32((raw + bits) & ((1u << kO1Log) - 1));
+                        cx = raw >> 28;
+                        if (cx == 15u) {
+                            cx = 13u + uniform32((lds(signs)[(uint32_t)(e >> 5) & (kSerialSigns - 1)] >> (e & 31u)) & 1u);
+                            e++;
+                        }
+                    }
+                    fin = true;
+                }
+                steps += n;
+                before = n;
+                if (l == 0) {
+                    sh_n[par] = n;
+                    sh_fin[par ^ 1u] = fin;
+                    sh_a[par ^ 1u] = a;
+                    sh_e[par ^ 1u] = e;
+                }
+            } else if (l == 0) {
+                sh_n[par] = 0;
+                sh_fin[par ^ 1u] = 2;
+            }
+        } else if (wv == 1) {
+            // expands the round before
+            const uint32_t n = uniform32(sh_n[par ^ 1u]);
+            const FZ_LDS uint32_t* lg = lds(log[par ^ 1u]);
+            FZ_GLB int16_t* out = glb(J.out);
+            constexpr int kB = 4;  // states a lane at a time, their table reads in flight together
+            for (uint32_t i0 = 0; i0 < n; i0 += 64 * kB) {
+                uint32_t raw[kB], last[kB];
+                uint8_t cnt[kB], single[kB];
+#pragma unroll
+                for (int q = 0; q < kB; q++) {
+                    const uint32_t i = i0 + 64u * q + l;
+                    const uint32_t v = i < n ? lg[i] : 0u;
+                    const uint32_t c = v >= kLogCold ? (v >> (kO1Log + 2)) & 15u : dm.perm(v >> (kO1Log + 2));
+                    raw[q] = dt[c << kO1Log | ((v >> 2) & ((1u << kO1Log) - 1))];
+                    cnt[q] = i < n;
+                    single[q] = i >= n || (v & kLogSingle);
+                }
+                // the symbol an entry ends with, and how many come before it
+#pragma unroll
+                for (int q = 0; q < kB; q++) last[q] = raw[q];
+                for (uint32_t k = 0; k < dm.run; k++) {
+                    bool walk = false;
+#pragma unroll
+                    for (int q = 0; q < kB; q++) {
+                        if (cnt[q] == k + 1 && !single[q] && (last[q] >> 24) < 0xF0u && ((last[q] >> 24) & 15u) == 0) {
+                            last[q] = dt[last[q] >> 28 << kO1Log | (last[q] & ((1u << kO1Log) - 1))];
+                            cnt[q]++;
+                            walk = true;
+                        }
+                    }
+                    if (!__ballot(walk)) break;
+                }
+                // places: counts and escapes of the states before; escaped values
+                uint64_t at[kB];
+                int code[kB];
+#pragma unroll
+                for (int q = 0; q < kB; q++) {
+                    uint32_t pre = cnt[q];
+                    if (dm.run) {
+#pragma unroll
+                        for (int d = 1; d < 64; d <<= 1) {
+                            const uint32_t o = __shfl_up(pre, d);
+                            if (l >= (uint32_t)d) pre += o;
+                        }
+                        at[q] = done + pre - cnt[q];
+                        done += uniform32(__shfl(pre, 63));
+                    } else {
+                        at[q] = done + l;
+                        done += (uint32_t)__popcll(__ballot(cnt[q] != 0));
+                    }
+                    const uint32_t sy = (last[q] >> 16) & 0xFFu;
+                    code[q] = (int)((sy >> 1) ^ (~(sy & 1) + 1));
+                    const bool esc = cnt[q] && last[q] >> 28 == 15u;
+                    const uint64_t em = __ballot(esc);
+                    if (esc) {
+                        const uint64_t ei = eo + (uint32_t)__popcll(em & ((1ull << l) - 1));
+                        code[q] = ei < novf ? (int)ov[ei] : 32767;
+                        bad = bad || ei >= novf;
+                    }
+                    eo += (uint32_t)__popcll(em);
+                }
+#pragma unroll
+                for (int q = 0; q < kB; q++) {
+                    if (cnt[q] && at[q] + cnt[q] <= m) {
+                        uint32_t rw = raw[q];
+                        for (uint32_t k = 1; k < cnt[q]; k++) {
+                            const uint32_t sy = (rw >> 16) & 0xFFu;
+                            out[at[q]++] = (int16_t)((sy >> 1) ^ (~(sy & 1) + 1));
+                            rw = dt[rw >> 28 << kO1Log | (rw & ((1u << kO1Log) - 1))];
+                        }
+                        out[at[q]] = (int16_t)code[q];
+                    } else if (cnt[q]) {
+                        bad = true;
+                    }
+                }
+            }
+            if (l == 0) sh_done[par ^ 1u] = done;
+        } else {
+            // two rounds ahead of where wave 0 was when this one began
+            const int64_t lo = words_for(uniform64((uint64_t)sh_a[par]));
+            if (lo < staged) {
+                stage_words(lo, staged, l, 64);
+                staged = lo;
+            }
+            const uint64_t to = (uniform64(sh_e[par]) + 2 * (kSerialLog + 4) + 64 + 63) & ~63ull;
+            if (to > esigns) {
+                stage_signs(esigns, to);
+                esigns = to;
+            }
+        }
+        __syncthreads();
+        // the round in which wave 0 had nothing left has expanded the last log; a stream that ran far
+        // below its first bit is corrupt
+        if (sh_fin[par ^ 1u] == 2) break;
+        if (sh_a[par ^ 1u] < -128) {
+            bad = true;
+            break;
+        }
+    }
+    if (wv == 1) {
+        bad = bad || done != m || eo != novf;
+        if (__ballot(bad) && l == 0) *J.err = 1;
+    } else if (wv == 0 && l == 0 && bad) {
+        *J.err = 1;
+    }
+    if (J.times && tid == 0) J.times[1] = __builtin_amdgcn_s_memrealtime();
 }
-
-// The chains of many calls (the batched decompress), one workgroup a chain.
-__global__ void __launch_bounds__(kSeqLanes) k_o1d_dense_jobs(const DenseJob* jobs) {
-    dense_chain(DenseJobSrc{jobs + blockIdx.x});
-}
-
 
 // ---------------------------------------------------------------- method 0 decode
 __device__ inline uint64_t get_msb_field(const uint8_t* buf, uint64_t off, int k) {
@@ -3559,6 +3572,8 @@ static void fse_dec_multi(const std::vector<FseDecItem>& items, int* err, DevAre
 // ever meet), are decoded from their start.
 constexpr uint64_t kSplitMinSymbols = 8192;
 constexpr double kSplitMinBits = 2.5;
+// Sequential chains of fewer take several steps a lookup (kSerialRun).
+constexpr double kSerialRunBits = 2.0;
 // In the batched decompress, so are chains of at most this many: many fields' sequential chains run
 // side by side in one launch.
 constexpr uint64_t kDeferSymbols = 1ull << 19;
@@ -3616,34 +3631,32 @@ static uint32_t hot_window(const double pi[kO1Ctx]) {
     return best;
 }
 
-// The renumbering of the contexts of a dense chain in segment g: contexts by their share under the
-// stationary distribution of the segment's context chain, the four largest first; with esc set,
-// 13 and 14 are among the four.
-static DenseMap dense_map(const uint8_t* host, uint64_t nf_off, bool esc) {
-    double pi[kO1Ctx];
-    context_shares(host, nf_off, pi);
+// The contexts of a segment's sequential chains that are kept in LDS: the largest by share, with both
+// that follow an escape first where escapes are frequent (or where they are among the largest anyway).
+static SerialMap serial_map(const double pi[kO1Ctx], double escapes, double bits) {
     int order[kO1Ctx];
     for (int a = 0; a < kO1Ctx; a++) order[a] = a;
-    std::stable_sort(order, order + kO1Ctx, [&](int x, int y) {
-        const bool fx = esc && (x == 13 || x == 14), fy = esc && (y == 13 || y == 14);
-        if (fx != fy) return fx;
-        return pi[x] > pi[y];
-    });
-    DenseMap dm{};
+    std::stable_sort(order, order + kO1Ctx, [&](int x, int y) { return pi[x] > pi[y]; });
+    auto rank = [&](int c) { return (int)(std::find(order, order + kO1Ctx, c) - order); };
+    SerialMap m{};
+    m.esc = escapes > 1.0 / 64 || (rank(13) < kSerialHot && rank(14) < kSerialHot);
+    if (m.esc)
+        std::stable_sort(order, order + kO1Ctx, [&](int x, int y) {
+            return (x >= 13 ? x - 13 : 2) < (y >= 13 ? y - 13 : 2);
+        });
     for (int r = 0; r < kO1Ctx; r++) {
-        dm.perm[r] = (uint8_t)order[r];
-        dm.inv[order[r]] = (uint8_t)r;
+        m.inv_nibbles |= (uint64_t)r << (4 * order[r]);
+        if (r < kSerialHot) m.perm_bytes |= (uint32_t)order[r] << (8 * r);
     }
-    dm.inv[15] = 15;
-    dm.perm[15] = 15;
-    dm.esc = esc ? 1u : 0u;
-    return dm;
+    m.run = bits < kSerialRunBits ? kSerialRun : 0;
+    return m;
 }
 
 // Sequential chains of several calls, decoded together (dense_batch_run).
 struct DenseBatch {
     std::mutex mu;
-    std::vector<DenseJob> jobs;
+    std::vector<SerialJob> jobs;
+    std::vector<SerialTables> tabs;
     uint64_t bytes = 0, codes = 0;
 };
 DenseBatch* dense_batch_create() { return new DenseBatch; }
@@ -3655,24 +3668,31 @@ size_t dense_batch_size(DenseBatch* b) {
 void dense_batch_clear(DenseBatch* b) {
     std::lock_guard<std::mutex> g(b->mu);
     b->jobs.clear();
+    b->tabs.clear();
     b->bytes = b->codes = 0;
+}
+// Re-encodes the tables and decodes the chains of the lists on st; djobs and dtabs have room for them.
+static void launch_serial(std::vector<SerialJob>& jobs, const std::vector<SerialTables>& tabs, SerialJob* djobs,
+                          SerialTables* dtabs, uint64_t bytes, uint64_t codes, hipStream_t st) {
+    FZ_LAUNCH("o1_serial_tables", 0, k_o1d_tables, dim3(kO1Ctx, (unsigned)tabs.size()), dim3(256), 0, st, dtabs);
+    FZ_LAUNCH("o1_decode_serial", bytes + codes * 2, k_o1d_serial, dim3((unsigned)jobs.size()), dim3(kSerialThreads), 0, st,
+              djobs);
+    FZ_HIP(hipGetLastError());
 }
 void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st) {
     std::lock_guard<std::mutex> g(b->mu);
     const size_t n = b->jobs.size();
     if (!n) return;
     if (n > 0x7fffffffu) throw std::length_error("too many sequential chains for one launch");
+    if (b->tabs.size() > 65535u) throw std::length_error("too many sequential segments for one launch");
     // longest chains first, so that the last workgroups to start are short ones
-    std::stable_sort(b->jobs.begin(), b->jobs.end(),
-                     [](const DenseJob& x, const DenseJob& y) { return x.c.hi - x.c.lo > y.c.hi - y.c.lo; });
-    DenseJob* dj = ws.take<DenseJob>(n);
-    // the job list stays in b until dense_batch_clear, after the launches have finished
-    FZ_HIP(hipMemcpyAsync(dj, b->jobs.data(), n * sizeof(DenseJob), hipMemcpyHostToDevice, st));
-    FZ_LAUNCH("o1_decode_dense_tables", 0, k_o1d_dense_tables_jobs, dim3((unsigned)n, (unsigned)kWalkCtx0), dim3(256), 0,
-              st, dj);
-    FZ_LAUNCH("o1_decode_dense", b->bytes + b->codes * 2, k_o1d_dense_jobs, dim3((unsigned)n), dim3(kSeqLanes), 0, st,
-              dj);
-    FZ_HIP(hipGetLastError());
+    std::stable_sort(b->jobs.begin(), b->jobs.end(), [](const SerialJob& x, const SerialJob& y) { return x.m > y.m; });
+    SerialJob* dj = ws.take<SerialJob>(n);
+    SerialTables* dtab = ws.take<SerialTables>(b->tabs.size());
+    // the lists stay in b until dense_batch_clear, after the launches have finished
+    h2d(dj, b->jobs.data(), n, st);
+    h2d(dtab, b->tabs.data(), b->tabs.size(), st);
+    launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, st);
 }
 
 // How a chain is decoded: from its start by one workgroup (k_o1d_dense), or split into parts. The
@@ -3744,7 +3764,8 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
                                int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer) {
     const int nch = (int)(chains.size() / 7);
     std::vector<O1Split> hc;
-    std::vector<O1DecChain> hd;
+    std::vector<SerialJob> hd;
+    std::vector<uint64_t> hd_seg;
     std::vector<SplitPlan> plans;
     std::vector<uint64_t> seg_of, novf_of;
     uint64_t dense_bytes = 0, dense_codes = 0, stream_bytes = 0, ncodes = 0;
@@ -3777,7 +3798,18 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         SplitPlan sp;
         if (!all_seq && !(defer && m <= kDeferSymbols)) sp = split_plan(m, c[6], bits, pi, host + nf_off[c[5]], keep_short);
         if (sp.cls == kSplitNone) {
-            hd.push_back(O1DecChain{c[0], c[1], c[2], c[3], c[4], c[6], c[5], pos0, x0, 0});
+            SerialJob k{};
+            k.cb = dev + c[0];
+            k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
+            k.ov = ovf + c[4];
+            k.out = out + c[2];
+            k.err = err;
+            k.m = m;
+            k.novf = c[6];
+            k.pos0 = pos0;
+            k.x0 = x0;
+            hd.push_back(k);
+            hd_seg.push_back(c[5]);
             dense_bytes += c[1];
             dense_codes += m;
             continue;
@@ -3813,38 +3845,46 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     hipStream_t dst = aux.stream ? aux.stream : st;
     const bool stats_on = getenv("FALCONS_DECODE_STATS") != nullptr;
     uint64_t* dense_times = nullptr;  // per sequential chain: clock at start and end (statistics only)
-    std::vector<DenseMap> maps;  // read by a copy in flight until the function returns
+    std::vector<SerialTables> tabs;   // one a segment; read by copies in flight until the function returns
+    if (!hd.empty()) {
+        for (size_t q = 0; q < hd.size();) {
+            size_t q1 = q;
+            double sm = 0, se = 0, sb = 0;
+            for (; q1 < hd.size() && hd_seg[q1] == hd_seg[q]; q1++) {
+                sm += (double)hd[q1].m;
+                se += (double)hd[q1].novf;
+                sb += (double)std::max<int64_t>(hd[q1].pos0, 0);
+            }
+            context_shares(host, nf_off[hd_seg[q]], pi);
+            SerialTables t{hd[q].dt, ws.take<uint32_t>((size_t)kO1Ctx << kO1Log), serial_map(pi, se / sm, sb / sm)};
+            for (; q < q1; q++) {
+                hd[q].et = t.et;
+                hd[q].map = t.map;
+            }
+            tabs.push_back(t);
+        }
+        if (stats_on && !defer) {
+            dense_times = ws.take<uint64_t>(2 * hd.size());
+            for (size_t q = 0; q < hd.size(); q++) hd[q].times = dense_times + 2 * q;
+        }
+    }
     if (!hd.empty() && defer) {
-        uint32_t* dtd = ws.take<uint32_t>(hd.size() * kWalkCtx0 * (1u << kO1Log));
-        std::vector<DenseJob> jobs(hd.size());
-        for (size_t q = 0; q < hd.size(); q++)
-            jobs[q] = DenseJob{dev, dt, ovf, out, err, dtd + q * kWalkCtx0 * (1u << kO1Log), hd[q],
-                               dense_map(host, nf_off[hd[q].dset], hd[q].novf * 16 > hd[q].hi - hd[q].lo)};
         std::lock_guard<std::mutex> g(defer->mu);
-        defer->jobs.insert(defer->jobs.end(), jobs.begin(), jobs.end());
+        defer->jobs.insert(defer->jobs.end(), hd.begin(), hd.end());
+        defer->tabs.insert(defer->tabs.end(), tabs.begin(), tabs.end());
         defer->bytes += dense_bytes;
         defer->codes += dense_codes;
     } else if (!hd.empty()) {
-        O1DecChain* ddc = ws.take<O1DecChain>(hd.size());
-        h2d(ddc, hd.data(), hd.size(), st);
-        // more than one escape in 16 symbols: the escape-dense step
-        maps.resize(hd.size());
-        for (size_t q = 0; q < hd.size(); q++)
-            maps[q] = dense_map(host, nf_off[hd[q].dset], hd[q].novf * 16 > hd[q].hi - hd[q].lo);
-        DenseMap* dmaps = ws.take<DenseMap>(hd.size());
-        h2d(dmaps, maps.data(), maps.size(), st);
+        SerialJob* dj = ws.take<SerialJob>(hd.size());
+        SerialTables* dtab = ws.take<SerialTables>(tabs.size());
+        h2d(dj, hd.data(), hd.size(), st);
+        h2d(dtab, tabs.data(), tabs.size(), st);
         // the second stream starts after every copy above
         if (aux.stream) {
             FZ_HIP(hipEventRecord(aux.fork, st));
             FZ_HIP(hipStreamWaitEvent(aux.stream, aux.fork, 0));
         }
-        uint32_t* dtd = ws.take<uint32_t>(hd.size() * kWalkCtx0 * (1u << kO1Log));
-        FZ_LAUNCH("o1_decode_dense_tables", 0, k_o1d_dense_tables, dim3((unsigned)hd.size(), (unsigned)kWalkCtx0),
-                  dim3(256), 0, dst, ddc, dt, dmaps, dtd);
-        if (stats_on) dense_times = ws.take<uint64_t>(2 * hd.size());
-        FZ_LAUNCH("o1_decode_dense", dense_bytes + dense_codes * 2, k_o1d_dense, dim3((unsigned)hd.size()), dim3(kSeqLanes), 0,
-                  dst, dev, ddc, dt, dmaps, dtd, ovf, out, err, dense_times);
-        FZ_HIP(hipGetLastError());
+        launch_serial(hd, tabs, dj, dtab, dense_bytes, dense_codes, dst);
     }
     struct Join {  // the caller's stream waits for the dense chains however this function exits
         const AuxStream& a;
@@ -3931,9 +3971,9 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
                     sc[q].hot0);
         fprintf(stderr, "\n");
         fprintf(stderr, "[o1 decode] %zu chains decoded from their start:", hd.size());
-        for (const O1DecChain& c : hd)
-            fprintf(stderr, " b%.2f/s%llu/esc%llu", (double)c.pos0 / (double)std::max<uint64_t>(1, c.hi - c.lo),
-                    (unsigned long long)c.dset, (unsigned long long)c.novf);
+        for (size_t q = 0; q < hd.size(); q++)
+            fprintf(stderr, " b%.2f/s%llu/esc%llu", (double)hd[q].pos0 / (double)std::max<uint64_t>(1, hd[q].m),
+                    (unsigned long long)hd_seg[q], (unsigned long long)hd[q].novf);
         fprintf(stderr, "\n");
         if (dense_times) {
             FZ_HIP(hipStreamSynchronize(dst));
@@ -3943,10 +3983,10 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             for (size_t q = 0; q < hd.size(); q++) {
                 const double ms = (double)(tt[2 * q + 1] - tt[2 * q]) / 1e5;  // 100 MHz clock
                 double ps[kO1Ctx];
-                context_shares(host, nf_off[hd[q].dset], ps);
+                context_shares(host, nf_off[hd_seg[q]], ps);
                 double share = 0;
-                for (int r = 0; r < kWalkCtxN; r++) share += ps[maps[q].perm[r]];
-                fprintf(stderr, " %.1f/%.0f/%.3f", ms, ms * 1e6 / (double)std::max<uint64_t>(1, hd[q].hi - hd[q].lo), share);
+                for (int r = 0; r < kSerialHot; r++) share += ps[hd[q].map.perm(r)];
+                fprintf(stderr, " %.1f/%.0f/%.3f", ms, ms * 1e6 / (double)std::max<uint64_t>(1, hd[q].m), share);
             }
             fprintf(stderr, "\n");
         }
