@@ -225,91 +225,148 @@ static inline unsigned nblk(uint64_t n, unsigned bs = 256) { return (unsigned)((
 // (in symbol order) goes to the k-th position of the walk j*step mod 2^tableLog, j = 0, 1, ...,
 // that lies at or below the high threshold. The walk is a permutation (step is odd), so it is
 // enumerated in parallel and ranked with a block scan. Within a symbol, positions in increasing
-// order get consecutive states: one thread per symbol scans the spread table.
+// order get consecutive states: each wave takes a quarter of the positions 64 at a time, and a
+// position's place among its symbol's is the symbol's count in the quarters and steps before plus the
+// lanes below that hold the same symbol (eight ballots). One thread per symbol scanning the whole
+// table, and scans by one lane, took 0.54 ms for the 15 tables of one segment, as long for a small
+// field as for a large one; this takes 0.04 ms.
 template <unsigned MaxLog>
 struct TableLdsT {
     int16_t norm[256];          // symbols above maxSym hold 0
     uint32_t cum[257];          // exclusive prefix of the counts (-1 counts as 1)
     uint32_t cump[257];         // exclusive prefix of the positive counts
-    uint32_t part[256];
+    union {
+        uint64_t part[4];       // scans: sums of the waves
+        uint16_t wcnt[4][256];  // positions of each symbol in the quarters before, then so far
+    };
     int32_t high;               // last position of the walk part; -1 when every count is -1
     int bad;
     uint8_t sym[1u << MaxLog];
 };
 using TableLds = TableLdsT<kFseMaxTableLog>;
 
+// Exclusive prefix of v over the 256 threads of a workgroup; *total their sum. part: four words of LDS.
+__device__ __forceinline__ uint64_t block_scan_u64(uint64_t v, uint64_t* part, uint64_t* total) {
+    const unsigned t = threadIdx.x, l = t & 63u, w = t >> 6;
+    uint64_t x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_up((unsigned long long)x, d);
+        if (l >= (unsigned)d) x += o;
+    }
+    __syncthreads();
+    if (l == 63) part[w] = x;
+    __syncthreads();
+    uint64_t before = 0, sum = 0;
+    for (unsigned i = 0; i < 4; i++) {
+        if (i < w) before += part[i];
+        sum += part[i];
+    }
+    __syncthreads();
+    *total = sum;
+    return before + x - v;
+}
+
 template <class TL>
 __device__ bool spread_parallel(TL& L, unsigned tl) {
     const unsigned t = threadIdx.x;
     const uint32_t ts = 1u << tl, mask = ts - 1, step = (ts >> 1) + (ts >> 3) + 3;
+    const int v = L.norm[t];
+    // counts, positive counts and -1 counts in one scan (at most 256 * 2^13 each)
+    const uint64_t cp = v > 0 ? (uint64_t)min(v, (int)ts) : 0u, low = v == -1 ? 1u : 0u;
+    uint64_t sum;
+    const uint64_t pre = block_scan_u64((cp + low) | cp << 22 | low << 44, L.part, &sum);
+    constexpr uint64_t m22 = (1u << 22) - 1;
+    L.cum[t] = (uint32_t)(pre & m22);
+    L.cump[t] = (uint32_t)(pre >> 22 & m22);
     if (t == 0) {
-        uint32_t c = 0, cp = 0;
-        int32_t high = (int32_t)ts - 1;
-        int bad = 0;
-        for (int s = 0; s < 256; s++) {
-            const int v = L.norm[s];
-            if (v < -1 || v > (int)ts) bad = 1;
-            L.cum[s] = c;
-            L.cump[s] = cp;
-            if (v == -1) {
-                c += 1;
-                if (c <= ts) L.sym[high--] = (uint8_t)s;
-            } else if (v > 0) {
-                c += (uint32_t)v;
-                cp += (uint32_t)v;
-            }
-        }
-        L.cum[256] = c;
-        L.cump[256] = cp;
-        if (c != ts) bad = 1;
-        L.high = high;
-        L.bad = bad;
+        L.cum[256] = (uint32_t)(sum & m22);
+        L.cump[256] = (uint32_t)(sum >> 22 & m22);
+        L.high = (int32_t)ts - 1 - (int32_t)(sum >> 44);
     }
-    __syncthreads();
-    if (L.bad) return false;
+    if (__syncthreads_or(v < -1 || v > (int)ts || (sum & m22) != ts)) return false;
+    if (low) L.sym[ts - 1 - (uint32_t)(pre >> 44)] = (uint8_t)t;
     const int32_t high = L.high;
     const uint32_t per = (ts + 255) / 256;  // walk steps per thread
     const uint32_t k0 = min(ts, t * per), k1 = min(ts, k0 + per);
-    uint32_t cnt = 0;
-    for (uint32_t k = k0; k < k1; k++) cnt += (int32_t)((k * step) & mask) <= high;
-    L.part[t] = cnt;
-    __syncthreads();
-    if (t == 0) {
-        uint32_t acc = 0;
-        for (int i = 0; i < 256; i++) { const uint32_t v = L.part[i]; L.part[i] = acc; acc += v; }
+    uint32_t rank = k0;
+    if (high + 1 != (int32_t)ts) {
+        uint32_t cnt = 0;
+        for (uint32_t k = k0; k < k1; k++) cnt += (int32_t)((k * step) & mask) <= high;
+        rank = (uint32_t)block_scan_u64(cnt, L.part, &sum);
     }
-    __syncthreads();
-    uint32_t rank = L.part[t];
+    int s = 0, hi = 256;  // last symbol with cump <= rank: the one whose counts hold rank
+    while (hi - s > 1) {
+        const int mid = (s + hi) >> 1;
+        if (L.cump[mid] <= rank) s = mid; else hi = mid;
+    }
     for (uint32_t k = k0; k < k1; k++) {
         const uint32_t pos = (k * step) & mask;
         if ((int32_t)pos > high) continue;
-        int lo = 0, hi = 256;  // last symbol with cump <= rank: the one whose counts hold rank
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (L.cump[mid] <= rank) lo = mid; else hi = mid;
-        }
-        L.sym[pos] = (uint8_t)lo;
+        while (s < 255 && L.cump[s + 1] <= rank) s++;
+        L.sym[pos] = (uint8_t)s;
         rank++;
     }
     __syncthreads();
     return true;
 }
 
+// After spread_parallel: f(position, symbol, place of the position among its symbol's, in order).
+template <class TL, class F>
+__device__ __forceinline__ void rank_positions(TL& L, unsigned tl, F&& f) {
+    const unsigned t = threadIdx.x, l = t & 63u, w = t >> 6;
+    const uint32_t ts = 1u << tl, span = max(64u, ts / 4);
+    const uint32_t u0 = min(ts, w * span), u1 = min(ts, u0 + span);
+    // lanes of this step that hold the same symbol
+    auto same = [&](uint32_t s, bool in) {
+        uint64_t m = __ballot(in);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const uint64_t z = __ballot((s >> b) & 1u);
+            m &= (s >> b) & 1u ? z : ~z;
+        }
+        return m;
+    };
+#pragma unroll
+    for (int i = 0; i < 4; i++) L.wcnt[w][l + 64 * i] = 0;
+    wave_lds_order();
+    for (uint32_t u = u0; u < u1; u += 64) {
+        const bool in = u + l < u1;
+        const uint32_t s = in ? L.sym[u + l] : 0u;
+        const uint64_t m = same(s, in);
+        if (in && (m & ((1ull << l) - 1)) == 0) L.wcnt[w][s] = (uint16_t)(L.wcnt[w][s] + __popcll(m));
+        wave_lds_order();
+    }
+    __syncthreads();
+    {
+        uint32_t acc = 0;
+        for (int i = 0; i < 4; i++) {
+            const uint32_t n = L.wcnt[i][t];
+            L.wcnt[i][t] = (uint16_t)acc;
+            acc += n;
+        }
+    }
+    __syncthreads();
+    for (uint32_t u = u0; u < u1; u += 64) {
+        const bool in = u + l < u1;
+        const uint32_t s = in ? L.sym[u + l] : 0u;
+        const uint64_t m = same(s, in);
+        const uint64_t before = m & ((1ull << l) - 1);
+        const uint32_t base = L.wcnt[w][s];
+        wave_lds_order();
+        if (in && before == 0) L.wcnt[w][s] = (uint16_t)(base + __popcll(m));
+        wave_lds_order();
+        if (in) f(u + l, s, base + (uint32_t)__popcll(before));
+    }
+}
+
 // FSE_buildCTable_wksp (fse_compress.c:65-155) after spread_parallel; thread t handles symbol t.
 template <class TL, class CT>
-__device__ void ctable_parallel(const TL& L, unsigned tl, unsigned maxSym, CT* ct) {
+__device__ void ctable_parallel(TL& L, unsigned tl, unsigned maxSym, CT* ct) {
     const unsigned t = threadIdx.x;
     const uint32_t ts = 1u << tl;
     const int nc = L.norm[t];
-    uint32_t slot = L.cum[t];
-    if (nc != 0) {
-        const uint32_t* w = reinterpret_cast<const uint32_t*>(L.sym);
-        for (uint32_t u4 = 0; u4 < ts / 4; u4++) {
-            const uint32_t v = w[u4];
-            for (int b = 0; b < 4; b++)
-                if (((v >> (8 * b)) & 0xFFu) == t) ct->stateTable[slot++] = (uint16_t)(ts + 4 * u4 + b);
-        }
-    }
+    rank_positions(L, tl, [&](uint32_t u, uint32_t s, uint32_t r) { ct->stateTable[L.cum[s] + r] = (uint16_t)(ts + u); });
     if (nc == 0) {
         ct->deltaNbBits[t] = ((tl + 1) << 16) - ts;
         ct->deltaFindState[t] = 0;
@@ -324,24 +381,21 @@ __device__ void ctable_parallel(const TL& L, unsigned tl, unsigned maxSym, CT* c
     if (t == 0) { ct->tableLog = tl; ct->maxSym = maxSym; }
 }
 
-// FSE_buildDTable (fse_decompress.c:70-127) after spread_parallel; thread t handles symbol t.
-template <class TL>
-__device__ void dtable_parallel(const TL& L, unsigned tl, DEntry* dt) {
-    const unsigned t = threadIdx.x;
+// FSE_buildDTable (fse_decompress.c:70-127) after spread_parallel. entry(symbol) goes into the top
+// four bits of nbBits.
+template <class TL, class X>
+__device__ void dtable_parallel(TL& L, unsigned tl, DEntry* dt, X&& extra) {
     const uint32_t ts = 1u << tl;
-    const int nc = L.norm[t];
-    if (nc == 0) return;
-    uint32_t next = (nc == -1) ? 1u : (uint32_t)nc;
-    const uint32_t* w = reinterpret_cast<const uint32_t*>(L.sym);
-    for (uint32_t u4 = 0; u4 < ts / 4; u4++) {
-        const uint32_t v = w[u4];
-        for (int k = 0; k < 4; k++)
-            if (((v >> (8 * k)) & 0xFFu) == t) {
-                const uint32_t ns = next++;
-                const uint32_t nb = tl - highbit32(ns);
-                dt[4 * u4 + k] = DEntry{(uint16_t)((ns << nb) - ts), (uint8_t)t, (uint8_t)nb};
-            }
-    }
+    rank_positions(L, tl, [&](uint32_t u, uint32_t s, uint32_t r) {
+        const int nc = L.norm[s];
+        const uint32_t ns = (nc == -1 ? 1u : (uint32_t)nc) + r;
+        const uint32_t nb = tl - highbit32(ns);
+        dt[u] = DEntry{(uint16_t)((ns << nb) - ts), (uint8_t)s, (uint8_t)(nb | extra(s) << 4)};
+    });
+}
+template <class TL>
+__device__ void dtable_parallel(TL& L, unsigned tl, DEntry* dt) {
+    dtable_parallel(L, tl, dt, [](uint32_t) { return 0u; });
 }
 
 // ---------------------------------------------------------------- FSE block (workgroup-wide)
@@ -1053,69 +1107,114 @@ __global__ void k_add_one(uint32_t* cnt, int total) {
 
 // o1_normalize (RleFse:410-477): FSE_normalizeCount at tableLog 13, with the reference's fallback
 // (proportional counts, surplus to the largest, deficit taken from the largest ones) when it fails
-// or when a context has at most one symbol. Runs in one lane; f receives the counts.
-__device__ void o1_normalize(const uint32_t* h, uint16_t* f) {
-    uint64_t total = 0;
-    int nonzero = 0;
-    for (int s = 0; s < kO1Sym; s++) { total += h[s]; nonzero += h[s] != 0; }
-    const int M = 1 << kO1Log;
-    bool done = false;
+// or when a context has at most one symbol. h and f are in LDS; f receives the counts. The first part
+// of FSE_normalizeCount runs with a thread per symbol; where its rounding leaves too much to give to
+// the largest count (its second method), and for the fallback, one lane does all of it.
+struct O1NormLds {
+    uint32_t h[kO1Sym];
     int16_t norm[kO1Sym];
-    if (total == 0) {
-        for (int s = 0; s < kO1Sym; s++) f[s] = 0;
-        f[0] = (uint16_t)M;
-        done = true;
-    } else if (nonzero > 1) {
-        if (normalize_count(norm, kO1Log, h, total, kO1Sym - 1) != kFseErr) {
-            for (int s = 0; s < kO1Sym; s++) f[s] = (uint16_t)norm[s];
-            done = true;
+    uint64_t part[4];
+    uint32_t best;
+    int sum;
+};
+__device__ void o1_normalize_lane(O1NormLds& L, uint64_t total, int nonzero) {
+    const uint32_t* h = L.h;
+    int16_t* f = L.norm;
+    const int M = 1 << kO1Log;
+    if (nonzero > 1 && normalize_count(f, kO1Log, h, total, kO1Sym - 1) != kFseErr) return;
+    int sum = 0, maxf = 0, argmax = 0;
+    for (int s = 0; s < kO1Sym; s++) {
+        if (h[s]) {
+            int v = (int)((uint64_t)h[s] * (uint64_t)M / total);
+            if (v == 0) v = 1;
+            f[s] = (int16_t)v;
+            sum += v;
+            if (v > maxf) { maxf = v; argmax = s; }
+        } else {
+            f[s] = 0;
         }
     }
-    if (!done) {
-        int sum = 0, maxf = 0, argmax = 0;
-        for (int s = 0; s < kO1Sym; s++) {
-            if (h[s]) {
-                int v = (int)((uint64_t)h[s] * (uint64_t)M / total);
-                if (v == 0) v = 1;
-                f[s] = (uint16_t)v;
-                sum += v;
-                if (v > maxf) { maxf = v; argmax = s; }
-            } else {
-                f[s] = 0;
-            }
-        }
-        int e = M - sum;
-        if (e > 0) {
-            f[argmax] = (uint16_t)(f[argmax] + e);
-        } else if (e < 0) {
-            e = -e;
-            int take = (maxf - 1 < e) ? (maxf - 1) : e;
-            f[argmax] = (uint16_t)(f[argmax] - take);
+    int e = M - sum;
+    if (e > 0) {
+        f[argmax] = (int16_t)(f[argmax] + e);
+    } else if (e < 0) {
+        e = -e;
+        int take = (maxf - 1 < e) ? (maxf - 1) : e;
+        f[argmax] = (int16_t)(f[argmax] - take);
+        e -= take;
+        while (e > 0) {
+            int mi = -1;
+            uint32_t mv = 1;
+            for (int s = 0; s < kO1Sym; s++)
+                if ((uint16_t)f[s] > mv) { mv = (uint16_t)f[s]; mi = s; }
+            if (mi < 0) break;
+            take = (int)(uint16_t)f[mi] - 1;
+            if (take > e) take = e;
+            f[mi] = (int16_t)(f[mi] - take);
             e -= take;
-            while (e > 0) {
-                int mi = -1;
-                uint32_t mv = 1;
-                for (int s = 0; s < kO1Sym; s++)
-                    if (f[s] > mv) { mv = f[s]; mi = s; }
-                if (mi < 0) break;
-                take = (int)f[mi] - 1;
-                if (take > e) take = e;
-                f[mi] = (uint16_t)(f[mi] - take);
-                e -= take;
-            }
         }
     }
+}
+// by the 256 threads of a workgroup, L.h set
+__device__ void o1_normalize(O1NormLds& L) {
+    const unsigned t = threadIdx.x;
+    const uint32_t c = L.h[t];
+    uint64_t sum;
+    block_scan_u64((uint64_t)c | (uint64_t)(c != 0) << 48, L.part, &sum);
+    const uint64_t total = sum & ((1ull << 48) - 1);
+    const int nonzero = (int)(sum >> 48);
+    if (total == 0) {
+        L.norm[t] = t == 0 ? (int16_t)(1 << kO1Log) : (int16_t)0;
+        __syncthreads();
+        return;
+    }
+    if (t == 0) {
+        L.best = 0;
+        L.sum = 0;
+    }
+    __syncthreads();
+    bool whole = nonzero > 1 && kO1Log >= min_table_log(total, kO1Sym - 1);
+    if (whole) {
+        const uint32_t rtb[8] = {0, 473195, 504333, 520860, 550000, 700000, 750000, 830000};
+        const uint64_t scale = 62 - kO1Log, step = ((uint64_t)1 << 62) / total, vStep = 1ull << (scale - 20);
+        int16_t p = 0;
+        int used = 0;
+        if (c != 0 && c <= (uint32_t)(total >> kO1Log)) {
+            p = -1;
+            used = 1;
+        } else if (c != 0) {
+            const uint64_t scaled = (uint64_t)c * step;
+            p = (int16_t)(scaled >> scale);
+            if (p < 8) p = (int16_t)(p + ((scaled - ((uint64_t)p << scale)) > vStep * rtb[p]));
+            used = p;
+            // the largest count, the first of equal ones
+            if (p > 0) atomicMax(&L.best, (uint32_t)p << 16 | (255u - t));
+        }
+        L.norm[t] = p;
+        if (used) atomicAdd(&L.sum, used);
+        __syncthreads();
+        const unsigned largest = L.best ? 255u - (L.best & 0xFFFFu) : 0u;
+        const int still = (1 << kO1Log) - L.sum;
+        const int lp = L.norm[largest];
+        __syncthreads();
+        whole = !(-still >= (lp >> 1));
+        if (whole && t == largest) L.norm[t] = (int16_t)(lp + still);
+    }
+    if (!whole && t == 0) o1_normalize_lane(L, total, nonzero);
+    __syncthreads();
 }
 
 // Encoding tables of every context of every segment: grid (contexts, segments).
 __global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint16_t* nf_all, CTable* ct_all) {
     __shared__ TableLds L;
+    __shared__ O1NormLds N;
     const unsigned t = threadIdx.x;
     const size_t c = (size_t)blockIdx.y * kO1Ctx + blockIdx.x;
-    uint16_t* nf = nf_all + c * kO1Sym;
-    if (t == 0) o1_normalize(cnt_all + c * kO1Sym, nf);
+    N.h[t] = cnt_all[c * kO1Sym + t];
     __syncthreads();
-    L.norm[t] = (int16_t)nf[t];
+    o1_normalize(N);
+    nf_all[c * kO1Sym + t] = (uint16_t)N.norm[t];
+    L.norm[t] = N.norm[t];
     __syncthreads();
     if (!spread_parallel(L, kO1Log)) return;  // cannot happen for counts from o1_normalize
     ctable_parallel(L, kO1Log, kO1Sym - 1, ct_all + c);
@@ -1492,17 +1591,11 @@ __global__ void __launch_bounds__(256) k_o1_dtables(const uint8_t* stream, const
         for (uint32_t u = t; u < (1u << kO1Log); u += blockDim.x) dt[u] = DEntry{0, 0, 0};
         return;
     }
-    dtable_parallel(L, kO1Log, dt);
-    __syncthreads();
     // the context that follows each entry's symbol rides in the top four bits of nbBits (15 after an
     // escape, whose context depends on the escaped value); readers mask nbBits with 15
-    for (uint32_t u = t; u < (1u << kO1Log); u += blockDim.x) {
-        DEntry d = dt[u];
-        const unsigned sy = d.symbol;
-        const uint32_t nc = sy == 255 ? 15u : (uint32_t)o1_ctx((int)((sy >> 1) ^ (~(sy & 1) + 1)));
-        d.nbBits = (uint8_t)(d.nbBits | (nc << 4));
-        dt[u] = d;
-    }
+    dtable_parallel(L, kO1Log, dt, [](uint32_t sy) {
+        return sy == 255 ? 15u : (uint32_t)o1_ctx((int)((sy >> 1) ^ (~(sy & 1) + 1)));
+    });
 }
 
 
