@@ -579,7 +579,7 @@ size_t gpu_compress(fz_ctx* ctx, DevArena& ws, fz_config& c, int dtype, void* d_
         void* sel_tmp = ws.take<uint8_t>(sel_bytes + 1);
         gen_anchors(dtype, false, d_data, unpred, G.anchors, st);
         gen_traverse(dtype, false, G.steps, 1, n, 0, d_data, codes, escval, GenEsc{}, st);
-        select_escapes(codes, ncodes, esc_idx, nesc_dev, sel_tmp, sel_bytes, st);
+        select_escapes(codes, ncodes, esc_idx, nesc_dev, sel_tmp, st);
         gen_gather_escapes(dtype, esc_idx, nesc_dev, ncodes, escval, static_cast<uint8_t*>(unpred) + nanchors * es, st);
     } else {
         const Plan P = make_plan(c.N, c.dims, c.interp_anchor_stride, c.interp_algo, c.interp_direction);
@@ -609,7 +609,7 @@ size_t gpu_compress(fz_ctx* ctx, DevArena& ws, fz_config& c, int dtype, void* d_
             for (const auto& p : P.passes)
                 interp_pass(dtype, false, p, d_data, codes, escval, lv, avx2, nullptr, 0, nullptr, st);
         }
-        select_escapes(codes, P.ncodes, esc_idx, nesc_dev, sel_tmp, sel_bytes, st);
+        select_escapes(codes, P.ncodes, esc_idx, nesc_dev, sel_tmp, st);
         gather_escapes(dtype, esc_idx, nesc_dev, P.ncodes, escval, static_cast<uint8_t*>(unpred) + P.nanchors * es,
                        st);
     }
@@ -755,7 +755,6 @@ struct DecompressCall {
     uint64_t* esc_idx = nullptr;
     uint64_t* nesc_dev = nullptr;
     void* sel_tmp = nullptr;
-    size_t sel_bytes = 0;
     std::unique_ptr<EntropyCall, void (*)(EntropyCall*)> ent{entropy_call_new(), entropy_call_free};
 };
 
@@ -798,8 +797,7 @@ void decompress_begin(DecompressCall& D, DevArena& ws, hipStream_t st, const fz_
     D.codes = ws.take<int16_t>(ncodes + 16);
     D.esc_idx = ws.take<uint64_t>(ncodes + 1);
     D.nesc_dev = ws.take<uint64_t>(1);
-    D.sel_bytes = select_escapes_scratch(ncodes);
-    D.sel_tmp = ws.take<uint8_t>(D.sel_bytes + 1);
+    D.sel_tmp = ws.take<uint8_t>(select_escapes_scratch(ncodes));
     FZ_HIP(hipStreamSynchronize(st));  // the host sources of the copies above (ratio) leave scope
     if (tm) tm->start();
     if (d_pre && nun) FZ_HIP(hipMemcpyAsync(D.d_unpred, d_pre + un_off, (size_t)nun * es, hipMemcpyDeviceToDevice, st));
@@ -823,7 +821,7 @@ void decompress_finish(DecompressCall& D, DevArena& ws, hipStream_t st) {
     int16_t* codes = D.codes;
     uint64_t* esc_idx = D.esc_idx;
     entropy_decode_end(D.ent.get(), ws, st);
-    select_escapes(codes, ncodes, esc_idx, D.nesc_dev, D.sel_tmp, D.sel_bytes, st);
+    select_escapes(codes, ncodes, esc_idx, D.nesc_dev, D.sel_tmp, st);
     uint64_t nesc = 0;
     FZ_HIP(hipMemcpyAsync(&nesc, D.nesc_dev, 8, hipMemcpyDeviceToHost, st));
     FZ_HIP(hipStreamSynchronize(st));

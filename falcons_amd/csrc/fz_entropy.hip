@@ -992,8 +992,7 @@ __global__ void __launch_bounds__(256) k_fse_dec_blocks(const FseBlk* blks, int*
 
 // ---------------------------------------------------------------- method 0 (RleFse:928-982)
 struct NonZero {
-    const int16_t* b;
-    __device__ __forceinline__ bool operator()(const uint64_t& i) const { return b[i] != 0; }
+    __device__ __forceinline__ bool operator()(int16_t c) const { return c != 0; }
 };
 
 __device__ inline int floor_log2_64(uint64_t v) { return 63 - __clzll((long long)v); }
@@ -1055,8 +1054,12 @@ __global__ void k_scatter_mantissas(const int16_t* bins, uint64_t n, const uint6
 
 // ---------------------------------------------------------------- method 1 (RleFse:582-751)
 struct IsO1Escape {
-    const int16_t* b;
-    __device__ __forceinline__ bool operator()(const uint64_t& i) const { return o1_sym(b[i]) == 255; }
+    __device__ __forceinline__ bool operator()(int16_t c) const { return o1_sym(c) == 255; }
+};
+struct CopyCode {
+    const int16_t* codes;
+    int16_t* out;
+    __device__ __forceinline__ void operator()(uint64_t k, uint64_t i) const { out[k] = codes[i]; }
 };
 
 // Exact per-context histogram of a segment (N < 2^20): the context resets to that of 0 at each
@@ -1569,10 +1572,6 @@ __global__ void k_o1_close(const int16_t* bins, O1Chains C, const CTable* ct_all
     blen[q] = (b0 + kO1Log + 1 + 7) >> 3;
 }
 
-__global__ void k_gather_i16(const int16_t* src, const uint64_t* idx, uint64_t n, int16_t* out) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = src[idx[i]];
-}
 
 // ---------------------------------------------------------------- method 1 decode
 // Decoding tables of every context of every segment, grid (contexts, segments); the counts are read
@@ -3087,8 +3086,7 @@ static size_t encode_method0(const int16_t* bins, uint64_t n, uint8_t* out, uint
     uint64_t* pos = ws.take<uint64_t>(n + 1);
     uint64_t* nsel = ws.take<uint64_t>(1);
     {
-        const size_t bytes = select_scratch_bytes(n);
-        select_indices(NonZero{bins}, n, pos, nsel, cub_scratch(ws, bytes), bytes, "rle_select_values", st);
+        select_indices(bins, n, NonZero{}, pos, nsel, cub_scratch(ws, select_scratch_bytes(n)), "rle_select_values", st);
     }
     uint64_t nv = 0;
     d2h(&nv, nsel, 1, st);
@@ -3276,19 +3274,6 @@ struct EscapeWorker {
     }
 };
 
-// below[q] = the number of sorted positions pos[0..n) under ends[q] (one lane per end).
-__global__ void k_count_below(const uint64_t* pos, uint64_t n, const uint64_t* ends, int nq, uint64_t* below) {
-    for (int q = threadIdx.x; q < nq; q += blockDim.x) {
-        const uint64_t v = ends[q];
-        uint64_t lo = 0, hi = n;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi) >> 1;
-            if (pos[mid] < v) lo = mid + 1; else hi = mid;
-        }
-        below[q] = lo;
-    }
-}
-
 static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint64_t cap, DevArena& ws,
                              hipStream_t st, const AuxStream& aux) {
     // the piece kernels read the codes in aligned 16-byte loads (arena allocations are 256-byte
@@ -3298,17 +3283,11 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
     if (S < 1) S = 1;
     if (S > 16) S = 16;
     const uint64_t seg = (n + S - 1) / S;
-    // escapes (sym 255) over the whole array, in index order
-    uint64_t* epos = ws.take<uint64_t>(n + 1);
+    // escaped codes (sym 255) of the whole array, in index order
+    int16_t* ovf = ws.take<int16_t>(n + 1);
     uint64_t* nsel = ws.take<uint64_t>(1);
-    {
-        const size_t bytes = select_scratch_bytes(n);
-        select_indices(IsO1Escape{bins}, n, epos, nsel, cub_scratch(ws, bytes), bytes, "o1_select_escapes", st);
-    }
-    uint64_t nesc = 0;
-    d2h(&nesc, nsel, 1, st);
-    int16_t* ovf = ws.take<int16_t>(nesc + 1);
-    if (nesc) FZ_LAUNCH("o1_gather_escapes", nesc * 10, k_gather_i16, dim3(nblk(nesc)), dim3(256), 0, st, bins, epos, nesc, ovf);
+    const SelTiles esc_tiles = select_codes(bins, n, IsO1Escape{}, CopyCode{bins, ovf}, nsel,
+                                            cub_scratch(ws, select_scratch_bytes(n)), "o1_select_escapes", st);
     // histograms and tables per segment
     uint32_t* cnt = ws.take<uint32_t>(S * kO1Ctx * kO1Sym);
     uint16_t* nf = ws.take<uint16_t>(S * kO1Ctx * kO1Sym);
@@ -3352,12 +3331,13 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         FZ_HIP(hipGetLastError());
     }
     {
-        // escapes below each chain's end: binary searches in the sorted escape positions
+        // escapes below each chain's end
         const int nb = (int)(S * kO1K);
         uint64_t* dends = ws.take<uint64_t>(nb);
         uint64_t* dbelow = ws.take<uint64_t>(nb);
         h2d(dends, ends.data(), nb, st);
-        FZ_LAUNCH("o1_escape_counts", 0, k_count_below, dim3(1), dim3(64), 0, st, epos, nesc, dends, nb, dbelow);
+        FZ_LAUNCH("o1_escape_counts", 0, k_sel_below<IsO1Escape>, dim3((unsigned)nb), dim3(256), 0, st, bins,
+                  n, IsO1Escape{}, esc_tiles.offs, esc_tiles.count, nsel, dends, dbelow);
         FZ_HIP(hipGetLastError());
         std::vector<uint64_t> below(nb);
         d2h(below.data(), dbelow, nb, st);

@@ -613,11 +613,6 @@ __global__ void k_gather_escapes(const uint64_t* idx, const uint64_t* nsel, cons
         out[i] = escval[idx[i]];
 }
 
-struct IsEscape {
-    const int16_t* codes;
-    __device__ __forceinline__ bool operator()(const uint64_t& i) const { return codes[i] == -32768; }
-};
-
 static inline unsigned blocks_for(uint64_t n, unsigned bs = 256) { return (unsigned)((n + bs - 1) / bs); }
 
 // ---------------- host-side launchers ----------------
@@ -780,8 +775,8 @@ void abs_error_bound(int dtype, const void* data, uint64_t n, int simd, int mode
 size_t select_escapes_scratch(uint64_t n) { return select_scratch_bytes(n); }
 
 void select_escapes(const int16_t* codes, uint64_t n, uint64_t* out_idx, uint64_t* nsel_dev, void* scratch,
-                    size_t scratch_bytes, hipStream_t st) {
-    select_indices(IsEscape{codes}, n, out_idx, nsel_dev, scratch, scratch_bytes, "select_escapes", st);
+                    hipStream_t st) {
+    select_indices(codes, n, IsEscape{}, out_idx, nsel_dev, scratch, "select_escapes", st);
 }
 
 void gather_escapes(int dtype, const uint64_t* idx, const uint64_t* nsel_dev, uint64_t max_n, const void* escval,

@@ -125,7 +125,7 @@ void abs_error_bound(int dtype, const void* data, uint64_t n, int simd, int mode
                      double psnr_factor, void* scratch, double* eb_dev, hipStream_t st);
 size_t select_escapes_scratch(uint64_t n);
 void select_escapes(const int16_t* codes, uint64_t n, uint64_t* out_idx, uint64_t* nsel_dev, void* scratch,
-                    size_t scratch_bytes, hipStream_t st);
+                    hipStream_t st);
 void gather_escapes(int dtype, const uint64_t* idx, const uint64_t* nsel_dev, uint64_t max_n, const void* escval,
                     void* out, hipStream_t st);
 

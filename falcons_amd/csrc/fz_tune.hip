@@ -87,11 +87,6 @@ __global__ void __launch_bounds__(256) k_tune_gather(const T* __restrict__ data,
     blocks[g] = data[idx];
 }
 
-struct IsEscape16 {
-    const int16_t* c;
-    __device__ __forceinline__ bool operator()(const uint64_t& i) const { return c[i] == -32768; }
-};
-
 // Unpredictable list of every block in order: its anchors, then its escapes in code order. Block b's
 // list starts at b*nanch + (escapes in the blocks before b).
 template <typename T>
@@ -178,7 +173,7 @@ struct Tuner {
         gen_traverse(dtype, false, G.steps, nblk, per, ncb, work, codes, escv, GenEsc{}, st);
         FZ_HIP(hipGetLastError());
         const uint64_t ncode = nblk * ncb;
-        select_indices(IsEscape16{codes}, ncode, esc, nesc_dev, sel_tmp, sel_bytes, "tune_escapes", st);
+        select_indices(codes, ncode, IsEscape{}, esc, nesc_dev, sel_tmp, "tune_escapes", st);
         uint64_t nesc = 0;
         FZ_HIP(hipMemcpyAsync(&nesc, nesc_dev, 8, hipMemcpyDeviceToHost, st));
         FZ_HIP(hipStreamSynchronize(st));
