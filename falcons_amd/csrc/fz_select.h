@@ -63,7 +63,7 @@ static __global__ void __launch_bounds__(1024) k_sel_scan(const uint32_t* counts
         uint32_t c[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) c[k] = t + k < ntiles ? counts[t + k] : 0u;
-        const uint32_t own = c[0] + c[1] + c[2] + c[3];  // at most 2^14 hits a thread, 2^24 a round
+        const uint32_t own = c[0] + c[1] + c[2] + c[3];  // sums of up to 2^17 a tile fit
         uint32_t inc = own;
 #pragma unroll
         for (uint32_t d = 1; d < 64; d <<= 1) {
