@@ -1226,20 +1226,35 @@ __global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint
 
 // ---- order-1 tANS encoding split into pieces --------------------------------------------------
 // A chain is encoded backwards: symbol hi-1 seeds the state (FSE_initCState2), then one encoder
-// step per symbol i = hi-2 .. lo. The steps are cut into pieces of kO1Piece consecutive steps,
+// step per symbol i = hi-2 .. lo. The steps are cut into pieces of consecutive steps,
 // piece 0 holding the first steps (i = hi-2 downwards). A piece's output bits depend on the state
 // it starts from, which the previous piece produces. Encoder steps are many-to-one (the low bits
-// of the state leave through the bitstream), so runs from different start states merge within a
-// few dozen steps; the pieces therefore run in parallel from a guessed state (k_o1_spec), then
-// each re-runs from its predecessor's end state until it meets its own logged trajectory
-// (k_o1_fix, repeated only while some piece fails to meet it), and finally every piece emits its
-// bits at its offset in the chain (k_o1_emit). The result is the sequential encoder's bitstream.
+// of the state leave through the bitstream), so runs from different start states merge, all but
+// a handful within a hundred steps and the last few within thousands. Every piece emits its bits at its
+// offset in the chain (k_o1_emit) once its start state is known, which is found in one of two ways;
+// the result is the sequential encoder's bitstream either way.
+// - Arrays of up to kSetMaxCodes codes, where a step's latency (its table is read from L2: 0.35 us with a
+//   state of its own in every lane, 0.13 us with a few) is all that counts: a wave a piece of kSetPiece steps follows every state that can enter the piece
+//   (k_o1_sets), and a walk over the pieces picks the true ones (k_o1_sets_walk).
+// - Longer arrays fill the chip with one lane a piece of kO1Piece steps: all run from a guessed state
+//   (k_o1_spec), then each re-runs from its predecessor's end state until it meets its own logged
+//   trajectory (k_o1_fix, repeated while some piece fails to meet it).
+// 540,000 codes, the order-1 stage without its side streams: guessed and repaired 1.4 to 6 ms (2 to 10
+// rounds, as slowly as the last states merge), by sets 0.25 ms; 86,000: 1.03 and 0.24 ms. By sets a
+// code costs 2.25 steps of a wave: 134 million codes, 2.7 ms guessed and repaired, would take 7.
 constexpr uint32_t kO1Piece = 1024;
+constexpr uint32_t kSetPiece = 256;
+constexpr uint64_t kSetMaxCodes = 7ull << 19;  // 3,584 pieces a chain: the walk's links fit 64 KB of LDS
+constexpr uint32_t kSetStates = 16;    // states followed through a piece
+constexpr uint32_t kSetWarm = 320;     // steps in front of a piece; the first 128 are searched for a rare symbol
+constexpr uint32_t kSetSearch = 128;
+constexpr uint32_t kSetWarmMax = 1344; // how far back the search goes
 
 struct O1Chains {        // device view of the chains of one call
     const uint64_t* c;   // 4 per chain: segment lo, chunk lo, chunk hi, segment
     const uint64_t* pfirst;  // first piece of each chain (exclusive scan), nchains + 1 entries
     int nchains;
+    uint32_t piece;          // steps of a piece
 };
 
 __device__ inline int o1_piece_chain(const O1Chains& C, uint64_t pid) {
@@ -1251,10 +1266,10 @@ __device__ inline int o1_piece_chain(const O1Chains& C, uint64_t pid) {
     return lo;
 }
 
-// Steps [s_hi down to s_lo] of piece p of a chain with symbols [lo, hi): s_hi = hi-2 - p*kO1Piece.
-__device__ inline void o1_piece_range(uint64_t lo, uint64_t hi, uint64_t p, uint64_t& s_hi, uint64_t& s_lo) {
-    s_hi = hi - 2 - p * kO1Piece;
-    s_lo = (s_hi + 1 > lo + kO1Piece) ? s_hi + 1 - kO1Piece : lo;
+// Steps [s_hi down to s_lo] of piece p of a chain with symbols [lo, hi): s_hi = hi-2 - p*piece.
+__device__ inline void o1_piece_range(uint32_t piece, uint64_t lo, uint64_t hi, uint64_t p, uint64_t& s_hi, uint64_t& s_lo) {
+    s_hi = hi - 2 - p * piece;
+    s_lo = (s_hi + 1 > lo + piece) ? s_hi + 1 - piece : lo;
 }
 
 __device__ inline uint32_t o1_seed_state(const int16_t* bins, uint64_t lo, uint64_t idx, const CTable* ct) {
@@ -1347,7 +1362,7 @@ __global__ void __launch_bounds__(256) k_o1_spec(const int16_t* bins, O1Chains C
     const bool staged = C.c[4 * q + 3] == wseg;
     const uint64_t p = pid - C.pfirst[q];
     uint64_t s_hi, s_lo;
-    o1_piece_range(lo, hi, p, s_hi, s_lo);
+    o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
     // piece 0 starts from the true seed; the others from the seed their own first symbol would give
     uint32_t st = o1_seed_state(bins, lo, p == 0 ? hi - 1 : s_hi, ct);
     uint64_t bits = 0;
@@ -1391,7 +1406,7 @@ __global__ void __launch_bounds__(256) k_o1_fix(const int16_t* bins, O1Chains C,
         const FZ_LDS uint32_t* dnb = lds(T.dnb);
         const FZ_LDS int32_t* dfs = lds(T.dfs);
         uint64_t s_hi, s_lo;
-        o1_piece_range(lo, hi, p, s_hi, s_lo);
+        o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
         uint32_t st = end_prev[pid - 1];
         int64_t delta = 0;
         bool met = false;
@@ -1526,9 +1541,11 @@ __device__ inline void rw_flush(RunWriter& W) {
 
 __global__ void __launch_bounds__(256) k_o1_emit(const int16_t* bins, O1Chains C, uint64_t npieces,
                                                  const CTable* ct_all, const uint32_t* end_state,
-                                                 const uint64_t* bitoff, uint32_t* words, uint64_t stride_words) {
+                                                 const uint64_t* bitoff, uint32_t* words, uint64_t stride_words,
+                                                 const uint64_t* failed) {
     __shared__ O1EncLds T;
     __shared__ __align__(16) uint32_t ring[256 * 16];
+    if (failed && *failed) return;
     const uint64_t first = (uint64_t)xcd_block() * blockDim.x;
     const uint64_t wseg = o1_stage_tables(T, C, npieces, ct_all, first);
     const uint64_t pid = first + threadIdx.x;
@@ -1541,7 +1558,7 @@ __global__ void __launch_bounds__(256) k_o1_emit(const int16_t* bins, O1Chains C
     const FZ_LDS int32_t* dfs = lds(T.dfs);
     const uint64_t p = pid - C.pfirst[q];
     uint64_t s_hi, s_lo;
-    o1_piece_range(lo, hi, p, s_hi, s_lo);
+    o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
     uint32_t st = p == 0 ? o1_seed_state(bins, lo, hi - 1, ct) : end_state[pid - 1];
     const uint64_t b0 = bitoff[pid];
     RunWriter W{words + q * stride_words, lds(ring + threadIdx.x * 16), b0 >> 5, 0, (uint32_t)(b0 & 31), true, false};
@@ -1554,11 +1571,195 @@ __global__ void __launch_bounds__(256) k_o1_emit(const int16_t* bins, O1Chains C
     rw_flush(W);
 }
 
+// The states that can enter a piece and what becomes of them: kSetStates slots a piece.
+struct O1Sets {
+    uint16_t *start, *end, *bits;
+    uint8_t* cnt;  // slots in use
+};
+
+// Steps hi_i down to lo_i for the state of every lane: the lanes read and look up 64 steps at once
+// (their symbols do not depend on the states), the next 64 in flight; a step then takes its two
+// numbers from the lane that holds them.
+__device__ __forceinline__ void o1_set_run(const int16_t* bins, uint64_t lo, uint64_t hi_i, uint64_t lo_i,
+                                           const CTable* ct, uint32_t& st, uint32_t& bits) {
+    if (hi_i < lo_i) return;
+    const uint32_t lane = threadIdx.x & 63u;
+    const FZ_GLB uint16_t* tab = glb(reinterpret_cast<const uint16_t*>(ct));
+    auto load = [&](uint64_t top, uint32_t& d, uint32_t& b) {
+        const uint64_t i = top >= lo_i + lane ? top - lane : lo_i;
+        const int cx = o1_ctx(i > lo ? bins[i - 1] : 0), sym = o1_sym(bins[i]);
+        d = ct[cx].deltaNbBits[sym];
+        b = (uint32_t)(cx * (sizeof(CTable) / 2) + offsetof(CTable, stateTable) / 2) + (uint32_t)ct[cx].deltaFindState[sym];
+    };
+    uint32_t d, b, dn, bn;
+    load(hi_i, dn, bn);
+    const uint64_t steps = hi_i - lo_i + 1;
+    for (uint64_t done = 0; done < steps; done += 64) {
+        d = dn;
+        b = bn;
+        if (done + 64 < steps) load(hi_i - done - 64, dn, bn);
+        auto step = [&](int k) {
+            const uint32_t nb = (st + (uint32_t)__builtin_amdgcn_readlane((int)d, k)) >> 16;
+            bits += nb;
+            st = tab[(st >> nb) + (uint32_t)__builtin_amdgcn_readlane((int)b, k)];
+        };
+        const int cnt = (int)min(steps - done, (uint64_t)64);
+        if (cnt == 64) {
+#pragma unroll 16
+            for (int k = 0; k < 64; k++) step(k);
+        } else {
+            for (int k = 0; k < cnt; k++) step(k);
+        }
+    }
+}
+
+// A wave a piece. After a step whose symbol has the normalized count c, only c of the 8,192 states are
+// left, whatever the state before: the symbol of the lowest count among 128 some way in front of the piece
+// gives the first set, one state a lane (a symbol of a count up to 64; none there, the search goes on
+// further back). On the way to the piece most of them merge: 5 are left in the median over fields at
+// bounds 1e-2 to 1e-4, at most 8 seen. failed: a piece without such a symbol, or with more than kSetStates
+// states left. Bound by the latency of the steps' table reads.
+__global__ void __launch_bounds__(256) k_o1_sets(const int16_t* bins, O1Chains C, uint64_t npieces, const CTable* ct_all,
+                                                 const uint16_t* nf, O1Sets B, uint64_t* failed) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t pid = uniform32((uint32_t)(xcd_block() * 4u + (threadIdx.x >> 6)));
+    if (pid >= npieces) return;
+    const int q = o1_piece_chain(C, pid);
+    const uint64_t lo = uniform64(C.c[4 * q + 1]), hi = uniform64(C.c[4 * q + 2]), seg = uniform64(C.c[4 * q + 3]);
+    const CTable* ct = ct_all + seg * kO1Ctx;
+    const uint16_t* norm = nf + seg * kO1Ctx * kO1Sym;
+    uint64_t s_hi, s_lo;
+    o1_piece_range(C.piece, lo, hi, pid - uniform64(C.pfirst[q]), s_hi, s_lo);
+    uint32_t st, bits = 0;
+    uint64_t from = hi - 1;  // the step before the first one run
+    uint32_t states = 1;
+    bool exact = true;
+    for (uint64_t warm = kSetWarm; s_hi + warm < hi - 1; warm += kSetSearch) {
+        // steps s_hi + warm downwards
+        uint32_t best = ~0u;
+#pragma unroll
+        for (uint32_t h = 0; h < kSetSearch; h += 64) {
+            const uint64_t i = s_hi + warm - h - lane;  // above s_lo: kSetWarm > kSetSearch
+            const uint32_t c = norm[o1_ctx(bins[i - 1]) * kO1Sym + o1_sym(bins[i])];
+            const uint32_t cc = c == 0xFFFFu ? 1u : c == 0 ? 0xFFFFu : c;  // -1 stands for 1
+            best = min(best, cc << 8 | (h + lane));
+        }
+#pragma unroll
+        for (uint32_t d = 32; d; d >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, (int)d, 64));
+        best = uniform32(best);
+        if (best >> 8 <= 64) {
+            exact = false;
+            from = s_hi + warm - (best & 255u);
+            states = best >> 8;
+            break;
+        }
+        if (warm + kSetSearch > kSetWarmMax) {
+            if (lane == 0) atomicOr(reinterpret_cast<unsigned long long*>(failed), 1ull);
+            return;
+        }
+    }
+    if (exact) {
+        st = o1_seed_state(bins, lo, hi - 1, ct);
+    } else {
+        const CTable& t = ct[o1_ctx(bins[from - 1])];
+        st = t.stateTable[t.deltaFindState[o1_sym(bins[from])] + (int32_t)(states + min(lane, states - 1))];
+    }
+    o1_set_run(bins, lo, from - 1, s_hi + 1, ct, st, bits);
+    // one slot for each state that is left
+    uint32_t cnt = 0, slot_state = uniform32(st);
+    for (uint64_t left = __ballot(1); left; cnt++) {
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)st, __ffsll((unsigned long long)left) - 1);
+        left &= ~__ballot(st == v);
+        if (lane == cnt) slot_state = v;
+    }
+    if (cnt > kSetStates) {
+        if (lane == 0) atomicOr(reinterpret_cast<unsigned long long*>(failed), 1ull);
+        return;
+    }
+    st = slot_state;
+    bits = 0;
+    if (lane < kSetStates) B.start[pid * kSetStates + lane] = lane < cnt ? (uint16_t)st : (uint16_t)0;
+    if (lane == 0) B.cnt[pid] = (uint8_t)cnt;
+    o1_set_run(bins, lo, s_hi, s_lo, ct, st, bits);
+    if (lane < cnt) {
+        B.end[pid * kSetStates + lane] = (uint16_t)st;
+        B.bits[pid * kSetStates + lane] = (uint16_t)bits;
+    }
+}
+
+// One workgroup a chain: every slot's end among the next piece's starts (it is there: a piece's set holds
+// what any state in front of it becomes), a walk over these links in LDS from the chain's seed, then
+// the end states and bit offsets of the pieces and the cleared words that k_o1_emit adds to. LDS: 17
+// bytes a piece.
+__global__ void __launch_bounds__(256) k_o1_sets_walk(O1Chains C, O1Sets B, uint32_t* end_state, uint64_t* bitoff,
+                                                      uint64_t* chain_bits, uint32_t* words, uint64_t stride_words,
+                                                      uint64_t* failed) {
+    extern __shared__ uint8_t link[];
+    __shared__ uint64_t part[4];
+    __shared__ uint32_t lost;
+    const uint32_t q = blockIdx.x, t = threadIdx.x;
+    const uint64_t p0 = C.pfirst[q];
+    const uint32_t np = (uint32_t)(C.pfirst[q + 1] - p0);
+    uint8_t* const pick = link + (uint64_t)np * kSetStates;
+    if (t == 0) lost = *failed != 0;  // read once: another chain's workgroup may be setting it
+    __syncthreads();
+    if (lost) return;
+    for (uint32_t u = t; u < np * kSetStates; u += blockDim.x) {
+        const uint32_t p = u / kSetStates, k = u % kSetStates;
+        uint32_t to = 0xFF;
+        if (p + 1 < np && k < B.cnt[p0 + p]) {
+            const uint16_t e = B.end[p0 * kSetStates + u];
+            const uint32_t m = B.cnt[p0 + p + 1];
+            for (uint32_t j = 0; j < m; j++)
+                if (B.start[(p0 + p + 1) * kSetStates + j] == e) to = j;
+        }
+        link[u] = (uint8_t)to;
+    }
+    __syncthreads();
+    if (t == 0) {
+        uint32_t cur = 0;
+        for (uint32_t p = 0; p < np; p++) {
+            pick[p] = (uint8_t)cur;
+            cur = link[p * kSetStates + cur];
+            if (cur >= kSetStates && p + 1 < np) {
+                lost = 1;
+                break;
+            }
+        }
+    }
+    __syncthreads();
+    if (lost) {
+        if (t == 0) atomicOr(reinterpret_cast<unsigned long long*>(failed), 1ull);
+        return;
+    }
+    uint64_t base = 0;
+    for (uint32_t b = 0; b < np; b += blockDim.x) {
+        const uint32_t p = b + t;
+        uint64_t bits = 0, sum;
+        if (p < np) {
+            const uint64_t at = (p0 + p) * kSetStates + pick[p];
+            end_state[p0 + p] = B.end[at];
+            bits = B.bits[at];
+        }
+        const uint64_t off = base + block_scan_u64(bits, part, &sum);
+        if (p < np) {
+            bitoff[p0 + p] = off;
+            words[q * stride_words + (off >> 5)] = 0;
+        }
+        base += sum;
+    }
+    if (t == 0) {
+        chain_bits[q] = base;
+        for (uint64_t w = base >> 5; w <= (base + kO1Log + 1) >> 5; w++) words[q * stride_words + w] = 0;
+    }
+}
+
 // Final state (kO1Log bits) and the end mark of every chain (BIT_closeCStream); byte length out.
 __global__ void k_o1_close(const int16_t* bins, O1Chains C, const CTable* ct_all, const uint32_t* end_state,
-                           const uint64_t* chain_bits, uint32_t* words, uint64_t stride_words, uint64_t* blen) {
+                           const uint64_t* chain_bits, uint32_t* words, uint64_t stride_words, uint64_t* blen,
+                           const uint64_t* failed) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= C.nchains) return;
+    if (q >= C.nchains || (failed && *failed)) return;
     const uint64_t lo = C.c[4 * q + 1], hi = C.c[4 * q + 2];
     if (hi <= lo) { blen[q] = 0; return; }
     const CTable* ct = ct_all + C.c[4 * q + 3] * kO1Ctx;
@@ -3519,87 +3720,123 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
     const uint64_t bstride = stride_words * 4;
     uint32_t* words = ws.take<uint32_t>(nch * stride_words);
     uint8_t* bufs = reinterpret_cast<uint8_t*>(words);
-    uint64_t* blen = ws.take<uint64_t>(nch);
-    // pieces of every chain (steps i = hi-2 .. lo)
-    std::vector<uint64_t> pfirst(nch + 1, 0);
-    for (int q = 0; q < nch; q++) {
-        const uint64_t clo = chains[4 * q + 1], chi = chains[4 * q + 2];
-        const uint64_t steps = (chi > clo + 1) ? chi - clo - 1 : 0;
-        pfirst[q + 1] = pfirst[q] + (steps + kO1Piece - 1) / kO1Piece;
-    }
-    const uint64_t np = pfirst[nch];
-    uint64_t* dpfirst = ws.take<uint64_t>(nch + 1);
-    h2d(dpfirst, pfirst.data(), nch + 1, st);
-    const O1Chains CH{dchains, dpfirst, nch};
-    uint16_t* slog = ws.take<uint16_t>(np * kO1Piece + 16);  // step-major: [step in piece][piece]
-    uint32_t* spec_end = ws.take<uint32_t>(np + 1);
-    uint32_t* end_a = ws.take<uint32_t>(np + 1);
-    uint32_t* end_b = ws.take<uint32_t>(np + 1);
-    uint64_t* spec_bits = ws.take<uint64_t>(np + 1);
-    uint64_t* nbits = ws.take<uint64_t>(np + 1);
-    uint8_t* chg_a = ws.take<uint8_t>(np + 1);
-    uint8_t* chg_b = ws.take<uint8_t>(np + 1);
-    unsigned int* any = ws.take<unsigned int>(1);
-    uint64_t* scan = ws.take<uint64_t>(np + 1);
-    uint64_t* bitoff = ws.take<uint64_t>(np + 1);
+    uint64_t* blen = ws.take<uint64_t>(nch + 1);  // lengths of the chains, and whether their sets failed
     uint64_t* chain_bits = ws.take<uint64_t>(nch);
-    if (np) {
-        FZ_LAUNCH("o1_encode_spec", n * 4, k_o1_spec, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog, spec_end, spec_bits);
-        FZ_HIP(hipGetLastError());
-        FZ_HIP(hipMemcpyAsync(nbits, spec_bits, np * 8, hipMemcpyDeviceToDevice, st));
-        // fix-up rounds; each round finalizes at least the next piece of every chain, so the loop
-        // ends within max-pieces-per-chain rounds
-        const uint32_t* end_prev = spec_end;
-        uint32_t* end_next = end_a;
-        const uint8_t* chg_prev = nullptr;
-        uint8_t* chg_next = chg_a;
-        uint64_t max_rounds = 1;
-        for (int q = 0; q < nch; q++) max_rounds = std::max<uint64_t>(max_rounds, pfirst[q + 1] - pfirst[q] + 1);
-        // Two rounds per host check: `any` counts the changes of the second only. A round after one
-        // with no change re-runs no piece and changes nothing, so the check ends the loop at the
-        // first pair whose second round saw no change.
-        for (uint64_t round = 0;;) {
-            if (round > max_rounds + 1) throw std::runtime_error("tANS piece fix-up did not settle");
-            for (int k = 0; k < 2; k++, round++) {
-                if (k == 1) FZ_HIP(hipMemsetAsync(any, 0, sizeof(unsigned int), st));
-                FZ_LAUNCH("o1_encode_fix", 0, k_o1_fix, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog,
-                          spec_end, spec_bits, end_prev, end_next, nbits, chg_prev, chg_next, any);
-                FZ_HIP(hipGetLastError());
-                end_prev = end_next;
-                end_next = (end_next == end_a) ? end_b : end_a;
-                chg_prev = chg_next;
-                chg_next = (chg_next == chg_a) ? chg_b : chg_a;
-            }
-            unsigned int h_any = 0;
-            d2h(&h_any, any, 1, st);
-            if (!h_any) break;
+    // The pieces of every chain (steps i = hi-2 .. lo), laid out on the host; the vector stays until the
+    // stream has been waited for.
+    auto lay_out = [&](uint32_t steps_piece, std::vector<uint64_t>& pfirst) {
+        pfirst.assign(nch + 1, 0);
+        for (int q = 0; q < nch; q++) {
+            const uint64_t clo = chains[4 * q + 1], chi = chains[4 * q + 2];
+            const uint64_t steps = (chi > clo + 1) ? chi - clo - 1 : 0;
+            pfirst[q + 1] = pfirst[q] + (steps + steps_piece - 1) / steps_piece;
         }
-        exclusive_scan_u64(nbits, scan, np, ws, st);
-        FZ_LAUNCH("o1_encode_offsets", 0, k_o1_offsets, dim3(nblk(np + nch)), dim3(256), 0, st, CH, np, scan, nbits, bitoff,
-                           chain_bits);
+        uint64_t* dpfirst = ws.take<uint64_t>(nch + 1);
+        h2d(dpfirst, pfirst.data(), nch + 1, st);
+        return O1Chains{dchains, dpfirst, nch, steps_piece};
+    };
+    std::vector<uint64_t> sets_first, pfirst;
+    const bool sets = n <= kSetMaxCodes;
+    uint64_t* failed = blen + nch;
+    if (sets) {
+        const O1Chains CH = lay_out(kSetPiece, sets_first);
+        const uint64_t np = sets_first[nch];
+        uint64_t most = 0;
+        for (int q = 0; q < nch; q++) most = std::max(most, sets_first[q + 1] - sets_first[q]);
+        O1Sets B{ws.take<uint16_t>(np * kSetStates + 1), ws.take<uint16_t>(np * kSetStates + 1),
+                 ws.take<uint16_t>(np * kSetStates + 1), ws.take<uint8_t>(np + 1)};
+        uint32_t* end_state = ws.take<uint32_t>(np + 1);
+        uint64_t* bitoff = ws.take<uint64_t>(np + 1);
+        FZ_HIP(hipMemsetAsync(failed, 0, sizeof(uint64_t), st));
+        if (np)
+            FZ_LAUNCH("o1_encode_sets", n * 4, k_o1_sets, dim3((unsigned)((np + 3) / 4)), dim3(256), 0, st, bins, CH, np, ct, nf,
+                      B, failed);
+        FZ_LAUNCH("o1_encode_walk", 0, k_o1_sets_walk, dim3((unsigned)nch), dim3(256), most * (kSetStates + 1), st, CH, B,
+                  end_state, bitoff, chain_bits, words, stride_words, failed);
+        if (np)
+            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, end_state, bitoff,
+                      words, stride_words, failed);
+        FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_state, chain_bits,
+                  words, stride_words, blen, failed);
         FZ_HIP(hipGetLastError());
-        FZ_LAUNCH("o1_encode_clear", 0, k_o1_clear_shared, dim3(nblk(np + nch)), dim3(256), 0, st, CH, np, bitoff, chain_bits,
-                           words, stride_words);
-        FZ_HIP(hipGetLastError());
-        FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, end_prev, bitoff, words,
-                           stride_words);
-        FZ_HIP(hipGetLastError());
-        FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_prev, chain_bits,
-                           words, stride_words, blen);
-    } else {
-        FZ_HIP(hipMemsetAsync(chain_bits, 0, nch * 8, st));
-        FZ_LAUNCH("o1_encode_clear", 0, k_o1_clear_shared, dim3(nblk(nch)), dim3(256), 0, st, CH, np, bitoff, chain_bits, words,
-                           stride_words);
-        FZ_HIP(hipGetLastError());
-        FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, spec_end, chain_bits,
-                           words, stride_words, blen);
     }
-    FZ_HIP(hipGetLastError());
+    auto guess_and_repair = [&]() {
+        const O1Chains CH = lay_out(kO1Piece, pfirst);
+        const uint64_t np = pfirst[nch];
+        uint16_t* slog = ws.take<uint16_t>(np * kO1Piece + 16);  // step-major: [step in piece][piece]
+        uint32_t* spec_end = ws.take<uint32_t>(np + 1);
+        uint32_t* end_a = ws.take<uint32_t>(np + 1);
+        uint32_t* end_b = ws.take<uint32_t>(np + 1);
+        uint64_t* spec_bits = ws.take<uint64_t>(np + 1);
+        uint64_t* nbits = ws.take<uint64_t>(np + 1);
+        uint8_t* chg_a = ws.take<uint8_t>(np + 1);
+        uint8_t* chg_b = ws.take<uint8_t>(np + 1);
+        unsigned int* any = ws.take<unsigned int>(1);
+        uint64_t* scan = ws.take<uint64_t>(np + 1);
+        uint64_t* bitoff = ws.take<uint64_t>(np + 1);
+        if (np) {
+            FZ_LAUNCH("o1_encode_spec", n * 4, k_o1_spec, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog, spec_end, spec_bits);
+            FZ_HIP(hipGetLastError());
+            FZ_HIP(hipMemcpyAsync(nbits, spec_bits, np * 8, hipMemcpyDeviceToDevice, st));
+            // fix-up rounds; each round finalizes at least the next piece of every chain, so the loop
+            // ends within max-pieces-per-chain rounds
+            const uint32_t* end_prev = spec_end;
+            uint32_t* end_next = end_a;
+            const uint8_t* chg_prev = nullptr;
+            uint8_t* chg_next = chg_a;
+            uint64_t max_rounds = 1;
+            for (int q = 0; q < nch; q++) max_rounds = std::max<uint64_t>(max_rounds, pfirst[q + 1] - pfirst[q] + 1);
+            // Two rounds per host check: `any` counts the changes of the second only. A round after one
+            // with no change re-runs no piece and changes nothing, so the check ends the loop at the
+            // first pair whose second round saw no change.
+            for (uint64_t round = 0;;) {
+                if (round > max_rounds + 1) throw std::runtime_error("tANS piece fix-up did not settle");
+                for (int k = 0; k < 2; k++, round++) {
+                    if (k == 1) FZ_HIP(hipMemsetAsync(any, 0, sizeof(unsigned int), st));
+                    FZ_LAUNCH("o1_encode_fix", 0, k_o1_fix, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog,
+                              spec_end, spec_bits, end_prev, end_next, nbits, chg_prev, chg_next, any);
+                    FZ_HIP(hipGetLastError());
+                    end_prev = end_next;
+                    end_next = (end_next == end_a) ? end_b : end_a;
+                    chg_prev = chg_next;
+                    chg_next = (chg_next == chg_a) ? chg_b : chg_a;
+                }
+                unsigned int h_any = 0;
+                d2h(&h_any, any, 1, st);
+                if (!h_any) break;
+            }
+            exclusive_scan_u64(nbits, scan, np, ws, st);
+            FZ_LAUNCH("o1_encode_offsets", 0, k_o1_offsets, dim3(nblk(np + nch)), dim3(256), 0, st, CH, np, scan, nbits, bitoff,
+                               chain_bits);
+            FZ_HIP(hipGetLastError());
+            FZ_LAUNCH("o1_encode_clear", 0, k_o1_clear_shared, dim3(nblk(np + nch)), dim3(256), 0, st, CH, np, bitoff, chain_bits,
+                               words, stride_words);
+            FZ_HIP(hipGetLastError());
+            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, end_prev, bitoff, words,
+                               stride_words, (const uint64_t*)nullptr);
+            FZ_HIP(hipGetLastError());
+            FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_prev, chain_bits,
+                               words, stride_words, blen, (const uint64_t*)nullptr);
+        } else {
+            FZ_HIP(hipMemsetAsync(chain_bits, 0, nch * 8, st));
+            FZ_LAUNCH("o1_encode_clear", 0, k_o1_clear_shared, dim3(nblk(nch)), dim3(256), 0, st, CH, np, bitoff, chain_bits, words,
+                               stride_words);
+            FZ_HIP(hipGetLastError());
+            FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, spec_end, chain_bits,
+                               words, stride_words, blen, (const uint64_t*)nullptr);
+        }
+        FZ_HIP(hipGetLastError());
+    };
+    if (!sets) guess_and_repair();
     // escape side streams, one block per segment
     if (aux.stream) ew.join();
     else escape_streams(ovf, ovf_off, S, oblock, ws, st);
-    std::vector<uint64_t> hblen(nch);
-    d2h(hblen.data(), blen, nch, st);
+    std::vector<uint64_t> hblen(nch + 1);
+    d2h(hblen.data(), blen, nch + (sets ? 1 : 0), st);
+    if (sets && hblen[nch]) {  // symbols too frequent or too flat for sets: nothing has been written yet
+        guess_and_repair();
+        d2h(hblen.data(), blen, nch, st);
+    }
     // assemble: [u64 S] then per segment [n][K][blen x4][novf x4][nf][streams][ovf block]
     uint64_t total = 8;
     for (uint64_t g = 0; g < S; g++) {
