@@ -399,256 +399,38 @@ __device__ void dtable_parallel(TL& L, unsigned tl, DEntry* dt) {
 }
 
 // ---------------------------------------------------------------- FSE block (workgroup-wide)
-// FSE_compress of one block of at most 64 K bytes (fse_compress.c:632-694), run by one workgroup.
-// The block is staged in LDS, histogram, spread and table build are shared by the workgroup, and
-// normalization, the table header and the two-state encode run on lane 0 against LDS only (its
-// input and its output bytes); the framed result is copied out by the whole workgroup.
+// FSE_compress of blocks of at most 64 K bytes (fse_compress.c:632-694), framed as in RleFse:150-176:
+// [0][raw] | [2][sym] | [1][u32 len][FSE bytes].
 // FSE_compress bounds the table log by FSE_DEFAULT_TABLELOG (11).
+//
+// The encode (fse_compress.c:578-628) emits symbols n-3 down to 0 alternately from two states, the
+// first of them seeded by symbol n-1 and the second by n-2 (in zfse's names: state 2 then state 1
+// for an even n, state 1 then state 2 for an odd one), then state 2's and state 1's final values
+// (tl bits each) and the end mark; the bytes are those bits LSB-first. A lane that follows each state
+// through its half of the symbols needs 32,768 dependent table steps of 80 ns for a block of 64 K.
+// Runs from two states under the same symbols do not soon become one (after 1,500 steps for the
+// classes of escaped codes, 12,000 for five equally frequent symbols), but after a symbol of count c
+// only c states of 2,048 are left, and a few dozen 300 steps on. So the two chains are cut into pieces of
+// 1,024 steps, a wave follows all states that a symbol in front of its piece leaves, one a lane at the
+// piece (k_fse_sets), and a walk from piece to piece picks the true ones, with the bits of every 128
+// steps noted on the way (k_fse_finish, which then writes the bits, 256 lanes a block). A piece that
+// more than 64 states reach (two symbols of equal counts: no two states ever meet) is run by the walk.
+// 138 blocks (9 million escapes of a 512^3 field at 1e-3): 2.6 ms -> 0.37; 765 blocks (50 million, at
+// 1e-4): 4.2 -> 1.9, the waves' LDS reads by then; one block of 35,000: 1.29 -> 0.23. Pieces of 512
+// steps run half as many steps twice: 2.4 ms for the 765 blocks, the others the same.
 constexpr unsigned kFblkLog = kFseDefaultTableLog;
-
-// The encoder's LDS: the block's histogram and its tables (a few KB, so that many blocks run on a
-// CU at once); the block's bytes are read from device memory and the FSE bytes go straight to the
-// block's output slot.
-constexpr uint32_t kFseTileWords = (256 * kFblkLog + 31) / 32 + 3;
-struct FseLds {
-    uint32_t count[256];
-    TableLdsT<kFblkLog> tab;
-    CTableT<kFblkLog> ct;
-    uint64_t result, nc, sbits;
-    uint32_t tl, maxSym;
-    uint32_t fin[2];     // the final values of state 2 and state 1
-    uint32_t part[4];    // per-wave sums
-    uint32_t tw[kFseTileWords];  // a tile's packed words (256 emissions of at most 11 bits, a carried word)
-};
-
-// Writes the FSE bytes (when the result is > 1) to fo, which has room for n + 1024 bytes. pre holds
-// n 16-bit values of scratch (the state before every symbol's step). Returns 0 (not compressible),
-// 1 (one symbol), kFseErr, or the compressed size.
-__device__ uint64_t fse_block_compress_wg(const uint8_t* src, uint32_t n, uint8_t* fo, FseLds& L, uint16_t* pre) {
-    const uint8_t* const src_in = src;
-    uint16_t* const pre_in = pre;
-    constexpr uint64_t kPending = ~1ull;
-    for (int s = threadIdx.x; s < 256; s += blockDim.x) L.count[s] = 0;
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) atomicAdd(&L.count[src[i]], 1u);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t r = kPending;
-        if (n <= 1) {
-            r = 0;
-        } else {
-            unsigned maxSym = 255;
-            while (!L.count[maxSym]) maxSym--;
-            uint32_t maxCount = 0;
-            for (unsigned s = 0; s <= maxSym; s++) maxCount = L.count[s] > maxCount ? L.count[s] : maxCount;
-            if (maxCount == n) r = 1;
-            else if (maxCount == 1 || maxCount < (n >> 7)) r = 0;
-            else {
-                const unsigned tl = optimal_table_log(kFseDefaultTableLog, n, maxSym);
-                for (unsigned s = maxSym + 1; s < 256; s++) L.tab.norm[s] = 0;
-                if (tl > kFblkLog || normalize_count(L.tab.norm, tl, L.count, n, maxSym) == kFseErr) {
-                    r = kFseErr;
-                } else {
-                    L.nc = write_ncount(fo, L.tab.norm, maxSym, tl);
-                    L.tl = tl;
-                    L.maxSym = maxSym;
-                }
-            }
-        }
-        L.result = r;
-    }
-    __syncthreads();
-    if (L.result != kPending) return L.result;
-    const unsigned tl = L.tl;
-    if (!spread_parallel(L.tab, tl)) {  // cannot happen for counts from normalize_count
-        if (threadIdx.x == 0) L.result = kFseErr;
-        __syncthreads();
-        return L.result;
-    }
-    ctable_parallel(L.tab, tl, L.maxSym, &L.ct);
-    __syncthreads();
-    // The encode (fse_compress.c:578-628) emits symbols n-3 down to 0 alternately from two states,
-    // the first of them seeded by symbol n-1 and the second by n-2 (in zfse's names: state 2 then
-    // state 1 for an even n, state 1 then state 2 for an odd one), then state 2's and state 1's
-    // final values (tl bits each) and the end mark; the bytes are those bits LSB-first. The two
-    // states never interact, so lanes 0 and 1 run one chain each, logging every symbol's state
-    // before its step (pre); the workgroup then scans the bit counts in emission order and packs
-    // the bits in parallel.
-    const FZ_LDS uint32_t* dnb = lds(L.ct.deltaNbBits);
-    const FZ_LDS int32_t* dfs = lds(L.ct.deltaFindState);
-    const FZ_LDS uint16_t* stt = lds(L.ct.stateTable);
-    if (threadIdx.x < 2) {
-        const uint32_t k = threadIdx.x;  // chain k emits e = k, k + 2, ... (symbol n - 3 - e)
-        const FZ_GLB uint8_t* src = glb(src_in);
-        FZ_GLB uint16_t* pre = glb(pre_in);
-        uint32_t s = init_state2(&L.ct, src[n - 1 - k]);
-        int64_t j = (int64_t)n - 3 - k;
-        // Four steps per round (symbols jj, jj - 2, jj - 4, jj - 6); the round's table values are
-        // read first (they do not depend on the state), and its symbols two rounds earlier, so that
-        // their loads are in flight for the eight steps before them. Three register sets take turns
-        // (no copies between them, which would wait for the loads); reads below symbol 0 are clamped
-        // to it and not used.
-        auto ld4 = [&](uint32_t (&g)[4], int64_t jj) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) g[r] = src[max(jj - 2 * r, (int64_t)0)];
-        };
-        auto round4 = [&](const uint32_t (&cur)[4], uint32_t (&ahead)[4], int64_t jj) {
-            ld4(ahead, jj - 16);
-            uint32_t d[4];
-            int32_t f[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                d[r] = dnb[cur[r]];
-                f[r] = dfs[cur[r]];
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                pre[jj - 2 * r] = (uint16_t)s;
-                const uint32_t nb = (s + d[r]) >> 16;
-                s = stt[(s >> nb) + f[r]];
-            }
-        };
-        uint32_t sa[4], sb[4], sc[4];
-        ld4(sa, j);
-        ld4(sb, j - 8);
-        // Wait for these first loads here, once (an empty statement that takes them as operands):
-        // the loop's head then needs only the waits of its own iterations; the compiler otherwise
-        // takes the head's wait from this entry path, where the loads were just issued.
-        asm volatile("" ::"v"(sa[0]), "v"(sa[1]), "v"(sa[2]), "v"(sa[3]), "v"(sb[0]), "v"(sb[1]), "v"(sb[2]),
-                     "v"(sb[3]));
-        for (;;) {
-            if (j < 6) break;
-            round4(sa, sc, j);
-            j -= 8;
-            if (j < 6) break;
-            round4(sb, sa, j);
-            j -= 8;
-            if (j < 6) break;
-            round4(sc, sb, j);
-            j -= 8;
-        }
-        for (; j >= 0; j -= 2) {
-            const uint32_t sym = src[j];
-            pre[j] = (uint16_t)s;
-            const uint32_t nb = (s + dnb[sym]) >> 16;
-            s = stt[(s >> nb) + dfs[sym]];
-        }
-        // state 2 is chain 0 for an even n, chain 1 for an odd one
-        L.fin[((n & 1u) == 0) == (k == 0) ? 0 : 1] = s;
-    }
-    __syncthreads();
-    // the bit counts in emission order, summed over the workgroup (one emission per thread per
-    // tile of blockDim.x, so the reads of pre and src coalesce)
-    const uint32_t m = n - 2;  // emissions e: symbol n - 3 - e
-    auto nbits_of = [&](uint32_t e) -> uint32_t {
-        const uint32_t j = n - 3 - e;
-        return (pre[j] + dnb[src[j]]) >> 16;
-    };
-    uint32_t mine = 0;
-    for (uint32_t e = threadIdx.x; e < m; e += blockDim.x) mine += nbits_of(e);
-    for (uint32_t d = 32; d; d >>= 1) mine += __shfl_xor(mine, d, 64);
-    if ((threadIdx.x & 63u) == 0) L.part[threadIdx.x >> 6] = mine;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t acc = 0;
-        for (uint32_t w = 0; w < blockDim.x / 64; w++) acc += L.part[w];
-        const uint64_t bits = acc + 2 * (uint64_t)tl + 1;
-        L.sbits = acc;
-        const uint64_t total = L.nc + (bits + 7) / 8;
-        L.result = (total >= n - 1) ? 0 : total;
-    }
-    __syncthreads();
-    if (L.result == 0) return 0;
-    // pack, tile by tile: each thread places its emission's bits in an LDS word buffer at its
-    // scanned offset; the tile's whole words are stored, the partial last one carries over
-    uint8_t* sb = fo + L.nc;
-    const uint32_t lead = (uint32_t)((uintptr_t)sb & 3u);  // stream bytes in front, in the first word
-    uint32_t* wbase = reinterpret_cast<uint32_t*>(sb - lead);
-    uint32_t* tb = L.tw;
-    for (uint32_t w = threadIdx.x; w < kFseTileWords; w += blockDim.x) tb[w] = 0;
-    __syncthreads();
-    if (threadIdx.x == 0 && lead) tb[0] = wbase[0] & ((1u << (8 * lead)) - 1u);  // the header's last bytes
-    uint64_t cur = 8 * (uint64_t)lead;  // bit position (from wbase) of the next emission
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    auto place = [&](uint64_t b, uint32_t v, uint32_t nb) {  // b: bit position from word cur >> 5
-        if (!nb) return;
-        v &= (1u << nb) - 1u;
-        const uint32_t wi = (uint32_t)(b >> 5), sh = (uint32_t)(b & 31u);
-        atomicOr(&tb[wi], v << sh);
-        if (sh + nb > 32) atomicOr(&tb[wi + 1], v >> (32 - sh));
-    };
-    auto drain = [&](uint64_t end) {  // store the whole words below bit `end`, keep the partial one
-        const uint64_t w0 = cur >> 5;
-        const uint32_t nw = (uint32_t)((end >> 5) - w0);
-        __syncthreads();
-        for (uint32_t w = threadIdx.x; w < nw; w += blockDim.x) wbase[w0 + w] = tb[w];
-        __syncthreads();
-        const uint32_t carry = tb[nw];
-        __syncthreads();
-        for (uint32_t w = threadIdx.x; w < kFseTileWords; w += blockDim.x) tb[w] = w == 0 ? carry : 0u;
-        __syncthreads();
-        cur = end;
-    };
-    for (uint32_t t0 = 0; t0 < m; t0 += blockDim.x) {
-        const uint32_t e = t0 + threadIdx.x;
-        uint32_t v = 0, nb = 0;
-        if (e < m) {
-            const uint32_t j = n - 3 - e;
-            v = pre[j];
-            nb = (v + dnb[src[j]]) >> 16;
-        }
-        // exclusive scan of nb over the tile: within the wave, then across the waves
-        uint32_t inc = nb;
-#pragma unroll
-        for (uint32_t d = 1; d < 64; d <<= 1) {
-            const uint32_t y = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += y;
-        }
-        if (lane == 63) L.part[wv] = inc;
-        __syncthreads();
-        uint32_t before = 0, tile = 0;
-        for (uint32_t w = 0; w < blockDim.x / 64; w++) {
-            const uint32_t pw = L.part[w];
-            if (w < wv) before += pw;
-            tile += pw;
-        }
-        place((cur & 31u) + before + inc - nb, v, nb);
-        drain(cur + tile);
-    }
-    if (threadIdx.x == 0) {
-        // state 2's and state 1's final values, then the end mark (BIT_closeCStream)
-        const uint64_t b = cur & 31u;
-        place(b, L.fin[0], tl);
-        place(b + tl, L.fin[1], tl);
-        place(b + 2 * tl, 1u, 1);
-    }
-    drain(cur + 2 * (uint64_t)tl + 1 + 31);  // the last partial word too
-    return L.result;
-}
-
-// Frames one class-byte block as in RleFse:150-176: [0][raw] | [2][sym] | [1][u32 len][FSE bytes].
-// Returns the framed length written to out.
-__device__ uint64_t frame_block_wg(const uint8_t* src, uint32_t len, uint8_t* out, FseLds& L, uint16_t* pre) {
-    const uint64_t r = fse_block_compress_wg(src, len, out + 5, L, pre);
-    uint64_t sz;
-    if (r == kFseErr || r == 0 || r >= len) {
-        if (threadIdx.x == 0) out[0] = 0;
-        for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) out[1 + i] = src[i];
-        sz = 1 + len;
-    } else if (r == 1) {
-        if (threadIdx.x == 0) { out[0] = 2; out[1] = src[0]; }
-        sz = 2;
-    } else {
-        if (threadIdx.x == 0) {
-            out[0] = 1;
-            const uint32_t rr = (uint32_t)r;
-            out[1] = (uint8_t)rr; out[2] = (uint8_t)(rr >> 8); out[3] = (uint8_t)(rr >> 16); out[4] = (uint8_t)(rr >> 24);
-        }
-        sz = 5 + r;  // the FSE bytes are in place
-    }
-    __syncthreads();
-    return sz;
-}
+constexpr uint32_t kFseGroup = 16;      // symbols of a load
+constexpr uint32_t kFseHists = 8;
+constexpr uint32_t kFseSub = 128;       // steps of a chain between noted states
+constexpr uint32_t kFsePiece = 1024;    // steps of a chain in a piece
+constexpr uint32_t kFseSubs = kFblk / (2 * kFseSub), kFsePieces = kFblk / (2 * kFsePiece);
+constexpr uint32_t kFseFields = kFsePiece / kFseSub + 1;
+constexpr uint32_t kFseWarm = 448;      // steps in front of a piece; the first 128 are searched
+constexpr uint32_t kFseSearch = 128;
+constexpr uint32_t kFseWarmFew = 704;   // up to here for a symbol of a count up to 256, then up to 1,024
+constexpr uint32_t kFseWarmMax = 8192;  // how far back the search goes
+constexpr uint32_t kFseLogWords = 2 * kFsePieces * kFseFields * 64;  // a block's noted states
+constexpr uint64_t kFsePending = ~1ull;
 
 // One FSE block of a batch: its input (class bytes, or a framed block to decode), its output and
 // its length in symbols (at most 64 K).
@@ -658,13 +440,449 @@ struct FseBlk {
     uint32_t len, pad;
 };
 
-// One workgroup per 64 K block (the blocks of every stream of a call in one launch); framed
-// blocks land in fixed slots.
-__global__ void __launch_bounds__(256) k_fse_blocks(const FseBlk* blks, uint8_t* slots, uint64_t* sizes, uint16_t* pre) {
-    __shared__ FseLds L;
-    const uint64_t b = blockIdx.x;
-    const uint64_t sz = frame_block_wg(blks[b].src, blks[b].len, slots + b * (kFblk + 1024), L, pre + b * kFblk);
-    if (threadIdx.x == 0) sizes[b] = sz;
+// What the kernels of a block hand on. result: 0 (not compressible), 1 (one symbol), kFseErr, or kFsePending.
+struct FseMeta {
+    CTableT<kFblkLog> ct;
+    uint64_t result;
+    uint32_t nc, tl;  // header bytes, table log
+};
+
+// 16 symbols ending below symbol h, the last of them in byte 15 (below symbol 0: zeros, not used).
+__device__ __forceinline__ void fse_group(const uint8_t* src, uint32_t h, uint32_t (&w)[4]) {
+    if (h >= kFseGroup) {
+        __builtin_memcpy(w, src + h - kFseGroup, kFseGroup);
+    } else {
+        w[0] = w[1] = w[2] = w[3] = 0;
+        for (uint32_t j = 0; j < h; j++) {
+            const uint32_t at = kFseGroup - h + j, v = (uint32_t)src[j] << (8 * (at & 3u));
+            w[0] |= at < 4 ? v : 0u;
+            w[1] |= at >= 4 && at < 8 ? v : 0u;
+            w[2] |= at >= 8 && at < 12 ? v : 0u;
+            w[3] |= at >= 12 ? v : 0u;
+        }
+    }
+}
+
+// Both chains over the symbols hi - 1 down to lo (hi - lo a multiple of 16, or lo == 0), the first
+// of them on chain 0. sink(value, bits) takes every emission in its order.
+template <class F>
+__device__ __forceinline__ void fse_run(const uint8_t* src, uint32_t hi, uint32_t lo, const CTableT<kFblkLog>& ct,
+                                        uint32_t& s0, uint32_t& s1, F&& sink) {
+    const FZ_LDS uint32_t* dnb = lds(ct.deltaNbBits);
+    const FZ_LDS int32_t* dfs = lds(ct.deltaFindState);
+    const FZ_LDS uint16_t* stt = lds(ct.stateTable);
+    uint32_t cur[4], nxt[4];
+    fse_group(src, hi, nxt);
+    for (uint32_t h = hi; h > lo;) {
+        const uint32_t cnt = min(h - lo, kFseGroup);
+#pragma unroll
+        for (int r = 0; r < 4; r++) cur[r] = nxt[r];
+        h -= cnt;
+        if (h > lo) fse_group(src, h, nxt);
+        auto pair = [&](uint32_t a, uint32_t b, bool two) {
+            const uint32_t n0 = (s0 + dnb[a]) >> 16;
+            sink(s0, n0);
+            s0 = stt[(s0 >> n0) + dfs[a]];
+            if (two) {
+                const uint32_t n1 = (s1 + dnb[b]) >> 16;
+                sink(s1, n1);
+                s1 = stt[(s1 >> n1) + dfs[b]];
+            }
+        };
+        if (cnt == kFseGroup) {
+#pragma unroll
+            for (int r = 3; r >= 0; r--) {
+                pair(cur[r] >> 24, cur[r] >> 16 & 255u, true);
+                pair(cur[r] >> 8 & 255u, cur[r] & 255u, true);
+            }
+        } else {  // the block's last symbols
+            for (uint32_t k = 0; k < cnt; k += 2) {
+                const uint32_t at = kFseGroup - 1 - k;  // odd: both bytes in one word
+                const uint32_t r = at >> 2, w = r == 3 ? cur[3] : r == 2 ? cur[2] : r == 1 ? cur[1] : cur[0];
+                pair(w >> (8 * (at & 3u)) & 255u, w >> (8 * (at & 3u) - 8) & 255u, k + 1 < cnt);
+            }
+        }
+    }
+}
+
+// Histogram, normalization, table header (to the block's slot) and encoding table of a block, by a
+// workgroup; normalization and header by lane 0 (a class stream has few symbols).
+__global__ void __launch_bounds__(256) k_fse_tables(const FseBlk* blks, uint8_t* slots, uint64_t slot, FseMeta* meta) {
+    __shared__ union {
+        uint32_t hist[kFseHists][256];  // one for every eighth lane: fewer adds to one word
+        TableLdsT<kFblkLog> tab;
+    } L;
+    __shared__ uint32_t count[256];
+    __shared__ CTableT<kFblkLog> ct;
+    __shared__ uint64_t result;
+    __shared__ uint32_t max_sym, log, head;
+    const uint8_t* src = blks[blockIdx.x].src;
+    const uint32_t n = blks[blockIdx.x].len, t = threadIdx.x;
+    FseMeta& M = meta[blockIdx.x];
+    for (uint32_t i = t; i < kFseHists * 256; i += blockDim.x) L.hist[i >> 8][i & 255u] = 0;
+    __syncthreads();
+    for (uint32_t i = t * kFseGroup; i < n; i += blockDim.x * kFseGroup) {
+        uint32_t* hist = L.hist[t & (kFseHists - 1)];
+        if (i + kFseGroup <= n) {
+            uint32_t w[4];
+            __builtin_memcpy(w, src + i, kFseGroup);
+#pragma unroll
+            for (int r = 0; r < 16; r++) atomicAdd(&hist[w[r >> 2] >> (8 * (r & 3)) & 255u], 1u);
+        } else {
+            for (uint32_t j = i; j < n; j++) atomicAdd(&hist[src[j]], 1u);
+        }
+    }
+    __syncthreads();
+    uint32_t c = 0;
+    for (uint32_t k = 0; k < kFseHists; k++) c += L.hist[k][t];
+    count[t] = c;
+    __syncthreads();
+    if (t == 0) {
+        uint64_t r = kFsePending;
+        head = log = max_sym = 0;
+        if (n <= 1) {
+            r = 0;
+        } else {
+            unsigned maxSym = 255;
+            while (!count[maxSym]) maxSym--;
+            uint32_t maxCount = 0;
+            for (unsigned s = 0; s <= maxSym; s++) maxCount = count[s] > maxCount ? count[s] : maxCount;
+            if (maxCount == n) r = 1;
+            else if (maxCount == 1 || maxCount < (n >> 7)) r = 0;
+            else {
+                const unsigned tl = optimal_table_log(kFseDefaultTableLog, n, maxSym);
+                for (unsigned s = maxSym + 1; s < 256; s++) L.tab.norm[s] = 0;
+                if (tl > kFblkLog || normalize_count(L.tab.norm, tl, count, n, maxSym) == kFseErr) {
+                    r = kFseErr;
+                } else {
+                    head = (uint32_t)write_ncount(slots + blockIdx.x * slot + 5, L.tab.norm, maxSym, tl);
+                    log = tl;
+                    max_sym = maxSym;
+                }
+            }
+        }
+        result = r;
+    }
+    __syncthreads();
+    if (result == kFsePending) {
+        if (spread_parallel(L.tab, log)) {
+            ctable_parallel(L.tab, log, max_sym, &ct);
+            __syncthreads();
+            const uint32_t* from = reinterpret_cast<const uint32_t*>(&ct);
+            uint32_t* to = reinterpret_cast<uint32_t*>(&M.ct);
+            for (uint32_t i = t; i < sizeof(ct) / 4; i += blockDim.x) to[i] = from[i];
+        } else {  // cannot happen for counts from normalize_count
+            __syncthreads();
+            if (t == 0) result = kFseErr;
+            __syncthreads();
+        }
+    }
+    if (t == 0) {
+        M.result = result;
+        M.nc = head;
+        M.tl = log;
+    }
+}
+
+__device__ __forceinline__ void fse_stage_table(CTableT<kFblkLog>& ct, const FseMeta& M) {
+    const uint32_t* from = reinterpret_cast<const uint32_t*>(&M.ct);
+    uint32_t* to = reinterpret_cast<uint32_t*>(&ct);
+    for (uint32_t i = threadIdx.x; i < sizeof(ct) / 4; i += blockDim.x) to[i] = from[i];
+    __syncthreads();
+}
+
+// Steps t0 up to t1 of a chain (step t codes symbol top[-2t]) for the R states of every lane: the lanes
+// look up 64 steps at once (their symbols do not depend on the states), the next 64 symbols in flight.
+template <int R>
+__device__ __forceinline__ void fse_set_run(const uint8_t* top, uint32_t t0, uint32_t t1, const CTableT<kFblkLog>& ct,
+                                            uint32_t (&st)[R], uint32_t& bits) {
+    if (t0 >= t1) return;
+    const uint32_t lane = threadIdx.x & 63u;
+    const FZ_LDS uint32_t* dnb = lds(ct.deltaNbBits);
+    const FZ_LDS int32_t* dfs = lds(ct.deltaFindState);
+    const FZ_LDS uint16_t* stt = lds(ct.stateTable);
+    auto load = [&](uint32_t t) { return (uint32_t)glb(top)[-2 * (int64_t)min(t + lane, t1 - 1)]; };
+    uint32_t next = load(t0);
+    for (uint32_t t = t0; t < t1; t += 64) {
+        const uint32_t d = dnb[next];
+        const int32_t f = dfs[next];
+        if (t + 64 < t1) next = load(t + 64);
+        auto step = [&](int k) {
+            const uint32_t dk = (uint32_t)__builtin_amdgcn_readlane((int)d, k);
+            const int32_t fk = __builtin_amdgcn_readlane(f, k);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint32_t nb = (st[r] + dk) >> 16;
+                if (r == 0) bits += nb;
+                st[r] = stt[(int32_t)(st[r] >> nb) + fk];
+            }
+        };
+        const int cnt = (int)min(t1 - t, 64u);
+        if (cnt == 64 && R == 1) {
+#pragma unroll 16
+            for (int k = 0; k < 64; k++) step(k);
+        } else {
+            for (int k = 0; k < cnt; k++) step(k);
+        }
+    }
+}
+
+// The different ones of a wave's states (at least 1 << tl, below twice that), Q a lane, the last one filling
+// the lanes left over. map: 64 words, list: 64 * Q states of LDS. False when there are more than that.
+template <int R, int Q>
+__device__ __forceinline__ bool fse_set_merge(const uint32_t (&st)[R], uint32_t (&out)[Q], uint32_t tl, FZ_LDS uint32_t* map,
+                                              FZ_LDS uint16_t* list) {
+    const uint32_t lane = threadIdx.x & 63u;
+    map[lane] = 0;
+    wave_lds_order();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t x = st[r] - (1u << tl);
+        __hip_atomic_fetch_or(&map[x >> 5], 1u << (x & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    wave_lds_order();
+    uint32_t w = map[lane], inc = __popc(w);
+    const uint32_t own = inc;
+#pragma unroll
+    for (uint32_t d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += y;
+    }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    if (total > 64 * Q) return false;
+    for (uint32_t at = inc - own; w; w &= w - 1) list[at++] = (uint16_t)((1u << tl) + lane * 32 + __ffs(w) - 1);
+    wave_lds_order();
+#pragma unroll
+    for (int r = 0; r < Q; r++) out[r] = list[min(r * 64 + lane, total - 1)];
+    wave_lds_order();
+    return true;
+}
+
+// The steps t0 up to t1 of a piece: every lane's state at the start, after each 128 steps and at the end, with
+// the bits of those steps.
+__device__ __forceinline__ void fse_log_piece(const uint8_t* top, uint32_t t0, uint32_t t1, const CTableT<kFblkLog>& ct,
+                                              uint32_t (&st)[1], uint32_t* log) {
+    for (uint32_t f = 0; f + 1 < kFseFields && t0 + f * kFseSub < t1; f++) {
+        const uint32_t at = st[0];
+        uint32_t bits = 0;
+        fse_set_run(top, t0 + f * kFseSub, min(t1, t0 + (f + 1) * kFseSub), ct, st, bits);
+        log[f * 64] = at | bits << 16;
+    }
+    log[(kFseFields - 1) * 64] = st[0];
+}
+
+// A wave a piece of a chain (grid: blocks, pieces of both chains / 4). Bound by the latency of the steps' LDS reads.
+__global__ void __launch_bounds__(256) k_fse_sets(const FseBlk* blks, const FseMeta* meta, uint32_t* logs) {
+    __shared__ CTableT<kFblkLog> ct;
+    __shared__ uint32_t maps[4][64];
+    __shared__ uint16_t lists[4][256];
+    const uint32_t b = blockIdx.x, lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t unit = uniform32(blockIdx.y * 4u + wv), k = unit & 1u, p = unit >> 1;
+    const uint32_t n = blks[b].len;
+    // n >= 3 where a result is pending; a chain's steps are the emissions k, k + 2, ... below n - 2
+    if (meta[b].result != kFsePending || blockIdx.y * 2u * kFsePiece >= (n - 1) / 2) return;
+    const uint32_t tl = meta[b].tl;
+    fse_stage_table(ct, meta[b]);
+    const uint32_t steps = (n - 1 - k) / 2, t0 = p * kFsePiece, t1 = min(steps, t0 + kFsePiece);
+    if (t0 >= steps) return;
+    const uint8_t* src = blks[b].src;
+    const uint8_t* top = src + (n - 3 - k);
+    FZ_LDS uint32_t* map = lds(maps[wv]);
+    FZ_LDS uint16_t* list = lds(lists[wv]);
+    uint32_t* log = logs + (uint64_t)b * kFseLogWords + (k * kFsePieces + p) * kFseFields * 64 + lane;
+    uint32_t st[1], from = 0, bits = 0;  // from: the first step that is left to run with one state a lane
+    bool found = false;
+    for (uint32_t warm = kFseWarm; !found;) {
+        if (t0 <= warm) {  // from the block's end, where the state is known
+            st[0] = init_state2(&ct, src[n - 1 - k]);
+            from = 0;
+            break;
+        }
+        if (warm > kFseWarmMax) {
+            log[0] = 0;  // no state is 0: the walk runs this piece
+            return;
+        }
+        uint32_t best = ~0u;
+#pragma unroll
+        for (uint32_t h = 0; h < kFseSearch; h += 64) {
+            const uint32_t d = ct.deltaNbBits[top[-2 * (int64_t)(t0 - warm + h + lane)]];
+            const uint32_t mb = (d >> 16) + 1;  // d = (mb << 16) - (c << mb)
+            best = min(best, ((mb << 16) - d) >> mb << 8 | (h + lane));
+        }
+#pragma unroll
+        for (uint32_t d = 32; d; d >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, (int)d, 64));
+        best = uniform32(best);
+        const uint32_t c = best >> 8;
+        if (c > (warm <= kFseWarmFew ? 256u : 1024u)) {
+            warm += kFseSearch;
+            continue;
+        }
+        // the c states that the symbol of step from - 1 leaves
+        from = t0 - warm + (best & 255u) + 1;
+        const uint16_t* image = ct.stateTable + (ct.deltaFindState[top[-2 * (int64_t)(from - 1)]] + (int32_t)c);
+        if (c <= 64) {
+            st[0] = image[min(lane, c - 1)];
+            break;
+        }
+        uint32_t s4[4];
+        bool room = true;
+        if (c <= 256) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) s4[r] = image[min(r * 64 + lane, c - 1)];
+        } else {
+            uint32_t s16[16];
+#pragma unroll
+            for (uint32_t r = 0; r < 16; r++) s16[r] = image[min(r * 64 + lane, c - 1)];
+            fse_set_run(top, from, from + 64, ct, s16, bits);  // at least 320 steps in front of the piece
+            from += 64;
+            room = fse_set_merge(s16, s4, tl, map, list);
+        }
+        while (room && !found && from < t0) {
+            const uint32_t to = min(from + 256, t0);
+            fse_set_run(top, from, to, ct, s4, bits);
+            from = to;
+            found = fse_set_merge(s4, st, tl, map, list);
+        }
+        warm *= 2;  // more than 64 are left: from further back
+    }
+    fse_set_run(top, from, t0, ct, st, bits);
+    fse_log_piece(top, t0, t1, ct, st, log);
+}
+static_assert(kFseWarm >= kFseSearch + 64 + 256, "the merging runs end in front of the piece");
+
+// A workgroup a block: the true states of both chains at every 256 symbols, the bits' places, the bits,
+// the frame. sizes: the framed length.
+__global__ void __launch_bounds__(256) k_fse_finish(const FseBlk* blks, const FseMeta* meta, uint32_t* logs,
+                                                    uint8_t* slots, uint64_t slot, uint64_t* sizes) {
+    __shared__ CTableT<kFblkLog> ct;
+    __shared__ uint64_t scan[4];
+    __shared__ uint32_t sub_state[kFseSubs], sub_bits[kFseSubs];  // states: chain 0 low, chain 1 high
+    __shared__ uint32_t fin[2];
+    __shared__ uint8_t pick[2][kFsePieces];
+    const uint32_t b = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    const uint8_t* src = blks[b].src;
+    const uint32_t n = blks[b].len;
+    uint8_t* out = slots + b * slot;
+    uint8_t* fo = out + 5;
+    uint64_t r = meta[b].result;
+    const uint32_t tl = meta[b].tl, nc = meta[b].nc;
+    if (r == kFsePending) {
+        fse_stage_table(ct, meta[b]);
+        const uint32_t m = n - 2;  // emissions: symbols n - 3 .. 0
+        if (wv < 2) {
+            const uint32_t k = wv, steps = (m - k + 1) / 2, np = (steps + kFsePiece - 1) / kFsePiece;
+            uint32_t* log = logs + (uint64_t)b * kFseLogWords + k * kFsePieces * kFseFields * 64 + lane;
+            uint32_t cur = uniform32(init_state2(&ct, src[n - 1 - k]));
+            for (uint32_t p0 = 0; p0 < np; p0 += 8) {
+                uint32_t s[8], e[8];
+#pragma unroll
+                for (uint32_t j = 0; j < 8; j++) {
+                    const uint32_t p = min(p0 + j, np - 1);
+                    s[j] = log[p * kFseFields * 64];
+                    e[j] = log[(p * kFseFields + kFseFields - 1) * 64];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 8; j++) {
+                    if (p0 + j < np) {
+                        const uint64_t hit = __ballot((s[j] & 0xFFFFu) == cur);
+                        const uint32_t w = hit ? (uint32_t)__ffsll((unsigned long long)hit) - 1u : 0u;
+                        if (lane == 0) pick[k][p0 + j] = (uint8_t)w;
+                        if (hit) {
+                            cur = (uint32_t)__builtin_amdgcn_readlane((int)e[j], (int)w) & 0xFFFFu;
+                        } else {  // a piece without a set
+                            uint32_t st[1] = {cur};
+                            const uint32_t t0 = (p0 + j) * kFsePiece;
+                            fse_log_piece(src + (n - 3 - k), t0, min(steps, t0 + kFsePiece), ct, st,
+                                          log + (p0 + j) * kFseFields * 64);
+                            cur = uniform32(st[0]);
+                        }
+                    }
+                }
+            }
+            if (lane == 0) fin[k] = cur;
+        }
+        __syncthreads();
+        const uint32_t hi = t * 2 * kFseSub < m ? m - t * 2 * kFseSub : 0u, lo = hi > 2 * kFseSub ? hi - 2 * kFseSub : 0u;
+        if (hi) {
+            uint32_t w[2] = {0, 0};
+            for (uint32_t k = 0; k < 2; k++) {
+                const uint32_t p = t / (kFseFields - 1), f = t % (kFseFields - 1);
+                if (t * kFseSub < (m - k + 1) / 2)  // m odd: chain 1 can end a piece earlier
+                    w[k] = logs[(uint64_t)b * kFseLogWords + ((k * kFsePieces + p) * kFseFields + f) * 64 + pick[k][p]];
+            }
+            sub_state[t] = (w[0] & 0xFFFFu) | w[1] << 16;
+            sub_bits[t] = (w[0] >> 16) + (w[1] >> 16);
+        }
+        __syncthreads();
+        uint64_t sbits;
+        const uint64_t off0 = block_scan_u64(hi ? sub_bits[t] : 0u, scan, &sbits);
+        const uint64_t total = nc + (sbits + 2 * (uint64_t)tl + 1 + 7) / 8;
+        r = total >= n - 1 ? 0 : total;
+        if (r) {
+            // Bits go to whole words from the last word boundary at or before the stream (the header's
+            // last bytes share it). A lane stores the words that only it reaches; a word that two lanes
+            // share is cleared first and takes its parts by atomics, as do those of the closing states.
+            uint8_t* sb = fo + nc;
+            const uint32_t lead = (uint32_t)((uintptr_t)sb & 3u);
+            uint32_t* wbase = reinterpret_cast<uint32_t*>(sb - lead);
+            const uint64_t off = off0 + 8 * lead, fin_bit = sbits + 8 * lead;
+            uint32_t head = 0;
+            if (t == 0)
+                for (uint32_t k = 0; k < lead && k < nc; k++) head |= (uint32_t)fo[nc - 1 - k] << (8 * (lead - 1 - k));
+            __syncthreads();
+            if (hi) wbase[off >> 5] = 0;
+            if (t == 0) {
+                const uint64_t last = (fin_bit + 2 * tl) >> 5;
+                for (uint64_t w = fin_bit >> 5; w <= last; w++) wbase[w] = 0;
+            }
+            __syncthreads();
+            if (t == 0 && lead) atomicOr(&wbase[0], head);
+            if (hi) {
+                uint32_t s0 = sub_state[t] & 0xFFFFu, s1 = sub_state[t] >> 16;
+                uint64_t acc = 0;
+                uint32_t have = (uint32_t)(off & 31u);
+                uint32_t* wp = wbase + (off >> 5);
+                bool first = true;  // the word is shared with the lane before
+                fse_run(src, hi, lo, ct, s0, s1, [&](uint32_t v, uint32_t nb) {
+                    acc |= (uint64_t)(v & ((1u << nb) - 1u)) << have;
+                    have += nb;
+                    if (have >= 32) {
+                        if (first) atomicOr(wp, (uint32_t)acc);
+                        else *wp = (uint32_t)acc;
+                        first = false;
+                        wp++;
+                        acc >>= 32;
+                        have -= 32;
+                    }
+                });
+                if (have && (uint32_t)acc) atomicOr(wp, (uint32_t)acc);  // shared with the lane after
+            }
+            if (t == 0) {
+                const uint32_t f0 = fin[n & 1u], f1 = fin[(n & 1u) ^ 1u];  // state 2 is chain 0 for an even n
+                const uint32_t mask = (1u << tl) - 1u, sh = (uint32_t)(fin_bit & 31u);
+                const uint64_t v = (uint64_t)(f0 & mask) | (uint64_t)(f1 & mask) << tl | 1ull << (2 * tl);
+                atomicOr(&wbase[fin_bit >> 5], (uint32_t)(v << sh));
+                if (sh + 2 * tl + 1 > 32) atomicOr(&wbase[(fin_bit >> 5) + 1], (uint32_t)(v << sh >> 32));
+            }
+        }
+    }
+    if (r == kFseErr || r == 0 || r >= n) {
+        if (t == 0) {
+            out[0] = 0;
+            sizes[b] = 1 + n;
+        }
+        for (uint32_t i = t; i < n; i += blockDim.x) out[1 + i] = src[i];
+    } else if (r == 1) {
+        if (t == 0) {
+            out[0] = 2;
+            out[1] = src[0];
+            sizes[b] = 2;
+        }
+    } else if (t == 0) {
+        out[0] = 1;
+        for (uint32_t k = 0; k < 4; k++) out[1 + k] = (uint8_t)((uint32_t)r >> (8 * k));
+        sizes[b] = 5 + r;
+    }
 }
 
 // Copies variable-size slots to their packed places (blks[b].dst, found by the host from the sizes).
@@ -3233,9 +3451,17 @@ struct FseBlocks {
         slots = ws.take<uint8_t>(nb * kFseSlot);
         sizes = ws.take<uint64_t>(nb);
         dblks = ws.take<FseBlk>(nb);
-        uint16_t* pre = ws.take<uint16_t>(nb * kFblk);
+        FseMeta* meta = ws.take<FseMeta>(nb);
+        uint32_t* logs = ws.take<uint32_t>(nb * kFseLogWords);
         h2d(dblks, blks.data(), nb, st);
-        FZ_LAUNCH("fse_blocks", 0, k_fse_blocks, dim3((unsigned)nb), dim3(256), 0, st, dblks, slots, sizes, pre);
+        uint32_t longest = 0;
+        for (const FseBlk& b : blks) longest = std::max(longest, b.len);
+        // two chains of up to (longest - 1) / 2 steps, four waves a workgroup
+        const unsigned pieces = std::max(1u, ((longest - 1) / 2 + kFsePiece - 1) / kFsePiece);
+        FZ_LAUNCH("fse_tables", 0, k_fse_tables, dim3((unsigned)nb), dim3(256), 0, st, dblks, slots, kFseSlot, meta);
+        FZ_LAUNCH("fse_sets", 0, k_fse_sets, dim3((unsigned)nb, (pieces + 1) / 2), dim3(256), 0, st, dblks, meta, logs);
+        FZ_LAUNCH("fse_finish", 0, k_fse_finish, dim3((unsigned)nb), dim3(256), 0, st, dblks, meta, logs, slots, kFseSlot,
+                  sizes);
         FZ_HIP(hipGetLastError());
     }
 };
@@ -3585,7 +3811,8 @@ static size_t escape_workspace_bound(const std::vector<uint64_t>& off, uint64_t 
     add(nb * kFseSlot);
     add(8 * nb);
     add(sizeof(FseBlk) * nb);
-    add(2 * nb * kFblk);
+    add(sizeof(FseMeta) * nb);
+    add(4 * nb * kFseLogWords);
     return bytes + (1u << 16);
 }
 
