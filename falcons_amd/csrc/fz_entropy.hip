@@ -1426,13 +1426,21 @@ __device__ void o1_normalize(O1NormLds& L) {
 }
 
 // Encoding tables of every context of every segment: grid (contexts, segments).
-__global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint16_t* nf_all, CTable* ct_all) {
+__global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint16_t* nf_all, CTable* ct_all, uint32_t* use) {
     __shared__ TableLds L;
     __shared__ O1NormLds N;
+    __shared__ uint32_t sum;
     const unsigned t = threadIdx.x;
     const size_t c = (size_t)blockIdx.y * kO1Ctx + blockIdx.x;
-    N.h[t] = cnt_all[c * kO1Sym + t];
+    if (t == 0) sum = 0;
     __syncthreads();
+    uint32_t h = cnt_all[c * kO1Sym + t];
+    N.h[t] = h;
+#pragma unroll
+    for (int d = 32; d; d >>= 1) h += __shfl_xor(h, d, 64);
+    if ((t & 63u) == 0) atomicAdd(&sum, h);
+    __syncthreads();
+    if (t == 0) use[c] = sum;
     o1_normalize(N);
     nf_all[c * kO1Sym + t] = (uint16_t)N.norm[t];
     L.norm[t] = N.norm[t];
@@ -1460,7 +1468,9 @@ __global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint
 // 540,000 codes, the order-1 stage without its side streams: guessed and repaired 1.4 to 6 ms (2 to 10
 // rounds, as slowly as the last states merge), by sets 0.25 ms; 86,000: 1.03 and 0.24 ms. By sets a
 // code costs 2.25 steps of a wave: 134 million codes, 2.7 ms guessed and repaired, would take 7.
-constexpr uint32_t kO1Piece = 1024;
+constexpr uint32_t kO1Piece = 1024, kO1PieceMin = 256;  // as many pieces as the chip has lanes in one round of workgroups
+constexpr uint32_t kEncThreads = 1024, kEmitThreads = 1024, kRingWords = 8;
+constexpr int kEncHot = 8, kEmitHot = 6;  // state tables in LDS: 158 KB with the per-symbol arrays (and the emit's rings)
 constexpr uint32_t kSetPiece = 256;
 constexpr uint64_t kSetMaxCodes = 7ull << 19;  // 3,584 pieces a chain: the walk's links fit 64 KB of LDS
 constexpr uint32_t kSetStates = 16;    // states followed through a piece
@@ -1495,103 +1505,160 @@ __device__ inline uint32_t o1_seed_state(const int16_t* bins, uint64_t lo, uint6
     return init_state2(&ct[o1_ctx(prev)], o1_sym(bins[idx]));
 }
 
-__device__ inline uint32_t o1_step(uint32_t& state, const CTable& ct, unsigned sym) {
-    const uint32_t nbOut = (uint32_t)(((uint64_t)state + ct.deltaNbBits[sym]) >> 16);
-    state = ct.stateTable[(state >> nbOut) + ct.deltaFindState[sym]];
-    return nbOut;
-}
-
-// The per-symbol arrays of one segment's 15 encoding tables, staged in LDS by a workgroup whose
-// pieces lie in that segment (a workgroup's 256 pieces span at most a segment boundary; pieces of
-// another segment read their tables from device memory). The state tables stay in device memory.
+// One segment's encoding tables in LDS: the per-symbol arrays of all 15 contexts, and the state tables
+// (16 KB each) of the H contexts that occur most often. With the state tables in L2 the lanes of a
+// full chip wait for its rate of requests (a lane reads one entry a step from anywhere in 240 KB: 160 G
+// steps/s, 0.84 ms for the steps of 134 million codes); with 8 of them in LDS a step waits for L2 only
+// in the waves that hold a rare context.
+template <int H>
 struct O1EncLds {
-    uint32_t dnb[kO1Ctx * kO1Sym];
-    int32_t dfs[kO1Ctx * kO1Sym];
+    // a symbol's deltaNbBits, and its deltaFindState + 8,192 * place of the context's state table: below H
+    // in st, else H + context
+    u32x2 sym[kO1Ctx * kO1Sym];
+    uint16_t st[(size_t)H << kO1Log];
+    uint32_t place[kO1Ctx + 1];
 };
-// Stages the arrays of the segment of the workgroup's first piece; returns that segment. Every
-// thread of the workgroup calls it.
-__device__ inline uint64_t o1_stage_tables(O1EncLds& T, const O1Chains& C, uint64_t npieces, const CTable* ct_all,
-                                           uint64_t first_pid) {
-    const uint64_t seg = C.c[4 * o1_piece_chain(C, min(first_pid, npieces - 1)) + 3];
-    const CTable* ct = ct_all + seg * kO1Ctx;
-    for (uint32_t u = threadIdx.x; u < kO1Ctx * kO1Sym; u += blockDim.x) {
-        T.dnb[u] = ct[u / kO1Sym].deltaNbBits[u % kO1Sym];
-        T.dfs[u] = ct[u / kO1Sym].deltaFindState[u % kO1Sym];
+template <int H>
+struct O1EncTab {
+    const FZ_LDS u32x2* sym;
+    const FZ_LDS uint16_t* st;
+    const FZ_GLB uint16_t* far;
+};
+// Stages the tables of segment seg. Every thread of the workgroup calls it.
+template <int H>
+__device__ inline O1EncTab<H> o1_stage_tables(O1EncLds<H>& T, const CTable* ct, const uint32_t* use) {
+    if (threadIdx.x < kO1Ctx) {
+        const uint32_t c = threadIdx.x, u = use[c];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < (uint32_t)kO1Ctx; j++) rank += use[j] > u || (use[j] == u && j < c) ? 1u : 0u;
+        T.place[c] = rank < (uint32_t)H ? rank : (uint32_t)H + c;
     }
     __syncthreads();
-    return seg;
+    for (uint32_t u = threadIdx.x; u < kO1Ctx * kO1Sym; u += blockDim.x) {
+        T.sym[u] = u32x2{ct[u / kO1Sym].deltaNbBits[u % kO1Sym],
+                         (uint32_t)ct[u / kO1Sym].deltaFindState[u % kO1Sym] + (T.place[u / kO1Sym] << kO1Log)};
+    }
+    for (uint32_t c = 0; c < (uint32_t)kO1Ctx; c++) {
+        if (T.place[c] >= (uint32_t)H) continue;
+        const uint32_t* from = reinterpret_cast<const uint32_t*>(ct[c].stateTable);
+        uint32_t* to = reinterpret_cast<uint32_t*>(T.st + (T.place[c] << kO1Log));
+        for (uint32_t i = threadIdx.x; i < 1u << (kO1Log - 1); i += blockDim.x) to[i] = from[i];
+    }
+    __syncthreads();
+    return O1EncTab<H>{lds(T.sym), lds(T.st),
+                       glb(reinterpret_cast<const uint16_t*>(ct)) + offsetof(CTable, stateTable) / 2};
 }
-// One encoder step in context cx: per-symbol values from LDS (staged) or device memory.
-__device__ __forceinline__ uint32_t o1_step_t(uint32_t& state, const CTable* ct, const FZ_LDS uint32_t* dnb,
-                                              const FZ_LDS int32_t* dfs, bool staged, int cx, unsigned sym) {
-    const uint32_t u = (uint32_t)cx * kO1Sym + sym;
-    const uint32_t d = staged ? dnb[u] : ct[cx].deltaNbBits[sym];
-    const int32_t f = staged ? dfs[u] : ct[cx].deltaFindState[sym];
-    const uint32_t nbOut = (uint32_t)(((uint64_t)state + d) >> 16);
-    state = ct[cx].stateTable[(state >> nbOut) + f];
-    return nbOut;
+// o1_ctx(prev) * 256 + o1_sym(code) in a few instructions: the context of a magnitude up to 12 is a nibble.
+__device__ __forceinline__ uint32_t o1_index(int code, int prev) {
+    const uint32_t a = min((uint32_t)(prev < 0 ? -prev : prev), 12u);
+    const uint32_t cx = ((uint32_t)(0xDBBBB99975310ull >> (4 * a)) & 15u) + ((uint32_t)prev >> 31);
+    return cx * kO1Sym + min(((uint32_t)code << 1) ^ (uint32_t)(code >> 31), 255u);
+}
+__host__ __device__ constexpr bool o1_index_holds() {
+    for (int v = 0; v < 40; v++) {
+        const int m = v <= 4 ? v - 1 : v <= 7 ? 4 : v <= 11 ? 5 : 6;
+        if ((int)(0xDBBBB99975310ull >> (4 * (v < 12 ? v : 12)) & 15u) != (v ? 1 + 2 * m : 0)) return false;
+    }
+    return true;
+}
+static_assert(o1_index_holds(), "the nibbles are o1_ctx");
+
+// The bits that a step of symbol d emits from a state, and the state after it.
+__device__ __forceinline__ uint32_t o1_step_bits(uint32_t state, u32x2 d) { return (state + d.x) >> 16; }
+template <int H>
+__device__ __forceinline__ uint32_t o1_step_next(const O1EncTab<H>& T, uint32_t state, u32x2 d, uint32_t bits) {
+    constexpr uint32_t kNear = (uint32_t)H << kO1Log;
+    const uint32_t at = (state >> bits) + d.y;
+    uint32_t v = T.st[min(at, kNear - 1)];
+    if (at >= kNear) {
+        const uint32_t j = at - kNear;
+        v = T.far[(j >> kO1Log) * (uint32_t)(sizeof(CTable) / 2) + (j & ((1u << kO1Log) - 1u))];
+    }
+    return v;
 }
 
-// Runs f(i, code, previous code) for the steps i = s_hi down to s_lo of a piece (previous code 0 at
-// the chain's first symbol lo), stopping early when f returns false. The codes come in aligned
-// 16-byte loads, eight at a time, the next eight in flight: one load per eight steps instead of two
-// scattered 2-byte loads per step (the lanes of a wave run pieces 2 KB apart). bins is 16-byte
-// aligned and its allocation extends to the next multiple of 16 bytes.
-template <typename F>
-__device__ __forceinline__ void o1_piece_codes(const int16_t* bins, uint64_t lo, uint64_t s_hi, uint64_t s_lo, F&& f) {
+// The lane's piece in a launch of whole workgroups a segment (every workgroup's pieces share the tables
+// that it stages); ~0 past the segment's last piece. seg: the workgroup's segment.
+__device__ __forceinline__ uint64_t o1_piece_of(const O1Chains& C, uint32_t groups, uint32_t& seg) {
+    const uint32_t b = xcd_block();
+    seg = b / groups;
+    const uint64_t pid = C.pfirst[seg * kO1K] + (uint64_t)(b % groups) * blockDim.x + threadIdx.x;
+    return pid < C.pfirst[(seg + 1) * kO1K] ? pid : ~0ull;
+}
+
+// Runs step(u, k) for the steps i = 8c + k from s_hi down to s_lo of a piece, u the step's o1_index
+// (previous code 0 at the chain's first symbol lo), begin(8c) before and more() after those of a group of
+// eight; ends early when more returns false. The codes come in aligned 16-byte loads, eight at a time,
+// the next eight in flight: one load per eight steps instead of two scattered 2-byte loads per step (the
+// lanes of a wave run pieces 1 KB and more apart). A step costs its instructions as much as its waits (16
+// waves a CU), so whole groups inside the piece, nearly all, run without tests of their bounds. bins is
+// 16-byte aligned and its allocation extends to the next multiple of 16 bytes.
+template <typename B, typename F, typename M>
+__device__ __forceinline__ void o1_piece_codes(const int16_t* bins, uint64_t lo, uint64_t s_hi, uint64_t s_lo, B&& begin,
+                                               F&& step, M&& more) {
     const u32x4* b4 = reinterpret_cast<const u32x4*>(bins);
     uint64_t c = s_hi >> 3;
     const uint64_t c_lo = s_lo >> 3;
     u32x4 cur = b4[c];
     u32x4 nxt = c > 0 ? b4[c - 1] : u32x4{0u, 0u, 0u, 0u};
     for (;;) {
+        const uint64_t base = 8 * c;
+        begin(base);
         int v[9];  // v[k + 1]: code 8c + k; v[0]: code 8c - 1
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             v[2 * k + 1] = (int)(int16_t)(cur[k] & 0xFFFFu);
-            v[2 * k + 2] = (int)(int16_t)(cur[k] >> 16);
+            v[2 * k + 2] = (int)cur[k] >> 16;
         }
-        v[0] = (int)(int16_t)(nxt[3] >> 16);
-        const uint64_t base = 8 * c;
+        v[0] = (int)nxt[3] >> 16;
+        if (base >= s_lo && base + 7 <= s_hi && base > lo) {
 #pragma unroll
-        for (int k = 7; k >= 0; k--) {
-            const uint64_t i = base + (uint64_t)k;
-            if (i > s_hi || i < s_lo) continue;
-            if (!f(i, v[k + 1], i > lo ? v[k] : 0)) return;
+            for (int k = 7; k >= 0; k--) step(o1_index(v[k + 1], v[k]), k);
+        } else {
+#pragma unroll
+            for (int k = 7; k >= 0; k--) {
+                const uint64_t i = base + (uint64_t)k;
+                if (i <= s_hi && i >= s_lo) step(o1_index(v[k + 1], i > lo ? v[k] : 0), k);
+            }
         }
-        if (c == c_lo) return;
+        if (c == c_lo || !more()) return;
         c--;
         cur = nxt;
         nxt = c > 0 ? b4[c - 1] : u32x4{0u, 0u, 0u, 0u};
     }
 }
+struct PieceNoop {
+    __device__ __forceinline__ void operator()(uint64_t) const {}
+    __device__ __forceinline__ bool operator()() const { return true; }
+};
 
-__global__ void __launch_bounds__(256) k_o1_spec(const int16_t* bins, O1Chains C, uint64_t npieces,
-                                                 const CTable* ct_all, uint16_t* slog, uint32_t* end_state,
-                                                 uint64_t* nbits) {
-    __shared__ O1EncLds T;
-    const uint64_t first = (uint64_t)xcd_block() * blockDim.x;
-    const uint64_t wseg = o1_stage_tables(T, C, npieces, ct_all, first);
-    const uint64_t pid = first + threadIdx.x;
-    if (pid >= npieces) return;
+__global__ void __launch_bounds__(kEncThreads) k_o1_spec(const int16_t* bins, O1Chains C, uint32_t groups, uint64_t npieces,
+                                                         const CTable* ct_all, const uint32_t* use, uint16_t* slog,
+                                                         uint32_t* end_state, uint64_t* nbits) {
+    __shared__ O1EncLds<kEncHot> L;
+    uint32_t seg;
+    const uint64_t pid = o1_piece_of(C, groups, seg);
+    const CTable* ct = ct_all + (size_t)seg * kO1Ctx;
+    const auto T = o1_stage_tables(L, ct, use + seg * kO1Ctx);
+    if (pid == ~0ull) return;
     const int q = o1_piece_chain(C, pid);
     const uint64_t lo = C.c[4 * q + 1], hi = C.c[4 * q + 2];
-    const CTable* ct = ct_all + C.c[4 * q + 3] * kO1Ctx;
-    const bool staged = C.c[4 * q + 3] == wseg;
     const uint64_t p = pid - C.pfirst[q];
     uint64_t s_hi, s_lo;
     o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
     // piece 0 starts from the true seed; the others from the seed their own first symbol would give
     uint32_t st = o1_seed_state(bins, lo, p == 0 ? hi - 1 : s_hi, ct);
-    uint64_t bits = 0;
-    const FZ_LDS uint32_t* dnb = lds(T.dnb);
-    const FZ_LDS int32_t* dfs = lds(T.dfs);
+    uint32_t bits = 0;
     // the log is step-major (step j of every piece side by side), so a wave's writes are coalesced
-    o1_piece_codes(bins, lo, s_hi, s_lo, [&](uint64_t i, int code, int pc) {
-        slog[(s_hi - i) * npieces + pid] = (uint16_t)st;
-        bits += o1_step_t(st, ct, dnb, dfs, staged, o1_ctx(pc), (unsigned)o1_sym(code));
-        return true;
-    });
+    uint16_t* log = slog + pid;
+    o1_piece_codes(bins, lo, s_hi, s_lo, PieceNoop{}, [&](uint32_t u, int) {
+        *log = (uint16_t)st;
+        log += npieces;
+        const u32x2 d = T.sym[u];
+        const uint32_t nb = o1_step_bits(st, d);
+        bits += nb;
+        st = o1_step_next(T, st, d, nb);
+    }, PieceNoop{});
     end_state[pid] = st;
     nbits[pid] = bits;
 }
@@ -1603,44 +1670,51 @@ __global__ void __launch_bounds__(256) k_o1_spec(const int16_t* bins, O1Chains C
 // re-run reached. A piece whose end state differs from end_prev marks itself changed, and its
 // successor runs again in the next round; after a round with no change every piece started from
 // its predecessor's true end state. Piece 0 of a chain starts from the true seed and never changes.
-__global__ void __launch_bounds__(256) k_o1_fix(const int16_t* bins, O1Chains C, uint64_t npieces,
-                                                const CTable* ct_all, const uint16_t* slog, const uint32_t* spec_end,
+__global__ void __launch_bounds__(kEncThreads) k_o1_fix(const int16_t* bins, O1Chains C, uint32_t groups, uint64_t npieces,
+                                                const CTable* ct_all, const uint32_t* use, const uint16_t* slog,
+                                                const uint32_t* spec_end,
                                                 const uint64_t* spec_bits, const uint32_t* end_prev,
                                                 uint32_t* end_next, uint64_t* nbits, const uint8_t* changed_prev,
                                                 uint8_t* changed_next, unsigned int* any_changed) {
-    __shared__ O1EncLds T;
-    const uint64_t first = (uint64_t)xcd_block() * blockDim.x;
-    const uint64_t wseg = o1_stage_tables(T, C, npieces, ct_all, first);
-    const uint64_t pid = first + threadIdx.x;
-    if (pid >= npieces) return;
-    const int q = o1_piece_chain(C, pid);
-    const uint64_t p = pid - C.pfirst[q];
+    __shared__ O1EncLds<kEncHot> L;
+    uint32_t seg;
+    const uint64_t pid = o1_piece_of(C, groups, seg);
+    int q = 0;
+    uint64_t p = 0;
+    bool again = false;
+    if (pid != ~0ull) {
+        q = o1_piece_chain(C, pid);
+        p = pid - C.pfirst[q];
+        again = p > 0 && (changed_prev == nullptr || changed_prev[pid - 1]);
+    }
+    O1EncTab<kEncHot> T{};
+    // the tables are staged where a lane needs them: after the first rounds that is in few workgroups
+    if (__syncthreads_or(again)) T = o1_stage_tables(L, ct_all + (size_t)seg * kO1Ctx, use + seg * kO1Ctx);
+    if (pid == ~0ull) return;
     uint32_t end = end_prev[pid];
     uint8_t ch = 0;
-    if (p > 0 && (changed_prev == nullptr || changed_prev[pid - 1])) {
+    if (again) {
         const uint64_t lo = C.c[4 * q + 1], hi = C.c[4 * q + 2];
-        const CTable* ct = ct_all + C.c[4 * q + 3] * kO1Ctx;
-        const bool staged = C.c[4 * q + 3] == wseg;
-        const FZ_LDS uint32_t* dnb = lds(T.dnb);
-        const FZ_LDS int32_t* dfs = lds(T.dfs);
         uint64_t s_hi, s_lo;
         o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
         uint32_t st = end_prev[pid - 1];
-        int64_t delta = 0;
+        int32_t delta = 0;
         bool met = false;
-        o1_piece_codes(bins, lo, s_hi, s_lo, [&](uint64_t i, int code, int pc) {
-            const uint32_t logged = slog[(s_hi - i) * npieces + pid];
-            if (st == logged) {
-                met = true;
-                return false;
-            }
-            const int cx = o1_ctx(pc);
-            const unsigned sym = (unsigned)o1_sym(code);
-            uint32_t ls = logged;
-            delta -= (int64_t)o1_step_t(ls, ct, dnb, dfs, staged, cx, sym);
-            delta += (int64_t)o1_step_t(st, ct, dnb, dfs, staged, cx, sym);
-            return true;
-        });
+        // The logged states of eight steps come together: a load a step would double a step's time, and
+        // the few lanes that are long without meeting their log decide a round's. After the states have
+        // met they stay together, so that the rest of the eight steps changes nothing.
+        uint32_t log8[8];
+        o1_piece_codes(bins, lo, s_hi, s_lo, [&](uint64_t base) {
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                log8[k] = slog[(s_hi - min(max(base + (uint64_t)k, s_lo), s_hi)) * npieces + pid];
+        }, [&](uint32_t u, int k) {
+            met = met || st == log8[k];
+            const u32x2 d = T.sym[u];
+            const uint32_t nb = o1_step_bits(st, d);
+            delta += (int32_t)nb - (int32_t)o1_step_bits(log8[k], d);
+            st = o1_step_next(T, st, d, nb);
+        }, [&]() { return !met; });
         nbits[pid] = (uint64_t)((int64_t)spec_bits[pid] + delta);
         const uint32_t e = met ? spec_end[pid] : st;
         if (e != end) {
@@ -1727,19 +1801,17 @@ __device__ inline void rw_word(RunWriter& W, uint32_t v) {
     } else if (!W.runs) {
         W.w[W.idx] = v;
     } else {
-        W.ring[W.idx & 15u] = v;
-        if ((W.idx & 15u) == 15u) {
+        W.ring[W.idx & (kRingWords - 1)] = v;
+        if ((W.idx & (kRingWords - 1)) == kRingWords - 1) {
             const FZ_LDS u32x4* r = reinterpret_cast<const FZ_LDS u32x4*>(W.ring);
-            u32x4* d = reinterpret_cast<u32x4*>(W.w + (W.idx - 15));
-            const u32x4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+            u32x4* d = reinterpret_cast<u32x4*>(W.w + (W.idx - (kRingWords - 1)));
+            const u32x4 r0 = r[0], r1 = r[1];
             d[0] = r0;
             d[1] = r1;
-            d[2] = r2;
-            d[3] = r3;
         }
     }
     W.idx++;
-    if ((W.idx & 15u) == 0) W.runs = true;
+    if ((W.idx & (kRingWords - 1)) == 0) W.runs = true;
 }
 __device__ inline void rw_put(RunWriter& W, uint32_t v, uint32_t nb) {
     if (!nb) return;
@@ -1753,39 +1825,36 @@ __device__ inline void rw_put(RunWriter& W, uint32_t v, uint32_t nb) {
 }
 __device__ inline void rw_flush(RunWriter& W) {
     if (W.runs)
-        for (uint64_t k = W.idx & ~(uint64_t)15; k < W.idx; k++) W.w[k] = W.ring[k & 15u];
+        for (uint64_t k = W.idx & ~(uint64_t)(kRingWords - 1); k < W.idx; k++) W.w[k] = W.ring[k & (kRingWords - 1)];
     if (W.n) atomicOr(&W.w[W.idx], (uint32_t)W.acc);
 }
 
-__global__ void __launch_bounds__(256) k_o1_emit(const int16_t* bins, O1Chains C, uint64_t npieces,
-                                                 const CTable* ct_all, const uint32_t* end_state,
-                                                 const uint64_t* bitoff, uint32_t* words, uint64_t stride_words,
-                                                 const uint64_t* failed) {
-    __shared__ O1EncLds T;
-    __shared__ __align__(16) uint32_t ring[256 * 16];
+__global__ void __launch_bounds__(kEmitThreads) k_o1_emit(const int16_t* bins, O1Chains C, uint32_t groups,
+                                                          const CTable* ct_all, const uint32_t* use,
+                                                          const uint32_t* end_state, const uint64_t* bitoff,
+                                                          uint32_t* words, uint64_t stride_words, const uint64_t* failed) {
+    __shared__ O1EncLds<kEmitHot> L;
+    __shared__ __align__(16) uint32_t ring[kEmitThreads * kRingWords];
     if (failed && *failed) return;
-    const uint64_t first = (uint64_t)xcd_block() * blockDim.x;
-    const uint64_t wseg = o1_stage_tables(T, C, npieces, ct_all, first);
-    const uint64_t pid = first + threadIdx.x;
-    if (pid >= npieces) return;
+    uint32_t seg;
+    const uint64_t pid = o1_piece_of(C, groups, seg);
+    const CTable* ct = ct_all + (size_t)seg * kO1Ctx;
+    const auto T = o1_stage_tables(L, ct, use + seg * kO1Ctx);
+    if (pid == ~0ull) return;
     const int q = o1_piece_chain(C, pid);
     const uint64_t lo = C.c[4 * q + 1], hi = C.c[4 * q + 2];
-    const CTable* ct = ct_all + C.c[4 * q + 3] * kO1Ctx;
-    const bool staged = C.c[4 * q + 3] == wseg;
-    const FZ_LDS uint32_t* dnb = lds(T.dnb);
-    const FZ_LDS int32_t* dfs = lds(T.dfs);
     const uint64_t p = pid - C.pfirst[q];
     uint64_t s_hi, s_lo;
     o1_piece_range(C.piece, lo, hi, p, s_hi, s_lo);
     uint32_t st = p == 0 ? o1_seed_state(bins, lo, hi - 1, ct) : end_state[pid - 1];
     const uint64_t b0 = bitoff[pid];
-    RunWriter W{words + q * stride_words, lds(ring + threadIdx.x * 16), b0 >> 5, 0, (uint32_t)(b0 & 31), true, false};
-    o1_piece_codes(bins, lo, s_hi, s_lo, [&](uint64_t, int code, int pc) {
-        const uint32_t st0 = st;
-        const uint32_t nbOut = o1_step_t(st, ct, dnb, dfs, staged, o1_ctx(pc), (unsigned)o1_sym(code));
-        rw_put(W, st0, nbOut);
-        return true;
-    });
+    RunWriter W{words + q * stride_words, lds(ring + threadIdx.x * kRingWords), b0 >> 5, 0, (uint32_t)(b0 & 31), true, false};
+    o1_piece_codes(bins, lo, s_hi, s_lo, PieceNoop{}, [&](uint32_t u, int) {
+        const u32x2 d = T.sym[u];
+        const uint32_t nb = o1_step_bits(st, d);
+        rw_put(W, st, nb);
+        st = o1_step_next(T, st, d, nb);
+    }, PieceNoop{});
     rw_flush(W);
 }
 
@@ -3850,6 +3919,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
     uint32_t* cnt = ws.take<uint32_t>(S * kO1Ctx * kO1Sym);
     uint16_t* nf = ws.take<uint16_t>(S * kO1Ctx * kO1Sym);
     CTable* ct = ws.take<CTable>(S * kO1Ctx);
+    uint32_t* use = ws.take<uint32_t>(S * kO1Ctx);
     FZ_HIP(hipMemsetAsync(cnt, 0, S * kO1Ctx * kO1Sym * 4, st));
     std::vector<uint64_t> chains;  // {seg lo, chunk lo, chunk hi, segment}
     std::vector<uint64_t> novf(S * kO1K), ovf_off(S + 1);
@@ -3934,7 +4004,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
             g_prof = nullptr;
         });
     }
-    FZ_LAUNCH("o1_tables", 0, k_o1_tables, dim3(kO1Ctx, (unsigned)S), dim3(256), 0, st, cnt, nf, ct);
+    FZ_LAUNCH("o1_tables", 0, k_o1_tables, dim3(kO1Ctx, (unsigned)S), dim3(256), 0, st, cnt, nf, ct, use);
     FZ_HIP(hipGetLastError());
     const int nch = (int)(S * kO1K);
     uint64_t* dchains = ws.take<uint64_t>(chains.size());
@@ -3962,6 +4032,12 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         h2d(dpfirst, pfirst.data(), nch + 1, st);
         return O1Chains{dchains, dpfirst, nch, steps_piece};
     };
+    // workgroups a segment in a launch of one lane a piece
+    auto groups_of = [&](const std::vector<uint64_t>& first, uint32_t threads) {
+        uint64_t most = 1;
+        for (uint64_t g = 0; g < S; g++) most = std::max(most, first[(g + 1) * kO1K] - first[g * kO1K]);
+        return (uint32_t)((most + threads - 1) / threads);
+    };
     std::vector<uint64_t> sets_first, pfirst;
     const bool sets = n <= kSetMaxCodes;
     uint64_t* failed = blen + nch;
@@ -3981,16 +4057,22 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         FZ_LAUNCH("o1_encode_walk", 0, k_o1_sets_walk, dim3((unsigned)nch), dim3(256), most * (kSetStates + 1), st, CH, B,
                   end_state, bitoff, chain_bits, words, stride_words, failed);
         if (np)
-            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, end_state, bitoff,
-                      words, stride_words, failed);
+            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3((unsigned)S * groups_of(sets_first, kEmitThreads)),
+                      dim3(kEmitThreads), 0, st, bins, CH, groups_of(sets_first, kEmitThreads), ct, use, end_state, bitoff, words,
+                      stride_words, failed);
         FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_state, chain_bits,
                   words, stride_words, blen, failed);
         FZ_HIP(hipGetLastError());
     }
     auto guess_and_repair = [&]() {
-        const O1Chains CH = lay_out(kO1Piece, pfirst);
+        // one round of workgroups of one a CU, whole ones for every segment
+        constexpr uint64_t kCus = 256;
+        const uint64_t lanes = std::max<uint64_t>(1, kCus / S) * kEncThreads - kO1K;  // a chain's last piece is a part
+        const uint32_t steps_piece = (uint32_t)std::min<uint64_t>(kO1Piece, std::max<uint64_t>(kO1PieceMin, ((seg + lanes - 1) / lanes + 15) & ~15ull));
+        const O1Chains CH = lay_out(steps_piece, pfirst);
         const uint64_t np = pfirst[nch];
-        uint16_t* slog = ws.take<uint16_t>(np * kO1Piece + 16);  // step-major: [step in piece][piece]
+        const uint32_t groups = groups_of(pfirst, kEncThreads);
+        uint16_t* slog = ws.take<uint16_t>(np * steps_piece + 16);  // step-major: [step in piece][piece]
         uint32_t* spec_end = ws.take<uint32_t>(np + 1);
         uint32_t* end_a = ws.take<uint32_t>(np + 1);
         uint32_t* end_b = ws.take<uint32_t>(np + 1);
@@ -4002,7 +4084,8 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         uint64_t* scan = ws.take<uint64_t>(np + 1);
         uint64_t* bitoff = ws.take<uint64_t>(np + 1);
         if (np) {
-            FZ_LAUNCH("o1_encode_spec", n * 4, k_o1_spec, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog, spec_end, spec_bits);
+            FZ_LAUNCH("o1_encode_spec", n * 4, k_o1_spec, dim3((unsigned)S * groups), dim3(kEncThreads), 0, st, bins, CH, groups, np,
+                      ct, use, slog, spec_end, spec_bits);
             FZ_HIP(hipGetLastError());
             FZ_HIP(hipMemcpyAsync(nbits, spec_bits, np * 8, hipMemcpyDeviceToDevice, st));
             // fix-up rounds; each round finalizes at least the next piece of every chain, so the loop
@@ -4020,8 +4103,8 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
                 if (round > max_rounds + 1) throw std::runtime_error("tANS piece fix-up did not settle");
                 for (int k = 0; k < 2; k++, round++) {
                     if (k == 1) FZ_HIP(hipMemsetAsync(any, 0, sizeof(unsigned int), st));
-                    FZ_LAUNCH("o1_encode_fix", 0, k_o1_fix, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, slog,
-                              spec_end, spec_bits, end_prev, end_next, nbits, chg_prev, chg_next, any);
+                    FZ_LAUNCH("o1_encode_fix", 0, k_o1_fix, dim3((unsigned)S * groups), dim3(kEncThreads), 0, st, bins, CH, groups, np, ct,
+                              use, slog, spec_end, spec_bits, end_prev, end_next, nbits, chg_prev, chg_next, any);
                     FZ_HIP(hipGetLastError());
                     end_prev = end_next;
                     end_next = (end_next == end_a) ? end_b : end_a;
@@ -4039,8 +4122,9 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
             FZ_LAUNCH("o1_encode_clear", 0, k_o1_clear_shared, dim3(nblk(np + nch)), dim3(256), 0, st, CH, np, bitoff, chain_bits,
                                words, stride_words);
             FZ_HIP(hipGetLastError());
-            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3(nblk(np)), dim3(256), 0, st, bins, CH, np, ct, end_prev, bitoff, words,
-                               stride_words, (const uint64_t*)nullptr);
+            FZ_LAUNCH("o1_encode_emit", n * 2, k_o1_emit, dim3((unsigned)S * groups_of(pfirst, kEmitThreads)), dim3(kEmitThreads), 0,
+                      st, bins, CH, groups_of(pfirst, kEmitThreads), ct, use, end_prev, bitoff, words, stride_words,
+                      (const uint64_t*)nullptr);
             FZ_HIP(hipGetLastError());
             FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_prev, chain_bits,
                                words, stride_words, blen, (const uint64_t*)nullptr);
