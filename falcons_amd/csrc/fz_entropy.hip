@@ -1467,7 +1467,7 @@ __global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint
 //   trajectory (k_o1_fix, repeated while some piece fails to meet it).
 // 540,000 codes, the order-1 stage without its side streams: guessed and repaired 1.4 to 6 ms (2 to 10
 // rounds, as slowly as the last states merge), by sets 0.25 ms; 86,000: 1.03 and 0.24 ms. By sets a
-// code costs 2.25 steps of a wave: 134 million codes, 2.7 ms guessed and repaired, would take 7.
+// code costs 2.25 steps of a wave: 134 million codes, 1.4 ms guessed, repaired and emitted, would take 7.
 constexpr uint32_t kO1Piece = 1024, kO1PieceMin = 256;  // as many pieces as the chip has lanes in one round of workgroups
 constexpr uint32_t kEncThreads = 1024, kEmitThreads = 1024, kRingWords = 8;
 constexpr int kEncHot = 8, kEmitHot = 6;  // state tables in LDS: 158 KB with the per-symbol arrays (and the emit's rings)
@@ -1508,8 +1508,10 @@ __device__ inline uint32_t o1_seed_state(const int16_t* bins, uint64_t lo, uint6
 // One segment's encoding tables in LDS: the per-symbol arrays of all 15 contexts, and the state tables
 // (16 KB each) of the H contexts that occur most often. With the state tables in L2 the lanes of a
 // full chip wait for its rate of requests (a lane reads one entry a step from anywhere in 240 KB: 160 G
-// steps/s, 0.84 ms for the steps of 134 million codes); with 8 of them in LDS a step waits for L2 only
-// in the waves that hold a rare context.
+// steps/s); with 8 of them in LDS a step waits for L2 only in the waves that hold a rare context, and
+// its instructions count as much. 134 million codes, one in 15 an escape: k_o1_spec 0.84 -> 0.40 ms,
+// k_o1_fix 0.85 -> 0.50, k_o1_emit (6 tables, the rings beside them) 0.95 -> 0.50; two codes in five an
+// escape: 1.40 -> 0.48, 2.2 -> 2.6 (beside the escapes' blocks, which come at once now), 0.93 -> 0.45.
 template <int H>
 struct O1EncLds {
     // a symbol's deltaNbBits, and its deltaFindState + 8,192 * place of the context's state table: below H
@@ -1781,18 +1783,18 @@ __device__ inline void ww_flush(WordWriter& W) {
     if (W.n) atomicOr(&W.w[W.idx], (uint32_t)W.acc);
 }
 
-// k_o1_emit's output: a lane's words pass through a 16-word LDS ring and leave in aligned 64-byte
+// k_o1_emit's output: a lane's words pass through an 8-word LDS ring and leave in aligned 32-byte
 // runs (the lanes of a wave write 131 K pieces' lines at once, and single-word stores leave partly
 // written lines to L2 evictions). The first word (shared with the previous piece) is OR-ed in; the
-// words before the first 64-byte boundary, and those after the last full run, go one by one; the last,
+// words before the first 32-byte boundary, and those after the last full run, go one by one; the last,
 // partial word (shared with the next piece) is OR-ed in.
 struct RunWriter {
     uint32_t* w;            // the chain's words
-    FZ_LDS uint32_t* ring;  // this lane's 16 words
+    FZ_LDS uint32_t* ring;  // this lane's kRingWords words
     uint64_t idx;           // the word being filled
     uint64_t acc;
     uint32_t n;
-    bool first, runs;       // runs: a 64-byte boundary has been passed
+    bool first, runs;       // runs: a 32-byte boundary has been passed
 };
 __device__ inline void rw_word(RunWriter& W, uint32_t v) {
     if (W.first) {
@@ -4012,7 +4014,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
     uint64_t maxcs = 0;
     for (uint64_t g = 0; g < S; g++) maxcs = std::max(maxcs, (seg_n[g] + kO1K - 1) / kO1K);
     // chain staging: 13 bits per symbol at most, plus the closing state; every chain's words start
-    // 64-byte aligned (k_o1_emit stores whole aligned 64-byte runs)
+    // 64-byte aligned (k_o1_emit stores whole aligned 32-byte runs)
     const uint64_t stride_words = ((maxcs * 2 + 4096 + 3) / 4 + 15) & ~(uint64_t)15;
     const uint64_t bstride = stride_words * 4;
     uint32_t* words = ws.take<uint32_t>(nch * stride_words);
@@ -4328,9 +4330,18 @@ constexpr uint64_t kSplitMinSymbols = 8192;
 constexpr double kSplitMinBits = 2.5;
 // Sequential chains of fewer take several steps a lookup (kSerialRun).
 constexpr double kSerialRunBits = 2.0;
-// In the batched decompress, so are chains of at most this many: many fields' sequential chains run
-// side by side in one launch.
+// In the batched decompress, chains of at most this many are handed to the batch, whose split chains run
+// in one set of launches, and whose other chains in one launch beside them: a field's own launches
+// leave most of the chip idle (192 chunks of 540,000 codes at bounds 1e-2 to 1e-4: 64 ms with all of
+// their chains decoded from their starts, 47 ms like this). The split chains of a batch share at most
+// kBatchSplitBytes of sets and graphs; chains past that are decoded from their start.
 constexpr uint64_t kDeferSymbols = 1ull << 19;
+constexpr double kBatchSplitBytes = 4.0 * (1ull << 30);
+// Alone, a chain of few bits a symbol runs 64 decoders 2,048 symbols ahead of every part in what the chip
+// has to spare. In a batch those steps are what the whole takes (256 of a lane a symbol, as many as L2
+// serves in 1.6 ns: 25 of 60 ms for the chunks above), so it runs 32 decoders 1,024 ahead, and the walk
+// decodes the few parts more that then lack their entry: 60 -> 49 ms.
+constexpr uint32_t kBatchWarm = 32 * 1024;
 
 // Stationary distribution of segment g's context chain (a code's context follows from the previous
 // code; an escape leads to 13 or 14, counted half each), from the normalized counts of its 15
@@ -4406,50 +4417,7 @@ static SerialMap serial_map(const double pi[kO1Ctx], double escapes, double bits
     return m;
 }
 
-// Sequential chains of several calls, decoded together (dense_batch_run).
-struct DenseBatch {
-    std::mutex mu;
-    std::vector<SerialJob> jobs;
-    std::vector<SerialTables> tabs;
-    uint64_t bytes = 0, codes = 0;
-};
-DenseBatch* dense_batch_create() { return new DenseBatch; }
-void dense_batch_destroy(DenseBatch* b) { delete b; }
-size_t dense_batch_size(DenseBatch* b) {
-    std::lock_guard<std::mutex> g(b->mu);
-    return b->jobs.size();
-}
-void dense_batch_clear(DenseBatch* b) {
-    std::lock_guard<std::mutex> g(b->mu);
-    b->jobs.clear();
-    b->tabs.clear();
-    b->bytes = b->codes = 0;
-}
-// Re-encodes the tables and decodes the chains of the lists on st; djobs and dtabs have room for them.
-static void launch_serial(std::vector<SerialJob>& jobs, const std::vector<SerialTables>& tabs, SerialJob* djobs,
-                          SerialTables* dtabs, uint64_t bytes, uint64_t codes, hipStream_t st) {
-    FZ_LAUNCH("o1_serial_tables", 0, k_o1d_tables, dim3(kO1Ctx, (unsigned)tabs.size()), dim3(256), 0, st, dtabs);
-    FZ_LAUNCH("o1_decode_serial", bytes + codes * 2, k_o1d_serial, dim3((unsigned)jobs.size()), dim3(kSerialThreads), 0, st,
-              djobs);
-    FZ_HIP(hipGetLastError());
-}
-void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st) {
-    std::lock_guard<std::mutex> g(b->mu);
-    const size_t n = b->jobs.size();
-    if (!n) return;
-    if (n > 0x7fffffffu) throw std::length_error("too many sequential chains for one launch");
-    if (b->tabs.size() > 65535u) throw std::length_error("too many sequential segments for one launch");
-    // longest chains first, so that the last workgroups to start are short ones
-    std::stable_sort(b->jobs.begin(), b->jobs.end(), [](const SerialJob& x, const SerialJob& y) { return x.m > y.m; });
-    SerialJob* dj = ws.take<SerialJob>(n);
-    SerialTables* dtab = ws.take<SerialTables>(b->tabs.size());
-    // the lists stay in b until dense_batch_clear, after the launches have finished
-    h2d(dj, b->jobs.data(), n, st);
-    h2d(dtab, b->tabs.data(), b->tabs.size(), st);
-    launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, st);
-}
-
-// How a chain is decoded: from its start by one workgroup (k_o1d_dense), or split into parts. The
+// How a chain is decoded: from its start by one workgroup (k_o1d_serial), or split into parts. The
 // split decoder follows, for every part, all states that its entry may be; what that costs is the
 // number of such states that live side by side, estimated from the chain's tables:
 //   mu   rate per symbol at which two decoders meet. It falls with the bits a symbol takes (a step
@@ -4511,6 +4479,152 @@ static SplitPlan split_plan(uint64_t m, uint64_t novf, double bits, const double
     return s;
 }
 
+// The split chains of a call or of a batch, in launch order, and what their kernels left (sc is read by a
+// copy on the stream: it stays until that has run).
+struct SplitRun {
+    std::vector<O1Split> sc;
+    std::vector<int> order;
+    O1SplitWs W{};
+    unsigned int* stats = nullptr;
+    uint64_t nparts = 0;
+};
+// Device bytes that split_launch takes for a chain, but for its few words a part.
+static double split_bytes(const O1Split& k, const SplitPlan& sp) {
+    return 12.0 * k.nsub * k.cap + 8.0 * (4.0 * sp.nodes * (double)k.m + 16.0 * k.nsub / k.parts);
+}
+static void split_launch(const std::vector<O1Split>& hc, const std::vector<SplitPlan>& plans, SplitRun& R, DevArena& ws,
+                         hipStream_t st) {
+    const int nc = (int)hc.size();
+    uint64_t stream_bytes = 0, ncodes = 0;
+    for (const O1Split& k : hc) {
+        stream_bytes += (uint64_t)k.len;
+        ncodes += k.m;
+    }
+    // chains of one size class side by side, for one launch each
+    std::vector<int>& order = R.order;
+    order.resize(nc);
+    for (int q = 0; q < nc; q++) order[q] = q;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hc[x].cls < hc[y].cls; });
+    std::vector<O1Split>& sc = R.sc;
+    sc.resize(nc);
+    uint64_t &nparts = R.nparts = 0, ncand = 0, nlanes = 0, nwaves = 0;
+    double pool = 0;
+    int cls_first[4] = {0, 0, 0, 0};
+    uint64_t cls_waves[3] = {0, 0, 0};
+    for (int i = 0; i < nc; i++) {
+        O1Split& k = sc[i] = hc[order[i]];
+        const SplitPlan& sp = plans[order[i]];
+        const uint64_t nw = (k.nsub - 1 + k.parts - 1) / k.parts;
+        k.tfirst = nparts;
+        k.cfirst = ncand;
+        k.wfirst = nlanes;
+        k.gfirst = nwaves;
+        nparts += k.nsub;
+        ncand += (uint64_t)k.nsub * k.cap;
+        nlanes += (((uint64_t)k.nsub << k.lgk) + 63) & ~63ull;
+        nwaves += nw;
+        cls_waves[k.cls] += nw;
+        for (uint32_t z = k.cls + 1; z < 4; z++) cls_first[z] = i + 1;
+        // twice what the estimate gives for two rounds, and some for each wave
+        pool += 4.0 * sp.nodes * (double)k.m + 16.0 * (double)nw;
+    }
+    O1Split* dch = ws.take<O1Split>(nc);
+    O1SplitWs& W = R.W;
+    W.cand = ws.take<uint32_t>(ncand);
+    W.edge = ws.take<uint32_t>(ncand);
+    W.exits = ws.take<uint32_t>(ncand);
+    W.hdr = ws.take<uint16_t>(nparts * kSplitRounds);
+    W.n0 = ws.take<uint8_t>(nparts);
+    W.wave = ws.take<uint2>((nwaves + 1) * kSplitRounds);
+    W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, 0xF0000000ull);
+    W.pool = ws.take<uint2>(W.pool_cap);
+    W.nparts = nparts;
+    W.res_state = ws.take<uint32_t>(nparts);
+    W.res_e = ws.take<uint64_t>(nparts);
+    W.res_off = ws.take<uint64_t>(nparts);
+    unsigned int* stats = R.stats = ws.take<unsigned int>(8 + nc);
+    W.pool_used = stats + 6 + nc;
+    h2d(dch, sc.data(), sc.size(), st);
+    FZ_HIP(hipMemsetAsync(stats, 0, (8 + nc) * sizeof(unsigned int), st));
+    FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(nlanes)), dim3(256), 0, st, dch, nc, nlanes, W);
+    for (int round = 0; round < kSplitRounds; round++)
+        for (int z = 2; z >= 0; z--) {
+            const int c0 = cls_first[z], cn = cls_first[z + 1] - c0;
+            const uint32_t nw = (uint32_t)cls_waves[z];
+            if (!cn || !nw) continue;
+            if (z == kSplitFew)
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[0]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+            else if (z == kSplitSome)
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[1]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+            else
+                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[2]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
+        }
+    FZ_LAUNCH("o1_split_walk", 0, k_o1s_walk, dim3(nc), dim3(kWalkThreads), 0, st, dch, nc, W, stats);
+    FZ_LAUNCH("o1_split_out", stream_bytes + ncodes * 2, k_o1s_out, dim3(nblk(nparts)), dim3(256), 0, st, dch, nc, W);
+    FZ_HIP(hipGetLastError());
+}
+
+// Sequential chains of several calls, decoded together (dense_batch_run).
+struct DenseBatch {
+    std::mutex mu;
+    std::vector<SerialJob> jobs;
+    std::vector<SerialTables> tabs;
+    uint64_t bytes = 0, codes = 0;
+    std::vector<O1Split> split;
+    std::vector<SplitPlan> plans;
+    double split_bytes = 0;
+    SplitRun run;
+};
+DenseBatch* dense_batch_create() { return new DenseBatch; }
+void dense_batch_destroy(DenseBatch* b) { delete b; }
+size_t dense_batch_size(DenseBatch* b) {
+    std::lock_guard<std::mutex> g(b->mu);
+    return b->jobs.size() + b->split.size();
+}
+void dense_batch_clear(DenseBatch* b) {
+    std::lock_guard<std::mutex> g(b->mu);
+    b->jobs.clear();
+    b->tabs.clear();
+    b->bytes = b->codes = 0;
+    b->split.clear();
+    b->plans.clear();
+    b->split_bytes = 0;
+}
+// Re-encodes the tables and decodes the chains of the lists on st; djobs and dtabs have room for them.
+static void launch_serial(std::vector<SerialJob>& jobs, const std::vector<SerialTables>& tabs, SerialJob* djobs,
+                          SerialTables* dtabs, uint64_t bytes, uint64_t codes, hipStream_t st) {
+    FZ_LAUNCH("o1_serial_tables", 0, k_o1d_tables, dim3(kO1Ctx, (unsigned)tabs.size()), dim3(256), 0, st, dtabs);
+    FZ_LAUNCH("o1_decode_serial", bytes + codes * 2, k_o1d_serial, dim3((unsigned)jobs.size()), dim3(kSerialThreads), 0, st,
+              djobs);
+    FZ_HIP(hipGetLastError());
+}
+void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStream& aux) {
+    std::lock_guard<std::mutex> g(b->mu);
+    const size_t n = b->jobs.size();
+    if (n > 0x7fffffffu) throw std::length_error("too many sequential chains for one launch");
+    if (b->tabs.size() > 65535u) throw std::length_error("too many sequential segments for one launch");
+    // the two decoders beside each other (neither needs what the other writes); the sequential one, which
+    // takes as long as its longest chain, is launched first
+    const bool beside = n && !b->split.empty() && aux.stream;
+    if (n) {
+        // longest chains first, so that the last workgroups to start are short ones
+        std::stable_sort(b->jobs.begin(), b->jobs.end(), [](const SerialJob& x, const SerialJob& y) { return x.m > y.m; });
+        SerialJob* dj = ws.take<SerialJob>(n);
+        SerialTables* dtab = ws.take<SerialTables>(b->tabs.size());
+        // the lists stay in b until dense_batch_clear, after the launches have finished
+        h2d(dj, b->jobs.data(), n, st);
+        h2d(dtab, b->tabs.data(), b->tabs.size(), st);
+        if (beside) {
+            FZ_HIP(hipEventRecord(aux.fork, st));
+            FZ_HIP(hipStreamWaitEvent(aux.stream, aux.fork, 0));
+        }
+        launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, beside ? aux.stream : st);
+        if (beside) FZ_HIP(hipEventRecord(aux.join, aux.stream));
+    }
+    if (!b->split.empty()) split_launch(b->split, b->plans, b->run, ws, st);
+    if (beside) FZ_HIP(hipStreamWaitEvent(st, aux.join, 0));
+}
+
 // defer: the sequential chains are handed to it instead of launched (their decode then runs in
 // dense_batch_run, after the work this call has queued on st).
 static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const std::vector<uint64_t>& chains,
@@ -4522,7 +4636,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     std::vector<uint64_t> hd_seg;
     std::vector<SplitPlan> plans;
     std::vector<uint64_t> seg_of, novf_of;
-    uint64_t dense_bytes = 0, dense_codes = 0, stream_bytes = 0, ncodes = 0;
+    uint64_t dense_bytes = 0, dense_codes = 0;
     // FALCONS_O1_SEQUENTIAL=1 decodes every chain from its start; FALCONS_O1_PARALLEL_SHORT=1 splits
     // short chains too (the tests of either decoder on small fields)
     const char* seq_env = getenv("FALCONS_O1_SEQUENTIAL");
@@ -4550,9 +4664,14 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             pi_seg = c[5];
         }
         SplitPlan sp;
-        if (!all_seq && !(defer && m <= kDeferSymbols)) sp = split_plan(m, c[6], bits, pi, host + nf_off[c[5]], keep_short);
-        if (sp.cls == kSplitNone) {
-            SerialJob k{};
+        if (!all_seq) sp = split_plan(m, c[6], bits, pi, host + nf_off[c[5]], keep_short);
+        const bool batched = defer && m <= kDeferSymbols;
+        if (batched && (sp.warm << sp.lgk) > kBatchWarm) {
+            sp.lgk = 5;
+            sp.warm = 1024;
+        }
+        if (sp.cls != kSplitNone) {
+            O1Split k{};
             k.cb = dev + c[0];
             k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
             k.ov = ovf + c[4];
@@ -4560,15 +4679,36 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             k.err = err;
             k.m = m;
             k.novf = c[6];
+            k.len = (int64_t)c[1];
             k.pos0 = pos0;
             k.x0 = x0;
-            hd.push_back(k);
-            hd_seg.push_back(c[5]);
-            dense_bytes += c[1];
-            dense_codes += m;
-            continue;
+            k.sub_bits = (uint32_t)std::max(2048.0, bits * sp.sub);
+            k.nsub = (uint32_t)std::max<int64_t>(1, (pos0 + k.sub_bits - 1) / k.sub_bits);
+            k.warm_bits = (uint32_t)(bits * sp.warm) + 64;
+            k.warm_steps = 2 * sp.warm;
+            k.lgk = sp.lgk;
+            k.cap = sp.cap;
+            k.parts = sp.parts;
+            k.max_sym = 8 * sp.sub;
+            k.hot0 = hot_window(pi);
+            k.cls = (uint32_t)sp.cls;
+            if (batched) {
+                const double need = split_bytes(k, sp);
+                std::lock_guard<std::mutex> g(defer->mu);
+                if (defer->split_bytes + need <= kBatchSplitBytes) {
+                    defer->split.push_back(k);
+                    defer->plans.push_back(sp);
+                    defer->split_bytes += need;
+                    continue;
+                }
+            } else {
+                hc.push_back(k);
+                plans.push_back(sp);
+                seg_of.push_back(c[5]);
+                continue;
+            }
         }
-        O1Split k{};
+        SerialJob k{};
         k.cb = dev + c[0];
         k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
         k.ov = ovf + c[4];
@@ -4576,24 +4716,12 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         k.err = err;
         k.m = m;
         k.novf = c[6];
-        k.len = (int64_t)c[1];
         k.pos0 = pos0;
         k.x0 = x0;
-        k.sub_bits = (uint32_t)std::max(2048.0, bits * sp.sub);
-        k.nsub = (uint32_t)std::max<int64_t>(1, (pos0 + k.sub_bits - 1) / k.sub_bits);
-        k.warm_bits = (uint32_t)(bits * sp.warm) + 64;
-        k.warm_steps = 2 * sp.warm;
-        k.lgk = sp.lgk;
-        k.cap = sp.cap;
-        k.parts = sp.parts;
-        k.max_sym = 8 * sp.sub;
-        k.hot0 = hot_window(pi);
-        k.cls = (uint32_t)sp.cls;
-        hc.push_back(k);
-        plans.push_back(sp);
-        seg_of.push_back(c[5]);
-        stream_bytes += c[1];
-        ncodes += m;
+        hd.push_back(k);
+        hd_seg.push_back(c[5]);
+        dense_bytes += c[1];
+        dense_codes += m;
     }
     // sequential chains run beside the rest, on the auxiliary stream when there is one
     hipStream_t dst = aux.stream ? aux.stream : st;
@@ -4652,70 +4780,14 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
     } join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
     if (hc.empty()) return;
+    SplitRun R;
+    split_launch(hc, plans, R, ws, st);
     const int nc = (int)hc.size();
-    // chains of one size class side by side, for one launch each
-    std::vector<int> order(nc);
-    for (int q = 0; q < nc; q++) order[q] = q;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hc[x].cls < hc[y].cls; });
-    std::vector<O1Split> sc(nc);
-    uint64_t nparts = 0, ncand = 0, nlanes = 0, nwaves = 0;
-    double pool = 0;
-    int cls_first[4] = {0, 0, 0, 0};
-    uint64_t cls_waves[3] = {0, 0, 0};
-    for (int i = 0; i < nc; i++) {
-        O1Split& k = sc[i] = hc[order[i]];
-        const SplitPlan& sp = plans[order[i]];
-        const uint64_t nw = (k.nsub - 1 + k.parts - 1) / k.parts;
-        k.tfirst = nparts;
-        k.cfirst = ncand;
-        k.wfirst = nlanes;
-        k.gfirst = nwaves;
-        nparts += k.nsub;
-        ncand += (uint64_t)k.nsub * k.cap;
-        nlanes += (((uint64_t)k.nsub << k.lgk) + 63) & ~63ull;
-        nwaves += nw;
-        cls_waves[k.cls] += nw;
-        for (uint32_t z = k.cls + 1; z < 4; z++) cls_first[z] = i + 1;
-        // twice what the estimate gives for two rounds, and some for each wave
-        pool += 4.0 * sp.nodes * (double)k.m + 16.0 * (double)nw;
-    }
-    O1Split* dch = ws.take<O1Split>(nc);
-    O1SplitWs W{};
-    W.cand = ws.take<uint32_t>(ncand);
-    W.edge = ws.take<uint32_t>(ncand);
-    W.exits = ws.take<uint32_t>(ncand);
-    W.hdr = ws.take<uint16_t>(nparts * kSplitRounds);
-    W.n0 = ws.take<uint8_t>(nparts);
-    W.wave = ws.take<uint2>((nwaves + 1) * kSplitRounds);
-    W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, 0xF0000000ull);
-    W.pool = ws.take<uint2>(W.pool_cap);
-    W.nparts = nparts;
-    W.res_state = ws.take<uint32_t>(nparts);
-    W.res_e = ws.take<uint64_t>(nparts);
-    W.res_off = ws.take<uint64_t>(nparts);
-    unsigned int* stats = ws.take<unsigned int>(8 + nc);
-    W.pool_used = stats + 6 + nc;
-    h2d(dch, sc.data(), sc.size(), st);
-    FZ_HIP(hipMemsetAsync(stats, 0, (8 + nc) * sizeof(unsigned int), st));
-    FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(nlanes)), dim3(256), 0, st, dch, nc, nlanes, W);
-    for (int round = 0; round < kSplitRounds; round++)
-        for (int z = 2; z >= 0; z--) {
-            const int c0 = cls_first[z], cn = cls_first[z + 1] - c0;
-            const uint32_t nw = (uint32_t)cls_waves[z];
-            if (!cn || !nw) continue;
-            if (z == kSplitFew)
-                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[0]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
-            else if (z == kSplitSome)
-                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[1]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
-            else
-                FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[2]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
-        }
-    FZ_LAUNCH("o1_split_walk", 0, k_o1s_walk, dim3(nc), dim3(kWalkThreads), 0, st, dch, nc, W, stats);
-    FZ_LAUNCH("o1_split_out", stream_bytes + ncodes * 2, k_o1s_out, dim3(nblk(nparts)), dim3(256), 0, st, dch, nc, W);
-    FZ_HIP(hipGetLastError());
+    const std::vector<O1Split>& sc = R.sc;
+    const std::vector<int>& order = R.order;
     if (stats_on) {
         std::vector<unsigned int> hsv(8 + nc);
-        d2h(hsv.data(), stats, 8 + nc, st);
+        d2h(hsv.data(), R.stats, 8 + nc, st);
         const unsigned int* hs = hsv.data();
         fprintf(stderr, "[o1 decode] chains (chain:exact subsequences/subsequences/escapes/bits a symbol/segment/"
                         "first LDS context of the walk):");
@@ -4746,7 +4818,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
                         "entries outside the set), %u nodes of %llu\n",
-                nc, (unsigned long long)nparts, hs[0] + hs[1], hs[0], hs[1], hs[6 + nc], (unsigned long long)W.pool_cap);
+                nc, (unsigned long long)R.nparts, hs[0] + hs[1], hs[0], hs[1], hs[6 + nc], (unsigned long long)R.W.pool_cap);
     }
 }
 

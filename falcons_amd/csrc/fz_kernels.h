@@ -170,7 +170,7 @@ struct DenseBatch;
 DenseBatch* dense_batch_create();
 void dense_batch_destroy(DenseBatch* b);
 size_t dense_batch_size(DenseBatch* b);
-void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st);
+void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStream& aux);
 void dense_batch_clear(DenseBatch* b);  // after dense_batch_run's launches have finished
 struct EntropyCall;
 EntropyCall* entropy_call_new();

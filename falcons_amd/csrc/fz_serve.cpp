@@ -194,7 +194,7 @@ constexpr size_t kGroupBytes = size_t(16) << 30;
 // (dec_call_begin, middle, finish; the call's workspace a slice of one group allocation), and
 // between the parts the longest-running kernels of the whole group run as one launch each on the
 // batch's own stream: after the first part, the FSE blocks of every item's class bytes; after the
-// second, every item's order-1 sequential chains. A pool of whole per-item calls keeps only a few
+// second, every item's order-1 chains (those split into parts, and those decoded from their start). A pool of whole per-item calls keeps only a few
 // kernels on the GPU at a time, each a handful of workgroups running for milliseconds; one launch
 // holds them all. An item whose parts do not fit its slice, or fail, is decompressed by a plain
 // call afterwards.
@@ -290,7 +290,7 @@ void decompress_grouped(fz_ctx* ctx, WorkerSet& wset, fz_batch_dec_item* items, 
             }
             rec[j] = hipEventRecord(R.ev[j], w->stream) == hipSuccess;
         }, wset.size());
-        shared([&] { dense_batch_run(R.batch, ctx->arena, cst); });
+        shared([&] { dense_batch_run(R.batch, ctx->arena, cst, ctx->aux); });
         wset.run(idx, [&](fz_ctx* w, int j) {
             fz_batch_dec_item& it = items[order[k0 + j]];
             if (ok[j]) {
