@@ -8,9 +8,10 @@
 //            gamma/FSE side stream.
 //
 // Data-parallel steps (sampling, delta, escape selection, context histograms, run/value extraction,
-// mantissa bit scatter, block framing, run expansion, prefix sums) run across the whole chip. The
-// tANS chains themselves are sequential state machines; each chain is run by one lane here and all
-// chains of a call run concurrently.
+// mantissa bit packing, block framing, run expansion, prefix sums) run across the whole chip. The
+// tANS and FSE chains are sequential state machines. They are cut into pieces, and what is followed
+// through a piece is every state that may enter it, or a guess that is repaired; a walk picks the true
+// ones. Chains that cannot be cut (decoding with many escapes) run in a workgroup each.
 #include <cstdio>
 #include <cstdlib>
 #include <stdexcept>
@@ -79,64 +80,6 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
 __device__ __forceinline__ void wave_lds_order() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-}
-
-struct BitW {  // LSB-first FSE bitstream writer (zfse/bitstream.h)
-    uint8_t* buf;
-    uint64_t pos;
-    uint64_t acc;
-    uint32_t n;
-};
-__device__ inline void bw_add(BitW& w, uint64_t v, uint32_t nb) {
-    if (!nb) return;
-    w.acc |= (v & ((1ull << nb) - 1)) << w.n;
-    w.n += nb;
-    while (w.n >= 8) {
-        w.buf[w.pos++] = (uint8_t)w.acc;
-        w.acc >>= 8;
-        w.n -= 8;
-    }
-}
-__device__ inline uint64_t bw_close(BitW& w) {
-    bw_add(w, 1, 1);
-    if (w.n) {
-        w.buf[w.pos++] = (uint8_t)w.acc;
-        w.acc = 0;
-        w.n = 0;
-    }
-    return w.pos;
-}
-template <class CT>
-__device__ inline void fse_encode(BitW& w, uint32_t& state, const CT& ct, unsigned sym) {
-    const uint32_t nbOut = (uint32_t)(((uint64_t)state + ct.deltaNbBits[sym]) >> 16);
-    bw_add(w, state, nbOut);
-    state = ct.stateTable[(state >> nbOut) + ct.deltaFindState[sym]];
-}
-
-struct BitR {  // backward reader of such a stream; bits below the start read as zero
-    const uint8_t* buf;
-    int64_t pos;
-};
-__device__ inline bool br_init(BitR& r, const uint8_t* buf, uint64_t size) {
-    r.buf = buf;
-    if (size < 1 || buf[size - 1] == 0) { r.pos = 0; return false; }
-    r.pos = (int64_t)(size - 1) * 8 + (int64_t)highbit32(buf[size - 1]);
-    return true;
-}
-__device__ inline uint32_t br_read(BitR& r, uint32_t nb) {
-    if (!nb) return 0;
-    const int64_t lo = r.pos - nb;
-    r.pos = lo;
-    uint32_t v = 0;
-    const int64_t b0 = lo >> 3;  // arithmetic shift: floor for negatives
-    const int sh = (int)(lo - b0 * 8);
-    uint64_t w = 0;
-    for (int j = 0; j < 4; j++) {
-        const int64_t b = b0 + j;
-        if (b >= 0) w |= (uint64_t)r.buf[b] << (8 * j);
-    }
-    v = (uint32_t)((w >> sh) & ((1ull << nb) - 1));
-    return v;
 }
 
 // Backward reader with a 64-bit window in registers: bits [lo, lo + 64) of the stream (bytes below the
@@ -1467,7 +1410,7 @@ __global__ void __launch_bounds__(256) k_o1_tables(const uint32_t* cnt_all, uint
 //   trajectory (k_o1_fix, repeated while some piece fails to meet it).
 // 540,000 codes, the order-1 stage without its side streams: guessed and repaired 1.4 to 6 ms (2 to 10
 // rounds, as slowly as the last states merge), by sets 0.25 ms; 86,000: 1.03 and 0.24 ms. By sets a
-// code costs 2.25 steps of a wave: 134 million codes, 1.4 ms guessed, repaired and emitted, would take 7.
+// code costs 2.25 steps of a wave: 134 million codes, 1.3 ms guessed, repaired and emitted, would take 7.
 constexpr uint32_t kO1Piece = 1024, kO1PieceMin = 256;  // as many pieces as the chip has lanes in one round of workgroups
 constexpr uint32_t kEncThreads = 1024, kEmitThreads = 1024, kRingWords = 8;
 constexpr int kEncHot = 8, kEmitHot = 6;  // state tables in LDS: 158 KB with the per-symbol arrays (and the emit's rings)
@@ -1509,9 +1452,9 @@ __device__ inline uint32_t o1_seed_state(const int16_t* bins, uint64_t lo, uint6
 // (16 KB each) of the H contexts that occur most often. With the state tables in L2 the lanes of a
 // full chip wait for its rate of requests (a lane reads one entry a step from anywhere in 240 KB: 160 G
 // steps/s); with 8 of them in LDS a step waits for L2 only in the waves that hold a rare context, and
-// its instructions count as much. 134 million codes, one in 15 an escape: k_o1_spec 0.84 -> 0.40 ms,
-// k_o1_fix 0.85 -> 0.50, k_o1_emit (6 tables, the rings beside them) 0.95 -> 0.50; two codes in five an
-// escape: 1.40 -> 0.48, 2.2 -> 2.6 (beside the escapes' blocks, which come at once now), 0.93 -> 0.45.
+// its instructions count as much. 134 million codes, one in 15 an escape: k_o1_spec 0.84 -> 0.37 ms,
+// k_o1_fix 0.85 -> 0.50, k_o1_emit (6 tables, the rings beside them) 0.95 -> 0.45; two codes in five an
+// escape: 1.40 -> 0.43, 2.2 -> 2.5 (beside the escapes' blocks, which come at once now), 0.93 -> 0.41.
 template <int H>
 struct O1EncLds {
     // a symbol's deltaNbBits, and its deltaFindState + 8,192 * place of the context's state table: below H
@@ -1590,43 +1533,66 @@ __device__ __forceinline__ uint64_t o1_piece_of(const O1Chains& C, uint32_t grou
 
 // Runs step(u, k) for the steps i = 8c + k from s_hi down to s_lo of a piece, u the step's o1_index
 // (previous code 0 at the chain's first symbol lo), begin(8c) before and more() after those of a group of
-// eight; ends early when more returns false. The codes come in aligned 16-byte loads, eight at a time,
-// the next eight in flight: one load per eight steps instead of two scattered 2-byte loads per step (the
-// lanes of a wave run pieces 1 KB and more apart). A step costs its instructions as much as its waits (16
-// waves a CU), so whole groups inside the piece, nearly all, run without tests of their bounds. bins is
-// 16-byte aligned and its allocation extends to the next multiple of 16 bytes.
+// eight; ends early when more returns false. A lane's codes come 32 at a time in four 16-byte loads of
+// the same 64 bytes, the next 32 in flight: the open lines of a full chip's lanes (one each, 33 MB) do not
+// stay in L2, and eight loads a line fetched the codes five times (k_o1_spec 0.40 ms, k_o1_emit 0.50; 0.37 and 0.45 so). A step costs its instructions as much
+// as its waits (16 waves a CU), so blocks of 32 inside the piece, nearly all, run without tests of their
+// bounds. bins is 16-byte aligned and its allocation extends to the next multiple of 16 bytes.
 template <typename B, typename F, typename M>
 __device__ __forceinline__ void o1_piece_codes(const int16_t* bins, uint64_t lo, uint64_t s_hi, uint64_t s_lo, B&& begin,
                                                F&& step, M&& more) {
     const u32x4* b4 = reinterpret_cast<const u32x4*>(bins);
-    uint64_t c = s_hi >> 3;
-    const uint64_t c_lo = s_lo >> 3;
-    u32x4 cur = b4[c];
-    u32x4 nxt = c > 0 ? b4[c - 1] : u32x4{0u, 0u, 0u, 0u};
-    for (;;) {
-        const uint64_t base = 8 * c;
-        begin(base);
-        int v[9];  // v[k + 1]: code 8c + k; v[0]: code 8c - 1
+    // v[k + 1]: code k of a group of eight; v[0]: the code in front of it
+    auto codes = [](u32x4 w, u32x4 before, int (&v)[9]) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            v[2 * k + 1] = (int)(int16_t)(cur[k] & 0xFFFFu);
-            v[2 * k + 2] = (int)cur[k] >> 16;
+            v[2 * k + 1] = (int)(int16_t)(w[k] & 0xFFFFu);
+            v[2 * k + 2] = (int)w[k] >> 16;
         }
-        v[0] = (int)nxt[3] >> 16;
-        if (base >= s_lo && base + 7 <= s_hi && base > lo) {
+        v[0] = (int)before[3] >> 16;
+    };
+    const u32x4 zero{0u, 0u, 0u, 0u};
+    u32x4 cur[4] = {zero, zero, zero, zero}, nxt[4] = {zero, zero, zero, zero};
+    uint64_t blk = s_hi >> 5;
+    const uint64_t blk_lo = s_lo >> 5;
+    auto inside = [&](uint64_t k) { return 32 * k >= s_lo && 32 * k + 31 <= s_hi && 32 * k > lo; };
+    if (inside(blk)) {
 #pragma unroll
-            for (int k = 7; k >= 0; k--) step(o1_index(v[k + 1], v[k]), k);
+        for (int g = 0; g < 4; g++) cur[g] = b4[4 * blk + g];
+    }
+    for (;;) {
+        if (blk > 0) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) nxt[g] = b4[4 * (blk - 1) + g];
+        }
+        int v[9];
+        if (inside(blk)) {
+#pragma unroll
+            for (int g = 3; g >= 0; g--) {
+                begin(32 * blk + 8 * g);
+                codes(cur[g], g > 0 ? cur[g - 1] : nxt[3], v);
+#pragma unroll
+                for (int k = 7; k >= 0; k--) step(o1_index(v[k + 1], v[k]), k);
+                if (!more()) return;
+            }
         } else {
+            for (int g = 3; g >= 0; g--) {
+                const uint64_t c = 4 * blk + g, base = 8 * c;
+                if (base > s_hi || base + 7 < s_lo) continue;
+                begin(base);
+                codes(b4[c], c > 0 ? b4[c - 1] : zero, v);
 #pragma unroll
-            for (int k = 7; k >= 0; k--) {
-                const uint64_t i = base + (uint64_t)k;
-                if (i <= s_hi && i >= s_lo) step(o1_index(v[k + 1], i > lo ? v[k] : 0), k);
+                for (int k = 7; k >= 0; k--) {
+                    const uint64_t i = base + (uint64_t)k;
+                    if (i <= s_hi && i >= s_lo) step(o1_index(v[k + 1], i > lo ? v[k] : 0), k);
+                }
+                if (!more()) return;
             }
         }
-        if (c == c_lo || !more()) return;
-        c--;
-        cur = nxt;
-        nxt = c > 0 ? b4[c - 1] : u32x4{0u, 0u, 0u, 0u};
+        if (blk == blk_lo) return;
+        blk--;
+#pragma unroll
+        for (int g = 0; g < 4; g++) cur[g] = nxt[g];
     }
 }
 struct PieceNoop {
@@ -1779,10 +1745,6 @@ __device__ inline void ww_put(WordWriter& W, uint32_t v, uint32_t nb) {
         W.n -= 32;
     }
 }
-__device__ inline void ww_flush(WordWriter& W) {
-    if (W.n) atomicOr(&W.w[W.idx], (uint32_t)W.acc);
-}
-
 // k_o1_emit's output: a lane's words pass through an 8-word LDS ring and leave in aligned 32-byte
 // runs (the lanes of a wave write 131 K pieces' lines at once, and single-word stores leave partly
 // written lines to L2 evictions). The first word (shared with the previous piece) is OR-ed in; the
@@ -4768,7 +4730,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         launch_serial(hd, tabs, dj, dtab, dense_bytes, dense_codes, dst);
     }
-    struct Join {  // the caller's stream waits for the dense chains however this function exits
+    struct Join {  // the caller's stream waits for the sequential chains however this function exits
         const AuxStream& a;
         hipStream_t st;
         bool on;

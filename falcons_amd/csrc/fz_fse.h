@@ -251,74 +251,6 @@ FZ_HD uint64_t read_ncount(int16_t* norm, unsigned* maxSym, unsigned* tableLog, 
     return (bit + 7) / 8;
 }
 
-// Symbol spread shared by the encoder and decoder tables; tableSymbol must hold 1<<tableLog bytes.
-// Returns false if the counts do not fill the table exactly.
-FZ_HD bool spread_symbols(uint8_t* tableSymbol, const int16_t* norm, unsigned maxSym, unsigned tableLog,
-                          uint32_t* highOut) {
-    const uint32_t tableSize = 1u << tableLog, mask = tableSize - 1;
-    const uint32_t step = (tableSize >> 1) + (tableSize >> 3) + 3;
-    uint32_t high = tableSize - 1;
-    for (uint32_t s = 0; s <= maxSym; s++)
-        if (norm[s] == -1) tableSymbol[high--] = (uint8_t)s;
-    uint32_t pos = 0;
-    for (uint32_t s = 0; s <= maxSym; s++)
-        for (int k = 0; k < norm[s]; k++) {
-            tableSymbol[pos] = (uint8_t)s;
-            pos = (pos + step) & mask;
-            while (pos > high) pos = (pos + step) & mask;
-        }
-    if (highOut) *highOut = high;
-    return pos == 0;
-}
-
-FZ_HD void build_ctable(CTable* ct, const int16_t* norm, unsigned maxSym, unsigned tableLog, uint8_t* scratch) {
-    const uint32_t tableSize = 1u << tableLog;
-    ct->tableLog = tableLog;
-    ct->maxSym = maxSym;
-    spread_symbols(scratch, norm, maxSym, tableLog, nullptr);
-    uint32_t cumul[257];
-    cumul[0] = 0;
-    for (uint32_t u = 1; u <= maxSym + 1; u++)
-        cumul[u] = cumul[u - 1] + (norm[u - 1] == -1 ? 1u : (uint32_t)norm[u - 1]);
-    for (uint32_t u = 0; u < tableSize; u++) {
-        const uint8_t s = scratch[u];
-        ct->stateTable[cumul[s]++] = (uint16_t)(tableSize + u);
-    }
-    unsigned total = 0;
-    for (unsigned s = 0; s <= maxSym; s++) {
-        const int nc = norm[s];
-        if (nc == 0) {
-            ct->deltaNbBits[s] = ((tableLog + 1) << 16) - (1u << tableLog);
-            ct->deltaFindState[s] = 0;
-        } else if (nc == -1 || nc == 1) {
-            ct->deltaNbBits[s] = (tableLog << 16) - (1u << tableLog);
-            ct->deltaFindState[s] = (int32_t)total - 1;
-            total++;
-        } else {
-            const uint32_t maxBitsOut = tableLog - highbit32((uint32_t)(nc - 1));
-            ct->deltaNbBits[s] = (maxBitsOut << 16) - ((uint32_t)nc << maxBitsOut);
-            ct->deltaFindState[s] = (int32_t)total - nc;
-            total += (unsigned)nc;
-        }
-    }
-}
-
-FZ_HD bool build_dtable(DEntry* dt, const int16_t* norm, unsigned maxSym, unsigned tableLog, uint8_t* scratch) {
-    const uint32_t tableSize = 1u << tableLog;
-    if (!spread_symbols(scratch, norm, maxSym, tableLog, nullptr)) return false;
-    uint16_t next[256];
-    for (uint32_t s = 0; s <= maxSym; s++) next[s] = norm[s] == -1 ? 1 : (uint16_t)norm[s];
-    for (uint32_t u = 0; u < tableSize; u++) {
-        const uint8_t s = scratch[u];
-        const uint32_t ns = next[s]++;
-        const uint8_t nb = (uint8_t)(tableLog - highbit32(ns));
-        dt[u].symbol = s;
-        dt[u].nbBits = nb;
-        dt[u].newState = (uint16_t)((ns << nb) - tableSize);
-    }
-    return true;
-}
-
 // FSE_initCState2 (zfse/fse.h:504-515)
 template <class CT>
 FZ_HD uint32_t init_state2(const CT* ct, unsigned sym) {
