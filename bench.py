@@ -54,8 +54,9 @@ def parse():
 
 
 # launch-profiler name -> kernel symbol, for the counter data of profiles/
-KERNEL_SYMBOLS = {"o1_decode_dense": "k_o1d_dense", "o1_decode_graph": "k_o1d_graph", "o1_decode_walk": "k_o1d_walk",
-                  "o1_decode_out": "k_o1d_out", "o1_encode_spec": "k_o1_spec", "o1_encode_emit": "k_o1_emit"}
+KERNEL_SYMBOLS = {"o1_decode_serial": "k_o1d_serial", "o1_split_warm": "k_o1s_warm", "o1_split_walk": "k_o1s_walk",
+                  "o1_split_out": "k_o1s_out", "o1_encode_spec": "k_o1_spec", "o1_encode_emit": "k_o1_emit",
+                  "interp_yx": ("k_yx<float, false>", "k_yx<float, true>")}
 
 
 def measured_traffic(name, a):
@@ -66,10 +67,13 @@ def measured_traffic(name, a):
         return None
     try:
         with open(os.path.join(ROOT, "profiles", prof)) as f:
-            k = json.load(f)["kernels"].get(KERNEL_SYMBOLS.get(name, name))
+            kernels = json.load(f)["kernels"]
+        names = KERNEL_SYMBOLS.get(name, name)
+        found = [kernels[k] for k in ([names] if isinstance(names, str) else names)]
     except (OSError, ValueError, KeyError):
         return None
-    return None if k is None else int(k["fetch_bytes"] + k["write_bytes"])
+    launches = sum(k["launches"] for k in found)
+    return int(sum((k["fetch_bytes"] + k["write_bytes"]) * k["launches"] for k in found) / launches)
 
 
 def log(msg):
