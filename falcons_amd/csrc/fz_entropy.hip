@@ -3927,17 +3927,29 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
                   (int)(s_sampled * kO1Ctx * kO1Sym));
         FZ_HIP(hipGetLastError());
     }
-    {
-        // escapes below each chain's end
-        const int nb = (int)(S * kO1K);
-        uint64_t* dends = ws.take<uint64_t>(nb);
-        uint64_t* dbelow = ws.take<uint64_t>(nb);
-        h2d(dends, ends.data(), nb, st);
-        FZ_LAUNCH("o1_escape_counts", 0, k_sel_below<IsO1Escape>, dim3((unsigned)nb), dim3(256), 0, st, bins,
-                  n, IsO1Escape{}, esc_tiles.offs, esc_tiles.count, nsel, dends, dbelow);
-        FZ_HIP(hipGetLastError());
-        std::vector<uint64_t> below(nb);
-        d2h(below.data(), dbelow, nb, st);
+    // escapes below each chain's end
+    const int nch = (int)(S * kO1K);
+    uint64_t* dends = ws.take<uint64_t>(nch);
+    uint64_t* dbelow = ws.take<uint64_t>(nch);
+    h2d(dends, ends.data(), nch, st);
+    FZ_LAUNCH("o1_escape_counts", 0, k_sel_below<IsO1Escape>, dim3((unsigned)nch), dim3(256), 0, st, bins, n, IsO1Escape{},
+              esc_tiles.offs, esc_tiles.count, nsel, dends, dbelow);
+    FZ_HIP(hipGetLastError());
+    if (aux.stream) {
+        FZ_HIP(hipEventRecord(aux.fork, st));
+        FZ_HIP(hipStreamWaitEvent(aux.stream, aux.fork, 0));
+    }
+    // The escape side streams need only the escaped values and their segment offsets: with a second
+    // stream they are coded there, beside the chains. Their counts are read over that stream, and only after
+    // the chains' first kernels are queued: the main stream has work meanwhile.
+    std::vector<EscapeBlock> oblock(S);
+    EscapeWorker ew;
+    bool counted = false;
+    auto start_escapes = [&]() {
+        if (counted) return;
+        counted = true;
+        std::vector<uint64_t> below(nch);
+        d2h(below.data(), dbelow, nch, aux.stream ? aux.stream : st);
         for (uint64_t g = 0; g < S; g++) {
             ovf_off[g] = e;
             for (int k = 0; k < kO1K; k++) {
@@ -3948,17 +3960,10 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
                 e = b;
             }
         }
-    }
-    ovf_off[S] = e;
-    // the escape side streams need only the escaped values and their segment offsets: with a
-    // second stream they are coded there, beside the chains
-    std::vector<EscapeBlock> oblock(S);
-    EscapeWorker ew;
-    if (aux.stream) {
+        ovf_off[S] = e;
+        if (!aux.stream) return;
         const size_t need = escape_workspace_bound(ovf_off, S);
         ew.sub.bind(ws.take<uint8_t>(need), need);
-        FZ_HIP(hipEventRecord(aux.fork, st));
-        FZ_HIP(hipStreamWaitEvent(aux.stream, aux.fork, 0));
         int dev = 0;
         FZ_HIP(hipGetDevice(&dev));
         LaunchProfiler* prof = g_prof;
@@ -3972,10 +3977,9 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
             }
             g_prof = nullptr;
         });
-    }
+    };
     FZ_LAUNCH("o1_tables", 0, k_o1_tables, dim3(kO1Ctx, (unsigned)S), dim3(256), 0, st, cnt, nf, ct, use);
     FZ_HIP(hipGetLastError());
-    const int nch = (int)(S * kO1K);
     uint64_t* dchains = ws.take<uint64_t>(chains.size());
     h2d(dchains, chains.data(), chains.size(), st);
     uint64_t maxcs = 0;
@@ -4032,6 +4036,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         FZ_LAUNCH("o1_encode_close", 0, k_o1_close, dim3(nblk(nch, 64)), dim3(64), 0, st, bins, CH, ct, end_state, chain_bits,
                   words, stride_words, blen, failed);
         FZ_HIP(hipGetLastError());
+        start_escapes();
     }
     auto guess_and_repair = [&]() {
         // one round of workgroups of one a CU, whole ones for every segment
@@ -4056,6 +4061,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
             FZ_LAUNCH("o1_encode_spec", n * 4, k_o1_spec, dim3((unsigned)S * groups), dim3(kEncThreads), 0, st, bins, CH, groups, np,
                       ct, use, slog, spec_end, spec_bits);
             FZ_HIP(hipGetLastError());
+            start_escapes();
             FZ_HIP(hipMemcpyAsync(nbits, spec_bits, np * 8, hipMemcpyDeviceToDevice, st));
             // fix-up rounds; each round finalizes at least the next piece of every chain, so the loop
             // ends within max-pieces-per-chain rounds
@@ -4108,6 +4114,7 @@ static size_t encode_method1(const int16_t* bins, uint64_t n, uint8_t* out, uint
         FZ_HIP(hipGetLastError());
     };
     if (!sets) guess_and_repair();
+    start_escapes();  // no chain has a step
     // escape side streams, one block per segment
     if (aux.stream) ew.join();
     else escape_streams(ovf, ovf_off, S, oblock, ws, st);
@@ -4188,8 +4195,7 @@ size_t entropy_encode(const int16_t* codes, uint64_t n, uint8_t* out, size_t out
     if (n < (uint64_t)20 * kO1Ctx * kO1Sym) method = 0;
     if (stats) { stats->method = method; stats->use_delta = use_delta; }
     const uint8_t save[5] = {(uint8_t)(method | (use_delta ? 0x80 : 0)), 0, 0, 0, 0};
-    FZ_HIP(hipMemcpyAsync(out, save, 5, hipMemcpyHostToDevice, st));
-    sync(st);
+    FZ_HIP(hipMemcpyAsync(out, save, 5, hipMemcpyHostToDevice, st));  // save lives until the encoders have waited
     const int16_t* bins = codes;
     if (use_delta && n > 0) {
         int16_t* d = ws.take<int16_t>(n);
