@@ -27,6 +27,7 @@
 #include "fz_fse.h"
 #include "fz_kernels.h"
 #include "fz_select.h"
+#include "fz_split.h"
 
 namespace fz {
 
@@ -2227,9 +2228,9 @@ struct O1SplitWs {
     uint32_t* exits;             // states in which paths leave the part
     uint16_t* hdr;               // [kSplitRounds][parts]: start states | exits << 8 after the round
     uint8_t* n0;                 // [parts]: start states from the warm-up
-    uint2* wave;                 // [graph waves][kSplitRounds]: first node in pool (~0: no room there), nodes
+    uint2* wave;                 // [graph waves][kSplitRounds]: first node in pool (kPoolNone: no room there), nodes
     uint2* pool;                 // nodes: edges for an escaped code >= 0 / < 0
-    unsigned int* pool_used;
+    NodeCount* pool_used;
     uint64_t pool_cap;
     uint64_t nparts;
     uint32_t* res_state;         // [parts]: entry, escape index and output offset on the true path
@@ -2580,13 +2581,10 @@ __global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, ui
     nn = min(nn, (uint32_t)NC);
     uint32_t at = 0;
     if (nn) {
-        if (l == 0) at = atomicAdd(ws.pool_used, nn);
+        if (l == 0) at = pool_first(atomicAdd(ws.pool_used, (NodeCount)nn), nn, ws.pool_cap);
         at = __builtin_amdgcn_readfirstlane(at);
-        if ((uint64_t)at + nn <= ws.pool_cap) {
+        if (at != kPoolNone)  // else the walk finds no node and decodes such parts exactly
             for (uint32_t i = l; i < nn; i += 64) ws.pool[at + i] = nodes[i];
-        } else {
-            at = ~0u;  // the walk finds no node and decodes such parts exactly
-        }
     }
     if (l == 0) ws.wave[gw * kSplitRounds + round] = make_uint2(at, nn);
     for (uint32_t i = l; i < np; i += 64) hdr[t0 + i] = (uint16_t)(ncand[i] | min(nex[i], cap) << 8);
@@ -2653,7 +2651,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
             bool room = true;
 #pragma unroll
             for (int z = 0; z < kSplitRounds; z++) {
-                const uint32_t n = room && rd[z].x != ~0u ? min(rd[z].y, NS - ns) : 0u;
+                const uint32_t n = room && rd[z].x != kPoolNone ? min(rd[z].y, NS - ns) : 0u;
                 for (uint32_t i0 = 0; i0 < n; i0 += 512) {
                     u32x2 v[8];
 #pragma unroll
@@ -2676,7 +2674,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
         const uint2* rw = ws.wave + (c.gfirst + u) * kSplitRounds;
         for (int z = 0; z < kSplitRounds; z++) {
             const uint2 v = rw[z];
-            if (tgt < v.y) return v.x == ~0u ? kSplitFail : glb(reinterpret_cast<const uint32_t*>(ws.pool))[2 * ((uint64_t)v.x + tgt) + neg];
+            if (tgt < v.y) return v.x == kPoolNone ? kSplitFail : glb(reinterpret_cast<const uint32_t*>(ws.pool))[2 * ((uint64_t)v.x + tgt) + neg];
             tgt -= v.y;
         }
         return kSplitFail;
@@ -2922,9 +2920,17 @@ __global__ void __launch_bounds__(256) k_o1s_out(const O1Split* ch, int nch, O1S
         rd.refill(cw);
         out[i++] = (int16_t)step();
     }
-    // the part's symbols are those that start above the next boundary
+    // the part's symbols are those that start above the next boundary, and leave the state and the
+    // escape that the walk entered the next part with
     const int64_t pos = 32 * rd.j + rd.have - cw.shift, stop = b - (int64_t)c.sub_bits;
-    if (bad || (last && e != novf) || (!last && o1 > o0 && (pos > stop || pos + (int64_t)nb <= stop))) *c.err = 1;
+    if (last) {
+        bad = bad || e != novf;
+    } else {
+        const uint32_t to = ws.res_state[t + 1];
+        bad = bad || pos != stop - (int64_t)(to >> 17) || idx != (to & 0x1FFFFu) || e != ws.res_e[t + 1] ||
+              (o1 > o0 && pos + (int64_t)nb <= stop);
+    }
+    if (bad) *c.err = 1;
 }
 
 // ---- chains decoded from their start ------------------------------------------------------------
@@ -4461,6 +4467,8 @@ struct SplitRun {
     unsigned int* stats = nullptr;
     uint64_t nparts = 0;
 };
+// 32-bit words of its statistics for nc chains: six counts, one a chain, then the pool's count.
+static int split_stats(int nc) { return (6 + nc + 1) / 2 * 2 + 2; }
 // Device bytes that split_launch takes for a chain, but for its few words a part.
 static double split_bytes(const O1Split& k, const SplitPlan& sp) {
     return 12.0 * k.nsub * k.cap + 8.0 * (4.0 * sp.nodes * (double)k.m + 16.0 * k.nsub / k.parts);
@@ -4509,16 +4517,19 @@ static void split_launch(const std::vector<O1Split>& hc, const std::vector<Split
     W.hdr = ws.take<uint16_t>(nparts * kSplitRounds);
     W.n0 = ws.take<uint8_t>(nparts);
     W.wave = ws.take<uint2>((nwaves + 1) * kSplitRounds);
-    W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, 0xF0000000ull);
+    W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, kPoolMax);
+    // FALCONS_O1_POOL_NODES: a test switch; the parts whose nodes find no room are decoded by the walk
+    if (const char* few = getenv("FALCONS_O1_POOL_NODES")) W.pool_cap = std::min<uint64_t>(W.pool_cap, std::strtoull(few, nullptr, 10));
     W.pool = ws.take<uint2>(W.pool_cap);
     W.nparts = nparts;
     W.res_state = ws.take<uint32_t>(nparts);
     W.res_e = ws.take<uint64_t>(nparts);
     W.res_off = ws.take<uint64_t>(nparts);
-    unsigned int* stats = R.stats = ws.take<unsigned int>(8 + nc);
-    W.pool_used = stats + 6 + nc;
+    const int nstats = split_stats(nc);
+    unsigned int* stats = R.stats = ws.take<unsigned int>(nstats);
+    W.pool_used = reinterpret_cast<NodeCount*>(stats + nstats - 2);
     h2d(dch, sc.data(), sc.size(), st);
-    FZ_HIP(hipMemsetAsync(stats, 0, (8 + nc) * sizeof(unsigned int), st));
+    FZ_HIP(hipMemsetAsync(stats, 0, nstats * sizeof(unsigned int), st));
     FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(nlanes)), dim3(256), 0, st, dch, nc, nlanes, W);
     for (int round = 0; round < kSplitRounds; round++)
         for (int z = 2; z >= 0; z--) {
@@ -4759,8 +4770,10 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     const std::vector<O1Split>& sc = R.sc;
     const std::vector<int>& order = R.order;
     if (stats_on) {
-        std::vector<unsigned int> hsv(8 + nc);
-        d2h(hsv.data(), R.stats, 8 + nc, st);
+        std::vector<unsigned int> hsv(split_stats(nc));
+        d2h(hsv.data(), R.stats, hsv.size(), st);
+        NodeCount nodes = 0;
+        memcpy(&nodes, &hsv[hsv.size() - 2], sizeof(nodes));
         const unsigned int* hs = hsv.data();
         fprintf(stderr, "[o1 decode] chains (chain:exact subsequences/subsequences/escapes/bits a symbol/segment/"
                         "first LDS context of the walk):");
@@ -4790,8 +4803,8 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             fprintf(stderr, "\n");
         }
         fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
-                        "entries outside the set), %u nodes of %llu\n",
-                nc, (unsigned long long)R.nparts, hs[0] + hs[1], hs[0], hs[1], hs[6 + nc], (unsigned long long)R.W.pool_cap);
+                        "entries outside the set), %llu nodes of %llu\n",
+                nc, (unsigned long long)R.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap);
     }
 }
 
