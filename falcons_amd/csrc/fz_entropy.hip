@@ -4458,8 +4458,7 @@ static SplitPlan split_plan(uint64_t m, uint64_t novf, double bits, const double
     return s;
 }
 
-// The split chains of a call or of a batch, in launch order, and what their kernels left (sc is read by a
-// copy on the stream: it stays until that has run).
+// The split chains of a call or of a batch, in launch order, and what their kernels left.
 struct SplitRun {
     std::vector<O1Split> sc;
     std::vector<int> order;
@@ -4609,17 +4608,25 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStrea
     if (beside) FZ_HIP(hipStreamWaitEvent(st, aux.join, 0));
 }
 
+// The lists of one call's chains. Copies on the call's stream read them: they stay until it has been waited for.
+struct O1Lists {
+    SplitRun split;
+    std::vector<SerialJob> serial;
+    std::vector<SerialTables> tabs;  // one a segment
+};
+
 // defer: the sequential chains are handed to it instead of launched (their decode then runs in
 // dense_batch_run, after the work this call has queued on st).
 static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const std::vector<uint64_t>& chains,
                                const std::vector<uint64_t>& nf_off, const DEntry* dt, const int16_t* ovf, int16_t* out,
-                               int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer) {
+                               int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer,
+                               O1Lists& lists) {
     const int nch = (int)(chains.size() / 7);
     std::vector<O1Split> hc;
-    std::vector<SerialJob> hd;
+    std::vector<SerialJob>& hd = lists.serial;
     std::vector<uint64_t> hd_seg;
     std::vector<SplitPlan> plans;
-    std::vector<uint64_t> seg_of, novf_of;
+    std::vector<uint64_t> seg_of;
     uint64_t dense_bytes = 0, dense_codes = 0;
     // FALCONS_O1_SEQUENTIAL=1 decodes every chain from its start; FALCONS_O1_PARALLEL_SHORT=1 splits
     // short chains too (the tests of either decoder on small fields)
@@ -4711,7 +4718,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     hipStream_t dst = aux.stream ? aux.stream : st;
     const bool stats_on = getenv("FALCONS_DECODE_STATS") != nullptr;
     uint64_t* dense_times = nullptr;  // per sequential chain: clock at start and end (statistics only)
-    std::vector<SerialTables> tabs;   // one a segment; read by copies in flight until the function returns
+    std::vector<SerialTables>& tabs = lists.tabs;
     if (!hd.empty()) {
         for (size_t q = 0; q < hd.size();) {
             size_t q1 = q;
@@ -4764,7 +4771,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
     } join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
     if (hc.empty()) return;
-    SplitRun R;
+    SplitRun& R = lists.split;
     split_launch(hc, plans, R, ws, st);
     const int nc = (int)hc.size();
     const std::vector<O1Split>& sc = R.sc;
@@ -4978,6 +4985,7 @@ struct EntropyCall {
     int* err = nullptr;
     int16_t* ovf = nullptr;       // method 1: escaped codes
     std::vector<uint8_t*> vcls;   // method 1: class bytes of every segment
+    O1Lists lists;                // method 1: its chains; entropy_decode_end waits for what reads them
     uint8_t* rcl = nullptr;       // method 0: run and value classes
     uint8_t* vcl = nullptr;
 };
@@ -5083,7 +5091,7 @@ void entropy_decode_middle(EntropyCall* E, DevArena& ws, hipStream_t st, const A
             d2h(&herr, err, 1, st);
             if (herr) throw std::invalid_argument("corrupt o1 tANS tables");
         }
-        o1_decode_parallel(host, dev, chains, nf_off, dt, ovf, out, err, ws, st, aux, defer);
+        o1_decode_parallel(host, dev, chains, nf_off, dt, ovf, out, err, ws, st, aux, defer, E->lists);
     } else {
         const uint64_t nr = Lay.nr, nv = Lay.nv, rbp = Lay.rbp, vbp = Lay.vbp;
         const uint64_t o_rman = Lay.o_rman, o_vman = Lay.o_vman;
