@@ -475,7 +475,8 @@ struct Timer {
 // Workspace a call is expected to take: the peak measured on k^-3 fields with the order-1 tANS
 // coder (34 B per float element to compress, 16 B to decompress) with a margin. The arena grows
 // beyond it on demand (RLE+FSE streams and escape-heavy fields take more), so these size the first
-// allocation and the admission of served requests, not a hard limit.
+// allocation and the admission of served requests, not a hard limit. The sets and graphs of the split
+// order-1 decoder come beside it, split_limit() at most; calls that are admitted by their workspace add that.
 size_t fz::compress_workspace_bytes(uint64_t n, int dtype) {
     const size_t es = elem_size(dtype);
     return n * (3 * es + 24) + (64u << 20);

@@ -31,10 +31,7 @@
 
 namespace fz {
 
-constexpr int kO1Ctx = 15;               // RleFseEncoder.hpp:344
-constexpr int kO1Sym = 256;              // :347 (255 = escape to the side stream)
-constexpr unsigned kO1Log = 13;          // :345
-constexpr int kO1K = 4;                  // :479
+constexpr int kO1K = 4;                  // RleFseEncoder.hpp:479
 constexpr uint64_t kO1Seg = 8ull << 20;  // :577
 constexpr uint32_t kFblk = 65536;        // :75
 
@@ -2212,12 +2209,10 @@ struct O1Split {
     uint32_t cls;         // graph size class
 };
 
-constexpr int kSplitRounds = 3;
 // Edges: target (16 bits: node, numbered through all rounds of its graph wave, or kSplitExit | exit),
 // symbols decoded << 16.
 constexpr uint32_t kSplitExit = 0xF000u, kSplitFail = 0xFFFFFFFFu;
 constexpr uint32_t kSplitMaxSym = 0xFFFEu;
-constexpr uint32_t kSplitMaxCap = 128;  // candidates a part holds at most
 constexpr int kSplitMaxParts = 16;   // parts a graph wave takes at most
 constexpr int kSplitMaxOrig = 256;   // origins it takes at most (parts * cap)
 
@@ -4303,17 +4298,14 @@ static void fse_dec_multi(const std::vector<FseDecItem>& items, int* err, DevAre
 
 // Order-1 tANS chains are given as 7 values each: stream offset, bytes, out lo, out hi, escape offset,
 // table set, escape count.
-// Chains of fewer symbols, or of fewer bits a symbol (where decoders started at guessed states hardly
-// ever meet), are decoded from their start.
-constexpr uint64_t kSplitMinSymbols = 8192;
-constexpr double kSplitMinBits = 2.5;
 // Sequential chains of fewer take several steps a lookup (kSerialRun).
 constexpr double kSerialRunBits = 2.0;
 // In the batched decompress, chains of at most this many are handed to the batch, whose split chains run
 // in one set of launches, and whose other chains in one launch beside them: a field's own launches
 // leave most of the chip idle (192 chunks of 540,000 codes at bounds 1e-2 to 1e-4: 64 ms with all of
-// their chains decoded from their starts, 47 ms like this). The split chains of a batch share at most
-// kBatchSplitBytes of sets and graphs; chains past that are decoded from their start.
+// their chains decoded from their starts, 47 ms like this). So are longer ones that their item's
+// region has no room for. The split chains of a batch share at most kBatchSplitBytes of sets and
+// graphs; chains past that are decoded from their start.
 constexpr uint64_t kDeferSymbols = 1ull << 19;
 constexpr double kBatchSplitBytes = 4.0 * (1ull << 30);
 // Alone, a chain of few bits a symbol runs 64 decoders 2,048 symbols ahead of every part in what the chip
@@ -4396,144 +4388,96 @@ static SerialMap serial_map(const double pi[kO1Ctx], double escapes, double bits
     return m;
 }
 
-// How a chain is decoded: from its start by one workgroup (k_o1d_serial), or split into parts. The
-// split decoder follows, for every part, all states that its entry may be; what that costs is the
-// number of such states that live side by side, estimated from the chain's tables:
-//   mu   rate per symbol at which two decoders meet. It falls with the bits a symbol takes (a step
-//        replaces that many bits of the 13-bit state): 5e-4 at 7.4 bits, 3e-4 at 6.2, 5e-5 at 3.2
-//        (measured on k^-3 fields), so 8e-6 * 2^(0.85 bits).
-//   pe   escapes per symbol by the tables, which is what a decoder off the true path meets. Every escape doubles the paths and meeting halves them: about 1 + 2 pe / mu live ones
-//        (counted on the CPU: 24 at 7.8 bits and an escape in 175 symbols, 130 at 7.4 and one in 36,
-//        over 900 at 3.0 and one in 250).
-// Split chains, by size class of the graph kernel; kSplitNone: from the start.
-enum { kSplitFew = 0, kSplitSome = 1, kSplitMany = 2, kSplitNone = 3 };
-constexpr int kSplitNodes[3] = {128, 512, 1024};
-struct SplitPlan {
-    int cls = kSplitNone;
-    double nodes = 0;  // nodes a symbol
-    uint32_t lgk = 0, warm = 0, cap = 0, parts = 0, sub = 0;  // warm, sub in symbols
+// A chain as its call finds it, and how it is to be decoded.
+struct O1Chain {
+    O1Split k;
+    SplitPlan plan;
+    uint64_t seg;
+    bool batched;  // handed to the batch
 };
-static SplitPlan split_plan(uint64_t m, uint64_t novf, double bits, const double pi[kO1Ctx], const uint8_t* norm,
-                            bool keep_short) {
-    SplitPlan s;
-    // a chain of few symbols is done sooner from its start than the split decoder's launches take
-    if (m < (keep_short ? 4096u : kSplitMinSymbols) || bits < kSplitMinBits) return s;
-    double pe = 0;
-    for (int a = 0; a < kO1Ctx; a++) {
-        int16_t v;
-        memcpy(&v, norm + 2 * ((size_t)a * kO1Sym + 255), 2);
-        pe += pi[a] * (v < 0 ? 1.0 : (double)v) / (double)(1u << kO1Log);
-    }
-    // the first chain of a segment holds most of its escapes (the coarse levels)
-    pe = std::max(pe, 0.25 * (double)novf / (double)m);
-    const double mu = 8e-6 * std::exp2(0.85 * bits);
-    const double live = 1.0 + 2.0 * pe / mu;
-    if (novf * 8 > m || live > (bits >= 6.0 ? 200.0 : bits >= 4.5 ? 60.0 : 10.0)) return s;
-    s.nodes = 1.5 * pe * live;
-    if (pe < 1.0 / 1024 && live <= 10.0) {
-        // Few states: long parts, and guessed decoders enough, early enough, for the true entry to be
-        // among their states in most parts before the first round (CPU counts on k^-3 fields, parts
-        // that the walk decodes exactly after three rounds: 6.2 bits, 8 decoders 512 symbols ahead 1 of
-        // 2000; 3.2 bits, 64 decoders 2048 ahead 2 of 750, 32 decoders 7).
-        s.cls = kSplitFew;
-        s.sub = m >= (1u << 20) ? (bits >= 5.5 ? 1024 : 2048) : m >= (1u << 18) ? 1024 : m >= (1u << 16) ? 512 : 256;
-        s.warm = bits >= 5.5 ? 512 : 2048;
-        s.lgk = bits >= 6.0 ? 3 : bits >= 5.5 ? 4 : 6;
-        s.cap = s.lgk <= 4 ? 16 : 32;
-        s.parts = s.lgk <= 4 ? 16 : 8;
-        while (s.parts > 1 && s.parts * s.nodes * s.sub > kSplitNodes[kSplitFew] / 3) s.parts /= 2;
-    } else {
-        // Escapes saturate the sets in a round or two whatever they start from: short parts and a short
-        // warm-up (same counts: none of 500 parts left at 16 decoders 256 symbols ahead).
-        s.sub = 256;
-        s.warm = 256;
-        s.lgk = 4;
-        const double nodes = s.nodes * s.sub;
-        // the estimate is about twice what is counted; past its table a graph is lost to the walk
-        if (nodes > 1.5 * kSplitNodes[kSplitMany]) return s;
-        s.cls = nodes <= kSplitNodes[kSplitSome] / 4 ? kSplitSome : kSplitMany;
-        s.cap = s.cls == kSplitSome ? 64 : kSplitMaxCap;
-        s.parts = s.cls == kSplitMany ? 1 : nodes <= kSplitNodes[kSplitSome] / 16 ? 4 : nodes <= kSplitNodes[kSplitSome] / 8 ? 2 : 1;
-    }
-    return s;
-}
 
 // The split chains of a call or of a batch, in launch order, and what their kernels left.
 struct SplitRun {
     std::vector<O1Split> sc;
-    std::vector<int> order;
+    std::vector<uint64_t> seg;
     O1SplitWs W{};
     unsigned int* stats = nullptr;
-    uint64_t nparts = 0;
+    uint64_t nlanes = 0, stream_bytes = 0, ncodes = 0;
+    int cls_first[4];
+    uint64_t cls_waves[3];
+    size_t bytes = 0;  // device memory
+    O1Split* dch = nullptr;
 };
 // 32-bit words of its statistics for nc chains: six counts, one a chain, then the pool's count.
 static int split_stats(int nc) { return (6 + nc + 1) / 2 * 2 + 2; }
-// Device bytes that split_launch takes for a chain, but for its few words a part.
-static double split_bytes(const O1Split& k, const SplitPlan& sp) {
-    return 12.0 * k.nsub * k.cap + 8.0 * (4.0 * sp.nodes * (double)k.m + 16.0 * k.nsub / k.parts);
-}
-static void split_launch(const std::vector<O1Split>& hc, const std::vector<SplitPlan>& plans, SplitRun& R, DevArena& ws,
-                         hipStream_t st) {
-    const int nc = (int)hc.size();
-    uint64_t stream_bytes = 0, ncodes = 0;
-    for (const O1Split& k : hc) {
-        stream_bytes += (uint64_t)k.len;
-        ncodes += k.m;
-    }
-    // chains of one size class side by side, for one launch each
-    std::vector<int>& order = R.order;
-    order.resize(nc);
-    for (int q = 0; q < nc; q++) order[q] = q;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return hc[x].cls < hc[y].cls; });
-    std::vector<O1Split>& sc = R.sc;
-    sc.resize(nc);
-    uint64_t &nparts = R.nparts = 0, ncand = 0, nlanes = 0, nwaves = 0;
+
+// Lays the chains out, those of one size class side by side for one launch each; at: the memory (null: only
+// its size is wanted, R.bytes).
+static void split_layout(const std::vector<O1Chain>& chains, SplitRun& R, uint8_t* at) {
+    R = SplitRun{};
+    std::vector<const O1Chain*> order;
+    for (const O1Chain& c : chains) order.push_back(&c);
+    std::stable_sort(order.begin(), order.end(), [](const O1Chain* x, const O1Chain* y) { return x->k.cls < y->k.cls; });
+    uint64_t nparts = 0, ncand = 0, nwaves = 0;
     double pool = 0;
-    int cls_first[4] = {0, 0, 0, 0};
-    uint64_t cls_waves[3] = {0, 0, 0};
-    for (int i = 0; i < nc; i++) {
-        O1Split& k = sc[i] = hc[order[i]];
-        const SplitPlan& sp = plans[order[i]];
-        const uint64_t nw = (k.nsub - 1 + k.parts - 1) / k.parts;
+    std::fill(R.cls_first, R.cls_first + 4, 0);
+    std::fill(R.cls_waves, R.cls_waves + 3, 0);
+    for (const O1Chain* c : order) {
+        R.sc.push_back(c->k);
+        R.seg.push_back(c->seg);
+        O1Split& k = R.sc.back();
+        const uint64_t nw = split_waves(c->plan, k.nsub);
         k.tfirst = nparts;
         k.cfirst = ncand;
-        k.wfirst = nlanes;
+        k.wfirst = R.nlanes;
         k.gfirst = nwaves;
         nparts += k.nsub;
         ncand += (uint64_t)k.nsub * k.cap;
-        nlanes += (((uint64_t)k.nsub << k.lgk) + 63) & ~63ull;
+        R.nlanes += (((uint64_t)k.nsub << k.lgk) + 63) & ~63ull;
         nwaves += nw;
-        cls_waves[k.cls] += nw;
-        for (uint32_t z = k.cls + 1; z < 4; z++) cls_first[z] = i + 1;
-        // twice what the estimate gives for two rounds, and some for each wave
-        pool += 4.0 * sp.nodes * (double)k.m + 16.0 * (double)nw;
+        R.cls_waves[k.cls] += nw;
+        for (uint32_t z = k.cls + 1; z < 4; z++) R.cls_first[z] = (int)R.sc.size();
+        pool += split_nodes(c->plan, k.m, k.nsub);
+        R.stream_bytes += (uint64_t)k.len;
+        R.ncodes += k.m;
     }
-    O1Split* dch = ws.take<O1Split>(nc);
+    const int nc = (int)R.sc.size();
+    auto take = [&](auto*& p, uint64_t n) {
+        p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(at + R.bytes);
+        R.bytes += (n * sizeof(*p) + 255) & ~(size_t)255;
+    };
     O1SplitWs& W = R.W;
-    W.cand = ws.take<uint32_t>(ncand);
-    W.edge = ws.take<uint32_t>(ncand);
-    W.exits = ws.take<uint32_t>(ncand);
-    W.hdr = ws.take<uint16_t>(nparts * kSplitRounds);
-    W.n0 = ws.take<uint8_t>(nparts);
-    W.wave = ws.take<uint2>((nwaves + 1) * kSplitRounds);
+    W.nparts = nparts;
     W.pool_cap = std::min<uint64_t>((uint64_t)pool + 4096, kPoolMax);
     // FALCONS_O1_POOL_NODES: a test switch; the parts whose nodes find no room are decoded by the walk
     if (const char* few = getenv("FALCONS_O1_POOL_NODES")) W.pool_cap = std::min<uint64_t>(W.pool_cap, std::strtoull(few, nullptr, 10));
-    W.pool = ws.take<uint2>(W.pool_cap);
-    W.nparts = nparts;
-    W.res_state = ws.take<uint32_t>(nparts);
-    W.res_e = ws.take<uint64_t>(nparts);
-    W.res_off = ws.take<uint64_t>(nparts);
+    take(R.dch, nc);
+    take(W.cand, ncand);
+    take(W.edge, ncand);
+    take(W.exits, ncand);
+    take(W.hdr, nparts * kSplitRounds);
+    take(W.n0, nparts);
+    take(W.wave, (nwaves + 1) * kSplitRounds);
+    take(W.pool, W.pool_cap);
+    take(W.res_state, nparts);
+    take(W.res_e, nparts);
+    take(W.res_off, nparts);
     const int nstats = split_stats(nc);
-    unsigned int* stats = R.stats = ws.take<unsigned int>(nstats);
-    W.pool_used = reinterpret_cast<NodeCount*>(stats + nstats - 2);
-    h2d(dch, sc.data(), sc.size(), st);
-    FZ_HIP(hipMemsetAsync(stats, 0, nstats * sizeof(unsigned int), st));
-    FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(nlanes)), dim3(256), 0, st, dch, nc, nlanes, W);
+    take(R.stats, nstats);
+    W.pool_used = reinterpret_cast<NodeCount*>(R.stats + nstats - 2);
+}
+static void split_launch(const SplitRun& R, hipStream_t st) {
+    const int nc = (int)R.sc.size(), nstats = split_stats(nc);
+    const O1SplitWs& W = R.W;
+    const int* cls_first = R.cls_first;
+    O1Split* dch = R.dch;
+    h2d(dch, R.sc.data(), R.sc.size(), st);
+    FZ_HIP(hipMemsetAsync(R.stats, 0, nstats * sizeof(unsigned int), st));
+    FZ_LAUNCH("o1_split_warm", 0, k_o1s_warm, dim3(nblk(R.nlanes)), dim3(256), 0, st, dch, nc, R.nlanes, W);
     for (int round = 0; round < kSplitRounds; round++)
         for (int z = 2; z >= 0; z--) {
             const int c0 = cls_first[z], cn = cls_first[z + 1] - c0;
-            const uint32_t nw = (uint32_t)cls_waves[z];
+            const uint32_t nw = (uint32_t)R.cls_waves[z];
             if (!cn || !nw) continue;
             if (z == kSplitFew)
                 FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[0]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
@@ -4542,8 +4486,8 @@ static void split_launch(const std::vector<O1Split>& hc, const std::vector<Split
             else
                 FZ_LAUNCH("o1_split_graph", 0, k_o1s_graph<kSplitNodes[2]>, dim3(nw), dim3(64), 0, st, dch + c0, cn, nw, round, W);
         }
-    FZ_LAUNCH("o1_split_walk", 0, k_o1s_walk, dim3(nc), dim3(kWalkThreads), 0, st, dch, nc, W, stats);
-    FZ_LAUNCH("o1_split_out", stream_bytes + ncodes * 2, k_o1s_out, dim3(nblk(nparts)), dim3(256), 0, st, dch, nc, W);
+    FZ_LAUNCH("o1_split_walk", 0, k_o1s_walk, dim3(nc), dim3(kWalkThreads), 0, st, dch, nc, W, R.stats);
+    FZ_LAUNCH("o1_split_out", R.stream_bytes + R.ncodes * 2, k_o1s_out, dim3(nblk(W.nparts)), dim3(256), 0, st, dch, nc, W);
     FZ_HIP(hipGetLastError());
 }
 
@@ -4553,8 +4497,7 @@ struct DenseBatch {
     std::vector<SerialJob> jobs;
     std::vector<SerialTables> tabs;
     uint64_t bytes = 0, codes = 0;
-    std::vector<O1Split> split;
-    std::vector<SplitPlan> plans;
+    std::vector<O1Chain> split;
     double split_bytes = 0;
     SplitRun run;
 };
@@ -4570,7 +4513,6 @@ void dense_batch_clear(DenseBatch* b) {
     b->tabs.clear();
     b->bytes = b->codes = 0;
     b->split.clear();
-    b->plans.clear();
     b->split_bytes = 0;
 }
 // Re-encodes the tables and decodes the chains of the lists on st; djobs and dtabs have room for them.
@@ -4604,7 +4546,13 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStrea
         launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, beside ? aux.stream : st);
         if (beside) FZ_HIP(hipEventRecord(aux.join, aux.stream));
     }
-    if (!b->split.empty()) split_launch(b->split, b->plans, b->run, ws, st);
+    if (!b->split.empty()) {
+        split_layout(b->split, b->run, nullptr);
+        uint8_t* mem = static_cast<uint8_t*>(ws.side(b->run.bytes, 0, (size_t)kBatchSplitBytes));
+        if (!mem) throw GpuError("no device memory for the split chains of the batch");
+        split_layout(b->split, b->run, mem);
+        split_launch(b->run, st);
+    }
     if (beside) FZ_HIP(hipStreamWaitEvent(st, aux.join, 0));
 }
 
@@ -4622,12 +4570,6 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
                                int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer,
                                O1Lists& lists) {
     const int nch = (int)(chains.size() / 7);
-    std::vector<O1Split> hc;
-    std::vector<SerialJob>& hd = lists.serial;
-    std::vector<uint64_t> hd_seg;
-    std::vector<SplitPlan> plans;
-    std::vector<uint64_t> seg_of;
-    uint64_t dense_bytes = 0, dense_codes = 0;
     // FALCONS_O1_SEQUENTIAL=1 decodes every chain from its start; FALCONS_O1_PARALLEL_SHORT=1 splits
     // short chains too (the tests of either decoder on small fields)
     const char* seq_env = getenv("FALCONS_O1_SEQUENTIAL");
@@ -4635,11 +4577,13 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     const char* par_env = getenv("FALCONS_O1_PARALLEL_SHORT");
     const bool keep_short = par_env && atoi(par_env) != 0;
     double pi[kO1Ctx];
-    uint64_t pi_seg = ~0ull;
+    uint64_t pi_seg = ~0ull, ncodes = 0;
+    std::vector<O1Chain> all;
     for (int q = 0; q < nch; q++) {
         const uint64_t* c = &chains[7 * q];
         const uint64_t m = c[3] - c[2];
         if (m == 0) continue;
+        ncodes += m;
         // initial state: the tableLog bits under the end mark (FSE_initDState)
         const uint8_t* b = host + c[0];
         const int64_t top = (int64_t)(c[1] - 1) * 8 + (int64_t)highbit32(b[c[1] - 1]);
@@ -4654,27 +4598,29 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             context_shares(host, nf_off[c[5]], pi);
             pi_seg = c[5];
         }
-        SplitPlan sp;
+        O1Chain x{};
+        x.seg = c[5];
+        x.batched = defer && m <= kDeferSymbols;
+        SplitPlan& sp = x.plan;
         if (!all_seq) sp = split_plan(m, c[6], bits, pi, host + nf_off[c[5]], keep_short);
-        const bool batched = defer && m <= kDeferSymbols;
-        if (batched && (sp.warm << sp.lgk) > kBatchWarm) {
+        if (x.batched && (sp.warm << sp.lgk) > kBatchWarm) {
             sp.lgk = 5;
             sp.warm = 1024;
         }
+        O1Split& k = x.k;
+        k.cb = dev + c[0];
+        k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
+        k.ov = ovf + c[4];
+        k.out = out + c[2];
+        k.err = err;
+        k.m = m;
+        k.novf = c[6];
+        k.len = (int64_t)c[1];
+        k.pos0 = pos0;
+        k.x0 = x0;
         if (sp.cls != kSplitNone) {
-            O1Split k{};
-            k.cb = dev + c[0];
-            k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
-            k.ov = ovf + c[4];
-            k.out = out + c[2];
-            k.err = err;
-            k.m = m;
-            k.novf = c[6];
-            k.len = (int64_t)c[1];
-            k.pos0 = pos0;
-            k.x0 = x0;
-            k.sub_bits = (uint32_t)std::max(2048.0, bits * sp.sub);
-            k.nsub = (uint32_t)std::max<int64_t>(1, (pos0 + k.sub_bits - 1) / k.sub_bits);
+            k.sub_bits = split_sub_bits(sp, bits);
+            k.nsub = (uint32_t)split_parts(pos0, k.sub_bits);
             k.warm_bits = (uint32_t)(bits * sp.warm) + 64;
             k.warm_steps = 2 * sp.warm;
             k.lgk = sp.lgk;
@@ -4683,36 +4629,71 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             k.max_sym = 8 * sp.sub;
             k.hot0 = hot_window(pi);
             k.cls = (uint32_t)sp.cls;
-            if (batched) {
-                const double need = split_bytes(k, sp);
-                std::lock_guard<std::mutex> g(defer->mu);
-                if (defer->split_bytes + need <= kBatchSplitBytes) {
-                    defer->split.push_back(k);
-                    defer->plans.push_back(sp);
-                    defer->split_bytes += need;
-                    continue;
-                }
+        }
+        all.push_back(x);
+    }
+    // The split chains of this call, as many as its memory may hold; the others are decoded from their start. In a
+    // batch, where the region of an item has no room for them, all of the item's go to the batch instead, which has
+    // memory of its own.
+    SplitRun& R = lists.split;
+    {
+        std::vector<SplitCand> cand;
+        uint64_t serial = 0;
+        double need = 0;
+        for (O1Chain& x : all) {
+            if (x.plan.cls == kSplitNone) serial = std::max(serial, x.k.m);
+            else if (!x.batched) cand.push_back(SplitCand{&x.plan, x.k.m, x.k.nsub});
+        }
+        // what the call takes after this: the re-encoded tables of sequential chains, the scratch of a scan
+        const size_t after = nf_off.size() * (sizeof(uint32_t) * kO1Ctx << kO1Log) + (1u << 20) + ncodes / 64;
+        const double head = 65536.0 + 256.0 * (double)cand.size();  // rounding, lists
+        const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - head;
+        for (const SplitCand& x : cand) need += x.bytes();
+        if (!defer) split_choose(cand, room, serial);
+        std::vector<O1Chain> own;
+        for (O1Chain& x : all) {
+            if (defer && need > room) x.batched = true;
+            if (x.plan.cls != kSplitNone && !x.batched) own.push_back(x);
+        }
+        if (!own.empty()) {
+            split_layout(own, R, nullptr);
+            if (uint8_t* mem = static_cast<uint8_t*>(ws.side(R.bytes, after, split_limit(ncodes)))) {
+                split_layout(own, R, mem);
             } else {
-                hc.push_back(k);
-                plans.push_back(sp);
-                seg_of.push_back(c[5]);
+                R = SplitRun{};
+                for (O1Chain& x : all)
+                    if (!x.batched) x.plan.cls = kSplitNone;
+            }
+        }
+    }
+    std::vector<SerialJob>& hd = lists.serial;
+    std::vector<uint64_t> hd_seg;
+    uint64_t dense_bytes = 0, dense_codes = 0;
+    for (const O1Chain& x : all) {
+        if (x.plan.cls != kSplitNone) {
+            if (!x.batched) continue;
+            const double need = split_bytes(x.plan, x.k.m, x.k.nsub);
+            std::lock_guard<std::mutex> g(defer->mu);
+            if (defer->split_bytes + need <= kBatchSplitBytes) {
+                defer->split.push_back(x);
+                defer->split_bytes += need;
                 continue;
             }
         }
         SerialJob k{};
-        k.cb = dev + c[0];
-        k.dt = reinterpret_cast<const uint32_t*>(dt + c[5] * kO1Ctx * (1u << kO1Log));
-        k.ov = ovf + c[4];
-        k.out = out + c[2];
+        k.cb = x.k.cb;
+        k.dt = x.k.dt;
+        k.ov = x.k.ov;
+        k.out = x.k.out;
         k.err = err;
-        k.m = m;
-        k.novf = c[6];
-        k.pos0 = pos0;
-        k.x0 = x0;
+        k.m = x.k.m;
+        k.novf = x.k.novf;
+        k.pos0 = x.k.pos0;
+        k.x0 = x.k.x0;
         hd.push_back(k);
-        hd_seg.push_back(c[5]);
-        dense_bytes += c[1];
-        dense_codes += m;
+        hd_seg.push_back(x.seg);
+        dense_bytes += (uint64_t)x.k.len;
+        dense_codes += x.k.m;
     }
     // sequential chains run beside the rest, on the auxiliary stream when there is one
     hipStream_t dst = aux.stream ? aux.stream : st;
@@ -4770,12 +4751,10 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             }
         }
     } join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
-    if (hc.empty()) return;
-    SplitRun& R = lists.split;
-    split_launch(hc, plans, R, ws, st);
-    const int nc = (int)hc.size();
+    if (R.sc.empty()) return;
+    split_launch(R, st);
     const std::vector<O1Split>& sc = R.sc;
-    const std::vector<int>& order = R.order;
+    const int nc = (int)sc.size();
     if (stats_on) {
         std::vector<unsigned int> hsv(split_stats(nc));
         d2h(hsv.data(), R.stats, hsv.size(), st);
@@ -4786,7 +4765,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
                         "first LDS context of the walk):");
         for (int q = 0; q < nc; q++)
             fprintf(stderr, " %d:%u/%u/esc%llu/b%.2f/s%llu/h%u", q, hs[6 + q], sc[q].nsub, (unsigned long long)sc[q].novf,
-                    (double)sc[q].pos0 / (double)std::max<uint64_t>(1, sc[q].m), (unsigned long long)seg_of[order[q]],
+                    (double)sc[q].pos0 / (double)std::max<uint64_t>(1, sc[q].m), (unsigned long long)R.seg[q],
                     sc[q].hot0);
         fprintf(stderr, "\n");
         fprintf(stderr, "[o1 decode] %zu chains decoded from their start:", hd.size());
@@ -4811,7 +4790,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
                         "entries outside the set), %llu nodes of %llu\n",
-                nc, (unsigned long long)R.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap);
+                nc, (unsigned long long)R.W.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap);
     }
 }
 

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -20,6 +21,8 @@ namespace fz {
 //
 // A bound arena (bind()) draws from one region of device memory the caller owns and never
 // allocates: a take() beyond the region throws instead of adding a block.
+//
+// side() gives memory that a call can do without: one region beside the blocks, for one user a call.
 class DevArena {
    public:
     ~DevArena() { release(); }
@@ -32,14 +35,14 @@ class DevArena {
     void reserve(size_t bytes) {
         bytes = (bytes + 255) & ~size_t(255);
         if (bytes <= cap_ || bound_) return;  // a bound arena cannot grow: its takes throw instead
-        if (used_ == 0 && !blocks_.empty() && blocks_[0].cap < bytes) release();  // regrow as one block
+        if (used_ == 0 && !blocks_.empty() && blocks_[0].cap < bytes) drop_blocks();  // regrow as one block
         if (blocks_.empty()) add_block(bytes);
         else add_block(bytes - cap_);
     }
     void reset() {
         cur_ = 0;
         off_ = 0;
-        used_ = 0;
+        used_ = side_used_ = 0;
     }
     template <typename T>
     T* take(size_t count) {
@@ -53,13 +56,44 @@ class DevArena {
         T* p = reinterpret_cast<T*>(static_cast<char*>(blocks_[cur_].p) + off_);
         off_ += bytes;
         used_ += bytes;
-        peak_ = used_ > peak_ ? used_ : peak_;
+        peak_ = std::max(peak_, used_ + side_used_);
         return p;
+    }
+    // The most that side() may give, when `after` bytes of takes are still to come.
+    size_t side_room(size_t after) const {
+        size_t most = side_most_;
+        if (bound_) most = blocks_.empty() || cur_ > 0 || off_ + after > blocks_[0].cap ? 0 : blocks_[0].cap - off_ - after;
+        // FALCONS_SIDE_BYTES: a test switch
+        if (const char* e = getenv("FALCONS_SIDE_BYTES")) most = std::min<size_t>(most, std::strtoull(e, nullptr, 10));
+        return most;
+    }
+    void set_side_most(size_t bytes) { side_most_ = bytes; }
+    // Null where there is no room (side_room) or the device has no such memory. The region is kept for the
+    // next call and regrown for a larger one: to twice the need, 256 MB at least, and `most` at most, as the
+    // hipFree that goes with it waits for the whole device.
+    void* side(size_t bytes, size_t after, size_t most) {
+        bytes = (bytes + 255) & ~size_t(255);
+        const size_t room = side_room(after);
+        if (bytes > room) return nullptr;
+        if (bound_) return take<uint8_t>(bytes);
+        if (bytes > side_.cap) {
+            drop_side();
+            const size_t cap = std::max(bytes, std::min(std::min(room, most), std::max(2 * bytes, size_t(256) << 20)));
+            void* p = nullptr;
+            if (hipMalloc(&p, cap) != hipSuccess) {
+                (void)hipGetLastError();  // it is the caller's to go another way
+                return nullptr;
+            }
+            side_ = Block{p, cap};
+        }
+        side_used_ = bytes;
+        peak_ = std::max(peak_, used_ + side_used_);
+        return side_.p;
     }
     size_t used() const { return used_; }
     // most taken at once since the last clear_peak()
     size_t peak() const { return peak_; }
-    void clear_peak() { peak_ = used_; }
+    void clear_peak() { peak_ = used_ + side_used_; }
     // Gives back everything taken after `mark` (a value of used()); the caller has finished with it
     // in stream order.
     void rewind(size_t mark) {
@@ -75,8 +109,19 @@ class DevArena {
             base += blocks_[k].cap;
         }
     }
-    size_t capacity() const { return cap_; }
+    size_t capacity() const { return cap_ + side_.cap; }
+    size_t side_capacity() const { return side_.cap; }
     void release() {
+        drop_blocks();
+        drop_side();
+    }
+
+   private:
+    struct Block {
+        void* p = nullptr;
+        size_t cap = 0;
+    };
+    void drop_blocks() {
         if (!bound_)
             for (Block& b : blocks_) (void)hipFree(b.p);
         blocks_.clear();
@@ -84,12 +129,11 @@ class DevArena {
         cur_ = 0;
         bound_ = false;
     }
-
-   private:
-    struct Block {
-        void* p;
-        size_t cap;
-    };
+    void drop_side() {
+        if (side_.p) (void)hipFree(side_.p);
+        side_ = Block{};
+        side_used_ = 0;
+    }
     void add_block(size_t bytes) {
         bytes = (bytes + 255) & ~size_t(255);
         if (bound_)
@@ -101,7 +145,9 @@ class DevArena {
         cap_ += bytes;
     }
     std::vector<Block> blocks_;
-    size_t cap_ = 0, used_ = 0, off_ = 0, peak_ = 0, cur_ = 0;
+    Block side_;
+    size_t cap_ = 0, used_ = 0, off_ = 0, peak_ = 0, cur_ = 0, side_used_ = 0;
+    size_t side_most_ = ~size_t(0) / 2;
     bool bound_ = false;
 };
 

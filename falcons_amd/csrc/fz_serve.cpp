@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "fz_ctx.h"
+#include "fz_split.h"
 
 namespace fz {
 
@@ -333,7 +334,7 @@ extern "C" int fz_decompress_batch(fz_ctx* ctx, fz_batch_dec_item* items, int n,
             size_t need = 0;
             for (int i = 0; i < n; i++)
                 need = std::max(need, decompress_workspace_bytes(items[i].conf.num, items[i].dtype, items[i].conf.num,
-                                                                 items[i].pre_len));
+                                                                 items[i].pre_len) + split_limit(items[i].conf.num));
             const int active = active_workers(ws, need, ws.held());
             ws.run(order, [&](fz_ctx* w, int i) {
                 fz_batch_dec_item& it = items[i];
@@ -362,7 +363,9 @@ struct Job {
     fz_request req;
     double t_submit;
     size_t field_bytes;  // device field buffer the request needs
-    size_t ws_bytes;     // workspace the request's call reserves (an upper bound)
+    size_t ws_bytes;     // workspace the request's call is expected to take
+    size_t side_bytes;   // the most that its split order-1 decoder may take beside
+    size_t bytes() const { return field_bytes + ws_bytes + side_bytes; }
 };
 
 struct Slot {
@@ -401,7 +404,8 @@ namespace {
 
 // Device bytes slot s holds after growing for job j.
 size_t held_after(const Slot& s, const Job& j) {
-    return std::max(s.ctx->arena.capacity(), j.ws_bytes) + std::max(s.field_cap, j.field_bytes);
+    const size_t side = s.ctx->arena.side_capacity(), blocks = s.ctx->arena.capacity() - side;
+    return std::max(blocks, j.ws_bytes) + std::max(side, j.side_bytes) + std::max(s.field_cap, j.field_bytes);
 }
 
 size_t held_total(const fz_server* S) {
@@ -420,7 +424,7 @@ bool admit(fz_server* S, int k, const Job& j) {
     size_t busy = 0;
     for (const Slot& o : S->slots)
         if (o.busy) busy += o.held();
-    if (busy + j.ws_bytes + j.field_bytes > S->budget) return false;
+    if (busy + j.bytes() > S->budget) return false;
     me.trim();
     if (others + held_after(me, j) <= S->budget) return true;
     for (size_t i = 0; i < S->slots.size(); i++) {
@@ -452,6 +456,7 @@ void run_job(fz_server* S, Slot& s, const Job& j, fz_result& r) {
                                       &mutated);
     } else {
         fz_config c;
+        ctx->arena.set_side_most(j.side_bytes);
         void* d = s.field;
         decompress_to_device(ctx, static_cast<const uint8_t*>(q.src), q.src_len, q.dtype, &d,
                              s.field_cap / es_of(q.dtype), &c, &o);
@@ -553,7 +558,7 @@ extern "C" int fz_server_submit(fz_server* S, const fz_request* r) {
     if (!S || !r) return FZ_ERR_INVALID_ARGUMENT;
     if (r->op != 0 && r->op != 1) return FZ_ERR_INVALID_ARGUMENT;
     if (r->dtype < FZ_FLOAT || r->dtype > FZ_INT64) return FZ_ERR_UNSUPPORTED;
-    Job j;
+    Job j{};
     j.req = *r;
     j.t_submit = now_ms();
     const size_t es = es_of(r->dtype);
@@ -566,10 +571,13 @@ extern "C" int fz_server_submit(fz_server* S, const fz_request* r) {
             return FZ_ERR_INVALID_ARGUMENT;
         j.field_bytes = c.num * es;
         j.ws_bytes = decompress_workspace_bytes(c.num, r->dtype, c.num, fz_prezstd_bound(&c, r->dtype));
+        j.side_bytes = split_limit(c.num);
     }
     std::lock_guard<std::mutex> g(S->m);
-    // a request larger than the whole budget can never run
+    // a request larger than the whole budget can never run; one that only fits without the split decoder's
+    // memory has its chains decoded from their start
     if (j.field_bytes + j.ws_bytes > S->budget) return FZ_ERR_INVALID_ARGUMENT;
+    j.side_bytes = std::min(j.side_bytes, S->budget - j.field_bytes - j.ws_bytes);
     S->pending.push_back(j);
     S->st.submitted++;
     S->st.max_pending = std::max<uint64_t>(S->st.max_pending, S->pending.size());
