@@ -4305,7 +4305,7 @@ constexpr double kSerialRunBits = 2.0;
 // leave most of the chip idle (192 chunks of 540,000 codes at bounds 1e-2 to 1e-4: 64 ms with all of
 // their chains decoded from their starts, 47 ms like this). So are longer ones that their item's
 // region has no room for. The split chains of a batch share at most kBatchSplitBytes of sets and
-// graphs; chains past that are decoded from their start.
+// graphs, and a quarter of the device memory that is free; chains past that are decoded from their start.
 constexpr uint64_t kDeferSymbols = 1ull << 19;
 constexpr double kBatchSplitBytes = 4.0 * (1ull << 30);
 // Alone, a chain of few bits a symbol runs 64 decoders 2,048 symbols ahead of every part in what the chip
@@ -4498,7 +4498,7 @@ struct DenseBatch {
     std::vector<SerialTables> tabs;
     uint64_t bytes = 0, codes = 0;
     std::vector<O1Chain> split;
-    double split_bytes = 0;
+    double split_bytes = 0, split_limit = 0;
     SplitRun run;
 };
 DenseBatch* dense_batch_create() { return new DenseBatch; }
@@ -4506,6 +4506,12 @@ void dense_batch_destroy(DenseBatch* b) { delete b; }
 size_t dense_batch_size(DenseBatch* b) {
     std::lock_guard<std::mutex> g(b->mu);
     return b->jobs.size() + b->split.size();
+}
+void dense_batch_limit(DenseBatch* b, size_t free_bytes) {
+    std::lock_guard<std::mutex> g(b->mu);
+    b->split_limit = std::min(kBatchSplitBytes, 0.25 * (double)free_bytes);
+    // FALCONS_BATCH_SPLIT_BYTES: a test switch
+    if (const char* most = getenv("FALCONS_BATCH_SPLIT_BYTES")) b->split_limit = std::min(b->split_limit, atof(most));
 }
 void dense_batch_clear(DenseBatch* b) {
     std::lock_guard<std::mutex> g(b->mu);
@@ -4523,19 +4529,38 @@ static void launch_serial(std::vector<SerialJob>& jobs, const std::vector<Serial
               djobs);
     FZ_HIP(hipGetLastError());
 }
+// A stream waits for what was queued on the second one, however the block ends.
+struct AuxJoin {
+    const AuxStream& a;
+    hipStream_t st;
+    bool on;
+    ~AuxJoin() {
+        if (!on) return;
+        (void)hipEventRecord(a.join, a.stream);
+        (void)hipStreamWaitEvent(st, a.join, 0);
+    }
+};
 void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStream& aux) {
     std::lock_guard<std::mutex> g(b->mu);
     const size_t n = b->jobs.size();
     if (n > 0x7fffffffu) throw std::length_error("too many sequential chains for one launch");
     if (b->tabs.size() > 65535u) throw std::length_error("too many sequential segments for one launch");
+    // all device memory before the first launch: without it nothing of the batch is under way
+    uint8_t* mem = nullptr;
+    if (!b->split.empty()) {
+        split_layout(b->split, b->run, nullptr);
+        mem = static_cast<uint8_t*>(ws.side(b->run.bytes, 0, (size_t)kBatchSplitBytes));
+        if (!mem) throw GpuError("no device memory for the split chains of the batch");
+        split_layout(b->split, b->run, mem);
+    }
+    SerialJob* dj = n ? ws.take<SerialJob>(n) : nullptr;
+    SerialTables* dtab = n ? ws.take<SerialTables>(b->tabs.size()) : nullptr;
     // the two decoders beside each other (neither needs what the other writes); the sequential one, which
     // takes as long as its longest chain, is launched first
-    const bool beside = n && !b->split.empty() && aux.stream;
+    const bool beside = n && mem && aux.stream;
     if (n) {
         // longest chains first, so that the last workgroups to start are short ones
         std::stable_sort(b->jobs.begin(), b->jobs.end(), [](const SerialJob& x, const SerialJob& y) { return x.m > y.m; });
-        SerialJob* dj = ws.take<SerialJob>(n);
-        SerialTables* dtab = ws.take<SerialTables>(b->tabs.size());
         // the lists stay in b until dense_batch_clear, after the launches have finished
         h2d(dj, b->jobs.data(), n, st);
         h2d(dtab, b->tabs.data(), b->tabs.size(), st);
@@ -4543,17 +4568,10 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStrea
             FZ_HIP(hipEventRecord(aux.fork, st));
             FZ_HIP(hipStreamWaitEvent(aux.stream, aux.fork, 0));
         }
-        launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, beside ? aux.stream : st);
-        if (beside) FZ_HIP(hipEventRecord(aux.join, aux.stream));
     }
-    if (!b->split.empty()) {
-        split_layout(b->split, b->run, nullptr);
-        uint8_t* mem = static_cast<uint8_t*>(ws.side(b->run.bytes, 0, (size_t)kBatchSplitBytes));
-        if (!mem) throw GpuError("no device memory for the split chains of the batch");
-        split_layout(b->split, b->run, mem);
-        split_launch(b->run, st);
-    }
-    if (beside) FZ_HIP(hipStreamWaitEvent(st, aux.join, 0));
+    AuxJoin join{aux, st, beside};
+    if (n) launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, beside ? aux.stream : st);
+    if (mem) split_launch(b->run, st);
 }
 
 // The lists of one call's chains. Copies on the call's stream read them: they stay until it has been waited for.
@@ -4674,7 +4692,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             if (!x.batched) continue;
             const double need = split_bytes(x.plan, x.k.m, x.k.nsub);
             std::lock_guard<std::mutex> g(defer->mu);
-            if (defer->split_bytes + need <= kBatchSplitBytes) {
+            if (defer->split_bytes + need <= defer->split_limit) {
                 defer->split.push_back(x);
                 defer->split_bytes += need;
                 continue;
@@ -4740,17 +4758,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         launch_serial(hd, tabs, dj, dtab, dense_bytes, dense_codes, dst);
     }
-    struct Join {  // the caller's stream waits for the sequential chains however this function exits
-        const AuxStream& a;
-        hipStream_t st;
-        bool on;
-        ~Join() {
-            if (on) {
-                (void)hipEventRecord(a.join, a.stream);
-                (void)hipStreamWaitEvent(st, a.join, 0);
-            }
-        }
-    } join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
+    AuxJoin join{aux, st, !hd.empty() && aux.stream != nullptr && !defer};
     if (R.sc.empty()) return;
     split_launch(R, st);
     const std::vector<O1Split>& sc = R.sc;

@@ -216,6 +216,9 @@ struct DenseBatch;
 DenseBatch* dense_batch_create();
 void dense_batch_destroy(DenseBatch* b);
 size_t dense_batch_size(DenseBatch* b);
+// Before the calls hand over chains: the device memory that is free, of which split chains get a part.
+void dense_batch_limit(DenseBatch* b, size_t free_bytes);
+// Throws, with nothing launched, where the memory for the chains cannot be had.
 void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStream& aux);
 void dense_batch_clear(DenseBatch* b);  // after dense_batch_run's launches have finished
 struct EntropyCall;

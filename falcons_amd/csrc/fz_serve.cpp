@@ -247,6 +247,9 @@ void decompress_grouped(fz_ctx* ctx, WorkerSet& wset, fz_batch_dec_item* items, 
             FZ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             R.ev.push_back(e);
         }
+        size_t left_b = 0;
+        FZ_HIP(hipMemGetInfo(&left_b, &total_b));
+        dense_batch_limit(R.batch, left_b + ctx->arena.side_capacity());
         std::vector<std::unique_ptr<DevArena>> ar(g);
         std::vector<std::unique_ptr<DecCall, void (*)(DecCall*)>> calls;
         std::vector<char> ok(g, 0), rec(g, 0);
@@ -260,12 +263,19 @@ void decompress_grouped(fz_ctx* ctx, WorkerSet& wset, fz_batch_dec_item* items, 
         std::vector<int> idx(g);
         std::iota(idx.begin(), idx.end(), 0);
         // a shared launch runs after every item's previous part: the items' events, recorded also
-        // after a failure, since work an item handed over reads what its stream has queued
+        // after a failure, since work an item handed over reads what its stream has queued. Where it fails
+        // (no device memory for it), every item of the group goes through the plain call.
         auto shared = [&](auto&& launch) {
-            for (size_t j = 0; j < g; j++)
-                if (rec[j]) FZ_HIP(hipStreamWaitEvent(cst, R.ev[j], 0));
-            launch();
-            FZ_HIP(hipEventRecord(R.done, cst));
+            try {
+                for (size_t j = 0; j < g; j++)
+                    if (rec[j]) FZ_HIP(hipStreamWaitEvent(cst, R.ev[j], 0));
+                launch();
+                FZ_HIP(hipEventRecord(R.done, cst));
+            } catch (...) {
+                (void)hipDeviceSynchronize();  // what reads the items' regions
+                (void)hipGetLastError();       // of this thread: the next launch must not report it
+                std::fill(ok.begin(), ok.end(), 0);
+            }
         };
         wset.run(idx, [&](fz_ctx* w, int j) {
             fz_batch_dec_item& it = items[order[k0 + j]];
