@@ -2207,6 +2207,8 @@ struct O1Split {
     uint32_t warm_steps;  // pairs of steps a warm-up decoder takes at most
     uint32_t hot0;        // the walk keeps the tables of contexts hot0 .. hot0 + 3 in LDS
     uint32_t cls;         // graph size class
+    uint32_t max_nodes;   // nodes a graph wave holds a round
+    uint32_t stage;       // nodes of a unit that the walk stages; the rest are read from memory
 };
 
 // Edges: target (16 bits: node, numbered through all rounds of its graph wave, or kSplitExit | exit),
@@ -2375,7 +2377,7 @@ __global__ void __launch_bounds__(256) k_o1s_warm(const O1Split* ch, int nch, ui
 // edges still to take are the tail of the node list, so there is no queue. Parts share a wave where
 // their edges are few (chains without escapes have a handful of start states). Steps run eight at a
 // time between looks at the table; a lane that has met its end waits for the rest.
-// NC: nodes a wave holds at most; past it, and where a table or the pool is full, the edges left stay
+// NC: nodes a wave holds at most (c.max_nodes is no more); past it, and where a table or the pool is full, the edges left stay
 // marked and the walk decodes such parts exactly.
 template <int NC>
 __global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, uint32_t nwaves, int round, O1SplitWs ws) {
@@ -2540,7 +2542,7 @@ __global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, ui
                               (idx | (esc ? 0xFu << kO1Log : 0u)), fresh);
         const uint64_t nmask = __ballot(fresh && esc);
         const uint32_t id = nn + (uint32_t)__popcll(nmask & below);
-        const bool full = nn + (uint32_t)__popcll(nmask) > (uint32_t)NC;
+        const bool full = nn + (uint32_t)__popcll(nmask) > c.max_nodes;
         if (fresh) {
             if (esc) {
                 if (id < (uint32_t)NC) {
@@ -2594,8 +2596,7 @@ __global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, ui
 constexpr int kWalkThreads = 512;
 constexpr uint32_t kWalkBuf = 65536;   // bytes of one buffer
 constexpr int64_t kWalkStage = 4096;   // bitstream bytes staged per window of an exact decode
-// Nodes of a unit that are staged, by size class; the rest are read from memory.
-__device__ __forceinline__ uint32_t walk_nodes(uint32_t cls) { return cls == 0 ? 64u : cls == 1 ? 512u : 1024u; }
+constexpr uint32_t kWalkNodes[3] = {64, 512, 1024};  // O1Split::stage by size class
 
 __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, int nch, O1SplitWs ws, unsigned int* stats) {
     __shared__ __align__(16) uint32_t mem[2 * kWalkBuf / 4];  // two buffers, or the hot tables
@@ -2608,7 +2609,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
     const uint32_t tid = threadIdx.x, l = tid & 63u, wv = tid >> 6;
     const bool lead = tid == 0;
     const uint32_t P = c.parts, pc = P * c.cap;  // candidates of a unit
-    const uint32_t NS = walk_nodes(c.cls);
+    const uint32_t NS = c.stage;
     // a unit's words: nodes (first, for their alignment), cand, edge, exits, start states of each part,
     // nodes staged
     const uint32_t o_cand = 2 * NS, o_edge = o_cand + pc, o_exit = o_edge + pc, o_n = o_exit + pc,
@@ -2676,6 +2677,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
     };
     uint32_t cur = c.x0 & ((1u << kO1Log) - 1);
     uint64_t e = 0, off = 0;
+    uint32_t far = 0;  // edges read from memory
     // signs of 64 escaped codes from index eb on (bit k: code eb + k is negative), the next 64 in flight
     uint64_t eb = 0, signs = 0;
     int vnext = 0;
@@ -2752,6 +2754,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
                         sum = ed >> 16;
                         tgt = ed & 0xFFFFu;
                         k++;
+                        far++;
                     }
                     po += sum;
                     pe += k - k0;
@@ -2831,6 +2834,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
         if (r < ngraph) stage_units(u0, lmem, 0, nwaves);
     }
     if (lead) {  // the last part
+        if (far) atomicAdd(&stats[2], far);
         ws.res_state[c.tfirst + r] = cur;
         ws.res_e[c.tfirst + r] = e;
         ws.res_off[c.tfirst + r] = off;
@@ -4594,6 +4598,9 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
     const bool all_seq = seq_env && atoi(seq_env) != 0;
     const char* par_env = getenv("FALCONS_O1_PARALLEL_SHORT");
     const bool keep_short = par_env && atoi(par_env) != 0;
+    // FALCONS_O1_GRAPH_NODES, FALCONS_O1_STAGE_NODES: test switches
+    auto few_nodes = [](const char* v) { return v ? (uint32_t)std::strtoul(v, nullptr, 10) : ~0u; };
+    const uint32_t graph_nodes = few_nodes(getenv("FALCONS_O1_GRAPH_NODES")), stage_nodes = few_nodes(getenv("FALCONS_O1_STAGE_NODES"));
     double pi[kO1Ctx];
     uint64_t pi_seg = ~0ull, ncodes = 0;
     std::vector<O1Chain> all;
@@ -4647,6 +4654,8 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             k.max_sym = 8 * sp.sub;
             k.hot0 = hot_window(pi);
             k.cls = (uint32_t)sp.cls;
+            k.max_nodes = std::min((uint32_t)kSplitNodes[sp.cls], graph_nodes);
+            k.stage = std::min(kWalkNodes[sp.cls], stage_nodes);
         }
         all.push_back(x);
     }
@@ -4770,11 +4779,11 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         memcpy(&nodes, &hsv[hsv.size() - 2], sizeof(nodes));
         const unsigned int* hs = hsv.data();
         fprintf(stderr, "[o1 decode] chains (chain:exact subsequences/subsequences/escapes/bits a symbol/segment/"
-                        "first LDS context of the walk):");
+                        "first LDS context of the walk/size class of its graphs):");
         for (int q = 0; q < nc; q++)
-            fprintf(stderr, " %d:%u/%u/esc%llu/b%.2f/s%llu/h%u", q, hs[6 + q], sc[q].nsub, (unsigned long long)sc[q].novf,
+            fprintf(stderr, " %d:%u/%u/esc%llu/b%.2f/s%llu/h%u/c%u", q, hs[6 + q], sc[q].nsub, (unsigned long long)sc[q].novf,
                     (double)sc[q].pos0 / (double)std::max<uint64_t>(1, sc[q].m), (unsigned long long)R.seg[q],
-                    sc[q].hot0);
+                    sc[q].hot0, sc[q].cls);
         fprintf(stderr, "\n");
         fprintf(stderr, "[o1 decode] %zu chains decoded from their start:", hd.size());
         for (size_t q = 0; q < hd.size(); q++)
@@ -4797,8 +4806,9 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             fprintf(stderr, "\n");
         }
         fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
-                        "entries outside the set), %llu nodes of %llu\n",
-                nc, (unsigned long long)R.W.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap);
+                        "entries outside the set), %llu nodes of %llu, %u edges from memory\n",
+                nc, (unsigned long long)R.W.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap,
+                hs[2]);
     }
 }
 
