@@ -356,9 +356,10 @@ __device__ void dtable_parallel(TL& L, unsigned tl, DEntry* dt) {
 // piece (k_fse_sets), and a walk from piece to piece picks the true ones, with the bits of every 128
 // steps noted on the way (k_fse_finish, which then writes the bits, 256 lanes a block). A piece that
 // more than 64 states reach (two symbols of equal counts: no two states ever meet) is run by the walk.
-// 138 blocks (9 million escapes of a 512^3 field at 1e-3): 2.6 ms -> 0.37; 765 blocks (50 million, at
-// 1e-4): 4.2 -> 1.9, the waves' LDS reads by then; one block of 35,000: 1.29 -> 0.23. Pieces of 512
-// steps run half as many steps twice: 2.4 ms for the 765 blocks, the others the same.
+// Escape classes of a 512^3 k^-3 field (one workgroup a block, two lanes at work -> these kernels): REL 1e-3, 14 blocks
+// (50,000 escapes), 2.06 -> 0.37 ms; 3.3e-4, 99 blocks (6 million), 2.75 -> 1.98, of which the walk 1.16: some
+// blocks hardly have a set; 1e-4, 1,036 blocks (67 million), 4.42 -> 2.04, the waves' LDS reads by then. One block of
+// 35,000: 1.29 -> 0.23. Pieces of 512 steps run half as many steps twice: 765 full blocks 2.4 ms against 1.9.
 constexpr unsigned kFblkLog = kFseDefaultTableLog;
 constexpr uint32_t kFseGroup = 16;      // symbols of a load
 constexpr uint32_t kFseHists = 8;
@@ -1452,9 +1453,9 @@ __device__ inline uint32_t o1_seed_state(const int16_t* bins, uint64_t lo, uint6
 // (16 KB each) of the H contexts that occur most often. With the state tables in L2 the lanes of a
 // full chip wait for its rate of requests (a lane reads one entry a step from anywhere in 240 KB: 160 G
 // steps/s); with 8 of them in LDS a step waits for L2 only in the waves that hold a rare context, and
-// its instructions count as much. 134 million codes, one in 15 an escape: k_o1_spec 0.84 -> 0.37 ms,
-// k_o1_fix 0.85 -> 0.50, k_o1_emit (6 tables, the rings beside them) 0.95 -> 0.45; two codes in five an
-// escape: 1.40 -> 0.43, 2.2 -> 2.5 (beside the escapes' blocks, which come at once now), 0.93 -> 0.41.
+// its instructions count as much. 134 million codes of a k^-3 field, REL 1e-3 (one in 2,700 an escape): k_o1_spec
+// 0.84 -> 0.36 ms, k_o1_fix 0.92 -> 0.49, k_o1_emit (6 tables, the rings beside them) 0.97 -> 0.45; 1e-4 (one in two):
+// 1.09 -> 0.39, 2.84 -> 2.38 (beside the escapes' blocks, which come at once now), 1.41 -> 0.41.
 template <int H>
 struct O1EncLds {
     // a symbol's deltaNbBits, and its deltaFindState + 8,192 * place of the context's state table: below H
@@ -2198,7 +2199,6 @@ struct O1Split {
     uint64_t cfirst;      // first slot of its candidate arrays (cap a part)
     uint64_t wfirst;      // first warm-up lane (a multiple of 64)
     uint64_t gfirst;      // first graph wave, over all chains
-    uint64_t lo;          // first code in the call's code array (alignment of the output)
     uint32_t x0, nsub, sub_bits, warm_bits;
     uint32_t lgk;         // 1 << lgk warm-up decoders a part
     uint32_t cap;         // candidates a part holds at most
@@ -3623,7 +3623,8 @@ static size_t encode_method0(const int16_t* bins, uint64_t n, uint8_t* out, uint
 // the bits of a tile, the tiles' sums are scanned, and every thread packs its 16 mantissas into
 // whole words. Nothing waits for the host before the coded sizes are read. Segment by segment, with a
 // scan of 8-byte bit counts and an atomic for every byte that a mantissa touches, the 15 segments of a
-// 512^3 field at 1e-4 (50 million escapes) took 5.4 ms beside their FSE blocks, all at once take 0.53.
+// 512^3 field at 1e-4 (67 million escapes) took 3.9 ms of kernels beside their FSE blocks and a host round trip each,
+// all at once take 0.57.
 __device__ __forceinline__ uint32_t ovf_zigzag1(int32_t f) { return (((uint32_t)f << 1) ^ (uint32_t)(f >> 31)) + 1u; }
 __device__ __forceinline__ uint32_t ovf_class(int32_t f) { return 31u - (uint32_t)__clz((int)ovf_zigzag1(f)); }
 

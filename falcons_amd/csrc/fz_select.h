@@ -5,10 +5,9 @@
 // A thread holds 16 consecutive codes (two 16-byte loads), a workgroup a tile of 4,096: the passes are
 // bound by the read of the codes (2 bytes each) for long arrays, and by the number of workgroups in
 // flight for short ones. Tiles of 65,536 codes read two bytes a thread at a time left a chunk of
-// 540,000 codes on 9 of 256 CUs. Count, scan and hand-out, on those tiles and here: 0.16 -> 0.02 ms
-// (86,000 codes, escapes of order-1 coding), 0.32 -> 0.08 ms (134 million, one code in 15 an escape),
-// 0.53 -> 0.30 ms (134 million, two in five); a batch of 192 chunks of 540,000 codes decodes in 64 ms
-// where it took 76.
+// 540,000 codes on 9 of 256 CUs. Count, scan, hand-out and what gathered the values, on those tiles and here, escapes
+// of order-1 coding: 0.16 -> 0.02 ms (86,000 codes), 0.32 -> 0.08 ms (134 million, one code in 2,700 an escape),
+// 0.74 -> 0.29 ms (134 million, one in two); a batch of 192 chunks of 540,000 codes decodes in 64 ms where it took 76.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
