@@ -2677,7 +2677,6 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
     };
     uint32_t cur = c.x0 & ((1u << kO1Log) - 1);
     uint64_t e = 0, off = 0;
-    uint32_t far = 0;  // edges read from memory
     // signs of 64 escaped codes from index eb on (bit k: code eb + k is negative), the next 64 in flight
     uint64_t eb = 0, signs = 0;
     int vnext = 0;
@@ -2754,7 +2753,6 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
                         sum = ed >> 16;
                         tgt = ed & 0xFFFFu;
                         k++;
-                        far++;
                     }
                     po += sum;
                     pe += k - k0;
@@ -2834,7 +2832,6 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
         if (r < ngraph) stage_units(u0, lmem, 0, nwaves);
     }
     if (lead) {  // the last part
-        if (far) atomicAdd(&stats[2], far);
         ws.res_state[c.tfirst + r] = cur;
         ws.res_e[c.tfirst + r] = e;
         ws.res_off[c.tfirst + r] = off;
@@ -4471,6 +4468,8 @@ static void split_layout(const std::vector<O1Chain>& chains, SplitRun& R, uint8_
     take(R.stats, nstats);
     W.pool_used = reinterpret_cast<NodeCount*>(R.stats + nstats - 2);
 }
+// What split_layout takes beside its chains' split_bytes, at most: roundings, lists, a few nodes.
+static size_t split_head(size_t nc) { return 65536 + (sizeof(O1Split) + 8) * nc; }
 static void split_launch(const SplitRun& R, hipStream_t st) {
     const int nc = (int)R.sc.size(), nstats = split_stats(nc);
     const O1SplitWs& W = R.W;
@@ -4551,12 +4550,11 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStrea
     if (n > 0x7fffffffu) throw std::length_error("too many sequential chains for one launch");
     if (b->tabs.size() > 65535u) throw std::length_error("too many sequential segments for one launch");
     // all device memory before the first launch: without it nothing of the batch is under way
+    const size_t need = (size_t)b->split_bytes + split_head(b->split.size());
     uint8_t* mem = nullptr;
     if (!b->split.empty()) {
-        split_layout(b->split, b->run, nullptr);
-        mem = static_cast<uint8_t*>(ws.side(b->run.bytes, 0, (size_t)kBatchSplitBytes));
+        mem = static_cast<uint8_t*>(ws.side(need, 0, (size_t)kBatchSplitBytes));
         if (!mem) throw GpuError("no device memory for the split chains of the batch");
-        split_layout(b->split, b->run, mem);
     }
     SerialJob* dj = n ? ws.take<SerialJob>(n) : nullptr;
     SerialTables* dtab = n ? ws.take<SerialTables>(b->tabs.size()) : nullptr;
@@ -4576,7 +4574,11 @@ void dense_batch_run(DenseBatch* b, DevArena& ws, hipStream_t st, const AuxStrea
     }
     AuxJoin join{aux, st, beside};
     if (n) launch_serial(b->jobs, b->tabs, dj, dtab, b->bytes, b->codes, beside ? aux.stream : st);
-    if (mem) split_launch(b->run, st);
+    if (mem) {
+        split_layout(b->split, b->run, mem);
+        if (b->run.bytes > need) throw std::logic_error("split chains of the batch: more memory than planned");
+        split_launch(b->run, st);
+    }
 }
 
 // The lists of one call's chains. Copies on the call's stream read them: they stay until it has been waited for.
@@ -4674,8 +4676,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         // what the call takes after this: the re-encoded tables of sequential chains, the scratch of a scan
         const size_t after = nf_off.size() * (sizeof(uint32_t) * kO1Ctx << kO1Log) + (1u << 20) + ncodes / 64;
-        const double head = 65536.0 + 256.0 * (double)cand.size();  // rounding, lists
-        const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - head;
+        const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - (double)split_head(cand.size());
         for (const SplitCand& x : cand) need += x.bytes();
         if (!defer) split_choose(cand, room, serial);
         std::vector<O1Chain> own;
@@ -4807,9 +4808,8 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             fprintf(stderr, "\n");
         }
         fprintf(stderr, "[o1 decode] %d split chains, %llu parts, walk decoded %u exactly (%u without a whole path, %u "
-                        "entries outside the set), %llu nodes of %llu, %u edges from memory\n",
-                nc, (unsigned long long)R.W.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap,
-                hs[2]);
+                        "entries outside the set), %llu nodes of %llu\n",
+                nc, (unsigned long long)R.W.nparts, hs[0] + hs[1], hs[0], hs[1], nodes, (unsigned long long)R.W.pool_cap);
     }
 }
 

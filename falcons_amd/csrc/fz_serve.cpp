@@ -247,9 +247,7 @@ void decompress_grouped(fz_ctx* ctx, WorkerSet& wset, fz_batch_dec_item* items, 
             FZ_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             R.ev.push_back(e);
         }
-        size_t left_b = 0;
-        FZ_HIP(hipMemGetInfo(&left_b, &total_b));
-        dense_batch_limit(R.batch, left_b + ctx->arena.side_capacity());
+        dense_batch_limit(R.batch, free_b - std::min(free_b, pool_bytes) + ctx->arena.side_capacity());
         std::vector<std::unique_ptr<DevArena>> ar(g);
         std::vector<std::unique_ptr<DecCall, void (*)(DecCall*)>> calls;
         std::vector<char> ok(g, 0), rec(g, 0);

@@ -1,6 +1,6 @@
 """The split order-1 decoder where a graph is not whole: each size class of its graphs with full tables of nodes (such
-parts are decoded one after another by the walk) and with nodes that the walk reads from memory, against the oracle
-bit for bit. The decoder's statistics say that the class and the path were the ones meant."""
+parts are decoded one after another by the walk) and with all or most nodes left to the walk to read from memory,
+against the oracle bit for bit. The decoder's statistics say that the class and the path were the ones meant."""
 import re
 
 import numpy as np
@@ -57,13 +57,12 @@ def test_split_paths(ctx, streams, monkeypatch, capfd, name, cls, switch, nodes)
     assert np.array_equal(got.reshape(-1).view(np.uint8), want.reshape(-1).view(np.uint8))
     chains = [int(c) for c in re.findall(r" \d+:\d+/\d+/esc\d+/b[\d.]+/s\d+/h\d+/c(\d+)", err)]
     assert chains == [cls] * 4, err[-2000:]
-    parts, exact, lost, used, far = (int(x) for x in re.search(
-        r"split chains, (\d+) parts, walk decoded (\d+) exactly \((\d+) without a whole path, .*, (\d+) nodes of \d+, "
-        r"(\d+) edges from memory", err).groups())
+    parts, exact, lost, used = (int(x) for x in re.search(
+        r"split chains, (\d+) parts, walk decoded (\d+) exactly \((\d+) without a whole path, .*, (\d+) nodes of \d+",
+        err).groups())
     if switch == "FALCONS_O1_GRAPH_NODES":
         waves = parts * 3  # at most: a part a wave, three rounds
         assert used <= nodes * waves and lost > 0
         assert exact > (parts // 2 if nodes == 0 else 20)
     else:
-        assert used > 1000 and exact < parts // 20
-        assert far > (50 if switch else -1)
+        assert used > 1000 and exact < parts // 20  # the escapes' edges are in the graphs
