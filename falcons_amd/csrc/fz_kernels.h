@@ -22,7 +22,8 @@ namespace fz {
 // A bound arena (bind()) draws from one region of device memory the caller owns and never
 // allocates: a take() beyond the region throws instead of adding a block.
 //
-// side() gives memory that a call can do without: one region beside the blocks, for one user a call.
+// side() gives memory that a call can do without, to one user a call: the end of the last block where the
+// call leaves it free, else a region beside the blocks.
 class DevArena {
    public:
     ~DevArena() { release(); }
@@ -42,12 +43,12 @@ class DevArena {
     void reset() {
         cur_ = 0;
         off_ = 0;
-        used_ = side_used_ = 0;
+        used_ = side_used_ = tail_ = 0;
     }
     template <typename T>
     T* take(size_t count) {
         const size_t bytes = ((count * sizeof(T)) + 255) & ~size_t(255);
-        while (cur_ < blocks_.size() && off_ + bytes > blocks_[cur_].cap) {  // the rest of this block is skipped
+        while (cur_ < blocks_.size() && off_ + bytes > open(cur_)) {  // the rest of this block is skipped
             used_ += blocks_[cur_].cap - off_;
             cur_++;
             off_ = 0;
@@ -68,7 +69,7 @@ class DevArena {
         return most;
     }
     void set_side_most(size_t bytes) { side_most_ = bytes; }
-    // Null where there is no room (side_room) or the device has no such memory. The region is kept for the
+    // Null where there is no room (side_room) or the device has no such memory. A region is kept for the
     // next call and regrown for a larger one: to twice the need, 256 MB at least, and `most` at most, as the
     // hipFree that goes with it waits for the whole device.
     void* side(size_t bytes, size_t after, size_t most) {
@@ -76,6 +77,15 @@ class DevArena {
         const size_t room = side_room(after);
         if (bytes > room) return nullptr;
         if (bound_) return take<uint8_t>(bytes);
+        const size_t last = blocks_.size() - 1;
+        if (!tail_ && cur_ < blocks_.size() &&
+            bytes + (cur_ == last ? off_ + after : 0) <= blocks_[last].cap) {
+            tail_ = bytes;
+            tail_block_ = last;
+            side_used_ = bytes;
+            peak_ = std::max(peak_, used_ + side_used_);
+            return static_cast<char*>(blocks_[last].p) + (blocks_[last].cap - bytes);
+        }
         if (bytes > side_.cap) {
             drop_side();
             const size_t cap = std::max(bytes, std::min(std::min(room, most), std::max(2 * bytes, size_t(256) << 20)));
@@ -121,11 +131,13 @@ class DevArena {
         void* p = nullptr;
         size_t cap = 0;
     };
+    // What takes may use of block k.
+    size_t open(size_t k) const { return blocks_[k].cap - (tail_ && k == tail_block_ ? tail_ : 0); }
     void drop_blocks() {
         if (!bound_)
             for (Block& b : blocks_) (void)hipFree(b.p);
         blocks_.clear();
-        cap_ = used_ = off_ = 0;
+        cap_ = used_ = off_ = tail_ = 0;
         cur_ = 0;
         bound_ = false;
     }
@@ -146,7 +158,7 @@ class DevArena {
     }
     std::vector<Block> blocks_;
     Block side_;
-    size_t cap_ = 0, used_ = 0, off_ = 0, peak_ = 0, cur_ = 0, side_used_ = 0;
+    size_t cap_ = 0, used_ = 0, off_ = 0, peak_ = 0, cur_ = 0, side_used_ = 0, tail_ = 0, tail_block_ = 0;
     size_t side_most_ = ~size_t(0) / 2;
     bool bound_ = false;
 };
