@@ -2208,7 +2208,7 @@ struct O1Split {
     uint32_t hot0;        // the walk keeps the tables of contexts hot0 .. hot0 + 3 in LDS
     uint32_t cls;         // graph size class
     uint32_t max_nodes;   // nodes a graph wave holds a round
-    uint32_t stage;       // nodes of a unit that the walk stages; the rest are read from memory
+    uint32_t stage;       // nodes of a unit that the walk stages (walk_nodes at most)
 };
 
 // Edges: target (16 bits: node, numbered through all rounds of its graph wave, or kSplitExit | exit),
@@ -2596,7 +2596,8 @@ __global__ void __launch_bounds__(64) k_o1s_graph(const O1Split* ch, int nch, ui
 constexpr int kWalkThreads = 512;
 constexpr uint32_t kWalkBuf = 65536;   // bytes of one buffer
 constexpr int64_t kWalkStage = 4096;   // bitstream bytes staged per window of an exact decode
-constexpr uint32_t kWalkNodes[3] = {64, 512, 1024};  // O1Split::stage by size class
+// Nodes of a unit that are staged at most, by size class; the rest are read from memory.
+__host__ __device__ constexpr uint32_t walk_nodes(uint32_t cls) { return cls == 0 ? 64u : cls == 1 ? 512u : 1024u; }
 
 __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, int nch, O1SplitWs ws, unsigned int* stats) {
     __shared__ __align__(16) uint32_t mem[2 * kWalkBuf / 4];  // two buffers, or the hot tables
@@ -2609,7 +2610,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
     const uint32_t tid = threadIdx.x, l = tid & 63u, wv = tid >> 6;
     const bool lead = tid == 0;
     const uint32_t P = c.parts, pc = P * c.cap;  // candidates of a unit
-    const uint32_t NS = c.stage;
+    const uint32_t NS = walk_nodes(c.cls);  // (a number from c, read in its place, makes the hops 2.5% slower)
     // a unit's words: nodes (first, for their alignment), cand, edge, exits, start states of each part,
     // nodes staged
     const uint32_t o_cand = 2 * NS, o_edge = o_cand + pc, o_exit = o_edge + pc, o_n = o_exit + pc,
@@ -2647,7 +2648,7 @@ __global__ void __launch_bounds__(kWalkThreads) k_o1s_walk(const O1Split* ch, in
             bool room = true;
 #pragma unroll
             for (int z = 0; z < kSplitRounds; z++) {
-                const uint32_t n = room && rd[z].x != kPoolNone ? min(rd[z].y, NS - ns) : 0u;
+                const uint32_t n = room && rd[z].x != kPoolNone ? min(rd[z].y, c.stage - ns) : 0u;
                 for (uint32_t i0 = 0; i0 < n; i0 += 512) {
                     u32x2 v[8];
 #pragma unroll
@@ -4413,8 +4414,7 @@ struct SplitRun {
 // 32-bit words of its statistics for nc chains: six counts, one a chain, then the pool's count.
 static int split_stats(int nc) { return (6 + nc + 1) / 2 * 2 + 2; }
 
-// Lays the chains out, those of one size class side by side for one launch each; at: the memory (null: only
-// its size is wanted, R.bytes).
+// Lays the chains out in the memory at `at`, those of one size class side by side for one launch each.
 static void split_layout(const std::vector<O1Chain>& chains, SplitRun& R, uint8_t* at) {
     R = SplitRun{};
     std::vector<const O1Chain*> order;
@@ -4658,7 +4658,7 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
             k.hot0 = hot_window(pi);
             k.cls = (uint32_t)sp.cls;
             k.max_nodes = std::min((uint32_t)kSplitNodes[sp.cls], graph_nodes);
-            k.stage = std::min(kWalkNodes[sp.cls], stage_nodes);
+            k.stage = std::min(walk_nodes((uint32_t)sp.cls), stage_nodes);
         }
         all.push_back(x);
     }
@@ -4678,18 +4678,21 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         const size_t after = nf_off.size() * (sizeof(uint32_t) * kO1Ctx << kO1Log) + (1u << 20) + ncodes / 64;
         const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - (double)split_head(cand.size());
         for (const SplitCand& x : cand) need += x.bytes();
+        const bool to_batch = defer && need > room;
         if (!defer) split_choose(cand, room, serial);
         std::vector<O1Chain> own;
+        need = (double)split_head(cand.size());
         for (O1Chain& x : all) {
-            if (defer && need > room) x.batched = true;
-            if (x.plan.cls != kSplitNone && !x.batched) own.push_back(x);
+            if (to_batch) x.batched = true;
+            if (x.plan.cls == kSplitNone || x.batched) continue;
+            need += split_bytes(x.plan, x.k.m, x.k.nsub);
+            own.push_back(x);
         }
         if (!own.empty()) {
-            split_layout(own, R, nullptr);
-            if (uint8_t* mem = static_cast<uint8_t*>(ws.side(R.bytes, after, split_limit(ncodes)))) {
+            if (uint8_t* mem = static_cast<uint8_t*>(ws.side((size_t)need, after, split_limit(ncodes)))) {
                 split_layout(own, R, mem);
+                if ((double)R.bytes > need) throw std::logic_error("split chains: more memory than planned");
             } else {
-                R = SplitRun{};
                 for (O1Chain& x : all)
                     if (!x.batched) x.plan.cls = kSplitNone;
             }
