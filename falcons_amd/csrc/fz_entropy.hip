@@ -2051,9 +2051,10 @@ __global__ void __launch_bounds__(256) k_o1_dtables(const uint8_t* stream, const
 }
 
 
-// Exact decoding of a stretch of one chain from a bitstream window staged in LDS, for the walk. win[k + kWinPad] holds chain byte wlo + k; the kWinPad bytes below are
-// zero when the window starts at the chain's first byte. The decoding tables of contexts
-// hot0 .. hot0 + kWalkCtxN - 1 sit in LDS (hot), the others are read from device memory.
+// Exact decoding of a stretch of one chain from a bitstream window staged in LDS, for the walk.
+// win[k + kWinPad] holds chain byte wlo + k; the kWinPad bytes below are zero when the window starts at
+// the chain's first byte. The decoding tables of contexts hot0 .. hot0 + kWalkCtxN - 1 sit in LDS (hot),
+// the others are read from device memory.
 constexpr int kWalkCtx0 = 11, kWalkCtxN = 4;  // contexts 11..14: after large codes, where escapes are dense
 constexpr int kWinPad = 16;
 constexpr int kSeqLanes = 64;       // the sequential decoders run as one wave
@@ -4588,8 +4589,8 @@ struct O1Lists {
     std::vector<SerialTables> tabs;  // one a segment
 };
 
-// defer: the sequential chains are handed to it instead of launched (their decode then runs in
-// dense_batch_run, after the work this call has queued on st).
+// defer: the sequential chains are handed to it instead of launched, and the split ones that are short or
+// find no room (their decode then runs in dense_batch_run, after the work this call has queued on st).
 static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const std::vector<uint64_t>& chains,
                                const std::vector<uint64_t>& nf_off, const DEntry* dt, const int16_t* ovf, int16_t* out,
                                int* err, DevArena& ws, hipStream_t st, const AuxStream& aux, DenseBatch* defer,
@@ -4676,7 +4677,8 @@ static void o1_decode_parallel(const uint8_t* host, const uint8_t* dev, const st
         }
         // what the call takes after this: the re-encoded tables of sequential chains, the scratch of a scan
         const size_t after = nf_off.size() * (sizeof(uint32_t) * kO1Ctx << kO1Log) + (1u << 20) + ncodes / 64;
-        const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - (double)split_head(cand.size());
+        const double room = (double)std::min<uint64_t>(split_limit(ncodes), ws.side_room(after)) - 256.0 -
+                            (double)split_head(cand.size());
         for (const SplitCand& x : cand) need += x.bytes();
         const bool to_batch = defer && need > room;
         if (!defer) split_choose(cand, room, serial);
