@@ -358,7 +358,7 @@ __device__ void dtable_parallel(TL& L, unsigned tl, DEntry* dt) {
 // more than 64 states reach (two symbols of equal counts: no two states ever meet) is run by the walk.
 // Escape classes of a 512^3 k^-3 field (one workgroup a block, two lanes at work -> these kernels): REL 1e-3, 14 blocks
 // (50,000 escapes), 2.06 -> 0.37 ms; 3.3e-4, 99 blocks (6 million), 2.75 -> 1.98, of which the walk 1.16: some
-// blocks hardly have a set; 1e-4, 1,036 blocks (67 million), 4.42 -> 2.04, the waves' LDS reads by then. One block of
+// blocks hardly have a set; 1e-4, 1,036 blocks (67 million), 4.42 -> 2.1, the waves' LDS reads by then. One block of
 // 35,000: 1.29 -> 0.23. Pieces of 512 steps run half as many steps twice: 765 full blocks 2.4 ms against 1.9.
 constexpr unsigned kFblkLog = kFseDefaultTableLog;
 constexpr uint32_t kFseGroup = 16;      // symbols of a load

@@ -144,7 +144,7 @@ inline double split_bytes(const SplitPlan& s, uint64_t m, uint64_t nsub) {
 // workspace count them beside what every call takes. 64 a code hold nearly every plan of a field of one segment
 // (16.8 million codes), where splitting saves most (a quarter of the field is one chain: 256^3 at REL 5e-4
 // 64 ms, 289 from the start). Fields of many segments have short chains and few segments with many
-// escapes: 512^3 takes 5 bytes a code at REL 8e-4 (44 ms, 204 from the start).
+// escapes: 512^3 takes 3 bytes a code at REL 8e-4 (44 ms, 204 from the start).
 inline uint64_t split_limit(uint64_t n) { return std::min<uint64_t>(64 * n, (1ull << 30) + 4 * n); }
 
 // Nodes of all split chains, for one symbol of the longest chain that is decoded from its start, above which splitting
